@@ -82,6 +82,15 @@ class BondEngine(object):
         # LDS state the edge array sits in L2 and computing measured 1.4 %
         # slower (L = 128)
         self.lattice_sweep = bool(L) and self.N > 16384
+        # a lattice relabelled where the tiles are not whole (L not a
+        # multiple of 8): pc_sweep_lattice takes it with its sides row by
+        # row, for its tiled sweep; the relabelled edge array serves the
+        # modes in which every node's code is in HBM
+        self.row_length, self.d_row_sides = 0, None
+        if not L and order is not None and self.N > 16384:
+            self.row_length = int(getattr(graph, 'lattice_length', 0) or 0)
+            if self.row_length and graph.node_sides is not None:
+                self.d_row_sides = torch.from_numpy(graph.node_sides.copy()).to(dev)
         self.rec_bytes = self.lib.pc_record_bytes(self.N)
         self.rec_torch = torch.int32 if self.rec_bytes == 4 else torch.int64
         self.rec_numpy = nat.record_dtype(self.N)
@@ -155,9 +164,15 @@ class BondEngine(object):
     def workspace_bytes(self, num_runs, state_mode=None):
         b = ctypes.c_uint64(0)
         mode = self.state_mode if state_mode is None else state_mode
-        nat.check(self.lib.pc_sweep_workspace_size(self.N, num_runs, mode,
-                                                   ctypes.byref(b)),
-                  'pc_sweep_workspace_size')
+        length = (self.lattice_length if self.lattice_sweep else 0) or self.row_length
+        if length:
+            nat.check(self.lib.pc_sweep_lattice_workspace_size(
+                length, num_runs, mode, ctypes.byref(b)),
+                'pc_sweep_lattice_workspace_size')
+        else:
+            nat.check(self.lib.pc_sweep_workspace_size(self.N, num_runs, mode,
+                                                       ctypes.byref(b)),
+                      'pc_sweep_workspace_size')
         return int(b.value)
 
     def occupancy(self, state_mode=None):
@@ -205,10 +220,13 @@ class BondEngine(object):
             chunk_state = torch.empty((R, C, nat.PC_STATE_WORDS),
                                       dtype=torch.int64, device=self.device)
         st = nat.stream_handle(torch)
-        if self.lattice_sweep:
+        rows = (self.row_length and self.state_mode == nat.PC_STATE_AUTO and
+                wb >= self.workspace_bytes(R))
+        if self.lattice_sweep or rows:
             nat.check(self.lib.pc_sweep_lattice(
-                self.lattice_length, 1 if self.lattice_tiled else 0,
-                nat.ptr(self.d_sides), self.span_first, nat.ptr(d_perm),
+                self.row_length if rows else self.lattice_length,
+                1 if self.lattice_tiled and not rows else 0,
+                nat.ptr(self.d_row_sides if rows else self.d_sides), self.span_first, nat.ptr(d_perm),
                 max(self.M, 1), R, nat.ptr(records), max(self.M, 1),
                 nat.ptr(span_step), nat.ptr(workspace), wb, self.merge_rounds,
                 self.state_mode, nat.ptr(chunk_state) if chunks else None, st),

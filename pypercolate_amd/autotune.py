@@ -91,7 +91,7 @@ def tune_sweep(engine, sample_runs=None, rounds=ROUND_CANDIDATES, modes=None,
     cache keeps one choice per graph and cap."""
     torch = engine.torch
     device = torch.cuda.get_device_properties(engine.device)
-    key = '{}|{}|{}'.format(device.gcnArchName, device.multi_processor_count,
+    key = 'tiled|{}|{}|{}'.format(device.gcnArchName, device.multi_processor_count,
                             graph_key(engine.graph))
     if max_runs:
         key += '|runs<={}'.format(int(max_runs))
@@ -107,6 +107,9 @@ def tune_sweep(engine, sample_runs=None, rounds=ROUND_CANDIDATES, modes=None,
             places = [nat.PC_STATE_LDS, nat.PC_STATE_HBM]
         modes = [p | w for p in places
                  for w in (nat.PC_SWEEP_ONE_WAVE, nat.PC_SWEEP_TWO_WAVES)]
+        if engine.N > 16384:
+            # square lattices: the library's tiled sweep (no placement asked)
+            modes.insert(0, nat.PC_STATE_AUTO)
     cus = device.multi_processor_count
     timings = {}
     best = None

@@ -1308,6 +1308,7 @@ static size_t rs_apply_lds_bytes(uint32_t n)
 // The largest code, 4P - 1, fits 16 bits; decoding is a shift and a mask
 // (the resolver's rounds are bound by the instructions they issue).
 struct LdsState {
+    static constexpr bool LDS = true;
     uint16_t *code;
     uint32_t P, shift;
     __device__ __forceinline__ uint32_t get(uint32_t i) const { return code[i]; }
@@ -1326,6 +1327,7 @@ struct LdsState {
 // 32-bit codes in HBM for larger N: bit 31 marks a root, bits 29-30 the
 // side, bits 0-28 the size.
 struct GlobalState {
+    static constexpr bool LDS = false;
     uint32_t *code;
     __device__ __forceinline__ uint32_t get(uint32_t i) const { return code[i]; }
     __device__ __forceinline__ void set(uint32_t i, uint32_t v) const { code[i] = v; }
@@ -1410,7 +1412,7 @@ __device__ __forceinline__ void find2(const St &st, uint32_t &x, uint32_t &cx,
     cx = st.get(x);
     cy = st.get(y);
     bool rx = st.is_root(cx), ry = st.is_root(cy);
-    if constexpr (std::is_same<St, LdsState>::value) {
+    if constexpr (St::LDS) {
         while (!(rx && ry)) {
             const uint32_t gx = st.get(rx ? x : cx);
             const uint32_t gy = st.get(ry ? y : cy);
@@ -1581,27 +1583,26 @@ struct LatticeEdges {
         return tiled ? ((((r >> 2) * (L >> 3) + (c >> 3)) << 5) | ((r & 3u) << 3) | (c & 7u))
                      : r * L + c;
     }
-    __device__ __forceinline__ int2 operator()(int32_t e) const
+    // bond x: its first node (r, c), and whether it goes down or to the right
+    __device__ __forceinline__ void bond(uint32_t x, uint32_t &r, uint32_t &c,
+                                         uint32_t &down) const
     {
-        const uint32_t x = (uint32_t)e;
-        uint32_t r = (uint32_t)((float)x * inv_d);
+        r = (uint32_t)((float)x * inv_d);
         // the float guess is off by at most one row either way
         if (r * d > x)
             --r;
         else if ((r + 1u) * d <= x)
             ++r;
         const uint32_t q = x - r * d;
-        uint32_t r2 = r, c = q, c2 = q + 1u;   // the last row: to the right
-        if (r + 1u < L) {
-            c = q >> 1;
-            if (q & 1u)
-                c2 = c + 1u;   // to the right
-            else {
-                r2 = r + 1u;   // down
-                c2 = c;
-            }
-        }
-        return make_int2((int32_t)node(r, c), (int32_t)node(r2, c2));
+        const bool last = r + 1u >= L;   // the last row: to the right only
+        c = last ? q : q >> 1;
+        down = last ? 0u : (~q & 1u);
+    }
+    __device__ __forceinline__ int2 operator()(int32_t e) const
+    {
+        uint32_t r, c, down;
+        bond((uint32_t)e, r, c, down);
+        return make_int2((int32_t)node(r, c), (int32_t)node(r + down, c + 1u - down));
     }
 };
 
@@ -2004,8 +2005,10 @@ __global__ __launch_bounds__(SPLIT ? (FOLDER ? 192 : 128) : 64) void sweep_globa
     const int32_t *__restrict__ perm, int64_t perm_stride,
     RecT *__restrict__ records, int64_t rec_stride,
     uint32_t *__restrict__ span_step, uint32_t *__restrict__ workspace,
-    uint32_t rounds, uint64_t *__restrict__ chunk_state)
+    uint32_t rounds, uint64_t *__restrict__ chunk_state,
+    const uint32_t *__restrict__ only)
 {
+    // only: sweep the runs marked there (NULL: every run)
     // the handoff: root slots, the roots' codes, then (FOLDER) the records
     __shared__ uint32_t claims[CLAIM_SLOTS];
     __shared__ uint32_t handoff[SPLIT ? SWEEP_HANDOFF_WORDS + (FOLDER ? 256u : 0u) : 1u];
@@ -2013,6 +2016,8 @@ __global__ __launch_bounds__(SPLIT ? (FOLDER ? 192 : 128) : 64) void sweep_globa
     const size_t cstride = (size_t)((M + 63u) / 64u) * PC_STATE_WORDS;
     const GlobalState st{workspace + (size_t)blockIdx.x * N};
     for (uint32_t r = blockIdx.x; r < R; r += gridDim.x) {
+        if (only && !only[r])
+            continue;
         sweep_run<GlobalState, RecT, CHUNKS, SPLIT, ES, FOLDER>(
             st, N, M, edges, sides, span_first != 0, rounds, claims, handoff,
             dirty, perm + (int64_t)r * perm_stride, records + (int64_t)r * rec_stride,
@@ -2102,6 +2107,651 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
             run(EdgeList{G.edges});
         __syncthreads();
     }
+}
+
+// ---------------------------------------------------------------------------
+// Tiled sweep of the square lattice (pc_sweep_lattice for lattices whose
+// union-find state does not fit LDS).  The lattice is cut into tiles of at
+// most TILE_SIDE x TILE_SIDE nodes.  A node with a bond into another tile is
+// open, and so is every cluster of a tile's own bonds that holds an open
+// node; the other clusters of a tile are closed: nothing outside the tile
+// can have joined them, so their sizes and sides are exact at every step.
+//   1. tile_scatter: each run's bonds, in step order, into one list per
+//      tile (its internal bonds); a bond between two tiles becomes an event;
+//   2. tile_sweep: one wavefront per (run, tile) merges the tile's internal
+//      bonds in step order with its state in LDS.  A merge of two closed
+//      clusters is final and its record is written.  A merge with an open
+//      cluster becomes an event: the open cluster, named by one of its open
+//      nodes, gains a closed cluster of known size, or joins another open
+//      one.  A closed cluster goes under the open root, whose code does not
+//      change, so such merges do not conflict over it: near and above the
+//      threshold, where most merges hit one large cluster, a batch resolves
+//      in one round;
+//   3. event_sweep: one wavefront per run merges the run's events in step
+//      order over the open nodes alone (0.05 N of them) and replaces every
+//      event by its record.
+// About 0.11 M of a random run's steps are events (64 x 64 tiles); the
+// others never leave LDS.  A tile-level merge of two open clusters that
+// outside bonds have already joined is found out in step 3 (record 0).
+// Untiled, with every node's code in HBM, the sweep moves 342 bytes per
+// addition in random lines at L = 1024.  Sweep with its chunk states, untiled
+// and tiled: L = 1024, 1000 runs 158 and 96 ms (lists 20, tiles 39, events 25,
+// chunk states 12); L = 256, 200 runs 3.67 and 1.53 ms; L = 181, 600 runs
+// 2.65 and 1.46 ms.  Bound by the wavefronts' dependent LDS round trips.
+//
+// Event record (half = half of a record's bits): the high half's top bit is
+// set (a final record's sizes are below 2^(half - 1) on both sides in step
+// 2, and step 3 reads a step before it writes it); low half: an open node's
+// id; its top bit clear for a gain (high half: size, sides << 12, and bit 14
+// set when the closed cluster is on the bond's u side), set for a join (high
+// half: the other open node's id).
+// ---------------------------------------------------------------------------
+#define TILE_SIDE 64u
+#define TILE_MAX_LENGTH 2048u
+#define TILE_CLAIM_BITS 10
+#define TILE_CLAIM_SLOTS (1u << TILE_CLAIM_BITS)
+#define TILE_SCATTER_BLOCKS 1024u // workgroups tile_scatter wants
+#define TILE_GROUPS 8u   // groups of 64 steps a wave of tile_scatter takes at once
+#define TILE_SHORT_STEPS (1u << 19) // up to so many edges a list entry has 32 bits
+
+// Tiles of h x w nodes (the last row and column of tiles may be smaller),
+// KH x KW of them.  mh, mw divide a coordinate by h and w (high half of the
+// product, exact below 2^16).  Ids of a tile's border nodes: per of them.
+struct TileGeo {
+    LatticeEdges lat;
+    uint32_t L, h, w, KH, KW, K, per, mh, mw, init_stride;
+    __host__ __device__ __forceinline__ uint32_t rows(uint32_t tr) const { return tr + 1u < KH ? h : L - (KH - 1u) * h; }
+    __host__ __device__ __forceinline__ uint32_t cols(uint32_t tc) const { return tc + 1u < KW ? w : L - (KW - 1u) * w; }
+    // internal bonds of a tile of hh x ww nodes, and the first list entry of
+    // tile (tr, tc) when the tiles' lists follow one another
+    __host__ __device__ static __forceinline__ uint32_t bonds(uint32_t hh, uint32_t ww) { return hh * (ww - 1u) + (hh - 1u) * ww; }
+    __host__ __device__ __forceinline__ uint32_t offset(uint32_t tr, uint32_t tc) const
+    {
+        const uint32_t hh = rows(tr);
+        return tr * ((KW - 1u) * bonds(h, w) + bonds(h, cols(KW - 1u))) + tc * bonds(hh, w);
+    }
+    __host__ __device__ __forceinline__ uint32_t bonds_of(uint32_t k) const { return bonds(rows(k / KW), cols(k % KW)); }
+    // place of border node (lr, lc) of a tile of hh rows among its ids
+    __device__ __forceinline__ uint32_t border(uint32_t lr, uint32_t lc, uint32_t hh) const
+    {
+        const uint32_t side = 2u * w + lr - 1u + (lc ? h - 2u : 0u);
+        return lr == 0u ? lc : lr + 1u == hh ? w + lc : side;
+    }
+};
+
+// A tile's union-find code: a parent's local index (below 0x1000), an open
+// root's place among the tile's ids (0x1000 + place), or a closed root's
+// (1 + sides) << 14 | size.
+#define TILE_OPEN 0x1000u
+#define TILE_CLOSED 0x4000u
+struct TileState {
+    static constexpr bool LDS = true;
+    uint16_t *code;
+    __device__ __forceinline__ uint32_t get(uint32_t i) const { return code[i]; }
+    __device__ __forceinline__ void set(uint32_t i, uint32_t v) const { code[i] = (uint16_t)v; }
+    __device__ __forceinline__ bool is_root(uint32_t v) const { return v >= TILE_OPEN; }
+};
+
+template <typename RecT>
+struct EventBits {
+    static constexpr uint32_t half = sizeof(RecT) * 4u;
+    static constexpr uint32_t top = 1u << (half - 1u);
+    static __device__ __forceinline__ RecT join(uint32_t a, uint32_t b) { return pack_record<RecT>(a | top, b | top); }
+    static __device__ __forceinline__ RecT gain(uint32_t open, uint32_t size, uint32_t f, bool closed_u)
+    {
+        return pack_record<RecT>(open, top | (closed_u ? 0x4000u : 0u) | (f << 12) | size);
+    }
+    static __device__ __forceinline__ bool is_event(RecT r) { return (r >> (2u * half - 1u)) != 0; }
+};
+
+// List entries: step, local index of u, and whether v is the node below u
+// (else the one to its right).
+template <typename ENT>
+struct TileEntry;
+template <>
+struct TileEntry<uint32_t> {
+    static __device__ __forceinline__ uint32_t make(uint32_t t, uint32_t u, uint32_t down) { return t | (u << 19) | (down << 31); }
+    static __device__ __forceinline__ void take(uint32_t e, uint32_t &t, uint32_t &u, uint32_t &down)
+    {
+        t = e & (TILE_SHORT_STEPS - 1u);
+        u = (e >> 19) & 0xFFFu;
+        down = e >> 31;
+    }
+};
+template <>
+struct TileEntry<uint64_t> {
+    static __device__ __forceinline__ uint64_t make(uint32_t t, uint32_t u, uint32_t down) { return (uint64_t)t | ((uint64_t)(u | (down << 31)) << 32); }
+    static __device__ __forceinline__ void take(uint64_t e, uint32_t &t, uint32_t &u, uint32_t &down)
+    {
+        t = (uint32_t)e;
+        u = (uint32_t)(e >> 32) & 0xFFFu;
+        down = (uint32_t)(e >> 63);
+    }
+};
+
+// Bond e in its tile: the tile k of its first node, that node's local row
+// and column, whether the bond goes down, and whether it leaves the tile.
+struct TileBond {
+    uint32_t k, tr, lr, lc, down;
+    bool cross;
+};
+__device__ __forceinline__ TileBond tile_bond(const TileGeo &g, int32_t e)
+{
+    uint32_t r, c, down;
+    g.lat.bond((uint32_t)e, r, c, down);
+    TileBond b;
+    b.tr = __umulhi(r, g.mh);
+    const uint32_t tc = __umulhi(c, g.mw);
+    b.lr = r - b.tr * g.h;
+    b.lc = c - tc * g.w;
+    b.k = b.tr * g.KW + tc;
+    b.down = down;
+    b.cross = down ? b.lr + 1u == g.h : b.lc + 1u == g.w;
+    return b;
+}
+
+// Initial codes of every tile's nodes and of the open nodes' own forest.
+__global__ __launch_bounds__(256) void tile_init_kernel(
+    TileGeo g, const uint8_t *__restrict__ sides, uint16_t *__restrict__ tiles,
+    uint32_t *__restrict__ open)
+{
+    const uint32_t k = blockIdx.x, tr = k / g.KW, tc = k % g.KW;
+    const uint32_t hh = g.rows(tr), ww = g.cols(tc);
+    for (uint32_t i = threadIdx.x; i < g.per; i += 256u)
+        open[k * g.per + i] = 0x80000001u;   // also the ids of no open node
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < g.init_stride; i += 256u) {
+        const uint32_t lr = i / g.w, lc = i % g.w;
+        uint32_t v = 0;
+        if (lr < hh && lc < ww) {
+            const uint32_t f = sides ? (uint32_t)sides[g.lat.node(tr * g.h + lr, tc * g.w + lc)] : 0u;
+            const bool is_open = (lr == 0u && tr) || (lr + 1u == hh && tr + 1u < g.KH) ||
+                                 (lc == 0u && tc) || (lc + 1u == ww && tc + 1u < g.KW);
+            v = ((1u + f) << 14) | 1u;
+            if (is_open) {
+                const uint32_t id = g.border(lr, lc, hh);
+                v = TILE_OPEN + id;
+                open[k * g.per + id] = 0x80000000u | (f << 29) | 1u;
+            }
+        }
+        tiles[(size_t)k * g.init_stride + i] = (uint16_t)v;
+    }
+}
+
+// Internal bonds per (run, segment of steps, tile), where a run's steps are
+// cut into nseg segments for several workgroups.
+__global__ __launch_bounds__(256) void tile_count_kernel(
+    TileGeo g, uint32_t M, uint32_t seg_steps, const int32_t *__restrict__ perm,
+    int64_t perm_stride, uint32_t *__restrict__ counts)
+{
+    extern __shared__ uint32_t tile_cnt[];
+    const uint32_t seg = blockIdx.x, nseg = gridDim.x;
+    for (uint32_t k = threadIdx.x; k < g.K; k += 256u)
+        tile_cnt[k] = 0u;
+    __syncthreads();
+    const int32_t *p = perm + (int64_t)blockIdx.y * perm_stride;
+    const uint32_t end = min(M, (seg + 1u) * seg_steps);
+    for (uint32_t t = seg * seg_steps + threadIdx.x; t < end; t += 256u) {
+        const uint32_t e = (uint32_t)p[t];
+        const TileBond b = tile_bond(g, (int32_t)min(e, M - 1u));
+        if (e < M && !b.cross)
+            atomicAdd(&tile_cnt[b.k], 1u);
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < g.K; k += 256u)
+        counts[((size_t)blockIdx.y * nseg + seg) * g.K + k] = tile_cnt[k];
+}
+
+// Counts to exclusive prefixes over a run's segments; odd[run] is set when a
+// tile's count is not its number of bonds.
+__global__ __launch_bounds__(256) void tile_scan_kernel(
+    TileGeo g, uint32_t nseg, uint32_t *__restrict__ counts, uint32_t *__restrict__ odd)
+{
+    uint32_t *c = counts + (size_t)blockIdx.x * nseg * g.K;
+    bool wrong = false;
+    for (uint32_t k = threadIdx.x; k < g.K; k += 256u) {
+        uint32_t acc = 0;
+        for (uint32_t s = 0; s < nseg; ++s) {
+            const uint32_t n = c[(size_t)s * g.K + k];
+            c[(size_t)s * g.K + k] = acc;
+            acc += n;
+        }
+        wrong |= acc != g.bonds_of(k);
+    }
+    const int any = __syncthreads_or(wrong);
+    if (threadIdx.x == 0u)
+        odd[blockIdx.x] = any ? 1u : 0u;
+}
+
+// The tiles' lists of a run (or of one segment of its steps): a stable
+// counting sort by tile of 256 * TILE_GROUPS steps at a time.  Every wave
+// ranks its 64 * TILE_GROUPS consecutive steps (match_label, and the wave's
+// own counter of each tile), the counters of the four waves become places
+// after the tile's cursor, and the entries are stored.  A row that is not a
+// permutation (some bond twice) may not fill the lists: such a run is marked
+// in odd[] and left to the untiled sweep.
+template <typename ENT, typename RecT>
+__global__ __launch_bounds__(256) void tile_scatter_kernel(
+    TileGeo g, uint32_t M, uint32_t tile_bits, uint32_t seg_steps,
+    const int32_t *__restrict__ perm, int64_t perm_stride,
+    const uint32_t *__restrict__ counts, ENT *__restrict__ lists, int64_t list_stride,
+    RecT *__restrict__ records, int64_t rec_stride, uint32_t *__restrict__ span_step,
+    uint32_t *__restrict__ odd)
+{
+    extern __shared__ uint32_t tile_dyn[];   // [4][K] wave counters, [K] cursors
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t seg = blockIdx.x, nseg = gridDim.x, run = blockIdx.y;
+    uint32_t *my = tile_dyn + wave * g.K, *cursor = tile_dyn + 4u * g.K;
+    for (uint32_t k = tid; k < g.K; k += 256u)
+        cursor[k] = g.offset(k / g.KW, k % g.KW) +
+                    (nseg > 1u ? counts[((size_t)run * nseg + seg) * g.K + k] : 0u);
+    if (seg == 0u && tid == 0u)
+        span_step[run] = PC_NO_SPAN;
+    if (nseg > 1u && odd[run])
+        return;
+    bool wrong = false;
+    const int32_t *p = perm + (int64_t)run * perm_stride;
+    ENT *list = lists + (int64_t)run * list_stride;
+    RecT *rec = records + (int64_t)run * rec_stride;
+    const uint32_t end = min(M, (seg + 1u) * seg_steps);
+    int32_t e[TILE_GROUPS];
+    uint32_t t0 = seg * seg_steps + wave * 64u * TILE_GROUPS + lane;
+#pragma unroll
+    for (uint32_t i = 0; i < TILE_GROUPS; ++i)
+        e[i] = t0 + i * 64u < end ? p[t0 + i * 64u] : -1;
+    for (uint32_t base = seg * seg_steps; base < end; base += 256u * TILE_GROUPS) {
+        for (uint32_t k = lane; k < g.K; k += 64u)
+            my[k] = 0u;
+        ENT ent[TILE_GROUPS];
+        uint32_t at[TILE_GROUPS];   // tile | rank << 12, or all ones
+#pragma unroll
+        for (uint32_t i = 0; i < TILE_GROUPS; ++i) {
+            const uint32_t t = t0 + i * 64u;
+            const bool ok = (uint32_t)e[i] < M;
+            const TileBond b = tile_bond(g, ok ? e[i] : 0);
+            const bool in = ok && !b.cross;
+            const uint64_t peers = match_label(b.k, tile_bits, __ballot(in));
+            at[i] = 0xFFFFFFFFu;
+            if (in) {
+                const uint32_t rank = lanes_below(peers);
+                const uint32_t before = my[b.k];
+                at[i] = b.k | ((before + rank) << 12);
+                if (rank == 0u)
+                    my[b.k] = before + (uint32_t)__popcll(peers);
+            } else if (ok) {
+                const uint32_t hh = g.rows(b.tr);
+                const uint32_t iu = b.k * g.per + g.border(b.lr, b.lc, hh);
+                const uint32_t kv = b.down ? b.k + g.KW : b.k + 1u;
+                const uint32_t iv = kv * g.per + (b.down ? b.lc : g.border(b.lr, 0u, hh));
+                rec[t] = EventBits<RecT>::join(iu, iv);
+            }
+            ent[i] = TileEntry<ENT>::make(t, b.lr * g.w + b.lc, b.down);
+        }
+        const uint32_t tn = t0 + 256u * TILE_GROUPS;
+#pragma unroll
+        for (uint32_t i = 0; i < TILE_GROUPS; ++i)
+            e[i] = tn + i * 64u < end ? p[tn + i * 64u] : -1;
+        __syncthreads();
+        for (uint32_t k = tid; k < g.K; k += 256u) {
+            uint32_t acc = cursor[k];
+#pragma unroll
+            for (uint32_t w = 0; w < 4u; ++w) {
+                const uint32_t n = tile_dyn[w * g.K + k];
+                tile_dyn[w * g.K + k] = acc;
+                acc += n;
+            }
+            cursor[k] = acc;
+            wrong |= acc > g.offset(k / g.KW, k % g.KW) + g.bonds_of(k);
+        }
+        if (__syncthreads_or(wrong))
+            break;
+#pragma unroll
+        for (uint32_t i = 0; i < TILE_GROUPS; ++i)
+            if (at[i] != 0xFFFFFFFFu)
+                list[my[at[i] & 0xFFFu] + (at[i] >> 12)] = ent[i];
+        t0 = tn;
+    }
+    if (nseg == 1u) {
+        for (uint32_t k = tid; k < g.K; k += 256u)
+            wrong |= cursor[k] != g.offset(k / g.KW, k % g.KW) + g.bonds_of(k);
+        const int any = __syncthreads_or(wrong);
+        if (tid == 0u)
+            odd[run] = any ? 1u : 0u;
+    }
+}
+
+// One tile of one run on one wavefront: 64 of the tile's bonds at a time
+// (lane = bond, in step order), as in sweep_run: finds, then rounds in which
+// every candidate claims its roots and merges if it is the earliest claimant
+// of each root it would change: of the closed one or ones, or, when both are
+// open, of both.  No budget of rounds: the earliest pending candidate always merges.  Blocks of
+// a run go to one XCD (shuf_block), whose L2 then collects the records that
+// the run's tiles write into shared lines.
+template <typename ENT, typename RecT>
+__global__ __launch_bounds__(64) void tile_sweep_kernel(
+    TileGeo g, uint32_t rn, const ENT *__restrict__ lists, int64_t list_stride,
+    const uint16_t *__restrict__ init, RecT *__restrict__ records,
+    int64_t rec_stride, uint32_t *__restrict__ span_step,
+    const uint32_t *__restrict__ odd)
+{
+    extern __shared__ uint32_t tile_lds[];
+    uint32_t *claims = tile_lds;
+    uint32_t rl, k;
+    if (!shuf_block(g.K, rn, rl, k) || odd[rl])
+        return;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t tr = k / g.KW, tc = k % g.KW;
+    const uint32_t n = TileGeo::bonds(g.rows(tr), g.cols(tc));
+    const uint32_t id0 = k * g.per;
+    const TileState st{(uint16_t *)(tile_lds + TILE_CLAIM_SLOTS)};
+    const ENT *list = lists + (int64_t)rl * list_stride + g.offset(tr, tc);
+    RecT *rec_out = records + (int64_t)rl * rec_stride;
+    {
+        const uint4 *src = (const uint4 *)(init + (size_t)k * g.init_stride);
+        uint4 *dst = (uint4 *)st.code;
+        for (uint32_t i = lane; i < g.init_stride / 8u; i += 64u)
+            dst[i] = src[i];
+    }
+    for (uint32_t i = lane; i < TILE_CLAIM_SLOTS; i += 64u)
+        claims[i] = 0u;
+    __syncthreads();
+
+    // list entries two batches ahead, the codes of the next batch's
+    // endpoints one batch ahead (a parent read early is still an ancestor)
+    ENT e0 = lane < n ? list[lane] : (ENT)0;
+    ENT e1 = 64u + lane < n ? list[64u + lane] : (ENT)0;
+    uint32_t hint_u = TILE_OPEN, hint_v = TILE_OPEN, tag = 0, span_at = PC_NO_SPAN;
+    for (uint32_t base = 0; base < n; base += 64u) {
+        uint32_t t, x, y, down;
+        TileEntry<ENT>::take(e0, t, x, down);
+        y = x + (down ? g.w : 1u);
+        const bool active = base + lane < n;
+        if (!active)
+            y = x = 0u;
+        e0 = e1;
+        e1 = base + 128u + lane < n ? list[base + 128u + lane] : (ENT)0;
+        x = st.is_root(hint_u) ? x : hint_u;
+        y = st.is_root(hint_v) ? y : hint_v;
+        uint32_t cx, cy;
+        find2(st, x, cx, y, cy);
+        {
+            uint32_t tn, un, dn;
+            TileEntry<ENT>::take(e0, tn, un, dn);
+            const bool more = base + 64u + lane < n;
+            hint_u = st.get(more ? un : 0u);
+            hint_v = st.get(more ? un + (dn ? g.w : 1u) : 0u);
+        }
+        bool cand = active && x != y;
+        RecT rec = 0;
+        while (__ballot(cand)) {
+            tag += 64u;
+            const uint32_t mine = tag + 63u - lane;
+            const bool open_x = cx < TILE_CLOSED, open_y = cy < TILE_CLOSED;
+            const uint32_t su = ((x * 0x9E3779u) & 0xFFFFFFu) >> (24 - TILE_CLAIM_BITS);
+            const uint32_t sv = ((y * 0x9E3779u) & 0xFFFFFFu) >> (24 - TILE_CLAIM_BITS);
+            // an open root is claimed only where two open ones may join: the
+            // join waits for every earlier candidate of either root, which
+            // else would name a root it was not yet joined with
+            const bool join = open_x && open_y;
+            const bool joins = __ballot(cand && join) != 0u;
+            if (cand && (!open_x || joins))
+                atomicMax(&claims[su], mine);
+            if (cand && (!open_y || joins))
+                atomicMax(&claims[sv], mine);
+            const bool go = cand && ((open_x && !join) || claims[su] == mine) &&
+                            ((open_y && !join) || claims[sv] == mine);
+            bool spans_here = false;
+            if (go) {
+                const uint32_t sx = cx & 0x3FFFu, sy = cy & 0x3FFFu;
+                // an open root is the parent of a closed one
+                const bool x_big = open_y ? open_x : (open_x || sx >= sy);
+                const uint32_t big = x_big ? x : y, small = x_big ? y : x;
+                st.set(small, big);
+                if (!open_x && !open_y) {
+                    const uint32_t f = ((cx >> 14) - 1u) | ((cy >> 14) - 1u);
+                    spans_here = f == 3u;
+                    st.set(big, ((1u + (f == 3u ? 0u : f)) << 14) | (sx + sy));
+                    rec = pack_record<RecT>(sx, sy);
+                } else {
+                    const uint32_t ix = id0 + cx - TILE_OPEN, iy = id0 + cy - TILE_OPEN;
+                    if (join)
+                        rec = EventBits<RecT>::join(ix, iy);
+                    else
+                        rec = EventBits<RecT>::gain(open_x ? ix : iy, open_x ? sy : sx,
+                                                    ((open_x ? cy : cx) >> 14) - 1u, open_y);
+                }
+            }
+            const uint64_t spans = __ballot(spans_here);
+            if (spans)
+                span_at = min(span_at, read_lane(t, (uint32_t)__builtin_ctzll(spans)) + 1u);
+            cand = cand && !go;
+            if (!__ballot(cand))
+                break;
+            if (cand)
+                find2(st, x, cx, y, cy);
+            cand = cand && x != y;
+        }
+        if (active)
+            rec_out[t] = rec;
+    }
+    if (lane == 0u && span_at != PC_NO_SPAN)
+        atomicMin(&span_step[rl], span_at);
+}
+
+// A run's open nodes with their codes in LDS (the HBM codes of GlobalState).
+struct OpenLdsState {
+    static constexpr bool LDS = true;
+    uint32_t *code;
+    __device__ __forceinline__ uint32_t get(uint32_t i) const { return code[i]; }
+    __device__ __forceinline__ void set(uint32_t i, uint32_t v) const { code[i] = v; }
+    __device__ __forceinline__ bool is_root(uint32_t v) const { return (v >> 31) != 0u; }
+    __device__ __forceinline__ uint32_t root(uint32_t size, uint32_t f) const { return 0x80000000u | (f << 29) | size; }
+    __device__ __forceinline__ void sync() const {}
+    __device__ __forceinline__ void decode(uint32_t v, uint32_t &size, uint32_t &f) const
+    {
+        size = v & 0x1FFFFFFFu;
+        f = (v >> 29) & 3u;
+    }
+};
+
+// A run's events in step order on one wavefront.  The records are scanned
+// EVENT_SCAN groups of 64 steps at a time (loaded one scan ahead), their
+// events appended to a ring in LDS, and taken from it 64 at a time (lane =
+// event) through the rounds of sweep_run: claims, independent merges and
+// star merges into the hub.  A gain's closed cluster is a root of its own
+// that no other event touches: it needs no claim and no store.
+#define EVENT_SCAN 4u
+#define EVENT_RING 512u
+
+template <typename RecT>
+constexpr uint32_t event_lds_words() { return CLAIM_SLOTS + EVENT_RING * (1u + sizeof(RecT) / 4u); }
+
+template <class St, typename RecT>
+__device__ __forceinline__ void event_run(const St &st, uint32_t M, RecT *rec_io,
+                                          uint32_t *claims, RecT *ring, uint32_t *ring_t,
+                                          uint32_t *span_step)
+{
+    const uint32_t lane = threadIdx.x;
+    constexpr uint32_t TOP = EventBits<RecT>::top;
+    uint32_t span_at = *span_step, tag = 0;
+    uint32_t head = 0, count = 0, pos = 0;
+    RecT ahead[EVENT_SCAN];
+#pragma unroll
+    for (uint32_t i = 0; i < EVENT_SCAN; ++i)
+        ahead[i] = i * 64u + lane < M ? rec_io[i * 64u + lane] : (RecT)0;
+    for (;;) {
+        while (count < 64u && pos < M) {
+            RecT cur[EVENT_SCAN];
+            const uint32_t next = pos + 64u * EVENT_SCAN;
+#pragma unroll
+            for (uint32_t i = 0; i < EVENT_SCAN; ++i) {
+                cur[i] = ahead[i];
+                ahead[i] = next + i * 64u + lane < M ? rec_io[next + i * 64u + lane] : (RecT)0;
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < EVENT_SCAN; ++i) {
+                const bool is = EventBits<RecT>::is_event(cur[i]);
+                const uint64_t b = __ballot(is);
+                if (is) {
+                    const uint32_t p = (head + count + lanes_below(b)) & (EVENT_RING - 1u);
+                    ring[p] = cur[i];
+                    ring_t[p] = pos + i * 64u + lane;
+                }
+                count += (uint32_t)__popcll(b);
+            }
+            pos = next;
+        }
+        if (!count)
+            break;
+        const uint32_t n = min(count, 64u);
+        const bool active = lane < n;
+        const uint32_t slot = (head + lane) & (EVENT_RING - 1u);
+        __syncthreads();
+        const RecT ev = active ? ring[slot] : (RecT)0;
+        const uint32_t t = active ? ring_t[slot] : 0u;
+        head += n;
+        count -= n;
+        uint32_t lo, hi;
+        unpack_record(ev, lo, hi);
+        const bool gain = active && !(lo & TOP);
+        const bool swap = gain && (hi & 0x4000u);   // the closed cluster is on u's side
+        uint32_t ru = active ? lo & (TOP - 1u) : 0u;
+        uint32_t rv = active && !gain ? hi & (TOP - 1u) : ru;
+        uint32_t cu, cv;
+        find2(st, ru, cu, rv, cv);
+        if (gain) {
+            rv = 0xFFFFFFFFu;
+            cv = st.root(hi & 0xFFFu, (hi >> 12) & 3u);
+        }
+        bool cand = active && ru != rv;
+        RecT rec = 0;
+        while (__ballot(cand)) {
+            tag += 64u;
+            const uint32_t mine = tag + 63u - lane;
+            const uint32_t su = claim_slot(ru), sv = claim_slot(rv);
+            if (cand)
+                atomicMax(&claims[su], mine);
+            if (cand && !gain)
+                atomicMax(&claims[sv], mine);
+            const uint32_t held_u = claims[su], held_v = gain ? mine : claims[sv];
+            const bool own_u = held_u == mine, own_v = held_v == mine;
+            bool go = cand && own_u && own_v;
+            uint64_t star = 0;
+            uint32_t hub = 0;
+            const uint64_t blocked = __ballot(cand && !go);
+            if (blocked) {
+                const uint32_t fl = (uint32_t)__builtin_ctzll(blocked);
+                hub = read_lane(own_u ? rv : ru, fl);
+                const bool at_u = ru == hub;
+                const bool touch = cand && (at_u || rv == hub);
+                const uint64_t tm = __ballot(touch);
+                const uint64_t bad = tm & ~__ballot(touch && (at_u ? own_v : own_u));
+                star = bad ? (tm & ((bad & (0u - bad)) - 1u)) : tm;
+                go = go && !touch;
+                const uint32_t hu = tag + 63u - held_u, hv = tag + 63u - held_v;
+                const bool late = cand && !go && !((star >> lane) & 1u) &&
+                                  (((star >> (hu & 63u)) & 1u) || ((star >> (hv & 63u)) & 1u));
+                const uint64_t lm = __ballot(late);
+                if (lm)
+                    star &= (lm & (0u - lm)) - 1u;
+            }
+            const bool in_star = (star >> lane) & 1u;
+            if (star) {
+                const bool at_u = ru == hub;
+                const uint32_t x = at_u ? rv : ru;
+                uint32_t sx, fx, sh, fh;
+                st.decode(at_u ? cv : cu, sx, fx);
+                st.decode(at_u ? cu : cv, sh, fh);
+                const uint32_t first = (uint32_t)__builtin_ctzll(star);
+                const uint32_t s_hub = read_lane(sh, first), f_hub = read_lane(fh, first);
+                const uint32_t incl = wave_scan_add(in_star ? sx : 0u);
+                const uint32_t total = read_lane(incl, 63u);
+                const uint64_t m1 = __ballot(in_star && (fx & 1u));
+                const uint64_t m2 = __ballot(in_star && (fx & 2u));
+                const uint32_t f_all = f_hub | (m1 ? 1u : 0u) | (m2 ? 2u : 0u);
+                if (in_star) {
+                    if (!gain)
+                        st.set(x, hub);
+                    const uint32_t sh_now = s_hub + incl - sx;
+                    rec = at_u != swap ? pack_record<RecT>(sh_now, sx) : pack_record<RecT>(sx, sh_now);
+                }
+                if (lane == first)
+                    st.set(hub, st.root(s_hub + total, f_all == 3u ? 0u : f_all));
+                if (f_all == 3u) {
+                    const uint32_t l1 = (f_hub & 1u) ? first : (uint32_t)__builtin_ctzll(m1);
+                    const uint32_t l2 = (f_hub & 2u) ? first : (uint32_t)__builtin_ctzll(m2);
+                    span_at = min(span_at, read_lane(t, max(l1, l2)) + 1u);
+                }
+            }
+            bool spans_here = false;
+            if (go) {
+                uint32_t sa, fa, sb, fb;
+                st.decode(cu, sa, fa);
+                st.decode(cv, sb, fb);
+                const bool a_big = gain || sa >= sb;
+                const uint32_t big = a_big ? ru : rv, small = a_big ? rv : ru;
+                const uint32_t f = fa | fb;
+                if (!gain)
+                    st.set(small, big);
+                st.set(big, st.root(sa + sb, f == 3u ? 0u : f));
+                rec = swap ? pack_record<RecT>(sb, sa) : pack_record<RecT>(sa, sb);
+                spans_here = f == 3u;
+            }
+            {
+                const uint64_t spans = __ballot(spans_here);
+                if (spans)
+                    span_at = min(span_at, read_lane(t, (uint32_t)__builtin_ctzll(spans)) + 1u);
+            }
+            cand = cand && !go && !in_star;
+            st.sync();
+            if (!__ballot(cand))
+                break;
+            if (cand) {
+                uint32_t z = gain ? ru : rv, cz = cv;
+                find2(st, ru, cu, z, cz);
+                if (!gain) {
+                    rv = z;
+                    cv = cz;
+                }
+            }
+            cand = cand && ru != rv;
+        }
+        if (active)
+            rec_io[t] = rec;
+    }
+    if (lane == 0u)
+        *span_step = span_at;
+}
+
+// Codes in LDS (LDS_STATE) or in the run's slot of `states`; both start from
+// `open` (tile_init_kernel).
+template <typename RecT, bool LDS_STATE>
+__global__ __launch_bounds__(64) void event_sweep_kernel(
+    uint32_t nodes, uint32_t M, const uint32_t *__restrict__ open,
+    uint32_t *__restrict__ states, RecT *__restrict__ records, int64_t rec_stride,
+    uint32_t *__restrict__ span_step, const uint32_t *__restrict__ odd)
+{
+    extern __shared__ __align__(16) uint32_t event_lds[];
+    if (odd[blockIdx.x])
+        return;
+    uint32_t *claims = event_lds, *ring_t = event_lds + CLAIM_SLOTS;
+    RecT *ring = (RecT *)(ring_t + EVENT_RING);
+    const uint32_t lane = threadIdx.x;
+    RecT *rec = records + (int64_t)blockIdx.x * rec_stride;
+    uint32_t *code = LDS_STATE ? event_lds + event_lds_words<RecT>()
+                               : states + (size_t)blockIdx.x * nodes;
+    for (uint32_t i = lane; i < CLAIM_SLOTS; i += 64u)
+        claims[i] = 0u;
+    for (uint32_t i = lane; i < nodes; i += 64u)
+        code[i] = open[i];
+    __threadfence_block();
+    __syncthreads();
+    if constexpr (LDS_STATE)
+        event_run<OpenLdsState, RecT>(OpenLdsState{code}, M, rec, claims, ring, ring_t,
+                                      span_step + blockIdx.x);
+    else
+        event_run<GlobalState, RecT>(GlobalState{code}, M, rec, claims, ring, ring_t,
+                                     span_step + blockIdx.x);
 }
 
 // Running per-run state (after some number of bonds).
@@ -3923,7 +4573,7 @@ static int sweep_launch(uint32_t num_nodes, uint32_t num_edges, ES edges,
     sweep_global_kernel<RT, CH, SP, ES, FO><<<(uint32_t)slots, threads, 0, s>>>(   \
         num_nodes, num_edges, num_runs, edges, d_node_sides,                   \
         span_on_first_merge, d_perm, perm_stride, (RT *)d_records, rec_stride, \
-        d_span_step, (uint32_t *)d_workspace, rounds, d_chunk_state)
+        d_span_step, (uint32_t *)d_workspace, rounds, d_chunk_state, nullptr)
 #define PC_SWEEP_GLOBAL_W(RT, CH)                                              \
     do {                                                                       \
         if (split)                                                             \
@@ -3971,6 +4621,208 @@ static LatticeEdges lattice_edges(uint32_t length, bool tiled)
     return LatticeEdges{length, d, 1.0f / (float)d, tiled ? 1u : 0u};
 }
 
+// ---------------------------------------------------------------------------
+// The tiled sweep's plan and launches
+// ---------------------------------------------------------------------------
+// Lattices it takes: state above the LDS limit, a side of at most
+// TILE_MAX_LENGTH.  False otherwise.
+static bool tile_geo(uint32_t length, bool tiled, TileGeo &g)
+{
+    if ((uint64_t)length * length <= kLdsMaxNodes || length > TILE_MAX_LENGTH)
+        return false;
+    g.lat = lattice_edges(length, tiled);
+    g.L = length;
+    g.KH = g.KW = (length + TILE_SIDE - 1u) / TILE_SIDE;
+    g.h = g.w = (length + g.KH - 1u) / g.KH;
+    g.K = g.KH * g.KW;
+    g.per = 2u * g.w + 2u * (g.h - 2u);
+    g.mh = (uint32_t)(((1ull << 32) + g.h - 1u) / g.h);
+    g.mw = (uint32_t)(((1ull << 32) + g.w - 1u) / g.w);
+    g.init_stride = (g.h * g.w + 7u) & ~7u;
+    return true;
+}
+
+// The workspace of a tiled sweep of num_runs runs whose lists are held for
+// `slab` runs at a time: the offsets of its parts, and its size.
+struct TilePlan {
+    uint64_t init, open, odd, states, counts, lists, list_bytes, bytes;
+    uint32_t nodes, slab;
+    bool lds;       // the open nodes' codes fit LDS
+    bool short_entries;
+};
+#define TILE_OPEN_LDS_NODES 18432u // 72 KiB of codes: two runs per CU
+
+static TilePlan tile_plan(const TileGeo &g, uint32_t num_runs, uint32_t slab)
+{
+    TilePlan p;
+    auto up = [](uint64_t v) { return (v + 255u) & ~(uint64_t)255u; };
+    const uint64_t M = 2ull * g.L * (g.L - 1u);
+    p.nodes = g.K * g.per;
+    p.slab = slab;
+    p.lds = p.nodes <= TILE_OPEN_LDS_NODES;
+    p.short_entries = M <= TILE_SHORT_STEPS;
+    p.init = 0;
+    p.open = up((uint64_t)g.K * g.init_stride * 2u);
+    p.odd = p.open + up((uint64_t)p.nodes * 4u);
+    p.states = p.odd + up((uint64_t)num_runs * 4u);
+    p.counts = p.states + (p.lds ? 0u : up((uint64_t)num_runs * p.nodes * 4u));
+    p.lists = p.counts + up(((uint64_t)slab + TILE_SCATTER_BLOCKS) * g.K * 4u);
+    p.list_bytes = up(M * (p.short_entries ? 4u : 8u));
+    p.bytes = p.lists + slab * p.list_bytes;
+    return p;
+}
+
+// Runs whose lists are held at a time: enough (run, tile) wavefronts to fill
+// the GPU several times over (16384), more where that takes no more memory
+// than the untiled sweep's codes.
+static uint32_t tile_slab(const TileGeo &g, uint32_t num_runs)
+{
+    const uint64_t slots = std::min(num_runs, kGlobalSlots);
+    const uint64_t same = slots * g.L * g.L * 4u / tile_plan(g, 1u, 1u).list_bytes;
+    const uint64_t fill = (16384u + g.K - 1u) / g.K;
+    return (uint32_t)std::min<uint64_t>(num_runs, std::max(same, fill));
+}
+
+extern "C" int pc_sweep_lattice_workspace_size(uint32_t length, uint32_t num_runs,
+                                               uint32_t state_mode, uint64_t *bytes)
+{
+    g_last_error[0] = 0;
+    if (!bytes)
+        return pc_fail(PC_EINVAL, "pc_sweep_lattice_workspace_size: bytes is NULL");
+    if (length == 0 || length > 16384u)
+        return pc_fail(PC_EINVAL, "pc_sweep_lattice_workspace_size: length must be in 1..16384");
+    const int rc = pc_sweep_workspace_size(length * length, num_runs, state_mode, bytes);
+    TileGeo g;
+    if (rc == PC_OK && num_runs && state_mode == PC_STATE_AUTO && tile_geo(length, false, g))
+        *bytes = std::max(*bytes, tile_plan(g, num_runs, tile_slab(g, num_runs)).bytes);
+    return rc;
+}
+
+template <typename ENT, typename RecT>
+static int tile_sweep_launch(const TileGeo &g, const TilePlan &p,
+                             const uint8_t *d_node_sides, const int32_t *d_perm,
+                             int64_t perm_stride, uint32_t num_runs, RecT *d_records,
+                             int64_t rec_stride, uint32_t *d_span_step, char *ws,
+                             uint32_t rounds, hipStream_t s)
+{
+    const uint32_t M = 2u * g.L * (g.L - 1u);
+    uint16_t *init = (uint16_t *)(ws + p.init);
+    uint32_t *open = (uint32_t *)(ws + p.open), *odd = (uint32_t *)(ws + p.odd);
+    uint32_t *counts = (uint32_t *)(ws + p.counts);
+    ENT *lists = (ENT *)(ws + p.lists);
+    const int64_t list_stride = (int64_t)(p.list_bytes / sizeof(ENT));
+    uint32_t bits = 0;
+    while ((1u << bits) < g.K)
+        ++bits;
+    tile_init_kernel<<<g.K, 256, 0, s>>>(g, d_node_sides, init, open);
+    PC_LAUNCH_CHECK("tile_init_kernel");
+    for (uint32_t r0 = 0; r0 < num_runs; r0 += p.slab) {
+        const uint32_t rn = std::min(p.slab, num_runs - r0);
+        const int32_t *perm = d_perm + (int64_t)r0 * perm_stride;
+        RecT *rec = d_records + (int64_t)r0 * rec_stride;
+        // a workgroup per run, or several where the runs are few: the steps
+        // of a segment then start where a count of the earlier ones says
+        uint32_t nseg = (TILE_SCATTER_BLOCKS + rn - 1u) / rn;
+        nseg = std::min(nseg, (M + 16383u) / 16384u);
+        const uint32_t quant = 256u * TILE_GROUPS;
+        const uint32_t seg = ((M + nseg - 1u) / nseg + quant - 1u) / quant * quant;
+        nseg = (M + seg - 1u) / seg;
+        if (nseg > 1u) {
+            tile_count_kernel<<<dim3(nseg, rn), 256, g.K * 4u, s>>>(g, M, seg, perm,
+                                                                    perm_stride, counts);
+            PC_LAUNCH_CHECK("tile_count_kernel");
+            tile_scan_kernel<<<rn, 256, 0, s>>>(g, nseg, counts, odd + r0);
+            PC_LAUNCH_CHECK("tile_scan_kernel");
+        }
+        tile_scatter_kernel<ENT, RecT><<<dim3(nseg, rn), 256, 5u * g.K * 4u, s>>>(
+            g, M, bits, seg, perm, perm_stride, counts, lists, list_stride, rec, rec_stride,
+            d_span_step + r0, odd + r0);
+        PC_LAUNCH_CHECK("tile_scatter_kernel");
+        const size_t lds = TILE_CLAIM_SLOTS * 4u + g.init_stride * 2u;
+        tile_sweep_kernel<ENT, RecT><<<shuf_blocks(g.K, rn), 64, lds, s>>>(
+            g, rn, lists, list_stride, init, rec, rec_stride, d_span_step + r0, odd + r0);
+        PC_LAUNCH_CHECK("tile_sweep_kernel");
+    }
+    const size_t ring = event_lds_words<RecT>() * 4u;
+    if (p.lds)
+        event_sweep_kernel<RecT, true><<<num_runs, 64, ring + p.nodes * 4u, s>>>(
+            p.nodes, M, open, nullptr, d_records, rec_stride, d_span_step, odd);
+    else
+        event_sweep_kernel<RecT, false><<<num_runs, 64, ring, s>>>(
+            p.nodes, M, open, (uint32_t *)(ws + p.states), d_records, rec_stride,
+            d_span_step, odd);
+    PC_LAUNCH_CHECK("event_sweep_kernel");
+    // runs whose row is not a permutation, with their codes in the lists'
+    // place
+    const uint64_t slots = p.slab * p.list_bytes / ((uint64_t)g.L * g.L * 4u);
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(std::min<uint64_t>(slots, num_runs), 256u);
+    sweep_global_kernel<RecT, false, true, LatticeEdges><<<grid, 128, 0, s>>>(
+        g.L * g.L, M, num_runs, g.lat, d_node_sides, 0, d_perm, perm_stride, d_records,
+        rec_stride, d_span_step, (uint32_t *)lists, rounds, nullptr, odd);
+    PC_LAUNCH_CHECK("sweep_global_kernel");
+    return PC_OK;
+}
+
+// The tiled sweep, if it takes this call: *taken tells.  Not taken: modes
+// that ask for a state or a number of wavefronts, auxiliary sides joined
+// from the first merge on, more than 2^31 grid blocks, or a workspace that
+// holds the lists of fewer than 4 runs (or of all runs).
+static int tile_sweep(uint32_t length, bool tiled, const uint8_t *d_node_sides,
+                      int32_t span_on_first_merge, const int32_t *d_perm,
+                      int64_t perm_stride, uint32_t num_runs, void *d_records,
+                      int64_t rec_stride, uint32_t *d_span_step, void *d_workspace,
+                      uint64_t workspace_bytes, uint32_t merge_rounds,
+                      uint32_t state_mode, uint64_t *d_chunk_state, void *stream,
+                      bool *taken)
+{
+    *taken = false;
+    TileGeo g;
+    const uint32_t rounds = merge_rounds ? merge_rounds : g_merge_rounds;
+    const int64_t M = 2ll * length * (length - 1ll);
+    if (state_mode != PC_STATE_AUTO || span_on_first_merge || num_runs == 0 || rounds > 64 ||
+        !tile_geo(length, tiled, g) || !d_workspace || ((uintptr_t)d_workspace & 15u) ||
+        !d_span_step || !d_perm || !d_records || perm_stride < M || rec_stride < M)
+        return PC_OK;
+    uint32_t slab = tile_slab(g, num_runs);
+    const TilePlan one = tile_plan(g, num_runs, 1u);
+    if (workspace_bytes < tile_plan(g, num_runs, slab).bytes) {
+        const uint64_t per_run = one.list_bytes + g.K * 4u;
+        const uint64_t base = one.bytes + 512u;
+        slab = workspace_bytes < base ? 0u : (uint32_t)std::min<uint64_t>(
+                   slab, 1u + (workspace_bytes - base) / per_run);
+        if (slab < std::min(num_runs, 4u))
+            return PC_OK;
+    }
+    // slabs of about the same size, in groups of eight runs
+    const uint32_t slabs = (num_runs + slab - 1u) / slab;
+    slab = std::min(slab, ((num_runs + slabs - 1u) / slabs + 7u) & ~7u);
+    if (slab > 65535u)
+        slab = 65528u;
+    const TilePlan p = tile_plan(g, num_runs, slab);
+    if (p.bytes > workspace_bytes || (uint64_t)(slab + 7u) * g.K > 0x7FFFFFFFu)
+        return PC_OK;
+    *taken = true;
+    hipStream_t s = as_stream(stream);
+    const bool u32rec = length * length <= kU32RecordMaxNodes;
+    int rc;
+    if (u32rec)
+        rc = tile_sweep_launch<uint32_t, uint32_t>(
+            g, p, d_node_sides, d_perm, perm_stride, num_runs, (uint32_t *)d_records,
+            rec_stride, d_span_step, (char *)d_workspace, rounds, s);
+    else if (p.short_entries)
+        rc = tile_sweep_launch<uint32_t, uint64_t>(
+            g, p, d_node_sides, d_perm, perm_stride, num_runs, (uint64_t *)d_records,
+            rec_stride, d_span_step, (char *)d_workspace, rounds, s);
+    else
+        rc = tile_sweep_launch<uint64_t, uint64_t>(
+            g, p, d_node_sides, d_perm, perm_stride, num_runs, (uint64_t *)d_records,
+            rec_stride, d_span_step, (char *)d_workspace, rounds, s);
+    if (rc == PC_OK && d_chunk_state)
+        rc = pc_chunk_scan(length * length, (uint32_t)M, num_runs, d_records, rec_stride,
+                           d_chunk_state, stream);
+    return rc;
+}
+
 extern "C" int pc_sweep_lattice(uint32_t length, int32_t tiled,
                                 const uint8_t *d_node_sides,
                                 int32_t span_on_first_merge, const int32_t *d_perm,
@@ -3987,6 +4839,13 @@ extern "C" int pc_sweep_lattice(uint32_t length, int32_t tiled,
     if (tiled && (length % 8u))
         return pc_fail(PC_EINVAL, "pc_sweep_lattice: the tiled order needs a multiple of 8");
     const uint32_t N = length * length, M = 2u * length * (length - 1u);
+    bool taken = false;
+    const int rc = tile_sweep(length, tiled != 0, d_node_sides, span_on_first_merge, d_perm,
+                              perm_stride, num_runs, d_records, rec_stride, d_span_step,
+                              d_workspace, workspace_bytes, merge_rounds, state_mode,
+                              d_chunk_state, stream, &taken);
+    if (taken)
+        return rc;
     return sweep_launch(N, M, lattice_edges(length, tiled != 0), true, d_node_sides,
                         span_on_first_merge, d_perm, perm_stride, num_runs,
                         d_records, rec_stride, d_span_step, d_workspace,

@@ -407,3 +407,91 @@ def test_hbm_sweep_with_fewer_slots_than_runs(gpu, chunks):
     if chunks:
         assert np.array_equal(part.chunk_state.cpu().numpy(),
                               full.chunk_state.cpu().numpy())
+
+
+def _tiled_and_untiled(eng, perm, chunks=True):
+    """The sweep as the library picks it and with every node's code in HBM."""
+    from pypercolate_amd import _native as nat
+    assert eng.state_mode == nat.PC_STATE_AUTO
+    auto = eng.sweep(perm, chunks=chunks)
+    eng.state_mode = nat.PC_STATE_HBM | nat.PC_SWEEP_TWO_WAVES
+    hbm = eng.sweep(perm, chunks=chunks)
+    eng.state_mode = nat.PC_STATE_AUTO
+    return auto, hbm
+
+
+def _same_sweep(a, b, chunks=True):
+    assert np.array_equal(a.records.cpu().numpy(), b.records.cpu().numpy())
+    assert np.array_equal(a.span_step.cpu().numpy(), b.span_step.cpu().numpy())
+    if chunks:
+        assert np.array_equal(a.chunk_state.cpu().numpy(), b.chunk_state.cpu().numpy())
+
+
+@pytest.mark.parametrize('length,runs', [(129, 5), (136, 9), (181, 40), (192, 3), (255, 2),
+                                         (256, 17), (257, 8), (512, 2), (513, 2), (700, 1)])
+def test_tiled_lattice_sweep_equals_untiled(gpu, length, runs):
+    """The tiled sweep's records, span steps and chunk states equal those of
+    the sweep with every node's code in HBM: whole and ragged tiles, 32- and
+    64-bit records (from 257), 32- and 64-bit list entries (from 513), open
+    nodes in LDS and in HBM (700), one workgroup per run or several."""
+    eng = BondEngine(_graph.square_lattice(length))
+    perm = eng.device_permutations(17, runs)
+    _same_sweep(*_tiled_and_untiled(eng, perm))
+
+
+@pytest.mark.parametrize('length', [130, 264])
+def test_tiled_lattice_sweep_orders(gpu, length):
+    """Orders that are far from random: the bonds in their own order and
+    reversed, all bonds down before those to the right, a far corner first;
+    and rows that are not permutations (one bond twice in another's place,
+    one bond throughout), which go through the untiled sweep, beside one
+    that is."""
+    eng = BondEngine(_graph.square_lattice(length))
+    M = eng.M
+    one = np.arange(M)
+    edges = eng.graph.edges
+    down = edges[:, 1] - edges[:, 0] == length
+    twice = np.random.RandomState(3).permutation(M)
+    twice[5] = twice[M // 2]
+    perm = eng.upload_permutations(np.stack(
+        [one, one[::-1], np.argsort(~down, kind='stable'), np.argsort(-edges[:, 1], kind='stable'),
+         twice, np.full(M, 7), np.random.RandomState(4).permutation(M)]))
+    _same_sweep(*_tiled_and_untiled(eng, perm))
+
+
+@pytest.mark.parametrize('sides', ['none', 'scattered'])
+def test_tiled_lattice_sweep_sides(gpu, sides):
+    """No spanning sides; and sides on nodes anywhere, so that clusters
+    inside a tile touch one side, or both."""
+    ga = _graph.square_lattice(200, spanning_cluster=False)
+    if sides == 'scattered':
+        rng = np.random.RandomState(8)
+        ga.node_sides = (rng.randint(0, 400, ga.num_nodes) % 3 *
+                         (rng.randint(0, 500, ga.num_nodes) == 0)).astype(np.uint8)
+        assert set(np.unique(ga.node_sides)) == {0, 1, 2}
+    eng = BondEngine(ga)
+    _same_sweep(*_tiled_and_untiled(eng, eng.device_permutations(23, 12)))
+
+
+def test_tiled_lattice_sweep_small_workspaces(gpu):
+    """Workspaces for the lists of some of the runs (slabs), and of too few
+    (the untiled sweep): the same records."""
+    eng = BondEngine(_graph.square_lattice(264))
+    perm = eng.device_permutations(29, 30)
+    full = eng.sweep(perm)
+    for nbytes in (eng.workspace_bytes(30) // 2, eng.workspace_bytes(10),
+                   2 * eng.N * 4, eng.N * 4):
+        ws = gpu.empty((nbytes,), dtype=gpu.uint8, device='cuda')
+        _same_sweep(eng.sweep(perm, workspace=ws), full)
+
+
+def test_tiled_lattice_sweep_matches_oracle(gpu):
+    """L = 300 (64-bit records): traces and exact sums over two numpy
+    permutations equal the oracle's."""
+    eng = BondEngine(_graph.square_lattice(300))
+    g = oracle.square_lattice_graph(300)
+    perms = oracle.randomstate_permutations(range(2), eng.M)
+    expect = oracle.bond_runs(g, perms)
+    res = eng.sweep(eng.upload_permutations(perms))
+    _check_traces(eng, res, expect)
+    _check_sums(eng, res, expect)
