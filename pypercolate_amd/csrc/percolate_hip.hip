@@ -2112,12 +2112,13 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 // ---------------------------------------------------------------------------
 // Tiled sweep of the square lattice (pc_sweep_lattice for lattices whose
 // union-find state does not fit LDS).  The lattice is cut into tiles of at
-// most TILE_SIDE x TILE_SIDE nodes.  A node with a bond into another tile is
+// most TILE_ROWS x TILE_COLS nodes.  A node with a bond into another tile is
 // open, and so is every cluster of a tile's own bonds that holds an open
 // node; the other clusters of a tile are closed: nothing outside the tile
 // can have joined them, so their sizes and sides are exact at every step.
 //   1. tile_scatter: each run's bonds, in step order, into one list per
-//      tile (its internal bonds); a bond between two tiles becomes an event;
+//      tile (its internal bonds); the record row, with an event for every
+//      bond between two tiles and 0 elsewhere;
 //   2. tile_sweep: one wavefront per (run, tile) merges the tile's internal
 //      bonds in step order with its state in LDS.  A merge of two closed
 //      clusters is final and its record is written.  A merge with an open
@@ -2127,7 +2128,7 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 //      change, so such merges do not conflict over it: near and above the
 //      threshold, where most merges hit one large cluster, a batch resolves
 //      in one round;
-//   3. event_sweep: one wavefront per run merges the run's events in step
+//   3. event_sweep: one workgroup per run merges the run's events in step
 //      order over the open nodes alone (0.05 N of them) and replaces every
 //      event by its record.
 // About 0.11 M of a random run's steps are events (64 x 64 tiles); the
@@ -2135,9 +2136,14 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 // outside bonds have already joined is found out in step 3 (record 0).
 // Untiled, with every node's code in HBM, the sweep moves 342 bytes per
 // addition in random lines at L = 1024.  Sweep with its chunk states, untiled
-// and tiled: L = 1024, 1000 runs 158 and 96 ms (lists 20, tiles 39, events 25,
-// chunk states 12); L = 256, 200 runs 3.67 and 1.53 ms; L = 181, 600 runs
-// 2.65 and 1.46 ms.  Bound by the wavefronts' dependent LDS round trips.
+// and tiled: L = 1024, 1000 runs 158 and 79 ms (lists 24, tiles 23, events 20,
+// chunk states 12); L = 256, 200 runs 3.67 and 1.3 ms; L = 181, 600 runs
+// 2.65 and 1.3 ms.  The tiles are bound by dependent LDS round trips (70 % of
+// a wavefront's cycles wait) and at L = 1024 by the records, which go out in
+// part-written lines: rows cleared in step order by tile_scatter, so that a
+// tile writes merges only, took them from 35 to 27 ms, a claim table of 512
+// slots instead of 1024 (15 wavefronts per CU, not 13) to 23 ms; 48 x 48 and
+// 32 x 64 tiles gain no more there than their events cost.
 //
 // Event record (half = half of a record's bits): the high half's top bit is
 // set (a final record's sizes are below 2^(half - 1) on both sides in step
@@ -2146,9 +2152,14 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 // set when the closed cluster is on the bond's u side), set for a join (high
 // half: the other open node's id).
 // ---------------------------------------------------------------------------
-#define TILE_SIDE 64u
+#ifndef TILE_ROWS
+#define TILE_ROWS 64u
+#define TILE_COLS 64u
+#endif
 #define TILE_MAX_LENGTH 2048u
-#define TILE_CLAIM_BITS 10
+#ifndef TILE_CLAIM_BITS
+#define TILE_CLAIM_BITS 9
+#endif
 #define TILE_CLAIM_SLOTS (1u << TILE_CLAIM_BITS)
 #define TILE_SCATTER_BLOCKS 1024u // workgroups tile_scatter wants
 #define TILE_GROUPS 8u   // groups of 64 steps a wave of tile_scatter takes at once
@@ -2378,13 +2389,17 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(
                 at[i] = b.k | ((before + rank) << 12);
                 if (rank == 0u)
                     my[b.k] = before + (uint32_t)__popcll(peers);
-            } else if (ok) {
+            }
+            RecT ev = 0;
+            if (ok && b.cross) {
                 const uint32_t hh = g.rows(b.tr);
                 const uint32_t iu = b.k * g.per + g.border(b.lr, b.lc, hh);
                 const uint32_t kv = b.down ? b.k + g.KW : b.k + 1u;
                 const uint32_t iv = kv * g.per + (b.down ? b.lc : g.border(b.lr, 0u, hh));
-                rec[t] = EventBits<RecT>::join(iu, iv);
+                ev = EventBits<RecT>::join(iu, iv);
             }
+            if (t < end)
+                rec[t] = ev;
             ent[i] = TileEntry<ENT>::make(t, b.lr * g.w + b.lc, b.down);
         }
         const uint32_t tn = t0 + 256u * TILE_GROUPS;
@@ -2456,30 +2471,23 @@ __global__ __launch_bounds__(64) void tile_sweep_kernel(
         claims[i] = 0u;
     __syncthreads();
 
-    // list entries two batches ahead, the codes of the next batch's
-    // endpoints one batch ahead (a parent read early is still an ancestor)
-    ENT e0 = lane < n ? list[lane] : (ENT)0;
-    ENT e1 = 64u + lane < n ? list[64u + lane] : (ENT)0;
+    // One batch: the bonds `cur`, with the codes of the next batch's
+    // endpoints (`next`) read before its merges (a parent read early is still
+    // an ancestor).
     uint32_t hint_u = TILE_OPEN, hint_v = TILE_OPEN, tag = 0, span_at = PC_NO_SPAN;
-    for (uint32_t base = 0; base < n; base += 64u) {
+    auto batch = [&](ENT cur, ENT next, bool active) __attribute__((always_inline)) {
         uint32_t t, x, y, down;
-        TileEntry<ENT>::take(e0, t, x, down);
+        TileEntry<ENT>::take(cur, t, x, down);
         y = x + (down ? g.w : 1u);
-        const bool active = base + lane < n;
-        if (!active)
-            y = x = 0u;
-        e0 = e1;
-        e1 = base + 128u + lane < n ? list[base + 128u + lane] : (ENT)0;
         x = st.is_root(hint_u) ? x : hint_u;
         y = st.is_root(hint_v) ? y : hint_v;
         uint32_t cx, cy;
         find2(st, x, cx, y, cy);
         {
             uint32_t tn, un, dn;
-            TileEntry<ENT>::take(e0, tn, un, dn);
-            const bool more = base + 64u + lane < n;
-            hint_u = st.get(more ? un : 0u);
-            hint_v = st.get(more ? un + (dn ? g.w : 1u) : 0u);
+            TileEntry<ENT>::take(next, tn, un, dn);
+            hint_u = st.get(un);
+            hint_v = st.get(un + (dn ? g.w : 1u));
         }
         bool cand = active && x != y;
         RecT rec = 0;
@@ -2531,8 +2539,26 @@ __global__ __launch_bounds__(64) void tile_sweep_kernel(
                 find2(st, x, cx, y, cy);
             cand = cand && x != y;
         }
-        if (active)
+        if (active && rec != 0)   // the others are 0 since tile_scatter
             rec_out[t] = rec;
+    };
+    // Entries are loaded two batches ahead, into registers that alternate: a
+    // load in a branch, or one whose register is copied at the end of the
+    // loop, would be waited for at once, with the stores before it.  Lanes
+    // past the end read the last entry again.
+    ENT e0 = list[min(lane, n - 1u)], e1 = list[min(64u + lane, n - 1u)];
+    uint32_t base = 0;
+    for (; base + 128u <= n; base += 128u) {
+        const ENT a = e0;
+        e0 = list[min(base + 128u + lane, n - 1u)];
+        batch(a, e1, true);
+        const ENT b = e1;
+        e1 = list[min(base + 192u + lane, n - 1u)];
+        batch(b, e0, true);
+    }
+    for (; base < n; base += 64u) {
+        batch(e0, e1, base + lane < n);
+        e0 = e1;
     }
     if (lane == 0u && span_at != PC_NO_SPAN)
         atomicMin(&span_step[rl], span_at);
@@ -2554,74 +2580,140 @@ struct OpenLdsState {
     }
 };
 
-// A run's events in step order on one wavefront.  The records are scanned
-// EVENT_SCAN groups of 64 steps at a time (loaded one scan ahead), their
-// events appended to a ring in LDS, and taken from it 64 at a time (lane =
-// event) through the rounds of sweep_run: claims, independent merges and
-// star merges into the hub.  A gain's closed cluster is a root of its own
-// that no other event touches: it needs no claim and no store.
+// A run's events in step order, on one workgroup: EVENT_FINDERS wavefronts
+// scan the records and find the events' roots, a window of
+// EVENT_FINDERS * 64 * EVENT_SCAN steps ahead of the wavefront that merges
+// them (the resolver), with one barrier per window.  Each finder takes a
+// segment of the window's steps (loaded a window ahead), appends its events
+// to its list in LDS and writes the roots found beside them; a find that
+// runs beside the merges of the window before may stop at a root linked
+// meanwhile, which is still an ancestor.  The resolver takes the events 64 at
+// a time (lane = event; fewer than 64 wait for the next window) through the
+// rounds of sweep_run: claims, independent merges and star merges into the
+// hub (one wavefront for all of it: L = 1024, 1000 runs 25 ms, now 20; L =
+// 256, 200 runs 0.67 ms, now 0.51).  A gain's closed cluster is a root of its own that no other event
+// touches: it needs no claim and no store.
 #define EVENT_SCAN 4u
-#define EVENT_RING 512u
+#define EVENT_FINDERS 3u
+#define EVENT_SEGMENT (64u * EVENT_SCAN)
+#define EVENT_WINDOW (EVENT_FINDERS * EVENT_SEGMENT)
+#define EVENT_GAIN 0x80000000u
 
-template <typename RecT>
-constexpr uint32_t event_lds_words() { return CLAIM_SLOTS + EVENT_RING * (1u + sizeof(RecT) / 4u); }
+// LDS: the claim table, then per event of two windows and of the waiting
+// ones its step, its first root, and its second root or (EVENT_GAIN set) the
+// closed cluster: order << 30 | sides << 28 | size; the lists' lengths.
+struct EventLds {
+    uint32_t claims[CLAIM_SLOTS];
+    uint32_t t[2u * EVENT_WINDOW + 64u], a[2u * EVENT_WINDOW + 64u], b[2u * EVENT_WINDOW + 64u];
+    uint32_t count[2u * EVENT_FINDERS + 2u];
+};
 
 template <class St, typename RecT>
 __device__ __forceinline__ void event_run(const St &st, uint32_t M, RecT *rec_io,
-                                          uint32_t *claims, RecT *ring, uint32_t *ring_t,
-                                          uint32_t *span_step)
+                                          EventLds &ev, uint32_t *span_step)
 {
-    const uint32_t lane = threadIdx.x;
+    const uint32_t lane = threadIdx.x & 63u, wave = uniform(threadIdx.x >> 6);
     constexpr uint32_t TOP = EventBits<RecT>::top;
-    uint32_t span_at = *span_step, tag = 0;
-    uint32_t head = 0, count = 0, pos = 0;
+    uint32_t *const claims = ev.claims;
+    const uint32_t windows = (M + EVENT_WINDOW - 1u) / EVENT_WINDOW;
+
+    // a finder's window w: the segment's events into half w & 1 of the lists
+    const uint32_t seg = wave ? (wave - 1u) * EVENT_SEGMENT : 0u;
     RecT ahead[EVENT_SCAN];
+    auto load = [&](uint32_t w) {
 #pragma unroll
-    for (uint32_t i = 0; i < EVENT_SCAN; ++i)
-        ahead[i] = i * 64u + lane < M ? rec_io[i * 64u + lane] : (RecT)0;
-    for (;;) {
-        while (count < 64u && pos < M) {
-            RecT cur[EVENT_SCAN];
-            const uint32_t next = pos + 64u * EVENT_SCAN;
+        for (uint32_t i = 0; i < EVENT_SCAN; ++i)
+            ahead[i] = rec_io[min(w * EVENT_WINDOW + seg + i * 64u + lane, M - 1u)];
+    };
+    auto find_window = [&](uint32_t w) {
+        RecT cur[EVENT_SCAN];
 #pragma unroll
-            for (uint32_t i = 0; i < EVENT_SCAN; ++i) {
-                cur[i] = ahead[i];
-                ahead[i] = next + i * 64u + lane < M ? rec_io[next + i * 64u + lane] : (RecT)0;
+        for (uint32_t i = 0; i < EVENT_SCAN; ++i)
+            cur[i] = ahead[i];
+        load(w + 1u);
+        const uint32_t at = (w & 1u) * EVENT_WINDOW + seg, t0 = w * EVENT_WINDOW + seg;
+        uint32_t n = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < EVENT_SCAN; ++i) {
+            const uint32_t t = t0 + i * 64u + lane;
+            const bool is = EventBits<RecT>::is_event(cur[i]) && t < M;
+            const uint64_t m = __ballot(is);
+            if (is) {
+                uint32_t lo, hi;
+                unpack_record(cur[i], lo, hi);
+                const uint32_t p = at + n + lanes_below(m);
+                ev.t[p] = t;
+                ev.a[p] = lo & (TOP - 1u);
+                ev.b[p] = (lo & TOP) ? hi & (TOP - 1u)
+                                     : EVENT_GAIN | ((hi & 0x4000u) << 16) |
+                                           ((hi & 0x3000u) << 16) | (hi & 0xFFFu);
             }
-#pragma unroll
-            for (uint32_t i = 0; i < EVENT_SCAN; ++i) {
-                const bool is = EventBits<RecT>::is_event(cur[i]);
-                const uint64_t b = __ballot(is);
-                if (is) {
-                    const uint32_t p = (head + count + lanes_below(b)) & (EVENT_RING - 1u);
-                    ring[p] = cur[i];
-                    ring_t[p] = pos + i * 64u + lane;
-                }
-                count += (uint32_t)__popcll(b);
-            }
-            pos = next;
+            n += (uint32_t)__popcll(m);
         }
-        if (!count)
-            break;
-        const uint32_t n = min(count, 64u);
+        if (lane == 0u)
+            ev.count[(w & 1u) * EVENT_FINDERS + wave - 1u] = n;
+        for (uint32_t i = lane; i < n; i += 64u) {
+            const uint32_t b = ev.b[at + i];
+            uint32_t x = ev.a[at + i], y = (b & EVENT_GAIN) ? x : b, cx, cy;
+            find2(st, x, cx, y, cy);
+            ev.a[at + i] = x;
+            if (!(b & EVENT_GAIN))
+                ev.b[at + i] = y;
+        }
+    };
+
+    uint32_t span_at = *span_step, tag = 0, waiting = 0;
+    if (wave) {
+        load(0u);
+        find_window(0u);
+    }
+    __syncthreads();
+    for (uint32_t w = 0; w < windows; ++w) {
+        if (wave) {
+            if (w + 1u < windows)
+                find_window(w + 1u);
+            st.sync();
+            __syncthreads();
+            continue;
+        }
+        uint32_t len[EVENT_FINDERS], total = waiting, done = 0;
+#pragma unroll
+        for (uint32_t f = 0; f < EVENT_FINDERS; ++f) {
+            len[f] = uniform(ev.count[(w & 1u) * EVENT_FINDERS + f]);
+            total += len[f];
+        }
+        // place of event i: the waiting ones, then the segments' lists
+        auto place = [&](uint32_t i) {
+            if (i < waiting)
+                return 2u * EVENT_WINDOW + i;
+            uint32_t j = i - waiting, p = (w & 1u) * EVENT_WINDOW;
+#pragma unroll
+            for (uint32_t f = 0; f + 1u < EVENT_FINDERS; ++f) {
+                const bool past = j >= len[f];
+                // the rest of the list, then the next segment
+                p += past ? EVENT_SEGMENT : 0u;
+                j -= past ? len[f] : 0u;
+                if (!past)
+                    break;
+            }
+            return p + j;
+        };
+        const bool last = w + 1u == windows;
+        while (total - done >= 64u || (last && done < total)) {
+        const uint32_t n = min(total - done, 64u);
         const bool active = lane < n;
-        const uint32_t slot = (head + lane) & (EVENT_RING - 1u);
-        __syncthreads();
-        const RecT ev = active ? ring[slot] : (RecT)0;
-        const uint32_t t = active ? ring_t[slot] : 0u;
-        head += n;
-        count -= n;
-        uint32_t lo, hi;
-        unpack_record(ev, lo, hi);
-        const bool gain = active && !(lo & TOP);
-        const bool swap = gain && (hi & 0x4000u);   // the closed cluster is on u's side
-        uint32_t ru = active ? lo & (TOP - 1u) : 0u;
-        uint32_t rv = active && !gain ? hi & (TOP - 1u) : ru;
+        const uint32_t slot = place(done + min(lane, n - 1u));
+        done += n;
+        const uint32_t t = ev.t[slot], eb = ev.b[slot];
+        const bool gain = active && (eb & EVENT_GAIN);
+        const bool swap = gain && (eb & 0x40000000u);   // the closed cluster is on u's side
+        uint32_t ru = ev.a[slot];
+        uint32_t rv = (eb & EVENT_GAIN) ? ru : eb;
         uint32_t cu, cv;
         find2(st, ru, cu, rv, cv);
         if (gain) {
             rv = 0xFFFFFFFFu;
-            cv = st.root(hi & 0xFFFu, (hi >> 12) & 3u);
+            cv = st.root(eb & 0xFFFu, (eb >> 28) & 3u);
         }
         bool cand = active && ru != rv;
         RecT rec = 0;
@@ -2718,40 +2810,49 @@ __device__ __forceinline__ void event_run(const St &st, uint32_t M, RecT *rec_io
         }
         if (active)
             rec_io[t] = rec;
+        }
+        // fewer than a batch are left: they wait in front of the next window
+        const uint32_t left = total - done;
+        if (lane < left) {
+            const uint32_t slot = place(done + lane);
+            const uint32_t t = ev.t[slot], a = ev.a[slot], b = ev.b[slot];
+            ev.t[2u * EVENT_WINDOW + lane] = t;
+            ev.a[2u * EVENT_WINDOW + lane] = a;
+            ev.b[2u * EVENT_WINDOW + lane] = b;
+        }
+        waiting = left;
+        st.sync();
+        __syncthreads();
     }
-    if (lane == 0u)
+    if (threadIdx.x == 0u)
         *span_step = span_at;
 }
 
 // Codes in LDS (LDS_STATE) or in the run's slot of `states`; both start from
 // `open` (tile_init_kernel).
 template <typename RecT, bool LDS_STATE>
-__global__ __launch_bounds__(64) void event_sweep_kernel(
+__global__ __launch_bounds__(64 * (1 + EVENT_FINDERS)) void event_sweep_kernel(
     uint32_t nodes, uint32_t M, const uint32_t *__restrict__ open,
     uint32_t *__restrict__ states, RecT *__restrict__ records, int64_t rec_stride,
     uint32_t *__restrict__ span_step, const uint32_t *__restrict__ odd)
 {
-    extern __shared__ __align__(16) uint32_t event_lds[];
+    extern __shared__ uint32_t event_codes[];
+    __shared__ EventLds ev;
+    constexpr uint32_t T = 64u * (1u + EVENT_FINDERS);
     if (odd[blockIdx.x])
         return;
-    uint32_t *claims = event_lds, *ring_t = event_lds + CLAIM_SLOTS;
-    RecT *ring = (RecT *)(ring_t + EVENT_RING);
-    const uint32_t lane = threadIdx.x;
     RecT *rec = records + (int64_t)blockIdx.x * rec_stride;
-    uint32_t *code = LDS_STATE ? event_lds + event_lds_words<RecT>()
-                               : states + (size_t)blockIdx.x * nodes;
-    for (uint32_t i = lane; i < CLAIM_SLOTS; i += 64u)
-        claims[i] = 0u;
-    for (uint32_t i = lane; i < nodes; i += 64u)
+    uint32_t *code = LDS_STATE ? event_codes : states + (size_t)blockIdx.x * nodes;
+    for (uint32_t i = threadIdx.x; i < CLAIM_SLOTS; i += T)
+        ev.claims[i] = 0u;
+    for (uint32_t i = threadIdx.x; i < nodes; i += T)
         code[i] = open[i];
     __threadfence_block();
     __syncthreads();
     if constexpr (LDS_STATE)
-        event_run<OpenLdsState, RecT>(OpenLdsState{code}, M, rec, claims, ring, ring_t,
-                                      span_step + blockIdx.x);
+        event_run<OpenLdsState, RecT>(OpenLdsState{code}, M, rec, ev, span_step + blockIdx.x);
     else
-        event_run<GlobalState, RecT>(GlobalState{code}, M, rec, claims, ring, ring_t,
-                                     span_step + blockIdx.x);
+        event_run<GlobalState, RecT>(GlobalState{code}, M, rec, ev, span_step + blockIdx.x);
 }
 
 // Running per-run state (after some number of bonds).
@@ -4632,8 +4733,10 @@ static bool tile_geo(uint32_t length, bool tiled, TileGeo &g)
         return false;
     g.lat = lattice_edges(length, tiled);
     g.L = length;
-    g.KH = g.KW = (length + TILE_SIDE - 1u) / TILE_SIDE;
-    g.h = g.w = (length + g.KH - 1u) / g.KH;
+    g.KH = (length + TILE_ROWS - 1u) / TILE_ROWS;
+    g.KW = (length + TILE_COLS - 1u) / TILE_COLS;
+    g.h = (length + g.KH - 1u) / g.KH;
+    g.w = (length + g.KW - 1u) / g.KW;
     g.K = g.KH * g.KW;
     g.per = 2u * g.w + 2u * (g.h - 2u);
     g.mh = (uint32_t)(((1ull << 32) + g.h - 1u) / g.h);
@@ -4650,7 +4753,8 @@ struct TilePlan {
     bool lds;       // the open nodes' codes fit LDS
     bool short_entries;
 };
-#define TILE_OPEN_LDS_NODES 18432u // 72 KiB of codes: two runs per CU
+#define TILE_OPEN_LDS_NODES 10240u  // 40 KiB of codes: two runs per CU
+#define TILE_OPEN_LDS_MOST 32768u   // 128 KiB: one run per CU
 
 static TilePlan tile_plan(const TileGeo &g, uint32_t num_runs, uint32_t slab)
 {
@@ -4659,7 +4763,9 @@ static TilePlan tile_plan(const TileGeo &g, uint32_t num_runs, uint32_t slab)
     const uint64_t M = 2ull * g.L * (g.L - 1u);
     p.nodes = g.K * g.per;
     p.slab = slab;
-    p.lds = p.nodes <= TILE_OPEN_LDS_NODES;
+    // in LDS also where it holds one run per CU, if the runs are that few
+    p.lds = p.nodes <= TILE_OPEN_LDS_NODES ||
+            (p.nodes <= TILE_OPEN_LDS_MOST && num_runs <= 256u);
     p.short_entries = M <= TILE_SHORT_STEPS;
     p.init = 0;
     p.open = up((uint64_t)g.K * g.init_stride * 2u);
@@ -4743,12 +4849,12 @@ static int tile_sweep_launch(const TileGeo &g, const TilePlan &p,
             g, rn, lists, list_stride, init, rec, rec_stride, d_span_step + r0, odd + r0);
         PC_LAUNCH_CHECK("tile_sweep_kernel");
     }
-    const size_t ring = event_lds_words<RecT>() * 4u;
+    const uint32_t threads = 64u * (1u + EVENT_FINDERS);
     if (p.lds)
-        event_sweep_kernel<RecT, true><<<num_runs, 64, ring + p.nodes * 4u, s>>>(
+        event_sweep_kernel<RecT, true><<<num_runs, threads, p.nodes * 4u, s>>>(
             p.nodes, M, open, nullptr, d_records, rec_stride, d_span_step, odd);
     else
-        event_sweep_kernel<RecT, false><<<num_runs, 64, ring, s>>>(
+        event_sweep_kernel<RecT, false><<<num_runs, threads, 0, s>>>(
             p.nodes, M, open, (uint32_t *)(ws + p.states), d_records, rec_stride,
             d_span_step, odd);
     PC_LAUNCH_CHECK("event_sweep_kernel");

@@ -428,12 +428,14 @@ def _same_sweep(a, b, chunks=True):
 
 
 @pytest.mark.parametrize('length,runs', [(129, 5), (136, 9), (181, 40), (192, 3), (255, 2),
-                                         (256, 17), (257, 8), (512, 2), (513, 2), (700, 1)])
+                                         (256, 17), (257, 8), (512, 2), (513, 2), (700, 1),
+                                         (1000, 1), (400, 300)])
 def test_tiled_lattice_sweep_equals_untiled(gpu, length, runs):
     """The tiled sweep's records, span steps and chunk states equal those of
     the sweep with every node's code in HBM: whole and ragged tiles, 32- and
     64-bit records (from 257), 32- and 64-bit list entries (from 513), open
-    nodes in LDS and in HBM (700), one workgroup per run or several."""
+    nodes in LDS (a run or several per CU) and in HBM (1000; 400 for more
+    than 256 runs), one workgroup per run or several."""
     eng = BondEngine(_graph.square_lattice(length))
     perm = eng.device_permutations(17, runs)
     _same_sweep(*_tiled_and_untiled(eng, perm))
