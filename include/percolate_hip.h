@@ -193,6 +193,21 @@ int pc_permute_randomstate(const uint32_t *d_seeds, uint32_t num_runs,
                            uint32_t num_edges, int32_t *d_perm,
                            int64_t perm_stride, void *stream);
 
+/*
+ * The same permutations with a workspace (8-byte aligned), for runs of more
+ * than 32768 and at most 2^21 edges: the swaps applied in two phases there
+ * too, position buckets of a run in turn from the top, one workgroup per
+ * run.  pc_permute_randomstate_workspace_size gives the bytes (0 for other
+ * sizes); with less, fewer runs are taken at a time, and without room for
+ * one, as for other sizes, the call is pc_permute_randomstate's.
+ */
+int pc_permute_randomstate_ws(const uint32_t *d_seeds, uint32_t num_runs,
+                              uint32_t num_edges, int32_t *d_perm,
+                              int64_t perm_stride, void *d_workspace,
+                              uint64_t workspace_bytes, void *stream);
+int pc_permute_randomstate_workspace_size(uint32_t num_edges, uint32_t num_runs,
+                                          uint64_t *bytes);
+
 /* Device workspace bytes pc_sweep needs (0 when the state is in LDS). */
 int pc_sweep_workspace_size(uint32_t num_nodes, uint32_t num_runs,
                             uint32_t state_mode, uint64_t *bytes);

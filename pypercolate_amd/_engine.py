@@ -155,9 +155,16 @@ class BondEngine(object):
         if out is None:
             out = torch.empty((n, max(self.M, 1)), dtype=torch.int32,
                               device=self.device)
-        nat.check(self.lib.pc_permute_randomstate(
+        b = ctypes.c_uint64(0)
+        nat.check(self.lib.pc_permute_randomstate_workspace_size(
+            self.M, n, ctypes.byref(b)), 'pc_permute_randomstate_workspace_size')
+        wb = int(b.value)
+        workspace = (torch.empty((wb,), dtype=torch.uint8, device=self.device)
+                     if wb else None)
+        nat.check(self.lib.pc_permute_randomstate_ws(
             nat.ptr(d_seeds), n, self.M, nat.ptr(out), max(self.M, 1),
-            nat.stream_handle(torch)), 'pc_permute_randomstate')
+            nat.ptr(workspace), wb, nat.stream_handle(torch)),
+            'pc_permute_randomstate_ws')
         return out
 
     # -- sweep ------------------------------------------------------------

@@ -977,7 +977,26 @@ __global__ __launch_bounds__(64) void permute_randomstate_kernel(
 // the result at i >= 1 is V(s) for the smallest step s > i with k_s = k_i,
 // or k_i itself without one, and the result at 0 is V(0).
 #define RS_APPLY_MAX 32768u
-#define RS_APPLY_T 1024u
+
+// The first words of MT19937 for a seed (init_genrand), by one wavefront: the
+// chain of 624 dependent steps runs on the scalar unit, a lane of a register
+// takes each word, and 64 words are stored at a time.
+__device__ __forceinline__ void mt_init(uint32_t seed, uint32_t *mt)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t x = uniform(seed);
+#pragma nounroll
+    for (uint32_t b = 0; b < MT_N; b += 64u) {
+        uint32_t v = 0;
+#pragma unroll
+        for (uint32_t l = 0; l < 64u; ++l) {
+            asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(x), "i"(l));
+            x = 1812433253u * (x ^ (x >> 30)) + (b + l + 1u);
+        }
+        if (b + lane < MT_N)
+            mt[b + lane] = v;
+    }
+}
 
 // Phase one.  The wave tempers 64 state words at a time (lane l holds word
 // base + l) and settles the whole block at once: for steps i, i-1, ... under
@@ -988,33 +1007,11 @@ __global__ __launch_bounds__(64) void permute_randomstate_kernel(
 // lanes below them.  The mask holds for c = i - m/2 more steps; when the
 // block accepts c words or more, the lanes after the c-th accepted one are
 // settled again under the next mask.
-__global__ __launch_bounds__(64) void randomstate_targets_kernel(
-    const uint32_t *__restrict__ seeds, uint32_t n, int32_t *__restrict__ perm,
-    int64_t stride)
+// mt_settle takes the words of one twist so; it returns the step reached.
+__device__ __forceinline__ uint32_t mt_settle(const uint32_t *mt, uint32_t i, int32_t *out)
 {
-    __shared__ uint32_t mt[MT_N];
-    const uint32_t lane = threadIdx.x;
-    int32_t *out = perm + (int64_t)blockIdx.x * stride;
-    if (lane == 0) {
-        uint32_t x = seeds[blockIdx.x];
-        mt[0] = x;
-        for (uint32_t i = 1; i < MT_N; ++i) {
-            x = 1812433253u * (x ^ (x >> 30)) + i;
-            mt[i] = x;
-        }
-        if (n)
-            out[0] = 0;
-    }
-    __syncthreads();
-    uint32_t pos = MT_N;
-    uint32_t i = n ? n - 1u : 0u;
-    while (i >= 1u) {
-        if (pos == MT_N) {
-            __syncthreads();
-            mt_twist(mt);
-            __syncthreads();
-            pos = 0;
-        }
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t pos = 0; pos < MT_N && i >= 1u;) {
         const uint32_t nw = min(64u, MT_N - pos);
         const uint32_t w = lane < nw ? mt_temper(mt[pos + lane]) : 0u;
         uint32_t l0 = 0;
@@ -1054,6 +1051,127 @@ __global__ __launch_bounds__(64) void randomstate_targets_kernel(
         } while (l0 < nw && i >= 1u);
         pos += nw;
     }
+    return i;
+}
+
+__global__ __launch_bounds__(64) void randomstate_targets_kernel(
+    const uint32_t *__restrict__ seeds, uint32_t n, int32_t *__restrict__ perm,
+    int64_t stride)
+{
+    __shared__ uint32_t mt[MT_N];
+    int32_t *out = perm + (int64_t)blockIdx.x * stride;
+    mt_init(seeds[blockIdx.x], mt);
+    if (threadIdx.x == 0u && n)
+        out[0] = 0;
+    uint32_t i = n ? n - 1u : 0u;
+    while (i >= 1u) {
+        __syncthreads();
+        mt_twist(mt);
+        __syncthreads();
+        i = mt_settle(mt, i, out);
+    }
+}
+
+// Phase one by a workgroup of 640 threads, thread t with state word t: a
+// twist is three steps of all threads (two barriers), and the 624 words are
+// settled together where the mask holds for all of them.  The word at place t
+// serves step i - (accepted words below t), of which there are at most t: it
+// is accepted for sure when x + t <= i, rejected for sure when x > i, and the
+// few in between (about 624^2 / 2 of every m + 1 words' worth) are decided in
+// order by the first wavefront.  Words around a change of mask, and the last
+// RST_SMALL steps, go through the blocks of 64 above on that wavefront.
+#define RST_T 640u
+#define RST_SMALL 8192u
+
+__global__ __launch_bounds__(RST_T) void randomstate_targets_wide_kernel(
+    const uint32_t *__restrict__ seeds, uint32_t n, int32_t *__restrict__ perm,
+    int64_t stride)
+{
+    constexpr uint32_t WAVES = RST_T / 64u, OUT = MT_N - MT_SHIFT;
+    __shared__ uint32_t mt[2][MT_N];
+    __shared__ uint32_t xs[RST_T];
+    __shared__ uint64_t accepted[WAVES], open[WAVES];
+    __shared__ uint32_t before[WAVES + 1u];
+    const uint32_t t = threadIdx.x, wave = uniform(t >> 6);
+    int32_t *out = perm + (int64_t)blockIdx.x * stride;
+    if (wave == 0u)
+        mt_init(seeds[blockIdx.x], mt[0]);
+    if (t == 0u && n)
+        out[0] = 0;
+    __syncthreads();
+    uint32_t i = n ? n - 1u : 0u;
+    for (uint32_t g = 0; i >= 1u; ++g) {
+        const uint32_t *old = mt[g & 1u];
+        uint32_t *now = mt[(g + 1u) & 1u];
+        uint32_t a = 0, b = 0, y = 0;
+        if (t < MT_N) {
+            a = old[t];
+            b = old[t + 1u < MT_N ? t + 1u : 0u];
+        }
+        if (t < OUT)
+            now[t] = y = mt_next_word(a, b, old[t + MT_SHIFT]);
+        __syncthreads();
+        if (t >= OUT && t < 2u * OUT)
+            now[t] = y = mt_next_word(a, b, now[t - OUT]);
+        __syncthreads();
+        if (t >= 2u * OUT && t < MT_N)
+            now[t] = y = mt_next_word(a, t + 1u < MT_N ? b : now[0], now[t - OUT]);
+        const uint32_t m = 0xFFFFFFFFu >> __builtin_clz(i);
+        if (i >= RST_SMALL && i - (m >> 1) > MT_N) {
+            const uint32_t x = mt_temper(y) & m;
+            const bool in = t < MT_N;
+            const uint64_t acc = __ballot(in && x + t <= i);
+            const uint64_t amb = __ballot(in && x <= i && x + t > i);
+            xs[t] = x;
+            if ((t & 63u) == 0u) {
+                accepted[wave] = acc;
+                open[wave] = amb;
+            }
+            __syncthreads();
+            if (wave == 0u) {
+                const uint32_t l = min(t, WAVES - 1u);
+                const uint64_t all = accepted[l], some = open[l];
+                uint32_t base = 0, at = 0;
+                uint64_t fin = 0;
+#pragma unroll
+                for (uint32_t w = 0; w < WAVES; ++w) {
+                    uint64_t ok = read_lane(all, w), left = read_lane(some, w);
+                    while (left) {
+                        const uint32_t z = (uint32_t)__builtin_ctzll(left);
+                        const uint32_t below = (uint32_t)__popcll(ok & ((1ull << z) - 1ull));
+                        if (uniform(xs[w * 64u + z]) + base + below <= i)
+                            ok |= 1ull << z;
+                        left &= left - 1ull;
+                    }
+                    if (t == w) {
+                        fin = ok;
+                        at = base;
+                    }
+                    base += (uint32_t)__popcll(ok);
+                }
+                if (t < WAVES) {
+                    accepted[t] = fin;
+                    before[t] = at;
+                }
+                if (t == 0u)
+                    before[WAVES] = base;
+            }
+            __syncthreads();
+            const uint64_t fin = accepted[wave];
+            if ((fin >> (t & 63u)) & 1ull)
+                out[i - before[wave] - lanes_below(fin)] = (int32_t)x;
+            i -= uniform(before[WAVES]);
+        } else {
+            __syncthreads();
+            if (wave == 0u) {
+                const uint32_t r = mt_settle(now, i, out);
+                if (t == 0u)
+                    before[WAVES] = r;
+            }
+            __syncthreads();
+            i = uniform(before[WAVES]);
+        }
+    }
 }
 
 // Smallest of the list entries ent[b..e) above thr, or 0xFFFF (entries are
@@ -1092,23 +1210,22 @@ __device__ __forceinline__ uint32_t opaque_v(uint32_t x)
     return x;
 }
 
-// Phase two, one workgroup of RS_APPLY_T threads per run of n <= RS_APPLY_MAX
-// edges, in place over the targets.  LDS holds 16-bit list cursors of the
+// Phase two, one workgroup of T threads per run of n <= T * PER edges, in place over the targets.  LDS holds 16-bit list cursors of the
 // positions in pairs and the lists of steps per target position (a counting
 // sort: counts, exclusive scan, placement; unordered within a list); every
-// thread owns indices j = tid + q * RS_APPLY_T and scans the list of k_j
+// thread owns indices j = tid + q * T (q < PER) and scans the list of k_j
 // once, for the smallest step above j and for whether j is the list's
 // smallest step (which then knows F(k_j)).  The list area is then reused for
 // V, which pointer jumping (V(p) <- V(V(p)) until nothing changes, over
 // position pairs) takes to the chain roots.  The loads of independent items
 // are issued together before any is waited for.  Dynamic LDS:
 // rs_apply_lds_bytes(n).
-__global__ __launch_bounds__(RS_APPLY_T) void randomstate_apply_kernel(
+template <uint32_t T, uint32_t PER>
+__global__ __launch_bounds__(T) void randomstate_apply_kernel(
     uint32_t n, int32_t *__restrict__ perm, int64_t stride)
 {
-    constexpr uint32_t T = RS_APPLY_T, PER = RS_APPLY_MAX / RS_APPLY_T;
     constexpr uint32_t PAIRS = PER / 2u, WAVES = T / 64u, LOOKUP = 0x8000u;
-    constexpr uint32_t GROUP = 4u;
+    constexpr uint32_t GROUP = PER < 4u ? PER : 4u;
     extern __shared__ uint32_t rsd[];
     const uint32_t words = (n + 2u) / 2u;   // 16-bit cursors of positions 0..n
     uint32_t *cur = rsd;
@@ -1287,6 +1404,296 @@ __global__ __launch_bounds__(RS_APPLY_T) void randomstate_apply_kernel(
             const uint32_t j = tf + (g + u) * T;
             if (j < n)
                 row[j] = (int32_t)val[u];
+        }
+    }
+}
+
+// The second phase for runs of more than RS_APPLY_MAX edges, which one
+// workgroup's LDS does not hold: positions are cut into buckets of at most
+// RSB_CAP positions and about as many steps targeting them, and one workgroup
+// per run takes the buckets from the top position down.  The steps of a run
+// are first grouped by the bucket of their target in the workspace; a bucket
+// is then the whole of phase two for its positions: the lists of its
+// positions (a counting sort in LDS), each step's successor and each
+// position's F from the lists, and V.  F(p) > p is a position of the same
+// bucket, resolved by pointer jumping in LDS, or of one done before, whose V
+// is in the workspace; so is the position whose V is a step's result.  The
+// result goes to the row, whose targets have all been read by then.
+// Bound by the LDS and barrier latencies of a bucket (about 20 us of a
+// workgroup each, 33 buckets at L = 256): 200 runs of L = 256 take 0.73 ms,
+// where the swaps walked in sequence took 37 ms; 512 threads instead of 1024
+// 0.87 ms.
+//
+// Buckets: the steps i >= x target a position below x with probability
+// x / (i + 1), so x + x ln(n / x) targets below x are expected; a bucket
+// spans RSB_WIDTH expected steps, or RSB_WIDTH positions near the top, where
+// fewer steps than positions remain.  Its bounds are multiples of a cell of
+// 2^shift positions (at most RSB_CELLS cells); the first cell holds up to
+// 2560 steps (2^21 edges), so at most 7760 steps are expected, and more than
+// RSB_CAP are 4.9 standard deviations off; the run is then walked in sequence.
+#define RSB_T 1024u
+#define RSB_CAP 8192u
+#define RSB_WIDTH 5200u
+#define RSB_CELLS 8192u
+#define RSB_BUCKETS 1024u
+#define RSB_MAX (1u << 21)
+#define RSB_SHORT (1u << 19)   // up to so many edges an entry has 32 bits
+
+struct RsbTable {
+    uint32_t nb;
+    uint32_t bounds[RSB_BUCKETS + 1u];
+    uint16_t cell[RSB_CELLS];
+};
+
+__device__ __forceinline__ uint32_t rsb_bucket(double x, double n)
+{
+    // expected steps below x, then positions, past the point n / e where a
+    // position expects one step
+    const double e = n * 0.36787944117144233, at = min(x, e);
+    const double g = at > 0.0 ? at + at * log(n / at) : 0.0;
+    return (uint32_t)((g + max(x - e, 0.0)) / (double)RSB_WIDTH);
+}
+
+__global__ __launch_bounds__(256) void randomstate_table_kernel(uint32_t n, uint32_t shift,
+                                                                RsbTable *__restrict__ t)
+{
+    const uint32_t cells = ((n - 1u) >> shift) + 1u;
+    for (uint32_t c = blockIdx.x * 256u + threadIdx.x; c < cells; c += gridDim.x * 256u) {
+        const uint32_t b = rsb_bucket((double)(c << shift), (double)n);
+        const uint32_t before = c ? rsb_bucket((double)((c - 1u) << shift), (double)n) : 0u;
+        t->cell[c] = (uint16_t)b;
+        if (c == 0u)
+            t->bounds[0] = 0u;
+        for (uint32_t j = before + 1u; j <= b; ++j)
+            t->bounds[j] = c << shift;
+        if (c + 1u == cells) {
+            t->nb = b + 1u;
+            t->bounds[b + 1u] = n;
+        }
+    }
+}
+
+// Smallest of the list entries ent[b..e) above thr, or all ones, and whether
+// an entry below thr exists.
+__device__ __forceinline__ uint32_t rsb_list_scan(const uint32_t *ent, uint32_t b,
+                                                  uint32_t e, uint32_t thr, bool &below)
+{
+    uint32_t best = 0xFFFFFFFFu;
+    bool lo = false;
+    for (uint32_t a = b; a < e; a += 2u) {
+        const uint32_t x = ent[a], y = ent[min(a + 1u, e - 1u)];
+        best = x > thr ? min(best, x) : best;
+        best = y > thr ? min(best, y) : best;
+        lo |= x < thr || y < thr;
+    }
+    below = lo;
+    return best;
+}
+
+template <typename ENT>
+__global__ __launch_bounds__(RSB_T) void randomstate_buckets_kernel(
+    uint32_t n, uint32_t runs, uint32_t shift, const RsbTable *__restrict__ table,
+    ENT *__restrict__ entries, uint32_t *values, int32_t *perm, int64_t stride)
+{
+    constexpr uint32_t T = RSB_T, PER = RSB_CAP / T, WAVES = T / 64u, DONE = 0x80000000u;
+    constexpr uint32_t STEP_BITS = sizeof(ENT) == 4u ? 19u : 32u;
+    __shared__ uint16_t cell[RSB_CELLS];
+    __shared__ uint32_t bounds[RSB_BUCKETS + 1u], start[RSB_BUCKETS + 1u], next[RSB_BUCKETS];
+    __shared__ uint32_t cur[RSB_CAP / 2u + 1u];   // 16-bit list cursors
+    __shared__ uint32_t list[RSB_CAP];            // the lists, then V
+    __shared__ uint32_t wsum[WAVES];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t nb = table->nb, cells = ((n - 1u) >> shift) + 1u;
+    for (uint32_t c = tid; c < cells; c += T)
+        cell[c] = table->cell[c];
+    for (uint32_t b = tid; b <= nb; b += T)
+        bounds[b] = table->bounds[b];
+    ENT *ent = entries + (size_t)blockIdx.x * n;
+    uint32_t *V = values + (size_t)blockIdx.x * n;
+    for (uint32_t run = blockIdx.x; run < runs; run += gridDim.x) {
+        int32_t *row = perm + (int64_t)run * stride;
+        for (uint32_t b = tid; b < nb; b += T)
+            next[b] = 0u;
+        __syncthreads();
+        // steps per bucket
+        for (uint32_t i0 = 0; i0 < n; i0 += 8u * T) {
+            uint32_t k[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u)
+                k[u] = (uint32_t)row[min(i0 + u * T + tid, n - 1u)];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u) {
+                const uint32_t i = i0 + u * T + tid;
+                if (i >= 1u && i < n)
+                    atomicAdd(&next[cell[k[u] >> shift]], 1u);
+            }
+        }
+        __syncthreads();
+        // their first entries; a thread owns two buckets
+        static_assert(2u * T >= RSB_BUCKETS, "two buckets a thread");
+        bool over = false;
+        {
+            const uint32_t c0 = 2u * tid < nb ? next[2u * tid] : 0u;
+            const uint32_t c1 = 2u * tid + 1u < nb ? next[2u * tid + 1u] : 0u;
+            over = c0 > RSB_CAP || c1 > RSB_CAP;
+            const uint32_t inc = wave_scan_add(c0 + c1);
+            if (lane == 63u)
+                wsum[wave] = inc;
+            __syncthreads();
+            uint32_t a = inc - c0 - c1;
+            for (uint32_t w = 0; w < wave; ++w)
+                a += wsum[w];
+            if (2u * tid < nb)
+                start[2u * tid] = next[2u * tid] = a;
+            if (2u * tid + 1u < nb)
+                start[2u * tid + 1u] = next[2u * tid + 1u] = a + c0;
+            if (tid == 0u)
+                start[nb] = n - 1u;
+        }
+        if (__syncthreads_or(over)) {
+            for (uint32_t j = tid; j < n; j += T)
+                V[j] = j;
+            __threadfence_block();
+            __syncthreads();
+            if (tid == 0u)
+                for (uint32_t i = n - 1u; i >= 1u; --i) {
+                    const uint32_t k = (uint32_t)row[i], a = V[i];
+                    V[i] = V[k];
+                    V[k] = a;
+                }
+            __threadfence_block();
+            __syncthreads();
+            for (uint32_t j = tid; j < n; j += T)
+                row[j] = (int32_t)V[j];
+            __syncthreads();
+            continue;
+        }
+        // the steps grouped by bucket: step, and place of the target in it
+        for (uint32_t i0 = 0; i0 < n; i0 += 8u * T) {
+            uint32_t k[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u)
+                k[u] = (uint32_t)row[min(i0 + u * T + tid, n - 1u)];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u) {
+                const uint32_t i = i0 + u * T + tid;
+                if (i >= 1u && i < n) {
+                    const uint32_t b = cell[k[u] >> shift];
+                    ent[atomicAdd(&next[b], 1u)] = (ENT)i | ((ENT)(k[u] - bounds[b]) << STEP_BITS);
+                }
+            }
+        }
+        __threadfence_block();
+        __syncthreads();
+        for (uint32_t b = nb; b-- > 0u;) {
+            const uint32_t lo = bounds[b], hi = bounds[b + 1u], W = hi - lo;
+            const uint32_t s0 = start[b], E = start[b + 1u] - s0;
+            if (W == 0u)
+                continue;
+            const uint32_t words = (W + 1u) / 2u;
+            uint32_t step[PER], pos[PER], succ[PER], first[PER];
+#pragma unroll
+            for (uint32_t q = 0; q < PER; ++q)
+                if (q * T < E) {
+                    const ENT e = ent[s0 + min(q * T + tid, E - 1u)];
+                    step[q] = (uint32_t)(e & (ENT)((1ull << STEP_BITS) - 1u));
+                    pos[q] = (uint32_t)((uint64_t)e >> STEP_BITS);
+                }
+            for (uint32_t w = tid; w < words; w += T)
+                cur[w] = 0u;
+            __syncthreads();
+#pragma unroll
+            for (uint32_t q = 0; q < PER; ++q)
+                if (q * T + tid < E)
+                    atomicAdd(&cur[pos[q] >> 1], 1u << ((pos[q] & 1u) * 16u));
+            __syncthreads();
+            // cur[p] = first slot of position p's list; a wave scans its
+            // share of the words, 64 at a time
+            {
+                const uint32_t chunk = ((words + WAVES - 1u) / WAVES + 63u) & ~63u;
+                const uint32_t w0 = min(wave * chunk, words), w1 = min(w0 + chunk, words);
+                uint32_t tot = 0;
+                for (uint32_t w = w0 + lane; w < w1; w += 64u)
+                    tot += (cur[w] & 0xFFFFu) + (cur[w] >> 16);
+                tot = read_lane(wave_scan_add(tot), 63u);
+                if (lane == 0u)
+                    wsum[wave] = tot;
+                __syncthreads();
+                uint32_t carry = 0;
+                for (uint32_t w = 0; w < wave; ++w)
+                    carry += wsum[w];
+                for (uint32_t c = w0; c < w1; c += 64u) {
+                    const uint32_t w = c + lane;
+                    const uint32_t x = w < w1 ? cur[w] : 0u;
+                    const uint32_t pair = (x & 0xFFFFu) + (x >> 16);
+                    const uint32_t inc = wave_scan_add(pair);
+                    const uint32_t a0 = carry + inc - pair;
+                    if (w < w1)
+                        cur[w] = a0 | ((a0 + (x & 0xFFFFu)) << 16);
+                    carry += read_lane(inc, 63u);
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t q = 0; q < PER; ++q)
+                if (q * T + tid < E) {
+                    const uint32_t sh = (pos[q] & 1u) * 16u;
+                    const uint32_t at = (atomicAdd(&cur[pos[q] >> 1], 1u << sh) >> sh) & 0xFFFFu;
+                    list[at] = step[q];
+                }
+            __syncthreads();
+            // successors, and F where the step is its list's smallest (all
+            // ones: none, or not the smallest): the cursor of p is now the
+            // end of its list, and p + 1's list starts there
+            auto half = [&](uint32_t p) { return (cur[p >> 1] >> ((p & 1u) * 16u)) & 0xFFFFu; };
+#pragma unroll
+            for (uint32_t q = 0; q < PER; ++q) {
+                succ[q] = first[q] = 0xFFFFFFFFu;
+                if (q * T + tid < E) {
+                    const uint32_t p = pos[q];
+                    bool below;
+                    succ[q] = rsb_list_scan(list, p ? half(p - 1u) : 0u, half(p), step[q], below);
+                    if (!below)
+                        first[q] = step[q] > lo + p ? step[q] : succ[q];
+                }
+            }
+            __syncthreads();
+            for (uint32_t j = tid; j < W; j += T)
+                list[j] = DONE | (lo + j);
+            __syncthreads();
+#pragma unroll
+            for (uint32_t q = 0; q < PER; ++q)
+                if (first[q] != 0xFFFFFFFFu)
+                    list[pos[q]] = first[q] >= hi ? DONE | V[first[q]] : first[q] - lo;
+            // pointer jumping to the ends of the chains inside the bucket
+            for (;;) {
+                __syncthreads();
+                bool open = false;
+                for (uint32_t j = tid; j < W; j += T) {
+                    const uint32_t v = list[j];
+                    if (!(v & DONE)) {
+                        const uint32_t nv = list[v];
+                        list[j] = nv;
+                        open |= !(nv & DONE);
+                    }
+                }
+                if (!__syncthreads_or(open))
+                    break;
+            }
+            for (uint32_t j = tid; j < W; j += T)
+                V[lo + j] = list[j] & ~DONE;
+            if (b == 0u && tid == 0u)
+                row[0] = (int32_t)(list[0] & ~DONE);
+#pragma unroll
+            for (uint32_t q = 0; q < PER; ++q)
+                if (q * T + tid < E) {
+                    const uint32_t s = succ[q];
+                    row[step[q]] = (int32_t)(s == 0xFFFFFFFFu ? lo + pos[q]
+                                             : s >= hi        ? V[s]
+                                                              : list[s - lo] & ~DONE);
+                }
+            __threadfence_block();
+            __syncthreads();
         }
     }
 }
@@ -5776,6 +6183,22 @@ extern "C" int pc_run_moments(const double *d_q, uint32_t num_p,
     return PC_OK;
 }
 
+// Targets of every run: a workgroup each while two fit every CU (200 runs of
+// 130560 edges: 0.47 ms, with a wavefront each 0.98; 600 of 79600: 0.70 and
+// 0.68).
+static int rs_targets(const uint32_t *d_seeds, uint32_t num_runs, uint32_t num_edges,
+                      int32_t *d_perm, int64_t perm_stride, hipStream_t s)
+{
+    if (num_runs <= 512u)
+        randomstate_targets_wide_kernel<<<num_runs, RST_T, 0, s>>>(d_seeds, num_edges, d_perm,
+                                                                   perm_stride);
+    else
+        randomstate_targets_kernel<<<num_runs, 64, 0, s>>>(d_seeds, num_edges, d_perm,
+                                                           perm_stride);
+    PC_LAUNCH_CHECK("randomstate_targets_kernel");
+    return PC_OK;
+}
+
 extern "C" int pc_permute_randomstate(const uint32_t *d_seeds, uint32_t num_runs,
                                       uint32_t num_edges, int32_t *d_perm,
                                       int64_t perm_stride, void *stream)
@@ -5790,11 +6213,24 @@ extern "C" int pc_permute_randomstate(const uint32_t *d_seeds, uint32_t num_runs
     hipStream_t s = as_stream(stream);
     if (num_edges <= RS_APPLY_MAX) {
         // targets, then all swaps at once (in place in the output rows)
-        randomstate_targets_kernel<<<num_runs, 64, 0, s>>>(d_seeds, num_edges, d_perm,
-                                                             perm_stride);
-        PC_LAUNCH_CHECK("randomstate_targets_kernel");
-        randomstate_apply_kernel<<<num_runs, RS_APPLY_T, rs_apply_lds_bytes(num_edges), s>>>(
-            num_edges, d_perm, perm_stride);
+        const int rc = rs_targets(d_seeds, num_runs, num_edges, d_perm, perm_stride, s);
+        if (rc != PC_OK)
+            return rc;
+        const size_t lds = rs_apply_lds_bytes(num_edges);
+        // as few threads and indices per thread as hold the run: 480 edges
+        // take 27 us with the largest form
+        if (num_edges <= 512u)
+            randomstate_apply_kernel<256u, 2u><<<num_runs, 256, lds, s>>>(num_edges, d_perm,
+                                                                          perm_stride);
+        else if (num_edges <= 4096u)
+            randomstate_apply_kernel<512u, 8u><<<num_runs, 512, lds, s>>>(num_edges, d_perm,
+                                                                          perm_stride);
+        else if (num_edges <= 8192u)
+            randomstate_apply_kernel<1024u, 8u><<<num_runs, 1024, lds, s>>>(num_edges, d_perm,
+                                                                            perm_stride);
+        else
+            randomstate_apply_kernel<1024u, 32u><<<num_runs, 1024, lds, s>>>(num_edges, d_perm,
+                                                                             perm_stride);
         PC_LAUNCH_CHECK("randomstate_apply_kernel");
         return PC_OK;
     }
@@ -5807,5 +6243,64 @@ extern "C" int pc_permute_randomstate(const uint32_t *d_seeds, uint32_t num_runs
             d_seeds, num_edges, d_perm, perm_stride);
     }
     PC_LAUNCH_CHECK("permute_randomstate_kernel");
+    return PC_OK;
+}
+
+// Slots of the bucketed second phase, and its workspace: the table, then
+// per slot the entries and the values.
+#define RSB_SLOTS 512u
+static uint64_t rsb_entry_bytes(uint32_t n) { return n <= RSB_SHORT ? 4u : 8u; }
+static bool rsb_takes(uint32_t n) { return n > RS_APPLY_MAX && n <= RSB_MAX; }
+
+extern "C" int pc_permute_randomstate_workspace_size(uint32_t num_edges, uint32_t num_runs,
+                                                     uint64_t *bytes)
+{
+    g_last_error[0] = 0;
+    if (!bytes)
+        return pc_fail(PC_EINVAL, "pc_permute_randomstate_workspace_size: bytes is NULL");
+    const uint64_t slots = std::min(num_runs, RSB_SLOTS);
+    *bytes = slots && rsb_takes(num_edges)
+                 ? sizeof(RsbTable) + 512u + slots * num_edges * (4u + rsb_entry_bytes(num_edges))
+                 : 0u;
+    return PC_OK;
+}
+
+extern "C" int pc_permute_randomstate_ws(const uint32_t *d_seeds, uint32_t num_runs,
+                                         uint32_t num_edges, int32_t *d_perm,
+                                         int64_t perm_stride, void *d_workspace,
+                                         uint64_t workspace_bytes, void *stream)
+{
+    g_last_error[0] = 0;
+    if (num_runs == 0 || num_edges == 0)
+        return PC_OK;
+    if (!d_seeds || !d_perm || perm_stride < (int64_t)num_edges)
+        return pc_fail(PC_EINVAL, "pc_permute_randomstate_ws: bad buffer");
+    const uint64_t eb = rsb_entry_bytes(num_edges), per_slot = num_edges * (4u + eb);
+    const uint64_t fixed = (sizeof(RsbTable) + 511u) & ~(uint64_t)255u;
+    // without room for a run the swaps are walked in sequence
+    if (!rsb_takes(num_edges) || !d_workspace || ((uintptr_t)d_workspace & 7u) ||
+        workspace_bytes < fixed + per_slot)
+        return pc_permute_randomstate(d_seeds, num_runs, num_edges, d_perm, perm_stride, stream);
+    const uint32_t slots = (uint32_t)std::min<uint64_t>(
+        std::min(num_runs, RSB_SLOTS), (workspace_bytes - fixed) / per_slot);
+    uint32_t shift = 0;
+    while (((num_edges - 1u) >> shift) >= RSB_CELLS)
+        ++shift;
+    RsbTable *table = (RsbTable *)d_workspace;
+    char *entries = (char *)d_workspace + fixed;
+    uint32_t *values = (uint32_t *)(entries + slots * num_edges * eb);
+    hipStream_t s = as_stream(stream);
+    randomstate_table_kernel<<<32, 256, 0, s>>>(num_edges, shift, table);
+    PC_LAUNCH_CHECK("randomstate_table_kernel");
+    const int rc = rs_targets(d_seeds, num_runs, num_edges, d_perm, perm_stride, s);
+    if (rc != PC_OK)
+        return rc;
+    if (eb == 4u)
+        randomstate_buckets_kernel<uint32_t><<<slots, RSB_T, 0, s>>>(
+            num_edges, num_runs, shift, table, (uint32_t *)entries, values, d_perm, perm_stride);
+    else
+        randomstate_buckets_kernel<uint64_t><<<slots, RSB_T, 0, s>>>(
+            num_edges, num_runs, shift, table, (uint64_t *)entries, values, d_perm, perm_stride);
+    PC_LAUNCH_CHECK("randomstate_buckets_kernel");
     return PC_OK;
 }

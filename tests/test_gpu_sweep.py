@@ -497,3 +497,28 @@ def test_tiled_lattice_sweep_matches_oracle(gpu):
     res = eng.sweep(eng.upload_permutations(perms))
     _check_traces(eng, res, expect)
     _check_sums(eng, res, expect)
+
+
+@pytest.mark.parametrize('M,runs', [(32769, 3), (40000, 1), (65537, 2), (130560, 5),
+                                    (524288, 2), (524289, 2), (2095104, 1)])
+def test_randomstate_permutations_in_buckets(gpu, M, runs):
+    """Runs above 32768 edges in position buckets (32-bit entries up to 2^19
+    edges, 64-bit above) equal numpy's, with a workspace for every run, for
+    one run, and for none (the swaps in sequence, for the smaller sizes)."""
+    import ctypes
+    from pypercolate_amd import _native as nat
+    eng = BondEngine(_graph.GraphArrays(M + 1, np.stack(
+        [np.arange(M), np.arange(1, M + 1)], axis=1)))
+    seeds = [3, 4294967295, 77, 0, 123456][:runs]
+    want = np.stack([np.random.RandomState(s).permutation(M) for s in seeds])
+    np.testing.assert_array_equal(eng.randomstate_permutations(seeds).cpu().numpy(), want)
+    b = ctypes.c_uint64(0)
+    nat.check(eng.lib.pc_permute_randomstate_workspace_size(M, 1, ctypes.byref(b)), 'size')
+    d_seeds = eng.upload_seeds(seeds)
+    for nbytes in [b.value] + ([0] if M <= 65537 else []):
+        ws = gpu.empty((nbytes,), dtype=gpu.uint8, device='cuda')
+        out = gpu.empty((runs, M), dtype=gpu.int32, device='cuda')
+        nat.check(eng.lib.pc_permute_randomstate_ws(
+            nat.ptr(d_seeds), runs, M, nat.ptr(out), M, nat.ptr(ws), nbytes,
+            nat.stream_handle(gpu)), 'pc_permute_randomstate_ws')
+        np.testing.assert_array_equal(out.cpu().numpy(), want)
