@@ -132,7 +132,95 @@ __device__ __forceinline__ uint32_t wave_scan_max(uint32_t x)
     return x;
 }
 
+// Inclusive prefix scans over the 64 lanes of a chunk's state in one go: the
+// maximum mx and the sums d2, d3, d4 (32 to 128 bits), in place with DPP adds
+// and carries (one instruction per word and step; the scans' steps alternate,
+// so no step waits for its own previous result).  Row shifts read 0 past a
+// row's edge; the two row broadcasts leave the rows they do not add to as they
+// are.  Against separate scans of moved copies: 26, 48 and 60 instructions
+// per chunk and step of the sums instead of 80 to 170.
+#define SCAN_SHR(n) "row_shr:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+#define SCAN_B15 "row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+#define SCAN_B31 "row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+#define SCAN_MAX(r, c) "v_max_u32_dpp " r ", " r ", " r " " c
+#define SCAN_ADD(r, c) "v_add_u32_dpp " r ", " r ", " r " " c
+#define SCAN_ADD_CO(r, c) "v_add_co_u32_dpp " r ", vcc, " r ", " r " " c
+#define SCAN_ADDC(r, c) "v_addc_co_u32_dpp " r ", vcc, " r ", " r ", vcc " c
+#define SCAN_64(lo, hi, c) SCAN_ADD_CO(lo, c) SCAN_ADDC(hi, c)
+#define SCAN_128(a, b, d, e, c) SCAN_ADD_CO(a, c) SCAN_ADDC(b, c) SCAN_ADDC(d, c) SCAN_ADDC(e, c)
+#define SCAN_STEPS(S) S(SCAN_SHR(1)) S(SCAN_SHR(2)) S(SCAN_SHR(4)) S(SCAN_SHR(8)) S(SCAN_B15) S(SCAN_B31)
+// sums over the rows of 16 lanes alone: the total in a row's last lane
+#define SCAN_ROWS(S) S(SCAN_SHR(1)) S(SCAN_SHR(2)) S(SCAN_SHR(4)) S(SCAN_SHR(8))
+// wait states between the compiler's write of an operand and the first DPP
+// read, and between the last write and a lane read
+#define SCAN_NOP "s_nop 1\n\t"
+
+#define SCAN_STEP_NARROW(c) SCAN_MAX("%0", c) SCAN_ADD("%1", c) SCAN_64("%2", "%3", c) SCAN_64("%4", "%5", c)
+#define SCAN_STEP_SUMS(c) SCAN_MAX("%0", c) SCAN_64("%1", "%2", c) SCAN_64("%3", "%4", c) SCAN_128("%5", "%6", "%7", "%8", c)
+#define SCAN_STEP_WIDE(c) SCAN_MAX("%0", c) SCAN_64("%1", "%2", c) SCAN_128("%3", "%4", "%5", "%6", c) SCAN_128("%7", "%8", "%9", "%10", c)
+
+struct Words128 {
+    uint32_t w[4];
+    __device__ __forceinline__ explicit Words128(u128 v)
+        : w{(uint32_t)v, (uint32_t)(v >> 32), (uint32_t)(v >> 64), (uint32_t)(v >> 96)} {}
+    __device__ __forceinline__ u128 value() const
+    {
+        return ((u128)(((uint64_t)w[3] << 32) | w[2]) << 64) | (((uint64_t)w[1] << 32) | w[0]);
+    }
+};
+
+#define SCAN_DEFINE(NAME, STEPS)                                                           \
+    __device__ __forceinline__ void NAME(uint32_t &mx, uint32_t &d2, uint64_t &d3,         \
+                                         uint64_t &d4)                                     \
+    {                                                                                      \
+        uint32_t a = (uint32_t)d3, b = (uint32_t)(d3 >> 32);                               \
+        uint32_t c = (uint32_t)d4, d = (uint32_t)(d4 >> 32);                               \
+        asm volatile(SCAN_NOP STEPS(SCAN_STEP_NARROW) SCAN_NOP                             \
+                     : "+v"(mx), "+v"(d2), "+v"(a), "+v"(b), "+v"(c), "+v"(d)::"vcc");     \
+        d3 = ((uint64_t)b << 32) | a;                                                      \
+        d4 = ((uint64_t)d << 32) | c;                                                      \
+    }                                                                                      \
+    __device__ __forceinline__ void NAME(uint32_t &mx, uint64_t &d2, uint64_t &d3,         \
+                                         u128 &d4)                                         \
+    {                                                                                      \
+        uint32_t a = (uint32_t)d2, b = (uint32_t)(d2 >> 32);                               \
+        uint32_t c = (uint32_t)d3, d = (uint32_t)(d3 >> 32);                               \
+        Words128 e(d4);                                                                    \
+        asm volatile(SCAN_NOP STEPS(SCAN_STEP_SUMS) SCAN_NOP                               \
+                     : "+v"(mx), "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e.w[0]),         \
+                       "+v"(e.w[1]), "+v"(e.w[2]), "+v"(e.w[3])::"vcc");                   \
+        d2 = ((uint64_t)b << 32) | a;                                                      \
+        d3 = ((uint64_t)d << 32) | c;                                                      \
+        d4 = e.value();                                                                    \
+    }                                                                                      \
+    __device__ __forceinline__ void NAME(uint32_t &mx, uint64_t &d2, u128 &d3, u128 &d4)   \
+    {                                                                                      \
+        uint32_t a = (uint32_t)d2, b = (uint32_t)(d2 >> 32);                               \
+        Words128 c(d3), e(d4);                                                             \
+        asm volatile(SCAN_NOP STEPS(SCAN_STEP_WIDE) SCAN_NOP                               \
+                     : "+v"(mx), "+v"(a), "+v"(b), "+v"(c.w[0]), "+v"(c.w[1]),             \
+                       "+v"(c.w[2]), "+v"(c.w[3]), "+v"(e.w[0]), "+v"(e.w[1]),             \
+                       "+v"(e.w[2]), "+v"(e.w[3])::"vcc");                                 \
+        d2 = ((uint64_t)b << 32) | a;                                                      \
+        d3 = c.value();                                                                    \
+        d4 = e.value();                                                                    \
+    }
+SCAN_DEFINE(scan_state, SCAN_STEPS)
+SCAN_DEFINE(scan_state_rows, SCAN_ROWS)
+
+// Lanes up to and including this one with the flag set.
+__device__ __forceinline__ uint32_t scan_count(bool flag)
+{
+    const uint64_t m = __ballot(flag);
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)) + (flag ? 1u : 0u);
+}
+
 __device__ __forceinline__ uint64_t umax64(uint64_t a, uint64_t b) { return a > b ? a : b; }
+
+// Lanes whose flag is set.  (__ballot compares the flag, widened to a
+// register, with 0: two vector instructions that a lane mask does not need.)
+__device__ __forceinline__ uint64_t ballot(bool flag) { return __builtin_amdgcn_ballot_w64(flag); }
 
 // The first active lane's value, as a wave-uniform (scalar) value.
 __device__ __forceinline__ uint32_t uniform(uint32_t v)
@@ -284,7 +372,7 @@ __device__ __forceinline__ uint64_t match_label(uint32_t label, uint32_t bits,
     uint32_t lo = (uint32_t)valid, hi = (uint32_t)(valid >> 32);
     for (uint32_t i = 0; i < bits; ++i) {
         const uint32_t s = (uint32_t)((int32_t)(label << (31u - i)) >> 31);
-        const uint64_t ones = __ballot(s != 0u);
+        const uint64_t ones = ballot(s != 0u);
         lo &= ~((uint32_t)ones ^ s);
         hi &= ~((uint32_t)(ones >> 32) ^ s);
     }
@@ -602,7 +690,7 @@ __global__ __launch_bounds__(64 * SHUF_W) void shuffle_scatter_kernel(
         for (uint32_t k = 0; k < 8u; ++k) {
             const uint32_t i = g * 512u + k * 64u + lane;
             const bool ok = i < ch.hi;
-            const uint64_t valid = __ballot(ok);
+            const uint64_t valid = ballot(ok);
             const uint32_t bkt = lb1 ? half16(key, k) >> (16u - lb1) : 0u;
             const uint64_t peers = match_label(bkt, lb1, valid);
             if (ok) {
@@ -730,7 +818,7 @@ __device__ void shuffle_group_lds(uint32_t n, uint32_t b, uint32_t run,
             for (uint32_t k = 0; k < 8u; ++k) {
                 const uint32_t j = g * 512u + k * 64u + lane;
                 const bool ok = j < n;
-                const uint64_t valid = __ballot(ok);
+                const uint64_t valid = ballot(ok);
                 const uint32_t s = lb ? half16(keys[gi], k) >> (16u - lb) : 0u;
                 const uint64_t peers = match_label(s, lb, valid);
                 if (ok) {
@@ -1020,8 +1108,8 @@ __device__ __forceinline__ uint32_t mt_settle(const uint32_t *mt, uint32_t i, in
             const uint32_t c = i - (m >> 1);
             const uint32_t x = w & m;
             const bool valid = lane >= l0 && lane < nw;
-            uint64_t acc = __ballot(valid && x + 63u <= i);
-            uint64_t amb = __ballot(valid && x <= i && x + 63u > i);
+            uint64_t acc = ballot(valid && x + 63u <= i);
+            uint64_t amb = ballot(valid && x <= i && x + 63u > i);
             while (amb) {
                 const uint32_t l = (uint32_t)__builtin_ctzll(amb);
                 const uint32_t below = (uint32_t)__popcll(acc & ((1ull << l) - 1ull));
@@ -1036,7 +1124,7 @@ __device__ __forceinline__ uint32_t mt_settle(const uint32_t *mt, uint32_t i, in
             uint32_t used;
             if (cnt >= c) {
                 // the c-th accepted lane takes the mask's last step
-                const uint32_t last = (uint32_t)__builtin_ctzll(__ballot(mine && below == c - 1u));
+                const uint32_t last = (uint32_t)__builtin_ctzll(ballot(mine && below == c - 1u));
                 if (mine && below < c)
                     out[i - below] = (int32_t)x;
                 used = c;
@@ -1120,8 +1208,8 @@ __global__ __launch_bounds__(RST_T) void randomstate_targets_wide_kernel(
         if (i >= RST_SMALL && i - (m >> 1) > MT_N) {
             const uint32_t x = mt_temper(y) & m;
             const bool in = t < MT_N;
-            const uint64_t acc = __ballot(in && x + t <= i);
-            const uint64_t amb = __ballot(in && x <= i && x + t > i);
+            const uint64_t acc = ballot(in && x + t <= i);
+            const uint64_t amb = ballot(in && x <= i && x + t > i);
             xs[t] = x;
             if ((t & 63u) == 0u) {
                 accepted[wave] = acc;
@@ -1853,24 +1941,32 @@ struct Wide {
 template <bool WIDE>
 struct Deltas {
     using MT = typename Wide<WIDE>::T;
-    uint32_t dmax; // size of the merged cluster (0: no merge)
-    uint32_t cnt;  // 1 for a merge
-    uint64_t d2;   // (a+b)^2 - a^2 - b^2
-    MT d3, d4;
+    using D2 = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
+    uint32_t dmax; // size s of the merged cluster (0: no merge)
+    D2 d2;         // s^2 - a^2 - b^2 = 2 q, q = a b
+    MT d3, d4;     // s^3 - a^3 - b^3 = 3 q s, s^4 - a^4 - b^4 = 2 q (2 s^2 - q)
     template <typename RecT>
     __device__ __forceinline__ explicit Deltas(RecT rec)
     {
         uint32_t a, b;
         unpack_record(rec, a, b);
-        const bool m = rec != 0;
-        dmax = m ? a + b : 0u;
-        cnt = m ? 1u : 0u;
-        const uint64_t ab = (uint64_t)a * b;
-        const uint64_t aa = (uint64_t)a * a, bb = (uint64_t)b * b;
-        d2 = 2u * ab;
-        d3 = (MT)3u * (MT)ab * (MT)(a + b);
-        d4 = (MT)(2u * ab) * (MT)(2u * aa + 3u * ab + 2u * bb);
+        const uint32_t s = a + b;
+        dmax = s;   // a record without a merge is 0
+        if constexpr (WIDE) {
+            // s <= 2^28
+            const uint64_t q = (uint64_t)a * b;
+            d2 = 2u * q;
+            d3 = (MT)q * (MT)(3u * s);
+            d4 = (MT)(2u * q) * (MT)(2u * ((uint64_t)s * s) - q);
+        } else {
+            // s <= 2^14: full-rate 24-bit products below 2^28
+            const uint32_t q = (uint32_t)__umul24(a, b);
+            d2 = 2u * q;
+            d3 = (uint64_t)q * (3u * s);
+            d4 = (uint64_t)(2u * q) * (2u * (uint32_t)__umul24(s, s) - q);
+        }
     }
+    __device__ __forceinline__ bool merge() const { return dmax != 0u; }
 };
 
 // Word w of a chunk-state entry: {max cluster size, merges, S2, S3 lo,
@@ -2139,12 +2235,13 @@ __device__ __forceinline__ void sweep_run(const St &st, uint32_t N, uint32_t M,
     // into the running state one batch later, off the resolver's chain
     RecT *rec_slots = (RecT *)(handoff + (HANDED ? 512u : 256u));
     auto fold_batch = [&](RecT rec) {
-        const Deltas<WIDE> d(rec);
-        cs_mx = umax64(cs_mx, (uint64_t)read_lane(wave_scan_max(d.dmax), 63u));
-        cs_merges += read_lane(wave_scan_add(d.cnt), 63u);
-        cs_s2 += read_lane(wave_scan_add(d.d2), 63u);
-        cs_s3 += read_lane(wave_scan_add(d.d3), 63u);
-        cs_s4 += read_lane(wave_scan_add(d.d4), 63u);
+        Deltas<WIDE> d(rec);
+        cs_merges += (uint32_t)__popcll(ballot(d.merge()));
+        scan_state(d.dmax, d.d2, d.d3, d.d4);
+        cs_mx = umax64(cs_mx, (uint64_t)read_lane(d.dmax, 63u));
+        cs_s2 += read_lane(d.d2, 63u);
+        cs_s3 += read_lane(d.d3, 63u);
+        cs_s4 += read_lane(d.d4, 63u);
     };
 
     for (uint32_t base = 0; base < M; base += 64u) {
@@ -2199,7 +2296,7 @@ __device__ __forceinline__ void sweep_run(const St &st, uint32_t N, uint32_t M,
             hint_v = st.get((uint32_t)uv_next.y);
         }
         bool cand = active && ru != rv;
-        uint64_t pending = __ballot(cand);
+        uint64_t pending = ballot(cand);
         RecT rec = 0;
 
         if (tag >= 0xFFFFFFFFu - 65u * 64u) {
@@ -2226,14 +2323,14 @@ __device__ __forceinline__ void sweep_run(const St &st, uint32_t N, uint32_t M,
             // earlier candidate also touches, all merge into the hub now
             uint64_t star = 0;
             uint32_t hub = 0;
-            const uint64_t blocked = __ballot(cand && !go);
+            const uint64_t blocked = ballot(cand && !go);
             if (blocked) {
                 const uint32_t fl = (uint32_t)__builtin_ctzll(blocked);
                 hub = read_lane(own_u ? rv : ru, fl);
                 const bool at_u = ru == hub;
                 const bool touch = cand && (at_u || rv == hub);
-                const uint64_t tm = __ballot(touch);
-                const uint64_t bad = tm & ~__ballot(touch && (at_u ? own_v : own_u));
+                const uint64_t tm = ballot(touch);
+                const uint64_t bad = tm & ~ballot(touch && (at_u ? own_v : own_u));
                 star = bad ? (tm & ((bad & (0u - bad)) - 1u)) : tm;
                 go = go && !touch;
                 // a pending candidate outside the star whose root's slot is
@@ -2243,12 +2340,12 @@ __device__ __forceinline__ void sweep_run(const St &st, uint32_t N, uint32_t M,
                 const uint32_t hu = tag + 63u - held_u, hv = tag + 63u - held_v;
                 const bool late = cand && !go && !((star >> lane) & 1u) &&
                                   (((star >> (hu & 63u)) & 1u) || ((star >> (hv & 63u)) & 1u));
-                const uint64_t lm = __ballot(late);
+                const uint64_t lm = ballot(late);
                 if (lm)
                     star &= (lm & (0u - lm)) - 1u;
             }
             const bool in_star = (star >> lane) & 1u;
-            const uint64_t freed = __ballot(go) | star;
+            const uint64_t freed = ballot(go) | star;
             if (star) {
                 // records in step order: the hub's size grows by the sizes
                 // absorbed by the earlier members (exclusive prefix sum)
@@ -2261,8 +2358,8 @@ __device__ __forceinline__ void sweep_run(const St &st, uint32_t N, uint32_t M,
                 const uint32_t s_hub = read_lane(sh, first), f_hub = read_lane(fh, first);
                 const uint32_t incl = wave_scan_add(in_star ? sx : 0u);
                 const uint32_t total = read_lane(incl, 63u);
-                const uint64_t m1 = __ballot(in_star && (fx & 1u));
-                const uint64_t m2 = __ballot(in_star && (fx & 2u));
+                const uint64_t m1 = ballot(in_star && (fx & 1u));
+                const uint64_t m2 = ballot(in_star && (fx & 2u));
                 const uint32_t f_all = f_hub | (m1 ? 1u : 0u) | (m2 ? 2u : 0u);
                 if (in_star) {
                     // (size on u's side, size on v's side), as every merge
@@ -2304,19 +2401,19 @@ __device__ __forceinline__ void sweep_run(const St &st, uint32_t N, uint32_t M,
                 spans_here = span_first || f == 3u;
             }
             {
-                const uint64_t spans = __ballot(spans_here);
+                const uint64_t spans = ballot(spans_here);
                 if (spans)
                     span_at = min(span_at, base + (uint32_t)__builtin_ctzll(spans) + 1u);
             }
             cand = cand && !go && !in_star;
             st.sync();
-            if (__ballot(cand)) {
+            if (ballot(cand)) {
                 // lanes still pending follow their roots past this round's merges
                 if (cand)
                     find2(st, ru, cu, rv, cv);
                 cand = cand && ru != rv;
             }
-            pending = __ballot(cand);
+            pending = ballot(cand);
             // a round that frees at most one candidate is resolving a chain
             // (typically through the largest cluster's root): the in-order
             // remainder does that more cheaply
@@ -3291,14 +3388,15 @@ __device__ __forceinline__ RunState<WIDE> load_state(const uint64_t *cs)
 // of the deltas of the chunk's records.
 template <bool WIDE>
 __device__ __forceinline__ RunState<WIDE> advance(const RunState<WIDE> &st0,
-                                                  const Deltas<WIDE> &d)
+                                                  Deltas<WIDE> d)
 {
     RunState<WIDE> st;
-    st.mx = umax64(st0.mx, (uint64_t)wave_scan_max(d.dmax));
-    st.merges = st0.merges + wave_scan_add(d.cnt);
-    st.s2 = st0.s2 + wave_scan_add(d.d2);
-    st.s3 = st0.s3 + wave_scan_add(d.d3);
-    st.s4 = st0.s4 + wave_scan_add(d.d4);
+    st.merges = st0.merges + scan_count(d.merge());
+    scan_state(d.dmax, d.d2, d.d3, d.d4);
+    st.mx = umax64(st0.mx, (uint64_t)d.dmax);
+    st.s2 = st0.s2 + d.d2;
+    st.s3 = st0.s3 + d.d3;
+    st.s4 = st0.s4 + d.d4;
     return st;
 }
 
@@ -3342,18 +3440,50 @@ __global__ __launch_bounds__(64) void chunk_delta_kernel(
     const uint32_t r = blockIdx.x / per_run, lane = threadIdx.x;
     const RecT *rec_r = records + (int64_t)r * rec_stride;
     uint64_t *out = chunk_state + (size_t)r * C * PC_STATE_WORDS;
-    const uint32_t c0 = (blockIdx.x % per_run) * CHUNK_DELTA_PER_BLOCK;
-    const uint32_t c1 = min(C, c0 + CHUNK_DELTA_PER_BLOCK);
-    for (uint32_t c = c0; c < c1; ++c) {
-        const uint32_t q = c * 64u + lane;
-        const Deltas<WIDE> d(q < M ? rec_r[q] : (RecT)0);
-        const uint64_t dmax = read_lane(wave_scan_max(d.dmax), 63u);
-        const uint64_t cnt = read_lane(wave_scan_add(d.cnt), 63u);
-        const uint64_t d2 = read_lane(wave_scan_add(d.d2), 63u);
-        const auto d3 = read_lane(wave_scan_add(d.d3), 63u);
-        const auto d4 = read_lane(wave_scan_add(d.d4), 63u);
-        if (lane < PC_STATE_WORDS)
-            out[(size_t)c * PC_STATE_WORDS + lane] = state_word(lane, dmax, cnt, d2, d3, d4);
+    const uint32_t c0 = (blockIdx.x % per_run) * CHUNK_DELTA_PER_BLOCK + lane / 16u;
+    // a row of 16 lanes per chunk, four records a lane (their order within a
+    // chunk does not matter to its totals): a quarter of the scan steps of a
+    // lane per record, and four of six levels.  With the scans in place, 10^4
+    // runs of L = 128 take 0.33 ms (1.35 before), 1000 of L = 1024 3.4 (10.8)
+    constexpr uint32_t ITER = CHUNK_DELTA_PER_BLOCK / 4u;
+    RecT rec[ITER][4];
+#pragma unroll
+    for (uint32_t i = 0; i < ITER; ++i)
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) {
+            const uint32_t q = (c0 + 4u * i) * 64u + u * 16u + lane % 16u;
+            rec[i][u] = rec_r[min(q, M - 1u)];
+            if (q >= M)
+                rec[i][u] = 0;
+        }
+#pragma unroll
+    for (uint32_t i = 0; i < ITER; ++i) {
+        const uint32_t c = c0 + 4u * i;
+        Deltas<WIDE> d(rec[i][0]);
+        uint32_t cnt = (uint32_t)__popcll(ballot(d.merge()) >> (lane & 48u) & 0xFFFFull);
+#pragma unroll
+        for (uint32_t u = 1; u < 4u; ++u) {
+            const Deltas<WIDE> e(rec[i][u]);
+            cnt += (uint32_t)__popcll(ballot(e.merge()) >> (lane & 48u) & 0xFFFFull);
+            d.dmax = max(d.dmax, e.dmax);
+            d.d2 += e.d2;
+            d.d3 += e.d3;
+            d.d4 += e.d4;
+        }
+        scan_state_rows(d.dmax, d.d2, d.d3, d.d4);
+        if (lane % 16u == 15u && c < C) {
+            const uint64_t hi3 = WIDE ? (uint64_t)((u128)d.d3 >> 64) : 0u;
+            const uint64_t hi4 = WIDE ? (uint64_t)((u128)d.d4 >> 64) : 0u;
+            uint64_t *w = out + (size_t)c * PC_STATE_WORDS;
+            w[0] = d.dmax;
+            w[1] = cnt;
+            w[2] = d.d2;
+            w[3] = (uint64_t)d.d3;
+            w[4] = hi3;
+            w[5] = (uint64_t)d.d4;
+            w[6] = hi4;
+            w[7] = 0u;
+        }
     }
 }
 
@@ -3381,9 +3511,11 @@ __global__ __launch_bounds__(64) void chunk_prefix_kernel(
             d3 |= (MT)w[4] << 64;
             d4 |= (MT)w[6] << 64;
         }
-        const uint32_t imax = wave_scan_max(dmax);
-        const uint64_t icnt = wave_scan_add(cnt), id2 = wave_scan_add(d2);
-        const MT id3 = wave_scan_add(d3), id4 = wave_scan_add(d4);
+        uint32_t imax = dmax;
+        const uint32_t icnt = wave_scan_add((uint32_t)cnt);
+        typename Deltas<WIDE>::D2 id2 = (typename Deltas<WIDE>::D2)d2;
+        MT id3 = d3, id4 = d4;
+        scan_state(imax, id2, id3, id4);
         // exclusive prefix: the sums minus the own chunk, the maximum of the
         // chunks before (the previous lane's inclusive maximum)
         uint32_t emax = (uint32_t)__shfl_up((int)imax, 1, 64);
@@ -3404,9 +3536,35 @@ __global__ __launch_bounds__(64) void chunk_prefix_kernel(
 
 // ---------------------------------------------------------------------------
 // Microcanonical sums: block (chunk c, run group g), lane = step.  Each lane
-// accumulates its step's sums over the group's runs in registers; groups
-// combine through multi-word atomics.
+// accumulates its step's sums over its wave's runs of the group in registers;
+// the waves add up in LDS, groups combine through multi-word atomics.
 // ---------------------------------------------------------------------------
+// Workgroups of one wave fill the GPU where there are 8192 of them with 32
+// runs each; they use no LDS, which the sweeps beside them hold (10^4 runs of
+// L = 128 as a pipeline: 8.3 ms, 9.5 with the form below).  Elsewhere the four
+// waves of a workgroup share 64 runs of a chunk and add up in LDS, so that a
+// fourth of the atomics remain (L = 100, 500 runs 0.121 -> 0.044 ms; L = 16,
+// 40 runs 13 -> 8 us).  Bound by vector issue.
+#define SUMS_BLOCKS 8192u
+#define SUMS_RUNS 32u
+
+// Product of two numbers below 2^24 (two full-rate instructions; __umul24
+// returns an int).
+__device__ __forceinline__ uint64_t mul24_wide(uint32_t a, uint32_t b)
+{
+    uint32_t hi;
+    asm("v_mul_hi_u32_u24 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    return ((uint64_t)hi << 32) | (uint32_t)__umul24(a, b);
+}
+
+// Square of a 64-bit number: three 32-bit products.
+__device__ __forceinline__ u128 square_u128(uint64_t x)
+{
+    const uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
+    const uint64_t ll = (uint64_t)lo * lo, lh = (uint64_t)lo * hi, hh = (uint64_t)hi * hi;
+    return (((u128)hh << 64) | ll) + ((u128)lh << 33);
+}
+
 __device__ __forceinline__ void square_u192(u128 x, uint64_t &w0, uint64_t &w1,
                                             uint64_t &w2)
 {
@@ -3420,22 +3578,61 @@ __device__ __forceinline__ void square_u192(u128 x, uint64_t &w0, uint64_t &w1,
     w2 = (uint64_t)(mid >> 64) + (uint64_t)(lh2 >> 64) + (uint64_t)hh;
 }
 
-template <typename RecT, bool WIDE>
-__global__ __launch_bounds__(64) void micro_sums_kernel(
+template <typename RecT, bool WIDE, uint32_t WAVES>
+__global__ __launch_bounds__(64 * WAVES) void micro_sums_kernel(
     uint32_t N, uint32_t M, uint32_t R, uint32_t runs_per_group,
     const RecT *__restrict__ records, int64_t rec_stride,
     const uint32_t *__restrict__ span_step,
     const uint64_t *__restrict__ chunk_state, uint64_t *__restrict__ sum1,
-    uint64_t *__restrict__ sum2)
+    uint64_t *__restrict__ sum2, bool store)
 {
+    // the waves' accumulators on their way to wave 0
+    constexpr uint32_t PARTS = WIDE ? 21u : 18u;
+    __shared__ uint64_t part[WAVES > 1u ? PARTS : 1u][64];
     using MT = typename Wide<WIDE>::T;
-    const uint32_t c = blockIdx.x, g = blockIdx.y, lane = threadIdx.x;
+    const uint32_t c = blockIdx.x, g = blockIdx.y, lane = threadIdx.x & 63u;
+    const uint32_t wave = uniform(threadIdx.x >> 6);
     const uint32_t C = (M + 63u) / 64u;
     const uint64_t S = (uint64_t)M + 1u;
     const uint32_t q = c * 64u + lane, s = q + 1u;
     const bool valid = q < M;
     const uint32_t r0 = g * runs_per_group;
     const uint32_t r1 = min(R, r0 + runs_per_group);
+
+    // the next run's state, record and spanning step, loaded a run ahead
+    RunState<WIDE> st_next;
+    RecT rec_next;
+    uint32_t span_next;
+    auto ahead = [&](uint32_t r) __attribute__((always_inline)) {
+        st_next = load_state<WIDE>(chunk_state + ((size_t)r * C + c) * PC_STATE_WORDS);
+        rec_next = records[(int64_t)r * rec_stride + min(q, M - 1u)];
+        span_next = span_step[r];
+    };
+    ahead(min(r0 + wave, R - 1u));
+
+    // wave 3's sums to wave 2, whose sum goes to wave 1, and on to wave 0
+    auto to_wave0 = [&](auto &&each) {
+        if constexpr (WAVES > 1u)
+        for (int w = WAVES - 1; w >= 0; --w) {
+            if ((int)wave == w) {
+                if (w + 1 < (int)WAVES)
+                    each([&](uint32_t i, auto &v) {
+                        using V = std::remove_reference_t<decltype(v)>;
+                        if constexpr (sizeof(V) == 16)
+                            v += (u128)part[i][lane] | ((u128)part[i + 1u][lane] << 64);
+                        else
+                            v += (V)part[i][lane];
+                    });
+                if (w > 0)
+                    each([&](uint32_t i, auto &v) {
+                        part[i][lane] = (uint64_t)v;
+                        if constexpr (sizeof(v) == 16)
+                            part[i + 1u][lane] = (uint64_t)(v >> 64);
+                    });
+            }
+            __syncthreads();
+        }
+    };
 
     u128 acc1[7];
     u128 acc2[7];
@@ -3458,27 +3655,44 @@ __global__ __launch_bounds__(64) void micro_sums_kernel(
         uint64_t n2[4] = {0, 0, 0, 0};  // sum x^2 of the same
         uint64_t m1_2 = 0, m1_3 = 0;    // sum x: moments 2 and 3
         u128 m1_4 = 0, m2_2 = 0, m2_3 = 0, m2_4 = 0;
-        for (uint32_t r = r0; r < r1; ++r) {
-            const RunState<false> st0 = load_state<false>(
-                chunk_state + ((size_t)r * C + c) * PC_STATE_WORDS);
-            const RecT rec = valid ? records[(int64_t)r * rec_stride + q] : (RecT)0;
-            const RunState<false> st = advance<false>(st0, Deltas<false>(rec));
-            uint64_t x[7];
-            observables<false>(st, N, s >= span_step[r], x);
+        for (uint32_t r = r0 + wave; r < r1; r += WAVES) {
+            const RunState<false> st0 = st_next;
+            const RecT rec = valid ? rec_next : (RecT)0;
+            const uint32_t span = span_next;
+            ahead(min(r + WAVES, r1 - 1u));
+            Deltas<false> d(rec);
+            const uint32_t merges = (uint32_t)st0.merges + scan_count(d.merge());
+            scan_state(d.dmax, d.d2, d.d3, d.d4);
+            const uint32_t mx = max((uint32_t)st0.mx, d.dmax), mx2 = (uint32_t)__umul24(mx, mx);
+            const uint32_t x[4] = {mx, s >= span ? 1u : 0u, N - merges - 1u, N - mx};
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const uint32_t v = (uint32_t)x[k];
-                n1[k] += v;
-                n2[k] += (uint64_t)(v * v);
+                n1[k] += x[k];
+                n2[k] += (uint32_t)__umul24(x[k], x[k]);
             }
-            const uint32_t v4 = (uint32_t)x[4];
-            m1_2 += v4;
-            m2_2 += (u128)((uint64_t)v4 * v4);
-            m1_3 += x[5];
-            m2_3 += (u128)x[5] * x[5];
-            m1_4 += x[6];
-            m2_4 += (u128)x[6] * x[6];
+            const uint32_t x4 = (uint32_t)st0.s2 + d.d2 - mx2;
+            m1_2 += x4;
+            m2_2 += (u128)((uint64_t)x4 * x4);
+            const uint64_t x5 = st0.s3 + d.d3 - (uint64_t)mx2 * mx;
+            m1_3 += x5;
+            m2_3 += square_u128(x5);
+            const uint64_t x6 = st0.s4 + d.d4 - (uint64_t)mx2 * mx2;
+            m1_4 += x6;
+            m2_4 += square_u128(x6);
         }
+        to_wave0([&](auto &&at) {
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) {
+                at(k, n1[k]);
+                at(4u + k, n2[k]);
+            }
+            at(8u, m1_2);
+            at(9u, m1_3);
+            at(10u, m1_4);
+            at(12u, m2_2);
+            at(14u, m2_3);
+            at(16u, m2_4);
+        });
         // column order of the sums: max, span, moments 0..4
         const int col[4] = {0, 1, 2, 3};
 #pragma unroll
@@ -3504,40 +3718,41 @@ __global__ __launch_bounds__(64) void micro_sums_kernel(
         u128 m2_2 = 0, m1_3 = 0, m1_4 = 0;
         u128 m2_3 = 0, m2_4 = 0;          // low 128 bits of sum x^2, moments 3 and 4
         uint64_t t2_3 = 0, t2_4 = 0;      // their top words
-        for (uint32_t r = r0; r < r1; ++r) {
-            const uint64_t *cs = chunk_state + ((size_t)r * C + c) * PC_STATE_WORDS;
-            const uint64_t mx0 = cs[0], merges0 = cs[1], s2_0 = cs[2], s3_0 = cs[3];
-            const u128 s4_0 = (u128)cs[5] | ((u128)cs[6] << 64);
-            const RecT rec = valid ? records[(int64_t)r * rec_stride + q] : (RecT)0;
+        for (uint32_t r = r0 + wave; r < r1; r += WAVES) {
+            const uint64_t mx0 = st_next.mx, merges0 = st_next.merges, s2_0 = st_next.s2,
+                           s3_0 = (uint64_t)st_next.s3;
+            const u128 s4_0 = st_next.s4;
+            const RecT rec = valid ? rec_next : (RecT)0;
+            const uint32_t span = span_next;
+            ahead(min(r + WAVES, r1 - 1u));
             uint32_t a, b;
             unpack_record(rec, a, b);
-            const bool merge = rec != 0;
-            const uint64_t ab = (uint64_t)a * b;
-            const uint64_t aa = (uint64_t)a * a, bb = (uint64_t)b * b;
-            const uint32_t dmax = merge ? a + b : 0u;
-            const uint64_t d2 = 2u * ab;
-            const uint64_t d3 = 3u * ab * (uint64_t)(a + b);
-            const u128 d4 = (u128)(2u * ab) * (u128)(2u * aa + 3u * ab + 2u * bb);
-            const uint64_t mx = umax64(mx0, (uint64_t)wave_scan_max(dmax));
-            const uint64_t merges = merges0 + wave_scan_add(merge ? 1u : 0u);
-            const uint64_t s2 = s2_0 + wave_scan_add(d2);
-            const uint64_t s3 = s3_0 + wave_scan_add(d3);
-            const u128 s4 = s4_0 + wave_scan_add(d4);
-            const uint64_t m2 = mx * mx;
-            const uint64_t x[4] = {mx, s >= span_step[r] ? 1u : 0u,
-                                   (uint64_t)N - merges - 1u, (uint64_t)N - mx};
+            // sizes below 2^21 + 1: 24-bit products, q <= 2^40
+            uint32_t mxd = a + b;
+            const uint32_t sz = mxd;
+            const uint64_t qq = mul24_wide(a, b);
+            uint64_t d2 = 2u * qq, d3 = qq * (3u * sz);
+            u128 d4 = (u128)(2u * qq) * (u128)(2u * mul24_wide(sz, sz) - qq);
+            const uint64_t merges = merges0 + scan_count(rec != 0);
+            scan_state(mxd, d2, d3, d4);
+            const uint32_t mx = max((uint32_t)mx0, mxd);
+            const uint64_t s2 = s2_0 + d2, s3 = s3_0 + d3;
+            const u128 s4 = s4_0 + d4;
+            const uint64_t m2 = mul24_wide(mx, mx);
+            const uint32_t x[4] = {mx, s >= span ? 1u : 0u, N - (uint32_t)merges - 1u,
+                                   N - mx};
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 n1[k] += x[k];
-                n2[k] += x[k] * x[k];
+                n2[k] += mul24_wide(x[k], x[k]);
             }
             const uint64_t x4 = s2 - m2, x5 = s3 - m2 * mx;
             const u128 x6 = s4 - (u128)m2 * m2;
             n1[4] += x4;
-            m2_2 += (u128)x4 * x4;
+            m2_2 += square_u128(x4);
             m1_3 += x5;
             {
-                const u128 sq = (u128)x5 * x5, before = m2_3;
+                const u128 sq = square_u128(x5), before = m2_3;
                 m2_3 += sq;
                 t2_3 += m2_3 < before ? 1u : 0u;
             }
@@ -3549,6 +3764,29 @@ __global__ __launch_bounds__(64) void micro_sums_kernel(
                 m2_4 += (u128)w0 | ((u128)w1 << 64);
                 t2_4 += w2 + (m2_4 < before ? 1u : 0u);
             }
+        }
+        {
+            // the carries of the two 192-bit sums go with their low words
+            u128 *const low[2] = {&m2_3, &m2_4};
+            uint64_t *const top[2] = {&t2_3, &t2_4};
+            to_wave0([&](auto &&at) {
+#pragma unroll
+                for (uint32_t k = 0; k < 5u; ++k)
+                    at(k, n1[k]);
+#pragma unroll
+                for (uint32_t k = 0; k < 4u; ++k)
+                    at(5u + k, n2[k]);
+                at(9u, m2_2);
+                at(11u, m1_3);
+                at(13u, m1_4);
+#pragma unroll
+                for (uint32_t k = 0; k < 2u; ++k) {
+                    const u128 before = *low[k];
+                    at(15u + 3u * k, *low[k]);
+                    *top[k] += *low[k] < before ? 1u : 0u;
+                    at(17u + 3u * k, *top[k]);
+                }
+            });
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -3565,7 +3803,19 @@ __global__ __launch_bounds__(64) void micro_sums_kernel(
         acc2_top[6] = t2_4;
     }
 
-    if (valid) {
+    if (wave)
+        return;
+    if (store && valid) {
+#pragma unroll
+        for (int k = 0; k < 7; ++k) {
+            uint64_t *w1 = sum1 + ((uint64_t)k * S + s) * 2u, *w2 = sum2 + ((uint64_t)k * S + s) * 3u;
+            w1[0] = (uint64_t)acc1[k];
+            w1[1] = (uint64_t)(acc1[k] >> 64);
+            w2[0] = (uint64_t)acc2[k];
+            w2[1] = (uint64_t)(acc2[k] >> 64);
+            w2[2] = acc2_top[k];
+        }
+    } else if (valid) {
 #pragma unroll
         for (int k = 0; k < 7; ++k) {
             atomic_add_u128(sum1 + ((uint64_t)k * S + s) * 2u, acc1[k]);
@@ -3579,8 +3829,17 @@ __global__ __launch_bounds__(64) void micro_sums_kernel(
         const u128 n = r1 - r0;
         const u128 x0[7] = {1, 0, N - 1u, N - 1u, N - 1u, N - 1u, N - 1u};
         for (int k = 0; k < 7; ++k) {
-            atomic_add_u128(sum1 + (uint64_t)k * S * 2u, n * x0[k]);
             const u128 sq = n * x0[k] * x0[k];
+            if (store) {
+                uint64_t *w1 = sum1 + (uint64_t)k * S * 2u, *w2 = sum2 + (uint64_t)k * S * 3u;
+                w1[0] = (uint64_t)(n * x0[k]);
+                w1[1] = (uint64_t)(n * x0[k] >> 64);
+                w2[0] = (uint64_t)sq;
+                w2[1] = (uint64_t)(sq >> 64);
+                w2[2] = 0u;
+                continue;
+            }
+            atomic_add_u128(sum1 + (uint64_t)k * S * 2u, n * x0[k]);
             atomic_add_u192(sum2 + (uint64_t)k * S * 3u, (uint64_t)sq,
                             (uint64_t)(sq >> 64), 0u);
         }
@@ -5430,7 +5689,21 @@ extern "C" int pc_microcanonical_sums(uint32_t num_nodes, uint32_t num_edges,
         return pc_fail(PC_EINVAL, "pc_microcanonical_sums: NULL buffer");
     hipStream_t s = as_stream(stream);
     const uint64_t S = (uint64_t)num_edges + 1u;
-    if (!accumulate) {
+    const uint32_t C = (num_edges + 63u) / 64u;
+    // enough waves to fill 256 CUs several times over, and enough runs a
+    // workgroup that its loop outweighs its 29 to 35 atomics a step
+    const uint32_t per32 = (num_runs + SUMS_RUNS - 1u) / SUMS_RUNS;
+    const bool one_wave = (uint64_t)C * per32 >= SUMS_BLOCKS;
+    uint32_t groups = C ? (SUMS_BLOCKS / (one_wave ? 1u : 4u) + C - 1u) / C : 1u;
+    groups = std::min(groups, one_wave ? per32 : (per32 + 1u) / 2u);
+    // at most 2^16 runs per group: the narrow 128-bit sum of squares of the
+    // fourth moment (each below 2^112) stays exact
+    groups = std::max(groups, num_runs / 65536u + (num_runs % 65536u != 0u));
+    const uint32_t rpg = groups ? (num_runs + groups - 1u) / groups : 0u;
+    groups = rpg ? (num_runs + rpg - 1u) / rpg : 0u;
+    // one group that does not accumulate stores its sums
+    const bool store = groups == 1u && !accumulate && num_edges;
+    if (!accumulate && !store) {
         fill_zero_kernel<<<1024, 256, 0, s>>>(d_sum1, 7u * S * 2u);
         fill_zero_kernel<<<1024, 256, 0, s>>>(d_sum2, 7u * S * 3u);
         PC_LAUNCH_CHECK("fill_zero_kernel");
@@ -5442,30 +5715,25 @@ extern "C" int pc_microcanonical_sums(uint32_t num_nodes, uint32_t num_edges,
         PC_LAUNCH_CHECK("step0_sums_kernel");
         return PC_OK;
     }
-    const uint32_t C = (num_edges + 63u) / 64u;
-    // enough blocks to fill 256 CUs several times over
-    uint32_t groups = (8192u + C - 1u) / C;
-    if (groups > num_runs)
-        groups = num_runs;
-    // at most 2^16 runs per group: the narrow 128-bit sum of squares of the
-    // fourth moment (each below 2^112) stays exact
-    if ((num_runs + groups - 1u) / groups > 65536u)
-        groups = (num_runs + 65535u) / 65536u;
-    const uint32_t rpg = (num_runs + groups - 1u) / groups;
-    groups = (num_runs + rpg - 1u) / rpg;
     const dim3 grid(C, groups);
+#define PC_SUMS(RT, WD)                                                               \
+    do {                                                                              \
+        if (one_wave)                                                                 \
+            micro_sums_kernel<RT, WD, 1u><<<grid, 64, 0, s>>>(                        \
+                num_nodes, num_edges, num_runs, rpg, (const RT *)d_records,           \
+                rec_stride, d_span_step, d_chunk_state, d_sum1, d_sum2, store);       \
+        else                                                                          \
+            micro_sums_kernel<RT, WD, 4u><<<grid, 256, 0, s>>>(                       \
+                num_nodes, num_edges, num_runs, rpg, (const RT *)d_records,           \
+                rec_stride, d_span_step, d_chunk_state, d_sum1, d_sum2, store);       \
+    } while (0)
     if (num_nodes <= kLdsMaxNodes)
-        micro_sums_kernel<uint32_t, false><<<grid, 64, 0, s>>>(
-            num_nodes, num_edges, num_runs, rpg, (const uint32_t *)d_records,
-            rec_stride, d_span_step, d_chunk_state, d_sum1, d_sum2);
+        PC_SUMS(uint32_t, false);
     else if (num_nodes <= kU32RecordMaxNodes)
-        micro_sums_kernel<uint32_t, true><<<grid, 64, 0, s>>>(
-            num_nodes, num_edges, num_runs, rpg, (const uint32_t *)d_records,
-            rec_stride, d_span_step, d_chunk_state, d_sum1, d_sum2);
+        PC_SUMS(uint32_t, true);
     else
-        micro_sums_kernel<uint64_t, true><<<grid, 64, 0, s>>>(
-            num_nodes, num_edges, num_runs, rpg, (const uint64_t *)d_records,
-            rec_stride, d_span_step, d_chunk_state, d_sum1, d_sum2);
+        PC_SUMS(uint64_t, true);
+#undef PC_SUMS
     PC_LAUNCH_CHECK("micro_sums_kernel");
     return PC_OK;
 }
