@@ -98,12 +98,12 @@ int pc_sweep_lattice(uint32_t length, int32_t tiled,
 
 /*
  * Device workspace bytes pc_sweep_lattice wants.  In mode PC_STATE_AUTO, for
- * lattices of more than 16384 nodes and a side of at most 2048, that is room
- * for the bond lists of its tiled sweep: tiles of at most 64 x 64 nodes whose
+ * a side of 96 to 2048 (from 65 on for at most 1024 runs), that is room for
+ * the bond lists of its tiled sweep: tiles of at most 64 x 64 nodes whose
  * own bonds are merged with their state in LDS, then the bonds between tiles
  * and the merges of clusters that reach a tile's border, per run.  With
  * pc_sweep_workspace_size bytes, or less, it still runs, with every node's
- * code in HBM where the lists do not fit.  The workspace must be 16-byte
+ * code in LDS or HBM as pc_sweep keeps it.  The workspace must be 16-byte
  * aligned for the tiled sweep.
  */
 int pc_sweep_lattice_workspace_size(uint32_t length, uint32_t num_runs,

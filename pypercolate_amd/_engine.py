@@ -82,12 +82,12 @@ class BondEngine(object):
         # LDS state the edge array sits in L2 and computing measured 1.4 %
         # slower (L = 128)
         self.lattice_sweep = bool(L) and self.N > 16384
-        # a lattice relabelled where the tiles are not whole (L not a
-        # multiple of 8): pc_sweep_lattice takes it with its sides row by
-        # row, for its tiled sweep; the relabelled edge array serves the
-        # modes in which every node's code is in HBM
+        # lattices whose edge array is swept otherwise (state in LDS, or a
+        # relabelling whose tiles are not whole): pc_sweep_lattice takes them
+        # with their sides row by row where it has a tiled sweep for them
+        # (a workspace of workspace_bytes for the number of runs)
         self.row_length, self.d_row_sides = 0, None
-        if not L and order is not None and self.N > 16384:
+        if not self.lattice_sweep and (self.N <= 16384 or order is not None):
             self.row_length = int(getattr(graph, 'lattice_length', 0) or 0)
             if self.row_length and graph.node_sides is not None:
                 self.d_row_sides = torch.from_numpy(graph.node_sides.copy()).to(dev)
@@ -171,7 +171,7 @@ class BondEngine(object):
     def workspace_bytes(self, num_runs, state_mode=None):
         b = ctypes.c_uint64(0)
         mode = self.state_mode if state_mode is None else state_mode
-        length = (self.lattice_length if self.lattice_sweep else 0) or self.row_length
+        length = self.lattice_length if self.lattice_sweep else self.row_length
         if length:
             nat.check(self.lib.pc_sweep_lattice_workspace_size(
                 length, num_runs, mode, ctypes.byref(b)),
@@ -227,8 +227,9 @@ class BondEngine(object):
             chunk_state = torch.empty((R, C, nat.PC_STATE_WORDS),
                                       dtype=torch.int64, device=self.device)
         st = nat.stream_handle(torch)
-        rows = (self.row_length and self.state_mode == nat.PC_STATE_AUTO and
-                wb >= self.workspace_bytes(R))
+        rows = (self.row_length and not self.lattice_sweep and wb and
+                self.state_mode == nat.PC_STATE_AUTO and
+                wb >= self.workspace_bytes(R) > 0)
         if self.lattice_sweep or rows:
             nat.check(self.lib.pc_sweep_lattice(
                 self.row_length if rows else self.lattice_length,

@@ -107,8 +107,8 @@ def tune_sweep(engine, sample_runs=None, rounds=ROUND_CANDIDATES, modes=None,
             places = [nat.PC_STATE_LDS, nat.PC_STATE_HBM]
         modes = [p | w for p in places
                  for w in (nat.PC_SWEEP_ONE_WAVE, nat.PC_SWEEP_TWO_WAVES)]
-        if engine.N > 16384:
-            # square lattices: the library's tiled sweep (no placement asked)
+        if engine.lattice_sweep or engine.row_length:
+            # the library's tiled sweep, with no placement asked
             modes.insert(0, nat.PC_STATE_AUTO)
     cus = device.multi_processor_count
     timings = {}

@@ -2614,9 +2614,9 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Tiled sweep of the square lattice (pc_sweep_lattice for lattices whose
-// union-find state does not fit LDS).  The lattice is cut into tiles of at
-// most TILE_ROWS x TILE_COLS nodes.  A node with a bond into another tile is
+// Tiled sweep of the square lattice (pc_sweep_lattice where tile_geo takes
+// it).  The lattice is cut into tiles of at
+// most TILE_SIDE x TILE_SIDE nodes.  A node with a bond into another tile is
 // open, and so is every cluster of a tile's own bonds that holds an open
 // node; the other clusters of a tile are closed: nothing outside the tile
 // can have joined them, so their sizes and sides are exact at every step.
@@ -2639,15 +2639,18 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 // others never leave LDS.  A tile-level merge of two open clusters that
 // outside bonds have already joined is found out in step 3 (record 0).
 // Untiled, with every node's code in HBM, the sweep moves 342 bytes per
-// addition in random lines at L = 1024.  Sweep with its chunk states, untiled
-// and tiled: L = 1024, 1000 runs 158 and 79 ms (lists 24, tiles 23, events 20,
-// chunk states 12); L = 256, 200 runs 3.67 and 1.3 ms; L = 181, 600 runs
-// 2.65 and 1.3 ms.  The tiles are bound by dependent LDS round trips (70 % of
-// a wavefront's cycles wait) and at L = 1024 by the records, which go out in
+// addition in random lines at L = 1024, and at L = 128 (codes in LDS) four
+// runs fill a CU.  Sweep with its chunk states, untiled and tiled: L = 1024,
+// 1000 runs 158 and 70 ms (lists 24, tiles 22, events 20, chunk states 4);
+// L = 256, 200 runs 3.67 and 1.1; L = 181, 600 runs 2.65 and 1.1; L = 128,
+// 10^4 runs (no chunk states) 7.06 and 5.05.  The tiles are bound by vector
+// issue (60 % of a wavefront's share of its SIMD at L = 256) and dependent
+// LDS round trips, and at L = 1024 by the records, which go out in
 // part-written lines: rows cleared in step order by tile_scatter, so that a
 // tile writes merges only, took them from 35 to 27 ms, a claim table of 512
-// slots instead of 1024 (15 wavefronts per CU, not 13) to 23 ms; 48 x 48 and
-// 32 x 64 tiles gain no more there than their events cost.
+// slots instead of 1024 (15 wavefronts per CU, not 13) to 23.  Codes that
+// are addresses, a claim slot without a multiply and both claims read at once
+// took 10^4 runs of L = 128 from 3.26 to 2.80 ms.
 //
 // Event record (half = half of a record's bits): the high half's top bit is
 // set (a final record's sizes are below 2^(half - 1) on both sides in step
@@ -2656,14 +2659,10 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 // set when the closed cluster is on the bond's u side), set for a join (high
 // half: the other open node's id).
 // ---------------------------------------------------------------------------
-#ifndef TILE_ROWS
-#define TILE_ROWS 64u
-#define TILE_COLS 64u
-#endif
+#define TILE_SIDE 64u
+#define TILE_LDS_LENGTH 96u
 #define TILE_MAX_LENGTH 2048u
-#ifndef TILE_CLAIM_BITS
 #define TILE_CLAIM_BITS 9
-#endif
 #define TILE_CLAIM_SLOTS (1u << TILE_CLAIM_BITS)
 #define TILE_SCATTER_BLOCKS 1024u // workgroups tile_scatter wants
 #define TILE_GROUPS 8u   // groups of 64 steps a wave of tile_scatter takes at once
@@ -2694,16 +2693,17 @@ struct TileGeo {
     }
 };
 
-// A tile's union-find code: a parent's local index (below 0x1000), an open
-// root's place among the tile's ids (0x1000 + place), or a closed root's
-// (1 + sides) << 14 | size.
-#define TILE_OPEN 0x1000u
+// A tile's union-find code, with nodes named by the byte offset of their code
+// (twice the local index, so a code is an address): a parent's offset (below
+// 0x2000), an open root's place among the tile's ids (0x2000 + place), or a
+// closed root's 0x4000 | sides << 12 | size.
+#define TILE_OPEN 0x2000u
 #define TILE_CLOSED 0x4000u
 struct TileState {
     static constexpr bool LDS = true;
-    uint16_t *code;
-    __device__ __forceinline__ uint32_t get(uint32_t i) const { return code[i]; }
-    __device__ __forceinline__ void set(uint32_t i, uint32_t v) const { code[i] = (uint16_t)v; }
+    char *code;
+    __device__ __forceinline__ uint32_t get(uint32_t i) const { return *(uint16_t *)(code + i); }
+    __device__ __forceinline__ void set(uint32_t i, uint32_t v) const { *(uint16_t *)(code + i) = (uint16_t)v; }
     __device__ __forceinline__ bool is_root(uint32_t v) const { return v >= TILE_OPEN; }
 };
 
@@ -2712,15 +2712,11 @@ struct EventBits {
     static constexpr uint32_t half = sizeof(RecT) * 4u;
     static constexpr uint32_t top = 1u << (half - 1u);
     static __device__ __forceinline__ RecT join(uint32_t a, uint32_t b) { return pack_record<RecT>(a | top, b | top); }
-    static __device__ __forceinline__ RecT gain(uint32_t open, uint32_t size, uint32_t f, bool closed_u)
-    {
-        return pack_record<RecT>(open, top | (closed_u ? 0x4000u : 0u) | (f << 12) | size);
-    }
     static __device__ __forceinline__ bool is_event(RecT r) { return (r >> (2u * half - 1u)) != 0; }
 };
 
-// List entries: step, local index of u, and whether v is the node below u
-// (else the one to its right).
+// List entries: step, local index of u (taken as its code's offset), and
+// whether v is the node below u (else the one to its right).
 template <typename ENT>
 struct TileEntry;
 template <>
@@ -2729,7 +2725,7 @@ struct TileEntry<uint32_t> {
     static __device__ __forceinline__ void take(uint32_t e, uint32_t &t, uint32_t &u, uint32_t &down)
     {
         t = e & (TILE_SHORT_STEPS - 1u);
-        u = (e >> 19) & 0xFFFu;
+        u = (e >> 18) & 0x1FFEu;
         down = e >> 31;
     }
 };
@@ -2739,7 +2735,7 @@ struct TileEntry<uint64_t> {
     static __device__ __forceinline__ void take(uint64_t e, uint32_t &t, uint32_t &u, uint32_t &down)
     {
         t = (uint32_t)e;
-        u = (uint32_t)(e >> 32) & 0xFFFu;
+        u = (uint32_t)(e >> 31) & 0x1FFEu;
         down = (uint32_t)(e >> 63);
     }
 };
@@ -2782,7 +2778,7 @@ __global__ __launch_bounds__(256) void tile_init_kernel(
             const uint32_t f = sides ? (uint32_t)sides[g.lat.node(tr * g.h + lr, tc * g.w + lc)] : 0u;
             const bool is_open = (lr == 0u && tr) || (lr + 1u == hh && tr + 1u < g.KH) ||
                                  (lc == 0u && tc) || (lc + 1u == ww && tc + 1u < g.KW);
-            v = ((1u + f) << 14) | 1u;
+            v = TILE_CLOSED | (f << 12) | 1u;
             if (is_open) {
                 const uint32_t id = g.border(lr, lc, hh);
                 v = TILE_OPEN + id;
@@ -2885,7 +2881,7 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(
             const bool ok = (uint32_t)e[i] < M;
             const TileBond b = tile_bond(g, ok ? e[i] : 0);
             const bool in = ok && !b.cross;
-            const uint64_t peers = match_label(b.k, tile_bits, __ballot(in));
+            const uint64_t peers = match_label(b.k, tile_bits, ballot(in));
             at[i] = 0xFFFFFFFFu;
             if (in) {
                 const uint32_t rank = lanes_below(peers);
@@ -2961,8 +2957,9 @@ __global__ __launch_bounds__(64) void tile_sweep_kernel(
     const uint32_t lane = threadIdx.x;
     const uint32_t tr = k / g.KW, tc = k % g.KW;
     const uint32_t n = TileGeo::bonds(g.rows(tr), g.cols(tc));
-    const uint32_t id0 = k * g.per;
-    const TileState st{(uint16_t *)(tile_lds + TILE_CLAIM_SLOTS)};
+    const uint32_t id0 = k * g.per - TILE_OPEN;   // an open code to its id
+    const TileState st{(char *)(tile_lds + TILE_CLAIM_SLOTS)};
+    const uint32_t below = 2u * g.w;   // from a node's code to the one below
     const ENT *list = lists + (int64_t)rl * list_stride + g.offset(tr, tc);
     RecT *rec_out = records + (int64_t)rl * rec_stride;
     {
@@ -2982,7 +2979,7 @@ __global__ __launch_bounds__(64) void tile_sweep_kernel(
     auto batch = [&](ENT cur, ENT next, bool active) __attribute__((always_inline)) {
         uint32_t t, x, y, down;
         TileEntry<ENT>::take(cur, t, x, down);
-        y = x + (down ? g.w : 1u);
+        y = x + (down ? below : 2u);
         x = st.is_root(hint_u) ? x : hint_u;
         y = st.is_root(hint_v) ? y : hint_v;
         uint32_t cx, cy;
@@ -2991,53 +2988,51 @@ __global__ __launch_bounds__(64) void tile_sweep_kernel(
             uint32_t tn, un, dn;
             TileEntry<ENT>::take(next, tn, un, dn);
             hint_u = st.get(un);
-            hint_v = st.get(un + (dn ? g.w : 1u));
+            hint_v = st.get(un + (dn ? below : 2u));
         }
         bool cand = active && x != y;
         RecT rec = 0;
-        while (__ballot(cand)) {
+        while (ballot(cand)) {
             tag += 64u;
             const uint32_t mine = tag + 63u - lane;
             const bool open_x = cx < TILE_CLOSED, open_y = cy < TILE_CLOSED;
-            const uint32_t su = ((x * 0x9E3779u) & 0xFFFFFFu) >> (24 - TILE_CLAIM_BITS);
-            const uint32_t sv = ((y * 0x9E3779u) & 0xFFFFFFu) >> (24 - TILE_CLAIM_BITS);
             // an open root is claimed only where two open ones may join: the
             // join waits for every earlier candidate of either root, which
             // else would name a root it was not yet joined with
             const bool join = open_x && open_y;
-            const bool joins = __ballot(cand && join) != 0u;
+            const bool joins = ballot(cand && join) != 0u;
+            const uint32_t su = (x >> 1) % TILE_CLAIM_SLOTS, sv = (y >> 1) % TILE_CLAIM_SLOTS;
             if (cand && (!open_x || joins))
                 atomicMax(&claims[su], mine);
             if (cand && (!open_y || joins))
                 atomicMax(&claims[sv], mine);
-            const bool go = cand && ((open_x && !join) || claims[su] == mine) &&
-                            ((open_y && !join) || claims[sv] == mine);
-            bool spans_here = false;
-            if (go) {
-                const uint32_t sx = cx & 0x3FFFu, sy = cy & 0x3FFFu;
-                // an open root is the parent of a closed one
-                const bool x_big = open_y ? open_x : (open_x || sx >= sy);
-                const uint32_t big = x_big ? x : y, small = x_big ? y : x;
+            const uint32_t held_x = claims[su], held_y = claims[sv];
+            const bool go = cand && ((open_x && !join) || held_x == mine) &&
+                            ((open_y && !join) || held_y == mine);
+            // an open root is the parent of a closed one
+            const uint32_t sx = cx & 0xFFFu, sy = cy & 0xFFFu;
+            const bool x_big = open_x || (!open_y && sx >= sy);
+            const bool closed = !open_x && !open_y;
+            const uint32_t big = x_big ? x : y, small = x_big ? y : x;
+            const uint32_t sides = (cx | cy) & 0x3000u;
+            const bool spans_here = go && closed && sides == 0x3000u;
+            if (go)
                 st.set(small, big);
-                if (!open_x && !open_y) {
-                    const uint32_t f = ((cx >> 14) - 1u) | ((cy >> 14) - 1u);
-                    spans_here = f == 3u;
-                    st.set(big, ((1u + (f == 3u ? 0u : f)) << 14) | (sx + sy));
-                    rec = pack_record<RecT>(sx, sy);
-                } else {
-                    const uint32_t ix = id0 + cx - TILE_OPEN, iy = id0 + cy - TILE_OPEN;
-                    if (join)
-                        rec = EventBits<RecT>::join(ix, iy);
-                    else
-                        rec = EventBits<RecT>::gain(open_x ? ix : iy, open_x ? sy : sx,
-                                                    ((open_x ? cy : cx) >> 14) - 1u, open_y);
-                }
+            if (go && closed)
+                st.set(big, TILE_CLOSED + (spans_here ? 0u : sides) + sx + sy);
+            if (go) {
+                const uint32_t ix = id0 + cx, iy = id0 + cy;
+                const uint32_t gain = ((open_x ? cy : cx) & 0x3FFFu) | EventBits<RecT>::top |
+                                      (open_x ? 0u : 0x4000u);
+                const uint32_t lo = join ? ix | EventBits<RecT>::top : open_x ? ix : iy;
+                const uint32_t hi = join ? iy | EventBits<RecT>::top : gain;
+                rec = pack_record<RecT>(closed ? sx : lo, closed ? sy : hi);
             }
-            const uint64_t spans = __ballot(spans_here);
+            const uint64_t spans = ballot(spans_here);
             if (spans)
                 span_at = min(span_at, read_lane(t, (uint32_t)__builtin_ctzll(spans)) + 1u);
             cand = cand && !go;
-            if (!__ballot(cand))
+            if (!ballot(cand))
                 break;
             if (cand)
                 find2(st, x, cx, y, cy);
@@ -3141,7 +3136,7 @@ __device__ __forceinline__ void event_run(const St &st, uint32_t M, RecT *rec_io
         for (uint32_t i = 0; i < EVENT_SCAN; ++i) {
             const uint32_t t = t0 + i * 64u + lane;
             const bool is = EventBits<RecT>::is_event(cur[i]) && t < M;
-            const uint64_t m = __ballot(is);
+            const uint64_t m = ballot(is);
             if (is) {
                 uint32_t lo, hi;
                 unpack_record(cur[i], lo, hi);
@@ -3221,7 +3216,7 @@ __device__ __forceinline__ void event_run(const St &st, uint32_t M, RecT *rec_io
         }
         bool cand = active && ru != rv;
         RecT rec = 0;
-        while (__ballot(cand)) {
+        while (ballot(cand)) {
             tag += 64u;
             const uint32_t mine = tag + 63u - lane;
             const uint32_t su = claim_slot(ru), sv = claim_slot(rv);
@@ -3234,20 +3229,20 @@ __device__ __forceinline__ void event_run(const St &st, uint32_t M, RecT *rec_io
             bool go = cand && own_u && own_v;
             uint64_t star = 0;
             uint32_t hub = 0;
-            const uint64_t blocked = __ballot(cand && !go);
+            const uint64_t blocked = ballot(cand && !go);
             if (blocked) {
                 const uint32_t fl = (uint32_t)__builtin_ctzll(blocked);
                 hub = read_lane(own_u ? rv : ru, fl);
                 const bool at_u = ru == hub;
                 const bool touch = cand && (at_u || rv == hub);
-                const uint64_t tm = __ballot(touch);
-                const uint64_t bad = tm & ~__ballot(touch && (at_u ? own_v : own_u));
+                const uint64_t tm = ballot(touch);
+                const uint64_t bad = tm & ~ballot(touch && (at_u ? own_v : own_u));
                 star = bad ? (tm & ((bad & (0u - bad)) - 1u)) : tm;
                 go = go && !touch;
                 const uint32_t hu = tag + 63u - held_u, hv = tag + 63u - held_v;
                 const bool late = cand && !go && !((star >> lane) & 1u) &&
                                   (((star >> (hu & 63u)) & 1u) || ((star >> (hv & 63u)) & 1u));
-                const uint64_t lm = __ballot(late);
+                const uint64_t lm = ballot(late);
                 if (lm)
                     star &= (lm & (0u - lm)) - 1u;
             }
@@ -3262,8 +3257,8 @@ __device__ __forceinline__ void event_run(const St &st, uint32_t M, RecT *rec_io
                 const uint32_t s_hub = read_lane(sh, first), f_hub = read_lane(fh, first);
                 const uint32_t incl = wave_scan_add(in_star ? sx : 0u);
                 const uint32_t total = read_lane(incl, 63u);
-                const uint64_t m1 = __ballot(in_star && (fx & 1u));
-                const uint64_t m2 = __ballot(in_star && (fx & 2u));
+                const uint64_t m1 = ballot(in_star && (fx & 1u));
+                const uint64_t m2 = ballot(in_star && (fx & 2u));
                 const uint32_t f_all = f_hub | (m1 ? 1u : 0u) | (m2 ? 2u : 0u);
                 if (in_star) {
                     if (!gain)
@@ -3294,13 +3289,13 @@ __device__ __forceinline__ void event_run(const St &st, uint32_t M, RecT *rec_io
                 spans_here = f == 3u;
             }
             {
-                const uint64_t spans = __ballot(spans_here);
+                const uint64_t spans = ballot(spans_here);
                 if (spans)
                     span_at = min(span_at, read_lane(t, (uint32_t)__builtin_ctzll(spans)) + 1u);
             }
             cand = cand && !go && !in_star;
             st.sync();
-            if (!__ballot(cand))
+            if (!ballot(cand))
                 break;
             if (cand) {
                 uint32_t z = gain ? ru : rv, cz = cv;
@@ -5391,18 +5386,28 @@ static LatticeEdges lattice_edges(uint32_t length, bool tiled)
 // ---------------------------------------------------------------------------
 // The tiled sweep's plan and launches
 // ---------------------------------------------------------------------------
-// Lattices it takes: state above the LDS limit, a side of at most
-// TILE_MAX_LENGTH.  False otherwise.
-static bool tile_geo(uint32_t length, bool tiled, TileGeo &g)
+// Lattices it takes, and their tiles; false otherwise.
+// - A side of at most TILE_MAX_LENGTH, and more than a tile's.
+// - Below TILE_LDS_LENGTH (a state that fits LDS several times a CU), batches
+//   of at most four runs per CU only: the sweep in milliseconds, untiled and
+//   tiled, is 0.784 and 0.842 for 4000 runs of L = 80, 0.296 and 0.252 for
+//   200; 2.68 and 2.36 for 8000 of L = 100, 7.06 and 5.05 for 10^4 of L = 128,
+//   0.66 and 0.47 for 200 of those.
+// - Tiles of at most 64 x 64 nodes, or 32 x 32 where those would leave the
+//   GPU with at most 2048 wavefronts (200 runs of L = 128: 0.52 and 0.43 ms,
+//   500 of L = 100: 0.40 and 0.38; more tiles make more events).
+static bool tile_geo(uint32_t length, bool tiled, uint32_t num_runs, TileGeo &g)
 {
-    if ((uint64_t)length * length <= kLdsMaxNodes || length > TILE_MAX_LENGTH)
+    if (length <= TILE_SIDE || length > TILE_MAX_LENGTH ||
+        (length < TILE_LDS_LENGTH && num_runs > 1024u))
         return false;
+    const uint32_t k64 = (length + TILE_SIDE - 1u) / TILE_SIDE;
+    const bool small = length <= 512u && (uint64_t)k64 * k64 * num_runs <= 2048u;
+    const uint32_t side = small ? TILE_SIDE / 2u : TILE_SIDE;
     g.lat = lattice_edges(length, tiled);
     g.L = length;
-    g.KH = (length + TILE_ROWS - 1u) / TILE_ROWS;
-    g.KW = (length + TILE_COLS - 1u) / TILE_COLS;
-    g.h = (length + g.KH - 1u) / g.KH;
-    g.w = (length + g.KW - 1u) / g.KW;
+    g.KH = g.KW = (length + side - 1u) / side;
+    g.h = g.w = (length + g.KH - 1u) / g.KH;
     g.K = g.KH * g.KW;
     g.per = 2u * g.w + 2u * (g.h - 2u);
     g.mh = (uint32_t)(((1ull << 32) + g.h - 1u) / g.h);
@@ -5465,7 +5470,8 @@ extern "C" int pc_sweep_lattice_workspace_size(uint32_t length, uint32_t num_run
         return pc_fail(PC_EINVAL, "pc_sweep_lattice_workspace_size: length must be in 1..16384");
     const int rc = pc_sweep_workspace_size(length * length, num_runs, state_mode, bytes);
     TileGeo g;
-    if (rc == PC_OK && num_runs && state_mode == PC_STATE_AUTO && tile_geo(length, false, g))
+    if (rc == PC_OK && num_runs && state_mode == PC_STATE_AUTO &&
+        tile_geo(length, false, num_runs, g))
         *bytes = std::max(*bytes, tile_plan(g, num_runs, tile_slab(g, num_runs)).bytes);
     return rc;
 }
@@ -5552,7 +5558,7 @@ static int tile_sweep(uint32_t length, bool tiled, const uint8_t *d_node_sides,
     const uint32_t rounds = merge_rounds ? merge_rounds : g_merge_rounds;
     const int64_t M = 2ll * length * (length - 1ll);
     if (state_mode != PC_STATE_AUTO || span_on_first_merge || num_runs == 0 || rounds > 64 ||
-        !tile_geo(length, tiled, g) || !d_workspace || ((uintptr_t)d_workspace & 15u) ||
+        !tile_geo(length, tiled, num_runs, g) || !d_workspace || ((uintptr_t)d_workspace & 15u) ||
         !d_span_step || !d_perm || !d_records || perm_stride < M || rec_stride < M)
         return PC_OK;
     uint32_t slab = tile_slab(g, num_runs);

@@ -413,6 +413,7 @@ def _tiled_and_untiled(eng, perm, chunks=True):
     """The sweep as the library picks it and with every node's code in HBM."""
     from pypercolate_amd import _native as nat
     assert eng.state_mode == nat.PC_STATE_AUTO
+    assert eng.workspace_bytes(perm.shape[0]) > 0
     auto = eng.sweep(perm, chunks=chunks)
     eng.state_mode = nat.PC_STATE_HBM | nat.PC_SWEEP_TWO_WAVES
     hbm = eng.sweep(perm, chunks=chunks)
@@ -427,12 +428,15 @@ def _same_sweep(a, b, chunks=True):
         assert np.array_equal(a.chunk_state.cpu().numpy(), b.chunk_state.cpu().numpy())
 
 
-@pytest.mark.parametrize('length,runs', [(129, 5), (136, 9), (181, 40), (192, 3), (255, 2),
-                                         (256, 17), (257, 8), (512, 2), (513, 2), (700, 1),
+@pytest.mark.parametrize('length,runs', [(65, 2), (65, 600), (80, 40), (95, 1024), (96, 1500),
+                                         (100, 3), (127, 700), (128, 200), (128, 1025),
+                                         (129, 5), (129, 300), (136, 9), (181, 40), (192, 3),
+                                         (255, 2), (256, 200), (257, 8), (512, 2), (513, 2), (700, 1),
                                          (1000, 1), (400, 300)])
 def test_tiled_lattice_sweep_equals_untiled(gpu, length, runs):
     """The tiled sweep's records, span steps and chunk states equal those of
-    the sweep with every node's code in HBM: whole and ragged tiles, 32- and
+    the sweep with every node's code in HBM: tiles of up to 32 x 32 nodes (few
+    runs) and 64 x 64, whole and ragged, state within the LDS limit, 32- and
     64-bit records (from 257), 32- and 64-bit list entries (from 513), open
     nodes in LDS (a run or several per CU) and in HBM (1000; 400 for more
     than 256 runs), one workgroup per run or several."""
@@ -441,7 +445,7 @@ def test_tiled_lattice_sweep_equals_untiled(gpu, length, runs):
     _same_sweep(*_tiled_and_untiled(eng, perm))
 
 
-@pytest.mark.parametrize('length', [130, 264])
+@pytest.mark.parametrize('length', [128, 130, 264])
 def test_tiled_lattice_sweep_orders(gpu, length):
     """Orders that are far from random: the bonds in their own order and
     reversed, all bonds down before those to the right, a far corner first;
