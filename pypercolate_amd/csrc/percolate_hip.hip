@@ -4445,11 +4445,13 @@ __global__ __launch_bounds__(256) void f64_to_f32_kernel(
 // precision; the dropped levels and the rounding of the 32-bit integers
 // leave a relative error near 1e-10 for non-negative columns.
 // ---------------------------------------------------------------------------
+// Bound by issue: a step is an FP64 MFMA of 64 cycles and, where no row's
+// window starts or ends, about seven vector instructions beside it (two
+// products, the ratio's broadcast, the load).  L = 1024, 4096 p in [0.3,
+// 0.7], 14 columns: 100 us, 127 with lane shuffles and window tests in every
+// step; the MFMAs alone take 35.
 #define FUSED_REANCHOR 1024
 #define FUSED_F64_UNROLL 8
-#ifndef FUSED_F64_AHEAD
-#define FUSED_F64_AHEAD 1
-#endif
 
 struct FusedCtx {
     const double *x;
@@ -4493,7 +4495,8 @@ __device__ __forceinline__ void walk_init(BinomWalk &b, const FusedCtx &f,
             ln = 1;
         }
     }
-    b.pq = b.p / (1.0 - b.p);
+    // (all mass at k = n when p is 1: no recursion)
+    b.pq = b.p >= 1.0 ? 0.0 : b.p / (1.0 - b.p);
     b.ka = max(k0, st);
     b.kend = min(k1, st + ln);
     b.anchor = b.ka < b.kend ? binom_pmf_outline((double)b.ka, b.n, b.p) : 0.0;
@@ -4530,10 +4533,12 @@ __device__ __forceinline__ bool fused_range(const FusedCtx &f, uint32_t p0,
                                             int64_t quant, int64_t &g_begin,
                                             int64_t &g_end, int64_t &per)
 {
+    // a lane per row, then the extremes over the rows of 16 lanes (all alike)
     int64_t lo = INT64_MAX, hi = 0;
-    for (uint32_t r = 0; r < 16 && p0 + r < f.P; ++r) {
-        const double p = f.ps[p0 + r];
-        int64_t st = f.start[p0 + r], ln = f.len[p0 + r];
+    const uint32_t row = p0 + threadIdx.x % 16u;
+    if (row < f.P) {
+        const double p = f.ps[row];
+        int64_t st = f.start[row], ln = f.len[row];
         if (p <= 0.0) {
             st = 0;
             ln = 1;
@@ -4541,9 +4546,16 @@ __device__ __forceinline__ bool fused_range(const FusedCtx &f, uint32_t p0,
             st = (int64_t)f.n;
             ln = 1;
         }
-        lo = min(lo, st);
-        hi = max(hi, st + ln);
+        lo = st;
+        hi = st + ln;
     }
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) {
+        lo = min(lo, (int64_t)__shfl_xor((long long)lo, off, 64));
+        hi = max(hi, (int64_t)__shfl_xor((long long)hi, off, 64));
+    }
+    lo = (int64_t)read_lane((uint64_t)lo, 0u);
+    hi = (int64_t)read_lane((uint64_t)hi, 0u);
     if (hi <= lo)
         return false;
     per = (hi - lo + slices - 1) / slices;
@@ -4553,7 +4565,32 @@ __device__ __forceinline__ bool fused_range(const FusedCtx &f, uint32_t p0,
     return g_begin < g_end;
 }
 
-__global__ __launch_bounds__(64) void canonical_fused_f64_kernel(
+static __device__ const double kOnes = 1.0;
+
+// Lanes FIRST .. FIRST + 7 of every row of 16 lanes, each to its whole row.
+template <int LANE>
+__device__ __forceinline__ double row_lane(double v)
+{
+    const uint64_t w = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)w, 0x150 + LANE, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(w >> 32), 0x150 + LANE, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <int FIRST>
+__device__ __forceinline__ void row_lanes(double v, double (&out)[FUSED_F64_UNROLL])
+{
+    static_assert(FUSED_F64_UNROLL == 8, "eight lanes");
+    out[0] = row_lane<FIRST>(v);
+    out[1] = row_lane<FIRST + 1>(v);
+    out[2] = row_lane<FIRST + 2>(v);
+    out[3] = row_lane<FIRST + 3>(v);
+    out[4] = row_lane<FIRST + 4>(v);
+    out[5] = row_lane<FIRST + 5>(v);
+    out[6] = row_lane<FIRST + 6>(v);
+    out[7] = row_lane<FIRST + 7>(v);
+}
+
+__global__ __launch_bounds__(64, 3) void canonical_fused_f64_kernel(
     FusedCtx f, uint32_t slices, double *__restrict__ partial)
 {
     const uint32_t lane = threadIdx.x, i = lane % 16u, q = lane / 16u;
@@ -4570,46 +4607,91 @@ __global__ __launch_bounds__(64) void canonical_fused_f64_kernel(
         walk_init(b, f, p0 + i, kq0, kq1);
         // the ratio (n - k + 1) / k depends on k only, shared by the 16 rows
         // of a lane group: each lane divides once per 16 steps, for step
-        // j0 + lane % 16 of group lane / 16, and the steps read it back
-        // with a lane shuffle
+        // j0 + lane % 16 of group lane / 16, and a step takes it from the
+        // lane of its row with a DPP broadcast
         double rr = 0.0;
-        // columns FUSED_F64_AHEAD chunks ahead (a miss to the MALL or HBM
-        // outlasts one chunk of MFMAs several times over)
-        double xq[FUSED_F64_AHEAD][FUSED_F64_UNROLL];
-#pragma unroll
-        for (int d = 0; d < FUSED_F64_AHEAD; ++d)
-#pragma unroll
-            for (int u = 0; u < FUSED_F64_UNROLL; ++u) {
-                const int64_t k = kq0 + d * FUSED_F64_UNROLL + u;
-                xq[d][u] = k < kq1 ? fused_x(f, k, c) : 0.0;
-            }
-        for (int64_t j0 = 0; j0 < Lq; j0 += FUSED_F64_UNROLL) {
+        // Columns one chunk ahead: column C reads a 1 over and over, lanes past
+        // it column 0 (their outputs are not kept); steps past the lane's
+        // range count as 0.
+        const double *xc = c == f.C ? &kOnes : f.x + (c < f.C ? c : 0u);
+        const int64_t stride = c == f.C ? 0 : f.x_stride;
+        const int64_t kl = max(kq1 - 1, (int64_t)0);
+        // the row's window within the lane's range, as steps of the walk
+        const int ja = (int)min(b.ka - kq0, (int64_t)1 << 30);
+        const int je = (int)min(max(b.kend - kq0, (int64_t)0), (int64_t)1 << 30);
+        double xn[FUSED_F64_UNROLL];
+        // FULL: the next chunk lies in every lane's range.  (Both forms of
+        // loads in one loop would be branches, whose loads are waited for
+        // where the branches meet.)
+        auto chunk = [&](int64_t j0, auto full) __attribute__((always_inline)) {
+            constexpr bool FULL = decltype(full)::value;
             double a[FUSED_F64_UNROLL], x[FUSED_F64_UNROLL];
+            const int64_t k0 = kq0 + j0, k1 = k0 + FUSED_F64_UNROLL;
+            const double *next = xc + k1 * stride;
 #pragma unroll
             for (int u = 0; u < FUSED_F64_UNROLL; ++u) {
-                x[u] = xq[0][u];
-#pragma unroll
-                for (int d = 0; d + 1 < FUSED_F64_AHEAD; ++d)
-                    xq[d][u] = xq[d + 1][u];
-                const int64_t k = kq0 + j0 + FUSED_F64_AHEAD * FUSED_F64_UNROLL + u;
-                xq[FUSED_F64_AHEAD - 1][u] = k < kq1 ? fused_x(f, k, c) : 0.0;
+                x[u] = xn[u];
+                if (!FULL) {
+                    x[u] = k0 + u < kq1 ? x[u] : 0.0;
+                    next = xc + min(k1 + u, kl) * stride;
+                }
+                xn[u] = *next;
+                if (FULL)
+                    next += stride;
             }
             if ((j0 & 15) == 0) {
                 const int64_t kr = g_begin + (int64_t)(lane / 16u) * Lq + j0 + (lane % 16u);
-                rr = (b.n - (double)kr + 1.0) / (double)kr;
+                rr = kr ? (b.n - (double)kr + 1.0) / (double)kr : 0.0;
             }
+            double ratio[FUSED_F64_UNROLL];
+            if (j0 & 8)
+                row_lanes<8>(rr, ratio);
+            else
+                row_lanes<0>(rr, ratio);
             const bool fresh = j0 > 0 && j0 % FUSED_REANCHOR == 0;
+            // where no row's window starts or ends in the chunk, a step is the
+            // two products alone: rows before their window, past it, or past P
+            // hold weight 0
+            const int j = (int)j0;
+            double direct = 0.0;
+            const bool anew = fresh && j > ja && j < je;
+            if (anew)
+                direct = binom_pmf_outline((double)k0, b.n, b.p);
+            const double w0 = b.w * ratio[0] * b.pq;
+            b.w = anew ? direct : w0;
+            const bool before = j + FUSED_F64_UNROLL <= ja;
+            if (ballot(before || j >= je || (j > ja && j + FUSED_F64_UNROLL <= je)) == ~0ull) {
+                a[0] = b.w;
 #pragma unroll
-            for (int u = 0; u < FUSED_F64_UNROLL; ++u) {
-                const double ratio = __shfl(rr, (int)(q * 16u) + (int)(j0 & 15) + u, 64);
-                a[u] = walk_step(b, kq0 + j0 + u, fresh && u == 0, ratio);
+                for (int u = 1; u < FUSED_F64_UNROLL; ++u)
+                    a[u] = b.w = b.w * ratio[u] * b.pq;
+            } else {
+#pragma unroll
+                for (int u = 0; u < FUSED_F64_UNROLL; ++u) {
+                    if (u)
+                        b.w = b.w * ratio[u] * b.pq;
+                    b.w = j + u == ja ? b.anchor : b.w;
+                    a[u] = j + u >= ja && j + u < je ? b.w : 0.0;
+                }
+                if (before || j + FUSED_F64_UNROLL >= je)
+                    b.w = 0.0;
             }
 #pragma unroll
             for (int u = 0; u < FUSED_F64_UNROLL; u += 2) {
                 acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], x[u], acc0, 0, 0, 0);
                 acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u + 1], x[u + 1], acc1, 0, 0, 0);
             }
-        }
+        };
+#pragma unroll
+        for (int u = 0; u < FUSED_F64_UNROLL; ++u)
+            xn[u] = xc[min(kq0 + u, kl) * stride];
+        // the last lane group has the shortest range
+        const int64_t jf = min(Lq, g_end - g_begin - 3 * Lq) - 2 * FUSED_F64_UNROLL;
+        int64_t j0 = 0;
+        for (; j0 <= jf; j0 += FUSED_F64_UNROLL)
+            chunk(j0, std::true_type());
+        for (; j0 < Lq; j0 += FUSED_F64_UNROLL)
+            chunk(j0, std::false_type());
     }
     // v_mfma_f64_16x16x4f64: register r holds D[q + 4r][i]
     for (int r = 0; r < 4; ++r) {
@@ -4735,10 +4817,26 @@ __global__ __launch_bounds__(256) void fused_reduce_kernel(
     const int64_t p = idx / C, c = idx % C;
     const uint32_t C1 = C + 1u;
     double num = 0.0, den = 0.0;
-    for (uint32_t s = 0; s < slices; ++s) {
-        const double *row = partial + ((int64_t)s * P + p) * C1;
-        num += row[c];
-        den += row[C];
+    const double *row = partial + p * C1;
+    const int64_t step = (int64_t)P * C1;
+    uint32_t s = 0;
+    for (; s + 8u <= slices; s += 8u) {
+        // eight slices' loads in flight, added in order
+        double v[8], w[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) {
+            v[u] = row[(s + u) * step + c];
+            w[u] = row[(s + u) * step + C];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 8u; ++u) {
+            num += v[u];
+            den += w[u];
+        }
+    }
+    for (; s < slices; ++s) {
+        num += row[s * step + c];
+        den += row[s * step + C];
     }
     out[idx] = num / den;
 }

@@ -130,3 +130,32 @@ def test_fused_deterministic_and_matches_unfused(gpu):
     unfused = E.contract(dx, E.binomial_weights(8000, ps), 'fp64_mfma').cpu().numpy()
     fused = E.canonical_fused(dx, ps, 'fp64_mfma').cpu().numpy()
     np.testing.assert_allclose(fused, unfused, rtol=1e-12)
+
+
+@pytest.mark.parametrize('n,ps', [(300, [0.0, 0.5, 1.0]), (5000, [1e-5, 0.3, 0.3, 0.999]),
+                                  (32512, np.linspace(0.0, 1.0, 33)),
+                                  (200000, np.linspace(0.49, 0.51, 50))])
+def test_fused_infinite_and_nan_columns(gpu, n, ps):
+    """An infinity inside a row's window makes that row's average of its
+    column infinite, a NaN makes it NaN; rows whose window (and whose
+    neighbours' windows) are far from them, and other columns, are as
+    without."""
+    rng = np.random.RandomState(n)
+    x = rng.rand(n + 1, 4)
+    ps = np.asarray(ps, dtype=np.float64)
+    clean = E.FusedPlan(gpu.from_numpy(x).cuda(), ps).run().cpu().numpy()
+    k = n // 3
+    y = x.copy()
+    y[k, 1], y[k, 2] = np.inf, np.nan
+    got = E.FusedPlan(gpu.from_numpy(y).cuda(), ps).run().cpu().numpy()
+    np.testing.assert_array_equal(got[:, [0, 3]], clean[:, [0, 3]])
+    start, length = E.binomial_windows(n, ps)
+    inside = (start <= k) & (k < start + length) & (ps > 0) & (ps < 1)
+    assert np.isnan(got[inside, 2]).all()
+    assert (np.isinf(got[inside, 1]) | np.isnan(got[inside, 1])).all()
+    # tiles of 16 sorted p share the steps of the union of their windows
+    tiles = np.arange(ps.size) // 16
+    lo = np.array([start[tiles == t].min() for t in tiles])
+    hi = np.array([(start + length)[tiles == t].max() for t in tiles])
+    far = (k < lo) | (k >= hi)
+    np.testing.assert_array_equal(got[far], clean[far])
