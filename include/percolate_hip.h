@@ -296,6 +296,15 @@ int pc_expand_traces(uint32_t num_nodes, uint32_t num_edges, uint32_t num_runs,
 int pc_binomial_window(uint32_t n, double p, int64_t *start, int64_t *len);
 
 /*
+ * The p grid of pc_canonical_fused on the device: d_ps[i] = ps[i] (ps on the
+ * host, read before the call returns) and the windows of pc_binomial_window
+ * at each, d_start[i] and d_len[i].  Kernels only, the values in their
+ * arguments, so nothing is copied or waited for.
+ */
+int pc_binomial_grid(uint32_t n, uint32_t num_p, const double *ps, double *d_ps,
+                     int64_t *d_start, int64_t *d_len, void *stream);
+
+/*
  * Binomial weights B(n, k; p) for num_p values p = d_ps[i] over the windows
  * (d_start[i], d_len[i]): d_w[i * kmax + j] = B(n, d_start[i] + j; p),
  * normalised to sum 1 over the window, 0 for j >= d_len[i].  Replaces the

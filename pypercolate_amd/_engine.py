@@ -659,7 +659,7 @@ class FusedPlan(object):
     windows share the tile's work) and the rows returned in the caller's
     order.  precision: 'fp64_mfma' or 'split_bf16'."""
 
-    def __init__(self, x, ps, precision='fp64_mfma'):
+    def __init__(self, x, ps, precision='fp64_mfma', _wait=True):
         torch = nat.torch_cuda()
         self.lib = nat.load_library()
         self.precision = nat.PRECISIONS.get(precision, precision)
@@ -672,14 +672,28 @@ class FusedPlan(object):
         self.n = self.S - 1
         ps = np.atleast_1d(np.asarray(ps, dtype=np.float64))
         self.P = ps.size
-        order = np.argsort(ps, kind='stable')
         self.ps = ps
-        start, length = binomial_windows(self.n, ps[order])
         dev = self.x.device
-        self.d_ps = torch.from_numpy(ps[order].copy()).to(dev)
-        self.d_start = torch.from_numpy(start).to(dev)
-        self.d_len = torch.from_numpy(length).to(dev)
-        self.unsort = torch.from_numpy(np.argsort(order).astype(np.int64)).to(dev)
+        if ps.ndim != 1 or not ((ps >= 0) & (ps <= 1)).all():
+            binomial_windows(self.n, ps)        # raises for the first bad p
+            ps = ps.ravel()
+        # a sorted grid needs no reordering of the rows
+        self.unsort = None
+        grid = ps
+        if self.P and not (ps[1:] >= ps[:-1]).all():
+            order = np.argsort(ps, kind='stable')
+            self.unsort = torch.from_numpy(np.argsort(order).astype(np.int64)).to(dev)
+            grid = ps[order]
+        grid = np.ascontiguousarray(grid)
+        buf = torch.empty((3, self.P), dtype=torch.int64, device=dev)
+        self.d_start, self.d_len = buf[0], buf[1]
+        self.d_ps = buf[2].view(torch.float64)
+        nat.check(self.lib.pc_binomial_grid(
+            self.n, self.P, ctypes.c_void_p(grid.ctypes.data), nat.ptr(self.d_ps),
+            nat.ptr(self.d_start), nat.ptr(self.d_len), nat.stream_handle(torch)),
+            'pc_binomial_grid')
+        if _wait:       # a plan may run on another stream than it was made on
+            torch.cuda.current_stream().synchronize()
         b = ctypes.c_uint64(0)
         nat.check(self.lib.pc_canonical_fused_workspace_size(
             self.P, self.C, self.precision, ctypes.byref(b)),
@@ -691,25 +705,31 @@ class FusedPlan(object):
                                       device=dev)
         self.out = None
 
-    def launch(self):
-        """Enqueue the kernels (sorted-order result in self.sorted_out)."""
+    def launch(self, out=None):
+        """Enqueue the kernels (sorted-order result in self.sorted_out, or
+        in out)."""
         torch = nat.torch_cuda()
         if self.P and self.C:
             nat.check(self.lib.pc_canonical_fused(
                 self.n, self.C, nat.ptr(self.x), self.C, self.P,
                 nat.ptr(self.d_ps), nat.ptr(self.d_start), nat.ptr(self.d_len),
-                nat.ptr(self.sorted_out), self.precision, nat.ptr(self.ws),
-                self.ws_bytes, nat.stream_handle(torch)), 'pc_canonical_fused')
+                nat.ptr(self.sorted_out if out is None else out), self.precision,
+                nat.ptr(self.ws), self.ws_bytes, nat.stream_handle(torch)),
+                'pc_canonical_fused')
 
     def run(self):
-        self.launch()
-        self.out = self.sorted_out[:self.P].index_select(0, self.unsort)
+        if self.unsort is None:
+            self.out = self.sorted_out.new_empty((self.P, self.C))
+            self.launch(self.out)
+        else:
+            self.launch()
+            self.out = self.sorted_out[:self.P].index_select(0, self.unsort)
         return self.out
 
 
 def canonical_fused(x, ps, precision='fp64_mfma'):
     """See FusedPlan: (P, C) float64 device tensor."""
-    return FusedPlan(x, ps, precision).run()
+    return FusedPlan(x, ps, precision, _wait=False).run()
 
 
 def micro_ci(sum1, sum2, num_edges, num_runs, alpha):

@@ -66,6 +66,7 @@ SIGNATURES = {
     'pc_binomial_window': (ctypes.c_int, [_u32, ctypes.c_double,
                                           ctypes.POINTER(_i64),
                                           ctypes.POINTER(_i64)]),
+    'pc_binomial_grid': (ctypes.c_int, [_u32, _u32, _vp, _vp, _vp, _vp, _vp]),
     'pc_binomial_weights': (ctypes.c_int, [_u32, _u32, _vp, _vp, _vp, _i64,
                                            _vp, _vp]),
     'pc_contract_workspace_size': (ctypes.c_int, [_u32, _u32, _i32,

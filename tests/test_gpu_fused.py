@@ -132,6 +132,32 @@ def test_fused_deterministic_and_matches_unfused(gpu):
     np.testing.assert_allclose(fused, unfused, rtol=1e-12)
 
 
+def test_grid_windows_equal_host_windows(gpu):
+    """The p grid and windows written by pc_binomial_grid (several launches'
+    worth, the ends of [0, 1] among them) equal pc_binomial_window's; a plan
+    over an unsorted grid returns the rows in the caller's order, a sorted
+    one a new tensor for every run, and a bad p raises."""
+    rng = np.random.RandomState(5)
+    for n in (1, 2, 47, 480, 32512, 2095104):
+        ps = np.sort(np.concatenate([[0.0, 1.0, 0.5, 1e-300, 1 - 2.0 ** -53], rng.rand(1000)]))
+        x = gpu.from_numpy(rng.rand(n + 1, 3)).cuda() if n < 40000 else \
+            gpu.zeros((n + 1, 3), dtype=gpu.float64, device='cuda')
+        plan = E.FusedPlan(x, ps)
+        start, length = E.binomial_windows(n, ps)
+        np.testing.assert_array_equal(plan.d_start.cpu().numpy(), start)
+        np.testing.assert_array_equal(plan.d_len.cpu().numpy(), length)
+        np.testing.assert_array_equal(plan.d_ps.cpu().numpy(), ps)
+        first = plan.run()
+        second = plan.run()
+        assert first.data_ptr() != second.data_ptr()
+        order = rng.permutation(ps.size)
+        shuffled = E.FusedPlan(x, ps[order]).run()
+        np.testing.assert_array_equal(shuffled.cpu().numpy(), first.cpu().numpy()[order])
+    for bad in (-0.1, 1.5, np.nan):
+        with pytest.raises(ValueError):
+            E.FusedPlan(x, [0.2, bad])
+
+
 @pytest.mark.parametrize('n,ps', [(300, [0.0, 0.5, 1.0]), (5000, [1e-5, 0.3, 0.3, 0.999]),
                                   (32512, np.linspace(0.0, 1.0, 33)),
                                   (200000, np.linspace(0.49, 0.51, 50))])
