@@ -17,6 +17,8 @@ percolation cluster spans once it contains nodes attached to both sides
 a pre-joined structure reports spanning from the first merge on.
 """
 
+from itertools import chain
+
 import numpy as np
 
 
@@ -132,6 +134,31 @@ def spanning_side_flags(node_index, auxiliary_node_attributes,
     return flags, False
 
 
+def _edges_in_order(perc_graph, nodes, index):
+    """The edges of perc_graph in networkx's order, as pairs of labels.
+
+    The edges of a subgraph view pass three layers of filters a neighbour
+    (3.8 ms a call of 40 runs on 32 x 32 nodes, 1.4 without), so the edges of a node
+    subgraph of a plain Graph are read from the graph below it: every
+    neighbour that is in the view and not before the node, in the graph's
+    own order.  Anything else (other classes, edge filters, views of views,
+    an adjacency in another order than the nodes) is asked itself."""
+    import networkx as nx
+    base = getattr(perc_graph, '_graph', None)
+    if (type(perc_graph) is nx.Graph and type(base) is nx.Graph
+            and not hasattr(base, '_graph')
+            and getattr(perc_graph, '_EDGE_OK', None) is nx.filters.no_filter
+            and isinstance(getattr(perc_graph, '_NODE_OK', None), nx.filters.show_nodes)
+            and list(base._adj) == list(base._node)):
+        adj = base._adj
+        get = index.get
+        return [(node, other) for i, node in enumerate(nodes)
+                for other in adj[node] if get(other, -1) >= i]
+    # a comprehension, not list(): list() asks the networkx views for their
+    # length first, which sums the degrees of every node
+    return [edge for edge in perc_graph.edges()]
+
+
 def from_percolation_graph(perc_graph, spanning_cluster=True,
                            auxiliary_node_attributes=None,
                            auxiliary_edge_attributes=None,
@@ -139,12 +166,10 @@ def from_percolation_graph(perc_graph, spanning_cluster=True,
     """GraphArrays of the keyword dict percolate.percolation_graph() returns
     (percolate/percolate.py:31-100), or of the same keywords passed to the
     percolate.hpc functions."""
-    # comprehensions, not list(): list() asks the networkx views for their
-    # length first, which sums the degrees of every node
     nodes = [node for node in perc_graph.nodes()]
     index = {node: i for i, node in enumerate(nodes)}
-    edge_list = [edge for edge in perc_graph.edges()]
-    edges = np.fromiter((index[node] for edge in edge_list for node in edge),
+    edge_list = _edges_in_order(perc_graph, nodes, index)
+    edges = np.fromiter(map(index.__getitem__, chain.from_iterable(edge_list)),
                         dtype=np.int32, count=2 * len(edge_list)).reshape(-1, 2)
     node_sides = None
     span_first = False

@@ -119,3 +119,43 @@ def test_locality_order_tiles_grid_nodes():
             idx = np.sort(order[sel])
             assert (np.diff(idx) == 1).all()
     assert _graph.locality_order(_graph.linear_chain(10)) is None
+
+
+def _views():
+    grid = nx.grid_2d_graph(6, 5)
+    loops = nx.Graph([(3, 1), (1, 1), (2, 3), (5, 2), (5, 5), (0, 3), (1, 2), (7, 0), (2, 2)])
+    mixed = nx.Graph([(1, 2.0), (2, 'a'), ('a', 1.0), ('b', 1), (2, 'b')])
+    few = nx.path_graph(40)
+    for name, g, keep in [('grid', grid, [n for n in grid if n[0]]), ('loops', loops, [5, 3, 2, 1]),
+                          ('mixed', mixed, ['a', 1, 2]), ('few', few, [7, 3, 4, 8, 30]),
+                          ('all', grid, list(grid)), ('none of them', loops, [3]),
+                          ('missing', grid, [(1, 1), (1, 2), (99, 99)])]:
+        yield name, g.subgraph(keep)
+    yield 'view of a view', grid.subgraph(list(grid)[3:]).subgraph(list(grid)[5:20])
+    yield 'edge filter', nx.subgraph_view(grid, filter_edge=lambda a, b: sum(a) % 2)
+    yield 'edge subgraph', grid.edge_subgraph(list(grid.edges())[::3])
+    yield 'node filter', nx.subgraph_view(grid, filter_node=lambda n: n[1] != 2)
+    yield 'filter on a view', nx.subgraph_view(grid.subgraph(list(grid)[3:]),
+                                               filter_edge=lambda a, b: a[0] != 3)
+    yield 'multigraph', nx.MultiGraph([(0, 1), (1, 2), (0, 1), (2, 3)]).subgraph([1, 0, 2])
+    yield 'directed', nx.DiGraph([(2, 1), (0, 2), (1, 0), (2, 3)]).subgraph([1, 0, 2])
+    changed = nx.Graph([(0, 1), (1, 2), (2, 3), (3, 0)])
+    view = changed.subgraph([0, 1, 2, 3, 9])
+    changed.remove_node(1)
+    changed.add_edges_from([(9, 3), (9, 1), (1, 2), (0, 2)])
+    yield 'changed after the view', view
+    yield 'no view', grid
+
+
+@pytest.mark.parametrize('name,view', list(_views()), ids=[n for n, _ in _views()])
+def test_edges_of_views_in_networkx_order(name, view):
+    """The edges read from below a subgraph view equal the view's own."""
+    a = _graph.from_percolation_graph(view, spanning_cluster=False)
+    expected = list(view.edges())
+    nodes = list(view.nodes())
+    assert a.nodes == nodes
+    assert [a.edge_labels(i) for i in range(a.num_edges)] == expected
+    assert [tuple(map(type, a.edge_labels(i))) for i in range(a.num_edges)] == \
+        [tuple(map(type, e)) for e in expected]
+    index = {n: i for i, n in enumerate(nodes)}
+    assert a.edges.tolist() == [[index[u], index[v]] for u, v in (e[:2] for e in expected)]
