@@ -427,12 +427,18 @@ class Pipeline(object):
         torch = self.torch
         eng = self.engine
         main = torch.cuda.current_stream()
-        ss0, ss1, sr = self.streams
+        nsub = (self.R + self.sub - 1) // self.sub
+        # one sub-batch without a draw ahead has nothing to overlap: all of
+        # it on the caller's stream (L = 16, 40 RandomState runs: 170 us a
+        # run() with the waits between four streams, 91 without)
+        side = nsub > 1 or self.prefetch
+        ss0, ss1, sr = self.streams if side else (main, main, main)
         sp = main
-        start = torch.cuda.Event()
-        start.record(main)
-        for s in self.streams:
-            s.wait_event(start)
+        if side:
+            start = torch.cuda.Event()
+            start.record(main)
+            for s in self.streams:
+                s.wait_event(start)
         self.sweep_events = []
         first = True
         fused = eng.fuse_chunk_states()
@@ -446,15 +452,15 @@ class Pipeline(object):
                                             workspace=self.perm_ws)
                 else:
                     eng.randomstate_permutations(self.d_seeds, out=self.perm)
-                have_all = torch.cuda.Event()
-                have_all.record(sp)
-        nsub = (self.R + self.sub - 1) // self.sub
+                if side:
+                    have_all = torch.cuda.Event()
+                    have_all.record(sp)
         for i, b0 in enumerate(range(0, self.R, self.sub)):
             n = min(self.sub, self.R - b0)
             ss = (ss0, ss1)[i & 1]
             perm = self.perm[b0:b0 + n]
             if self.permute_ahead:
-                have_perm = have_all
+                have_perm = have_all if side else None
             else:
                 with torch.cuda.stream(sp):
                     if self.d_seeds is None:
@@ -462,9 +468,12 @@ class Pipeline(object):
                                                 workspace=self.perm_ws)
                     else:
                         eng.randomstate_permutations(self.d_seeds[b0:b0 + n], out=perm)
-                    have_perm = torch.cuda.Event()
-                    have_perm.record(sp)
-            ss.wait_event(have_perm)
+                    have_perm = None
+                    if side:
+                        have_perm = torch.cuda.Event()
+                        have_perm.record(sp)
+            if side:
+                ss.wait_event(have_perm)
             with torch.cuda.stream(ss):
                 e0 = torch.cuda.Event(enable_timing=True)
                 e0.record(ss)
@@ -476,7 +485,8 @@ class Pipeline(object):
                 e1 = torch.cuda.Event(enable_timing=True)
                 e1.record(ss)
             self.sweep_events.append((e0, e1))
-            sr.wait_event(e1)
+            if side:
+                sr.wait_event(e1)
             with torch.cuda.stream(sr):
                 if not fused:
                     res.chunk_state = eng.chunk_scan(res, out=self.state[b0:b0 + n])
@@ -498,10 +508,11 @@ class Pipeline(object):
         if self.prefetch:
             self.cur = 1 - self.cur
             self.prefetched = True
-        for s in self.streams:
-            done = torch.cuda.Event()
-            done.record(s)
-            main.wait_event(done)
+        if side:
+            for s in self.streams:
+                done = torch.cuda.Event()
+                done.record(s)
+                main.wait_event(done)
         return self.sum1, self.sum2
 
     def sweep_ms(self):
