@@ -93,3 +93,43 @@ def test_run_moments(gpu, R, cols):
     np.testing.assert_allclose(mean.cpu().numpy(), mu, rtol=1e-13)
     d2 = ((q - mu[:, None, :]) ** 2).sum(axis=1)
     np.testing.assert_allclose(m2.cpu().numpy(), d2, rtol=1e-10, atol=1e-12)
+
+
+@pytest.mark.parametrize('S,lens,C', [
+    (1, [1], 64), (2, [2], 65), (3, [1, 2, 3, 0, 3], 64), (4, [4, 0, 1, 3, 2], 66),
+    (15, list(range(16)) * 5, 127), (16, [16] * 64, 128), (17, [17, 3, 16, 1] * 17, 129),
+    (31, [5, 0, 31] * 43, 70), (33, [33, 1, 2, 15, 16, 17] * 11, 191),
+    (700, [3, 700, 64, 1, 350] * 26, 65), (2500, [1200] * 200, 4096)])
+def test_contract_wide_windows(gpu, S, lens, C):
+    """The wide kernel's blocks of 16 steps against windows of every length
+    and phase (shorter than the four weights a lane reads, empty, starting
+    and ending inside a block, the last ending at the last step), p and
+    column counts around its tiles, with and without K-slices, and the
+    columns of a wider X."""
+    rng = np.random.RandomState(S + C)
+    lens = np.minimum(np.array(lens, dtype=np.int64), S)
+    start = np.array([rng.randint(0, S - n + 1) for n in lens], dtype=np.int64)
+    start[-1] = S - lens[-1]
+    if S == 2500:       # neighbouring p share most of their steps
+        start = np.sort(start)
+    kmax = max(int(lens.max()), 1)
+    w = rng.rand(len(lens), kmax) - 0.3
+    x = np.ascontiguousarray(rng.rand(S, C) * 10.0 ** (np.arange(C) % 5))
+    wt = E.Weights(S - 1, np.zeros(len(lens)), gpu.from_numpy(start).cuda(),
+                   gpu.from_numpy(lens).cuda(), kmax, gpu.from_numpy(w).cuda())
+    wt.host_start, wt.host_length = start, lens
+    ref = _numpy_contract(x, wt)[0]
+    mag = np.array([np.abs(w[i, :n]) @ x[a:a + n]        # sum of |w X|
+                    for i, (a, n) in enumerate(zip(start, lens))])
+    q = E.contract(gpu.from_numpy(x).cuda(), wt, 'fp64_mfma').cpu().numpy()
+    assert (np.abs(q - ref) <= 1e-13 * mag).all()
+    # an infinite step outside every window changes nothing
+    used = np.zeros(S, dtype=bool)
+    for a, n in zip(start, lens):
+        used[a:a + n] = True
+    lo, hi = (np.nonzero(used)[0][[0, -1]] if used.any() else (0, S - 1))
+    y = x.copy()
+    y[:lo] = np.inf
+    y[hi + 1:] = np.nan
+    z = E.contract(gpu.from_numpy(y).cuda(), wt, 'fp64_mfma').cpu().numpy()
+    np.testing.assert_array_equal(z, q)
