@@ -379,6 +379,32 @@ __device__ __forceinline__ uint64_t match_label(uint32_t label, uint32_t bits,
     return ((uint64_t)hi << 32) | lo;
 }
 
+// match_label through LDS: every lane sets its bit in the mask of its label's
+// low MATCH_BITS bits, a table of the wave's own (all zero before and after),
+// and reads the mask back; only the bits above cost a ballot, of four vector
+// instructions each.  Lanes outside `ok` get no peers.  The kernels that group
+// by label are bound by vector issue (80 to 92 % busy with a ballot for each
+// of 7 to 9 bits), so this pays: grouping by 512 labels, 2.1e9 edges, 7.1 ms
+// with ballots and labels drawn twice, 5.0; whole runs of 32512 edges (10^4)
+// 1.17 ms, 0.97 (5, 6 and 8 bits here: 1.08, 1.03 and 1.32, where the tables
+// leave room for fewer workgroups).
+#define MATCH_BITS 7u
+#define MATCH_WORDS (2u << MATCH_BITS)   // 32-bit words of a wave's table
+
+__device__ __forceinline__ uint64_t match_label_lds(uint32_t label, uint32_t bits,
+                                                    bool ok, unsigned long long *table)
+{
+    unsigned long long *slot = table + (label & ((1u << MATCH_BITS) - 1u));
+    uint64_t peers = 0;
+    if (ok) {
+        __hip_atomic_fetch_or(slot, 1ull << (threadIdx.x & 63u), __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_WORKGROUP);
+        peers = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    return bits > MATCH_BITS ? match_label(label >> MATCH_BITS, bits - MATCH_BITS, peers) : peers;
+}
+
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -427,29 +453,24 @@ __device__ __forceinline__ void shuffle_sub(E *a, uint32_t c, uint32_t st,
                                             uint32_t run, uint32_t b, uint32_t k0,
                                             uint32_t k1)
 {
-    uint32_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
-    uint32_t h = 8u, u = 0u, v = 0u;
-    for (uint32_t j = c - 1u; j >= 1u; --j) {
-        const uint32_t r = j + 1u;
-        if (h == 8u) {
-            const u32x4 w = shuf_philox(st, run, b, (3u << 28) | u, k0, k1);
-            w0 = w.x;
-            w1 = w.y;
-            w2 = w.z;
-            w3 = w.w;
-            ++u;
-            h = 0u;
+    uint32_t v = 0u;
+    // eight draws a Philox call
+    for (uint32_t j0 = c - 1u, u = 0u; (int32_t)j0 >= 1; j0 -= 8u, ++u) {
+        const u32x4 w = shuf_philox(st, run, b, (3u << 28) | u, k0, k1);
+#pragma unroll
+        for (uint32_t h = 0; h < 8u; ++h) {
+            const uint32_t j = j0 - h, r = j + 1u;
+            if ((int32_t)j < 1)
+                break;
+            // 16-bit word times r <= 2^15 + 1: a 24-bit multiply is exact
+            uint32_t m = __umul24(half16(w, h), r);
+            if (__builtin_expect((m & 0xFFFFu) < r, 0))
+                m = shuffle_redraw(m, r, st, run, b, k0, k1, v);
+            const uint32_t k = m >> 16;
+            const E t = a[j];
+            a[j] = a[k];
+            a[k] = t;
         }
-        const uint32_t wd = (h & 4u) ? ((h & 2u) ? w3 : w2) : ((h & 2u) ? w1 : w0);
-        // 16-bit word times r <= 2^15 + 1: a 24-bit multiply is exact
-        uint32_t m = __umul24((wd >> ((h & 1u) * 16u)) & 0xFFFFu, r);
-        ++h;
-        if (__builtin_expect((m & 0xFFFFu) < r, 0))
-            m = shuffle_redraw(m, r, st, run, b, k0, k1, v);
-        const uint32_t k = m >> 16;
-        const E t = a[j];
-        a[j] = a[k];
-        a[k] = t;
     }
 }
 
@@ -628,10 +649,11 @@ __global__ __launch_bounds__(64 * SHUF_W) void shuffle_scatter_kernel(
     uint32_t chunks, uint32_t r0, uint32_t rn, const uint32_t *__restrict__ counts,
     int32_t *__restrict__ perm, int64_t stride)
 {
-    __shared__ int32_t sval[SHUF_CHUNK];
-    __shared__ uint16_t slab[SHUF_CHUNK];
+    __shared__ unsigned long long masks[SHUF_W * MATCH_WORDS / 2u];
+    __shared__ uint32_t sorted[SHUF_CHUNK];   // label << 16 | place in the chunk
     __shared__ uint32_t wsum[SHUF_W];
-    extern __shared__ uint32_t dyn[];  // [SHUF_W][nb1] bases, lstart, gbase
+    extern __shared__ uint32_t dyn[];  // [SHUF_W][nb1] bases, [nb1] moves
+    constexpr uint32_t GPW = SHUF_CHUNK / (512u * SHUF_W);
     const uint32_t T = 64u * SHUF_W, tid = threadIdx.x, lane = tid & 63u,
                    wave = tid >> 6;
     const uint32_t nb1 = 1u << lb1;
@@ -639,25 +661,29 @@ __global__ __launch_bounds__(64 * SHUF_W) void shuffle_scatter_kernel(
     if (!shuf_block(chunks, rn, rl, c))
         return;
     const uint32_t r = r0 + rl, run = first_run + r;
-    uint32_t *base = dyn, *lstart = dyn + SHUF_W * nb1, *gbase = lstart + nb1;
+    uint32_t *base = dyn, *move = dyn + SHUF_W * nb1;
     uint32_t *my = base + wave * nb1;
     for (uint32_t i = tid; i < SHUF_W * nb1; i += T)
         base[i] = 0u;
+    for (uint32_t i = tid; i < SHUF_W * MATCH_WORDS / 2u; i += T)
+        masks[i] = 0ull;
     __syncthreads();
     const ShufChunk ch = shuf_chunk(c, M);
-    for (uint32_t g = ch.g0; g < ch.g1; ++g) {
-        const u32x4 key = lb1 ? shuf_philox((g << 6) | lane, run, 0u, 1u << 28, k0, k1)
-                              : u32x4{0, 0, 0, 0};
+    u32x4 keys[GPW];
+#pragma unroll
+    for (uint32_t gi = 0; gi < GPW; ++gi) {
+        const uint32_t g = ch.g0 + gi;
+        keys[gi] = shuf_philox((g << 6) | lane, run, 0u, 1u << 28, k0, k1);
 #pragma unroll
         for (uint32_t k = 0; k < 8u; ++k) {
             const uint32_t i = g * 512u + k * 64u + lane;
-            if (i < ch.hi)
-                atomicAdd(&my[lb1 ? half16(key, k) >> (16u - lb1) : 0u], 1u);
+            if (g < ch.g1 && i < ch.hi)
+                atomicAdd(&my[half16(keys[gi], k) >> (16u - lb1)], 1u);
         }
     }
     __syncthreads();
     // local bucket starts (exclusive over buckets of the chunk's totals),
-    // per-wave local bases, and the chunk's global base of each bucket
+    // per-wave local bases, and from there to the chunk's place in the bucket
     {
         const uint32_t per = (nb1 + T - 1u) / T;
         const uint32_t a = min(tid * per, nb1), e = min(a + per, nb1);
@@ -673,8 +699,7 @@ __global__ __launch_bounds__(64 * SHUF_W) void shuffle_scatter_kernel(
         for (uint32_t w = 0; w < wave; ++w)
             acc += wsum[w];
         for (uint32_t b = a; b < e; ++b) {
-            lstart[b] = acc;
-            gbase[b] = counts[((uint64_t)r * nb1 + b) * chunks + c];
+            move[b] = counts[((uint64_t)r * nb1 + b) * chunks + c] - acc;
             for (uint32_t w = 0; w < (uint32_t)SHUF_W; ++w) {
                 const uint32_t n = base[w * nb1 + b];
                 base[w * nb1 + b] = acc;
@@ -683,21 +708,19 @@ __global__ __launch_bounds__(64 * SHUF_W) void shuffle_scatter_kernel(
         }
     }
     __syncthreads();
-    for (uint32_t g = ch.g0; g < ch.g1; ++g) {
-        const u32x4 key = lb1 ? shuf_philox((g << 6) | lane, run, 0u, 1u << 28, k0, k1)
-                              : u32x4{0, 0, 0, 0};
+#pragma unroll
+    for (uint32_t gi = 0; gi < GPW; ++gi) {
+        const uint32_t g = ch.g0 + gi;
 #pragma unroll
         for (uint32_t k = 0; k < 8u; ++k) {
             const uint32_t i = g * 512u + k * 64u + lane;
-            const bool ok = i < ch.hi;
-            const uint64_t valid = ballot(ok);
-            const uint32_t bkt = lb1 ? half16(key, k) >> (16u - lb1) : 0u;
-            const uint64_t peers = match_label(bkt, lb1, valid);
+            const bool ok = g < ch.g1 && i < ch.hi;
+            const uint32_t bkt = half16(keys[gi], k) >> (16u - lb1);
+            const uint64_t peers = match_label_lds(bkt, lb1, ok, masks + wave * (MATCH_WORDS / 2u));
             if (ok) {
                 const uint32_t rank = lanes_below(peers);
                 const uint32_t at = my[bkt];
-                sval[at + rank] = (int32_t)i;
-                slab[at + rank] = (uint16_t)bkt;
+                sorted[at + rank] = bkt << 16 | (i - ch.lo);
                 if (rank == 0u)
                     my[bkt] = at + (uint32_t)__popcll(peers);
             }
@@ -707,8 +730,8 @@ __global__ __launch_bounds__(64 * SHUF_W) void shuffle_scatter_kernel(
     int32_t *row = perm + (int64_t)r * stride;
     const uint32_t n = ch.hi - ch.lo;
     for (uint32_t t = tid; t < n; t += T) {
-        const uint32_t b = slab[t];
-        row[gbase[b] + (t - lstart[b])] = sval[t];
+        const uint32_t v = sorted[t];
+        row[move[v >> 16] + t] = (int32_t)(ch.lo + (v & 0xFFFFu));
     }
 }
 
@@ -727,13 +750,13 @@ __host__ __device__ __forceinline__ uint32_t shuf_hist_words(uint32_t cap)
 // ent[] (16-bit), Fisher-Yates of each sub-bucket (one thread each), then
 // a[t] = old a[ent[t]] (all loads in flight together, all stores after a
 // barrier), or a[t] = ent[t] when a is the identity (IDENT: the whole run
-// is one bucket).  hist holds W * hw words, wsum W; GPW bounds the groups
-// of 512 positions a wave labels.
+// is one bucket).  hist holds W * hw words, wsum W, masks W tables of
+// match_label_lds; GPW bounds the groups of 512 positions a wave labels.
 template <int W, int GPW, bool IDENT>
 __device__ void shuffle_group_lds(uint32_t n, uint32_t b, uint32_t run,
                                   uint32_t k0, uint32_t k1, int32_t *a,
                                   uint16_t *ent, uint32_t *hist, uint32_t hw,
-                                  uint32_t *wsum)
+                                  uint32_t *wsum, unsigned long long *masks)
 {
     const uint32_t T = 64u * W, tid = threadIdx.x, wave = tid >> 6,
                    lane = tid & 63u;
@@ -747,6 +770,8 @@ __device__ void shuffle_group_lds(uint32_t n, uint32_t b, uint32_t run,
 
     for (uint32_t i = tid; i < W * hw; i += T)
         hist[i] = 0u;
+    for (uint32_t i = tid; i < W * (MATCH_WORDS / 2u); i += T)
+        masks[i] = 0ull;
     __syncthreads();
 
     // labels of this wave's positions (8 per Philox call, kept for the
@@ -818,9 +843,8 @@ __device__ void shuffle_group_lds(uint32_t n, uint32_t b, uint32_t run,
             for (uint32_t k = 0; k < 8u; ++k) {
                 const uint32_t j = g * 512u + k * 64u + lane;
                 const bool ok = j < n;
-                const uint64_t valid = ballot(ok);
                 const uint32_t s = lb ? half16(keys[gi], k) >> (16u - lb) : 0u;
-                const uint64_t peers = match_label(s, lb, valid);
+                const uint64_t peers = match_label_lds(s, lb, ok, masks + wave * (MATCH_WORDS / 2u));
                 if (ok) {
                     const uint32_t rank = lanes_below(peers);
                     const uint32_t sh = (s & 1u) * 16u;
@@ -888,7 +912,8 @@ __global__ __launch_bounds__(64 * W) void shuffle_group_kernel(
         IDENT ? (W == 2 ? SHUF_SMALL_CAP : SHUF_WHOLE) : SHUF_GROUP_CAP;
     constexpr int GPW = (int)(CAP / (512u * W));
     const uint32_t hw = shuf_hist_words(cap);
-    uint32_t *hist = gdyn, *wsum = gdyn + W * hw;
+    unsigned long long *masks = (unsigned long long *)gdyn;
+    uint32_t *hist = gdyn + W * MATCH_WORDS, *wsum = hist + W * hw;
     uint16_t *ent = (uint16_t *)(wsum + W);
     const uint32_t b = blockIdx.x, r = r0 + blockIdx.y;
     const uint32_t run = first_run + r;
@@ -909,12 +934,12 @@ __global__ __launch_bounds__(64 * W) void shuffle_group_kernel(
             shuffle_wide(a, n, run, b, k0, k1);
         return;
     }
-    shuffle_group_lds<W, GPW, IDENT>(n, b, run, k0, k1, a, ent, hist, hw, wsum);
+    shuffle_group_lds<W, GPW, IDENT>(n, b, run, k0, k1, a, ent, hist, hw, wsum, masks);
 }
 
 static size_t shuf_group_lds_bytes(uint32_t W, uint32_t cap)
 {
-    return (size_t)(W * shuf_hist_words(cap) + W) * 4u + (((size_t)cap * 2u + 3u) & ~(size_t)3u);
+    return (size_t)(W * (MATCH_WORDS + shuf_hist_words(cap)) + W) * 4u + (((size_t)cap * 2u + 3u) & ~(size_t)3u);
 }
 
 // ---------------------------------------------------------------------------
@@ -5376,7 +5401,7 @@ extern "C" int pc_permute_philox(uint64_t seed, uint64_t first_run,
                                                       counts, starts);
         PC_LAUNCH_CHECK("shuffle_scan_kernel");
         shuffle_scatter_kernel<<<shuf_blocks(chunks, rn), 64 * SHUF_W,
-                                 (SHUF_W + 2u) * nb1 * 4u, s>>>(
+                                 (SHUF_W + 1u) * nb1 * 4u, s>>>(
             k0, k1, fr, num_edges, lb1, chunks, r0, rn, counts, d_perm, perm_stride);
         PC_LAUNCH_CHECK("shuffle_scatter_kernel");
         shuffle_group_kernel<4, false><<<dim3(nb1, rn), 256,

@@ -552,3 +552,16 @@ def test_sums_groups(gpu, length, runs, sub):
         x = cols[k][:, steps].astype(object)
         assert (got1[k][steps] == x.sum(axis=0)).all(), k
         assert (got2[k][steps] == (x * x).sum(axis=0)).all(), k
+
+
+@pytest.mark.parametrize('M', [63, 4095, 8191, 8192, 8193, 16385, 32767, 131073, 1048577])
+def test_device_permutation_label_bits(gpu, M):
+    """Around the edge counts at which the labels gain a bit (0 to 9 bits: 7
+    are matched through LDS, the rest by ballots) and the chunks and groups
+    end: the oracle's permutations."""
+    eng = BondEngine(_graph.GraphArrays(M + 1, np.stack(
+        [np.arange(M), np.arange(1, M + 1)], axis=1)))
+    got = eng.device_permutations(seed=77, num_runs=3, first_run=9).cpu().numpy()
+    want = oracle.bucket_permutations(77, 9, 3, M)
+    for r in range(3):
+        np.testing.assert_array_equal(got[r], want[r], err_msg='run {}'.format(r))
