@@ -156,8 +156,11 @@ __device__ __forceinline__ uint32_t wave_scan_max(uint32_t x)
 #define SCAN_NOP "s_nop 1\n\t"
 
 #define SCAN_STEP_NARROW(c) SCAN_MAX("%0", c) SCAN_ADD("%1", c) SCAN_64("%2", "%3", c) SCAN_64("%4", "%5", c)
-#define SCAN_STEP_SUMS(c) SCAN_MAX("%0", c) SCAN_64("%1", "%2", c) SCAN_64("%3", "%4", c) SCAN_128("%5", "%6", "%7", "%8", c)
+#define SCAN_96(a, b, d, c) SCAN_ADD_CO(a, c) SCAN_ADDC(b, c) SCAN_ADDC(d, c)
+#define SCAN_STEP_96(c) SCAN_MAX("%0", c) SCAN_64("%1", "%2", c) SCAN_64("%3", "%4", c) SCAN_96("%5", "%6", "%7", c)
 #define SCAN_STEP_WIDE(c) SCAN_MAX("%0", c) SCAN_64("%1", "%2", c) SCAN_128("%3", "%4", "%5", "%6", c) SCAN_128("%7", "%8", "%9", "%10", c)
+
+typedef unsigned _BitInt(96) u96;
 
 struct Words128 {
     uint32_t w[4];
@@ -181,17 +184,17 @@ struct Words128 {
         d4 = ((uint64_t)d << 32) | c;                                                      \
     }                                                                                      \
     __device__ __forceinline__ void NAME(uint32_t &mx, uint64_t &d2, uint64_t &d3,         \
-                                         u128 &d4)                                         \
+                                         u96 &d4)                                          \
     {                                                                                      \
         uint32_t a = (uint32_t)d2, b = (uint32_t)(d2 >> 32);                               \
         uint32_t c = (uint32_t)d3, d = (uint32_t)(d3 >> 32);                               \
-        Words128 e(d4);                                                                    \
-        asm volatile(SCAN_NOP STEPS(SCAN_STEP_SUMS) SCAN_NOP                               \
-                     : "+v"(mx), "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e.w[0]),         \
-                       "+v"(e.w[1]), "+v"(e.w[2]), "+v"(e.w[3])::"vcc");                   \
+        uint32_t e = (uint32_t)d4, f = (uint32_t)(d4 >> 32), g = (uint32_t)(d4 >> 64);     \
+        asm volatile(SCAN_NOP STEPS(SCAN_STEP_96) SCAN_NOP                                 \
+                     : "+v"(mx), "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e), "+v"(f),     \
+                       "+v"(g)::"vcc");                                                    \
         d2 = ((uint64_t)b << 32) | a;                                                      \
         d3 = ((uint64_t)d << 32) | c;                                                      \
-        d4 = e.value();                                                                    \
+        d4 = ((u96)g << 64) | ((u96)f << 32) | e;                                          \
     }                                                                                      \
     __device__ __forceinline__ void NAME(uint32_t &mx, uint64_t &d2, u128 &d3, u128 &d4)   \
     {                                                                                      \
@@ -3564,9 +3567,15 @@ __global__ __launch_bounds__(64) void chunk_prefix_kernel(
 // L = 128 as a pipeline: 8.3 ms, 9.5 with the form below).  Elsewhere the four
 // waves of a workgroup share 64 runs of a chunk and add up in LDS, so that a
 // fourth of the atomics remain (L = 100, 500 runs 0.121 -> 0.044 ms; L = 16,
-// 40 runs 13 -> 8 us).  Bound by vector issue.
+// 40 runs 13 -> 8 us).  Bound by vector issue: 112 to 150 instructions a
+// record.  With the squares added up limb by limb in doubles (SquareSum)
+// instead of as 128- and 192-bit integers (255 instructions), and the sums of
+// N - max left to the end, 1000 runs of L = 1024 take 7.9 ms, not 12.7 (their
+// records alone: 3.5); 600 of L = 181 0.19, not 0.26; 200 of L = 256 0.158,
+// not 0.180; a sub-batch of L = 128 beside its sweeps 0.19, not 0.21.
 #define SUMS_BLOCKS 8192u
 #define SUMS_RUNS 32u
+#define SUMS_MOST 1024u   // runs a group may hold: what the bounds below allow
 
 // Product of two numbers below 2^24 (two full-rate instructions; __umul24
 // returns an int).
@@ -3577,26 +3586,60 @@ __device__ __forceinline__ uint64_t mul24_wide(uint32_t a, uint32_t b)
     return ((uint64_t)hi << 32) | (uint32_t)__umul24(a, b);
 }
 
-// Square of a 64-bit number: three 32-bit products.
-__device__ __forceinline__ u128 square_u128(uint64_t x)
+// Product of numbers below 2^44 and 2^44 (the high words' below 2^24).
+__device__ __forceinline__ u96 mul_u96(uint64_t p, uint64_t q)
 {
-    const uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
-    const uint64_t ll = (uint64_t)lo * lo, lh = (uint64_t)lo * hi, hh = (uint64_t)hi * hi;
-    return (((u128)hh << 64) | ll) + ((u128)lh << 33);
+    const uint32_t pl = (uint32_t)p, ph = (uint32_t)(p >> 32), ql = (uint32_t)q,
+                   qh = (uint32_t)(q >> 32);
+    const uint64_t t0 = (uint64_t)pl * ql, t1 = (uint64_t)pl * qh + (t0 >> 32),
+                   t2 = (uint64_t)ph * ql + (uint32_t)t1;
+    const uint32_t hi = (uint32_t)__umul24(ph, qh) + (uint32_t)(t1 >> 32) + (uint32_t)(t2 >> 32);
+    return ((u96)hi << 64) | ((u96)(uint32_t)t2 << 32) | (uint32_t)t0;
 }
 
-__device__ __forceinline__ void square_u192(u128 x, uint64_t &w0, uint64_t &w1,
-                                            uint64_t &w2)
-{
-    const uint64_t lo = (uint64_t)x, hi = (uint64_t)(x >> 64);
-    const u128 ll = (u128)lo * lo;
-    const u128 lh2 = ((u128)lo * hi) << 1; // < 2^129 only if hi >= 2^64: hi < 2^32 here
-    const u128 hh = (u128)hi * hi;
-    w0 = (uint64_t)ll;
-    const u128 mid = (ll >> 64) + (u128)(uint64_t)lh2;
-    w1 = (uint64_t)mid;
-    w2 = (uint64_t)(mid >> 64) + (uint64_t)(lh2 >> 64) + (uint64_t)hh;
-}
+// Sum of the squares of numbers of K limbs of B <= 21 bits: a sum for every
+// product of two limbs, put together once at the end, so that a square costs
+// no carries.  The sums are doubles, whose multiply-adds run at full rate
+// (64-bit integer ones: 9.3 ms where these take 7.9), and exact: SUMS_MOST
+// products below 2^42 stay below 2^53.
+template <int K, int B>
+struct SquareSum {
+    static_assert(2 * B <= 42, "exact in a double");
+    double sum[K * (K + 1) / 2] = {};
+    __device__ __forceinline__ void add(const uint32_t *limb)
+    {
+        double l[K];
+#pragma unroll
+        for (int i = 0; i < K; ++i)
+            l[i] = (double)limb[i];
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < K; ++i)
+#pragma unroll
+            for (int j = i; j < K; ++j)
+                sum[n] = __builtin_fma(l[i], l[j], sum[n]), ++n;
+    }
+    // low 128 bits, and the word above
+    __device__ __forceinline__ u128 value(uint64_t &top) const
+    {
+        u128 lo = 0;
+        top = 0;
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < K; ++i)
+#pragma unroll
+            for (int j = i; j < K; ++j) {
+                const u128 v = (u128)(uint64_t)sum[n++] << (i == j ? 0 : 1);
+                const int shift = B * (i + j);
+                const u128 part = shift < 128 ? v << (shift & 127) : (u128)0;
+                lo += part;
+                top += lo < part ? 1u : 0u;
+                top += shift >= 128 ? (uint64_t)(v << (shift & 127))
+                                    : shift ? (uint64_t)(v >> ((128 - shift) & 127)) : 0u;
+            }
+        return lo;
+    }
+};
 
 template <typename RecT, bool WIDE, uint32_t WAVES>
 __global__ __launch_bounds__(64 * WAVES) void micro_sums_kernel(
@@ -3665,41 +3708,53 @@ __global__ __launch_bounds__(64 * WAVES) void micro_sums_kernel(
     }
 
     if constexpr (!WIDE) {
-        // N <= 2^14 and at most 2^16 runs per group bound every accumulator:
-        // max, #clusters - 1 and N - max are below 2^14 (squares below 2^28,
-        // group sums of squares below 2^44); the spanning flag is 0 or 1;
-        // moment 2 is below N^2 / 2 (square below 2^54), moment 3 below
-        // N^3 / 4 (group sum below 2^56), moment 4 below N^4 / 8.  So the
-        // narrow columns use 32- and 64-bit arithmetic, exact all the same.
+        // N <= 2^14 and at most SUMS_MOST runs per group bound every
+        // accumulator: max, #clusters - 1 and N - max are below 2^14 (group
+        // sums of squares below 2^38); the spanning flag is 0 or 1; moment 2
+        // is below N^2 / 2 (squares below 2^54), moment 3 below N^3 / 4 =
+        // 2^40, moment 4 below N^4 / 8 = 2^53.  The sums of N - max follow
+        // from those of max.
         uint32_t n1[4] = {0, 0, 0, 0};  // sum x: max, span, #clusters - 1, N - max
         uint64_t n2[4] = {0, 0, 0, 0};  // sum x^2 of the same
-        uint64_t m1_2 = 0, m1_3 = 0;    // sum x: moments 2 and 3
-        u128 m1_4 = 0, m2_2 = 0, m2_3 = 0, m2_4 = 0;
+        uint64_t m1_2 = 0, m1_3 = 0, m1_4 = 0;   // sum x: moments 2 to 4
+        uint64_t sq_2 = 0;
+        SquareSum<2, 20> sq_3;
+        SquareSum<3, 18> sq_4;
+        uint32_t count = 0;
         for (uint32_t r = r0 + wave; r < r1; r += WAVES) {
             const RunState<false> st0 = st_next;
             const RecT rec = valid ? rec_next : (RecT)0;
             const uint32_t span = span_next;
             ahead(min(r + WAVES, r1 - 1u));
+            ++count;
             Deltas<false> d(rec);
             const uint32_t merges = (uint32_t)st0.merges + scan_count(d.merge());
             scan_state(d.dmax, d.d2, d.d3, d.d4);
             const uint32_t mx = max((uint32_t)st0.mx, d.dmax), mx2 = (uint32_t)__umul24(mx, mx);
-            const uint32_t x[4] = {mx, s >= span ? 1u : 0u, N - merges - 1u, N - mx};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                n1[k] += x[k];
-                n2[k] += (uint32_t)__umul24(x[k], x[k]);
-            }
+            const uint32_t x2 = N - merges - 1u;
+            n1[0] += mx;
+            n2[0] += mx2;
+            n1[1] += s >= span ? 1u : 0u;
+            n1[2] += x2;
+            n2[2] += (uint32_t)__umul24(x2, x2);
             const uint32_t x4 = (uint32_t)st0.s2 + d.d2 - mx2;
             m1_2 += x4;
-            m2_2 += (u128)((uint64_t)x4 * x4);
+            sq_2 += (uint64_t)x4 * x4;
             const uint64_t x5 = st0.s3 + d.d3 - (uint64_t)mx2 * mx;
             m1_3 += x5;
-            m2_3 += square_u128(x5);
             const uint64_t x6 = st0.s4 + d.d4 - (uint64_t)mx2 * mx2;
             m1_4 += x6;
-            m2_4 += square_u128(x6);
+            const uint32_t l5[2] = {(uint32_t)x5 & 0xFFFFFu, (uint32_t)(x5 >> 20)};
+            const uint32_t l6[3] = {(uint32_t)x6 & 0x3FFFFu, (uint32_t)(x6 >> 18) & 0x3FFFFu,
+                                    (uint32_t)(x6 >> 36)};
+            sq_3.add(l5);
+            sq_4.add(l6);
         }
+        n2[1] = n1[1];
+        n1[3] = count * N - n1[0];
+        n2[3] = (uint64_t)count * N * N + n2[0] - 2ull * N * n1[0];
+        uint64_t none;
+        u128 m2_2 = sq_2, m2_3 = sq_3.value(none), m2_4 = sq_4.value(none);
         to_wave0([&](auto &&at) {
 #pragma unroll
             for (uint32_t k = 0; k < 4u; ++k) {
@@ -3727,64 +3782,72 @@ __global__ __launch_bounds__(64 * WAVES) void micro_sums_kernel(
         acc1[6] = m1_4;
         acc2[6] = m2_4;
     } else {
-        // N <= 2^21 (the sums' limit) and at most 2^16 runs per group: S3 is
-        // below N^3 <= 2^63 (its deltas and scan stay in 64 bits), max,
-        // #clusters - 1 and N - max are below 2^21 (group sums of squares
-        // below 2^58), moment 2 below 2^42 (its square below 2^84), moment 3
-        // below 2^63 (square below 2^126) and moment 4 below 2^84 (square
-        // below 2^168).  Only moments 3 and 4 need 192-bit sums of squares.
+        // N <= 2^21 (the sums' limit) and at most SUMS_MOST runs per group:
+        // S3 is below N^3 <= 2^63 (its deltas and scan stay in 64 bits), S4
+        // at most N^4 <= 2^84 (96 bits); max, #clusters - 1 and N - max are
+        // at most 2^21 (group sums below 2^32, of squares below 2^53),
+        // moment 2 below 2^42, moment 3 below 2^63 and moment 4 below 2^84:
+        // two, three and four limbs of 21 bits.  The sums of N - max follow
+        // from those of max.
         uint64_t n1[5] = {0, 0, 0, 0, 0}; // sum x: max, span, #clusters - 1, N - max, moment 2
         uint64_t n2[4] = {0, 0, 0, 0};    // sum x^2 of the first four
-        u128 m2_2 = 0, m1_3 = 0, m1_4 = 0;
-        u128 m2_3 = 0, m2_4 = 0;          // low 128 bits of sum x^2, moments 3 and 4
-        uint64_t t2_3 = 0, t2_4 = 0;      // their top words
+        uint32_t s_mx = 0, s_span = 0, s_cl = 0, count = 0;
+        u96 s_3 = 0, s_4 = 0;             // sum x: moments 3 and 4
+        SquareSum<2, 21> sq_2;
+        SquareSum<3, 21> sq_3;
+        SquareSum<4, 21> sq_4;
+        constexpr uint32_t LIMB = (1u << 21) - 1u;
         for (uint32_t r = r0 + wave; r < r1; r += WAVES) {
-            const uint64_t mx0 = st_next.mx, merges0 = st_next.merges, s2_0 = st_next.s2,
-                           s3_0 = (uint64_t)st_next.s3;
-            const u128 s4_0 = st_next.s4;
+            const uint32_t mx0 = (uint32_t)st_next.mx, merges0 = (uint32_t)st_next.merges;
+            const uint64_t s2_0 = st_next.s2, s3_0 = (uint64_t)st_next.s3;
+            const u96 s4_0 = (u96)st_next.s4;
             const RecT rec = valid ? rec_next : (RecT)0;
             const uint32_t span = span_next;
             ahead(min(r + WAVES, r1 - 1u));
+            ++count;
             uint32_t a, b;
             unpack_record(rec, a, b);
             // sizes below 2^21 + 1: 24-bit products, q <= 2^40
             uint32_t mxd = a + b;
             const uint32_t sz = mxd;
             const uint64_t qq = mul24_wide(a, b);
-            uint64_t d2 = 2u * qq, d3 = qq * (3u * sz);
-            u128 d4 = (u128)(2u * qq) * (u128)(2u * mul24_wide(sz, sz) - qq);
-            const uint64_t merges = merges0 + scan_count(rec != 0);
+            uint64_t d2 = 2u * qq;
+            uint64_t d3 = (uint64_t)(uint32_t)qq * (3u * sz) +
+                          ((uint64_t)(uint32_t)__umul24((uint32_t)(qq >> 32), 3u * sz) << 32);
+            u96 d4 = mul_u96(2u * qq, 2u * mul24_wide(sz, sz) - qq);
+            const uint32_t merges = merges0 + scan_count(rec != 0);
             scan_state(mxd, d2, d3, d4);
-            const uint32_t mx = max((uint32_t)mx0, mxd);
-            const uint64_t s2 = s2_0 + d2, s3 = s3_0 + d3;
-            const u128 s4 = s4_0 + d4;
+            const uint32_t mx = max(mx0, mxd), cl = N - merges - 1u;
             const uint64_t m2 = mul24_wide(mx, mx);
-            const uint32_t x[4] = {mx, s >= span ? 1u : 0u, N - (uint32_t)merges - 1u,
-                                   N - mx};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                n1[k] += x[k];
-                n2[k] += mul24_wide(x[k], x[k]);
-            }
-            const uint64_t x4 = s2 - m2, x5 = s3 - m2 * mx;
-            const u128 x6 = s4 - (u128)m2 * m2;
+            s_mx += mx;
+            n2[0] += m2;
+            s_span += s >= span ? 1u : 0u;
+            s_cl += cl;
+            n2[2] += mul24_wide(cl, cl);
+            const uint64_t x4 = s2_0 + d2 - m2;
+            const uint64_t x5 = s3_0 + d3 - ((uint64_t)(uint32_t)m2 * mx +
+                                             ((uint64_t)(uint32_t)__umul24((uint32_t)(m2 >> 32), mx) << 32));
+            const u96 x6 = s4_0 + d4 - mul_u96(m2, m2);
             n1[4] += x4;
-            m2_2 += square_u128(x4);
-            m1_3 += x5;
-            {
-                const u128 sq = square_u128(x5), before = m2_3;
-                m2_3 += sq;
-                t2_3 += m2_3 < before ? 1u : 0u;
-            }
-            m1_4 += x6;
-            {
-                uint64_t w0, w1, w2;
-                square_u192(x6, w0, w1, w2);
-                const u128 before = m2_4;
-                m2_4 += (u128)w0 | ((u128)w1 << 64);
-                t2_4 += w2 + (m2_4 < before ? 1u : 0u);
-            }
+            s_3 += x5;
+            s_4 += x6;
+            const uint32_t l4[2] = {(uint32_t)x4 & LIMB, (uint32_t)(x4 >> 21)};
+            const uint32_t l5[3] = {(uint32_t)x5 & LIMB, (uint32_t)(x5 >> 21) & LIMB,
+                                    (uint32_t)(x5 >> 42)};
+            const uint32_t l6[4] = {(uint32_t)x6 & LIMB, (uint32_t)(x6 >> 21) & LIMB,
+                                    (uint32_t)(x6 >> 42) & LIMB, (uint32_t)(x6 >> 63)};
+            sq_2.add(l4);
+            sq_3.add(l5);
+            sq_4.add(l6);
         }
+        n1[0] = s_mx;
+        n1[1] = n2[1] = s_span;
+        n1[2] = s_cl;
+        n1[3] = (uint64_t)count * N - s_mx;
+        n2[3] = (uint64_t)count * N * N + n2[0] - 2ull * N * s_mx;
+        uint64_t none, t2_3, t2_4;
+        u128 m2_2 = sq_2.value(none), m2_3 = sq_3.value(t2_3), m2_4 = sq_4.value(t2_4);
+        u128 m1_3 = s_3, m1_4 = s_4;
         {
             // the carries of the two 192-bit sums go with their low words
             u128 *const low[2] = {&m2_3, &m2_4};
@@ -5872,9 +5935,8 @@ extern "C" int pc_microcanonical_sums(uint32_t num_nodes, uint32_t num_edges,
     const bool one_wave = (uint64_t)C * per32 >= SUMS_BLOCKS;
     uint32_t groups = C ? (SUMS_BLOCKS / (one_wave ? 1u : 4u) + C - 1u) / C : 1u;
     groups = std::min(groups, one_wave ? per32 : (per32 + 1u) / 2u);
-    // at most 2^16 runs per group: the narrow 128-bit sum of squares of the
-    // fourth moment (each below 2^112) stays exact
-    groups = std::max(groups, num_runs / 65536u + (num_runs % 65536u != 0u));
+    // the bounds of the sums in a group
+    groups = std::max(groups, num_runs / SUMS_MOST + (num_runs % SUMS_MOST != 0u));
     const uint32_t rpg = groups ? (num_runs + groups - 1u) / groups : 0u;
     groups = rpg ? (num_runs + rpg - 1u) / rpg : 0u;
     // one group that does not accumulate stores its sums

@@ -565,3 +565,31 @@ def test_device_permutation_label_bits(gpu, M):
     want = oracle.bucket_permutations(77, 9, 3, M)
     for r in range(3):
         np.testing.assert_array_equal(got[r], want[r], err_msg='run {}'.format(r))
+
+
+@pytest.mark.parametrize('N,runs', [(16384, 2500), (16385, 1100), (1 << 21, 2)])
+def test_sums_at_their_bounds(gpu, N, runs):
+    """Two clusters of half the nodes each, the largest moments there are,
+    at the node counts where the sums' arithmetic changes or ends and with
+    more runs than one group holds: sums and sums of squares in closed
+    form."""
+    h = N // 2
+    eng = BondEngine(_graph.GraphArrays(N, np.stack([np.arange(N - 1), np.arange(1, N)], axis=1)))
+    order = np.concatenate([np.arange(h - 1), np.arange(h, N - 1), [h - 1]])
+    perm = gpu.from_numpy(order.astype(np.int32)).cuda().repeat(runs, 1)
+    res = eng.sweep(perm)
+    s1, s2 = eng.microcanonical_sums(res)
+    steps = np.unique(np.concatenate([np.arange(40), np.arange(h - 70, h + 70),
+                                      np.linspace(0, N - 1, 300).astype(int),
+                                      np.arange(N - 70, N)]))
+    at = gpu.from_numpy(steps).cuda()
+    s1 = s1[:, at].cpu().numpy().view(np.uint64)
+    s2 = s2[:, at].cpu().numpy().view(np.uint64)
+    for j, s in enumerate(int(v) for v in steps):
+        sizes = [s + 1] if s < h else [h, s - h + 2] if s < N - 1 else [N]
+        singles = N - sum(sizes)
+        big = max(sizes)
+        x = [big, 0] + [singles + sum(c ** k for c in sizes) - big ** k for k in range(5)]
+        for k in range(7):
+            assert sum(int(w) << (64 * i) for i, w in enumerate(s1[k, j])) == runs * x[k], (s, k)
+            assert sum(int(w) << (64 * i) for i, w in enumerate(s2[k, j])) == runs * x[k] ** 2, (s, k)
