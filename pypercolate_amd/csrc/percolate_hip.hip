@@ -2669,7 +2669,7 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 // Untiled, with every node's code in HBM, the sweep moves 342 bytes per
 // addition in random lines at L = 1024, and at L = 128 (codes in LDS) four
 // runs fill a CU.  Sweep with its chunk states, untiled and tiled: L = 1024,
-// 1000 runs 158 and 70 ms (lists 24, tiles 22, events 20, chunk states 4);
+// 1000 runs 158 and 63 ms (lists 19, tiles 19, events 20, chunk states 4);
 // L = 256, 200 runs 3.67 and 1.1; L = 181, 600 runs 2.65 and 1.1; L = 128,
 // 10^4 runs (no chunk states) 7.06 and 5.05.  The tiles are bound by vector
 // issue (60 % of a wavefront's share of its SIMD at L = 256) and dependent
@@ -2693,8 +2693,19 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 #define TILE_CLAIM_BITS 9
 #define TILE_CLAIM_SLOTS (1u << TILE_CLAIM_BITS)
 #define TILE_SCATTER_BLOCKS 1024u // workgroups tile_scatter wants
-#define TILE_GROUPS 8u   // groups of 64 steps a wave of tile_scatter takes at once
-#define TILE_SHORT_STEPS (1u << 19) // up to so many edges a list entry has 32 bits
+// Groups of 64 steps a wave of tile_scatter takes at once: a turn of the four
+// waves then gives a tile's list 1024 * groups / tiles bytes.  With eight and
+// more than TILE_MANY tiles, lists and lines fill in small pieces: 16 groups
+// took 1000 runs of L = 1024 (256 tiles) from 17.0 to 15.1 ms, 300 of L = 700
+// (121) 2.44 to 2.27, 1000 of L = 384 (36) 1.85 to 1.70; 600 of L = 181 (9)
+// 0.157 to 0.179, so fewer tiles keep eight, and so do segments of fewer than
+// TILE_LONG_SEGMENT steps, where a turn is a large part (200 runs of L = 256,
+// 64 tiles, segments of 22000: 0.115 to 0.138).
+#define TILE_GROUPS 8u
+#define TILE_GROUPS_MANY 16u
+#define TILE_MANY 32u
+#define TILE_LONG_SEGMENT 65536u
+#define TILE_WINDOW (1u << 19)  // the steps that a list entry can tell apart
 
 // Tiles of h x w nodes (the last row and column of tiles may be smaller),
 // KH x KW of them.  mh, mw divide a coordinate by h and w (high half of the
@@ -2721,6 +2732,9 @@ struct TileGeo {
     }
 };
 
+// Windows of the list entries' steps in a run of M.
+__host__ __device__ __forceinline__ uint32_t tile_windows(uint32_t M) { return (M + TILE_WINDOW - 1u) / TILE_WINDOW; }
+
 // A tile's union-find code, with nodes named by the byte offset of their code
 // (twice the local index, so a code is an address): a parent's offset (below
 // 0x2000), an open root's place among the tile's ids (0x2000 + place), or a
@@ -2743,28 +2757,19 @@ struct EventBits {
     static __device__ __forceinline__ bool is_event(RecT r) { return (r >> (2u * half - 1u)) != 0; }
 };
 
-// List entries: step, local index of u (taken as its code's offset), and
-// whether v is the node below u (else the one to its right).
-template <typename ENT>
-struct TileEntry;
-template <>
-struct TileEntry<uint32_t> {
-    static __device__ __forceinline__ uint32_t make(uint32_t t, uint32_t u, uint32_t down) { return t | (u << 19) | (down << 31); }
+// List entries: step modulo TILE_WINDOW, local index of u (taken as its code's
+// offset), and whether v is the node below u (else the one to its right).
+// Where a run has more steps, tile_scatter notes how far each list has come
+// at every multiple of TILE_WINDOW.  (With 64-bit entries that hold the whole
+// step, 1000 runs of L = 1024 took 19.1 ms to scatter and 20.2 to sweep; with
+// these 17.0 and 19.4, in two slabs of runs instead of four.)
+struct TileEntry {
+    static __device__ __forceinline__ uint32_t make(uint32_t t, uint32_t u, uint32_t down) { return (t & (TILE_WINDOW - 1u)) | (u << 19) | (down << 31); }
     static __device__ __forceinline__ void take(uint32_t e, uint32_t &t, uint32_t &u, uint32_t &down)
     {
-        t = e & (TILE_SHORT_STEPS - 1u);
+        t = e & (TILE_WINDOW - 1u);
         u = (e >> 18) & 0x1FFEu;
         down = e >> 31;
-    }
-};
-template <>
-struct TileEntry<uint64_t> {
-    static __device__ __forceinline__ uint64_t make(uint32_t t, uint32_t u, uint32_t down) { return (uint64_t)t | ((uint64_t)(u | (down << 31)) << 32); }
-    static __device__ __forceinline__ void take(uint64_t e, uint32_t &t, uint32_t &u, uint32_t &down)
-    {
-        t = (uint32_t)e;
-        u = (uint32_t)(e >> 31) & 0x1FFEu;
-        down = (uint32_t)(e >> 63);
     }
 };
 
@@ -2863,20 +2868,22 @@ __global__ __launch_bounds__(256) void tile_scan_kernel(
 }
 
 // The tiles' lists of a run (or of one segment of its steps): a stable
-// counting sort by tile of 256 * TILE_GROUPS steps at a time.  Every wave
-// ranks its 64 * TILE_GROUPS consecutive steps (match_label, and the wave's
+// counting sort by tile of 256 * GROUPS steps at a time.  Every wave
+// ranks its 64 * GROUPS consecutive steps (match_label, and the wave's
 // own counter of each tile), the counters of the four waves become places
 // after the tile's cursor, and the entries are stored.  A row that is not a
 // permutation (some bond twice) may not fill the lists: such a run is marked
 // in odd[] and left to the untiled sweep.
-template <typename ENT, typename RecT>
+template <typename RecT, uint32_t GROUPS>
 __global__ __launch_bounds__(256) void tile_scatter_kernel(
     TileGeo g, uint32_t M, uint32_t tile_bits, uint32_t seg_steps,
     const int32_t *__restrict__ perm, int64_t perm_stride,
-    const uint32_t *__restrict__ counts, ENT *__restrict__ lists, int64_t list_stride,
-    RecT *__restrict__ records, int64_t rec_stride, uint32_t *__restrict__ span_step,
-    uint32_t *__restrict__ odd)
+    const uint32_t *__restrict__ counts, uint32_t *__restrict__ lists, int64_t list_stride,
+    uint32_t *__restrict__ windows, RecT *__restrict__ records, int64_t rec_stride,
+    uint32_t *__restrict__ span_step, uint32_t *__restrict__ odd)
 {
+    // a window starts at the start of some turn of the loop below
+    static_assert(TILE_WINDOW % (256u * GROUPS) == 0u, "turns must meet the windows' starts");
     extern __shared__ uint32_t tile_dyn[];   // [4][K] wave counters, [K] cursors
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t seg = blockIdx.x, nseg = gridDim.x, run = blockIdx.y;
@@ -2890,21 +2897,26 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(
         return;
     bool wrong = false;
     const int32_t *p = perm + (int64_t)run * perm_stride;
-    ENT *list = lists + (int64_t)run * list_stride;
+    uint32_t *list = lists + (int64_t)run * list_stride;
     RecT *rec = records + (int64_t)run * rec_stride;
     const uint32_t end = min(M, (seg + 1u) * seg_steps);
-    int32_t e[TILE_GROUPS];
-    uint32_t t0 = seg * seg_steps + wave * 64u * TILE_GROUPS + lane;
+    int32_t e[GROUPS];
+    uint32_t t0 = seg * seg_steps + wave * 64u * GROUPS + lane;
 #pragma unroll
-    for (uint32_t i = 0; i < TILE_GROUPS; ++i)
+    for (uint32_t i = 0; i < GROUPS; ++i)
         e[i] = t0 + i * 64u < end ? p[t0 + i * 64u] : -1;
-    for (uint32_t base = seg * seg_steps; base < end; base += 256u * TILE_GROUPS) {
+    for (uint32_t base = seg * seg_steps; base < end; base += 256u * GROUPS) {
         for (uint32_t k = lane; k < g.K; k += 64u)
             my[k] = 0u;
-        ENT ent[TILE_GROUPS];
-        uint32_t at[TILE_GROUPS];   // tile | rank << 12, or all ones
+        if (M > TILE_WINDOW && base % TILE_WINDOW == 0u) {
+            uint32_t *to = windows + ((size_t)run * tile_windows(M) + base / TILE_WINDOW) * g.K;
+            for (uint32_t k = tid; k < g.K; k += 256u)
+                to[k] = cursor[k];
+        }
+        uint32_t ent[GROUPS];
+        uint32_t at[GROUPS];   // tile | rank << 12, or all ones
 #pragma unroll
-        for (uint32_t i = 0; i < TILE_GROUPS; ++i) {
+        for (uint32_t i = 0; i < GROUPS; ++i) {
             const uint32_t t = t0 + i * 64u;
             const bool ok = (uint32_t)e[i] < M;
             const TileBond b = tile_bond(g, ok ? e[i] : 0);
@@ -2928,11 +2940,11 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(
             }
             if (t < end)
                 rec[t] = ev;
-            ent[i] = TileEntry<ENT>::make(t, b.lr * g.w + b.lc, b.down);
+            ent[i] = TileEntry::make(t, b.lr * g.w + b.lc, b.down);
         }
-        const uint32_t tn = t0 + 256u * TILE_GROUPS;
+        const uint32_t tn = t0 + 256u * GROUPS;
 #pragma unroll
-        for (uint32_t i = 0; i < TILE_GROUPS; ++i)
+        for (uint32_t i = 0; i < GROUPS; ++i)
             e[i] = tn + i * 64u < end ? p[tn + i * 64u] : -1;
         __syncthreads();
         for (uint32_t k = tid; k < g.K; k += 256u) {
@@ -2949,7 +2961,7 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(
         if (__syncthreads_or(wrong))
             break;
 #pragma unroll
-        for (uint32_t i = 0; i < TILE_GROUPS; ++i)
+        for (uint32_t i = 0; i < GROUPS; ++i)
             if (at[i] != 0xFFFFFFFFu)
                 list[my[at[i] & 0xFFFu] + (at[i] >> 12)] = ent[i];
         t0 = tn;
@@ -2970,10 +2982,10 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(
 // open, of both.  No budget of rounds: the earliest pending candidate always merges.  Blocks of
 // a run go to one XCD (shuf_block), whose L2 then collects the records that
 // the run's tiles write into shared lines.
-template <typename ENT, typename RecT>
+template <typename RecT>
 __global__ __launch_bounds__(64) void tile_sweep_kernel(
-    TileGeo g, uint32_t rn, const ENT *__restrict__ lists, int64_t list_stride,
-    const uint16_t *__restrict__ init, RecT *__restrict__ records,
+    TileGeo g, uint32_t rn, const uint32_t *__restrict__ lists, int64_t list_stride,
+    const uint32_t *__restrict__ windows, const uint16_t *__restrict__ init, RecT *__restrict__ records,
     int64_t rec_stride, uint32_t *__restrict__ span_step,
     const uint32_t *__restrict__ odd)
 {
@@ -2988,7 +3000,8 @@ __global__ __launch_bounds__(64) void tile_sweep_kernel(
     const uint32_t id0 = k * g.per - TILE_OPEN;   // an open code to its id
     const TileState st{(char *)(tile_lds + TILE_CLAIM_SLOTS)};
     const uint32_t below = 2u * g.w;   // from a node's code to the one below
-    const ENT *list = lists + (int64_t)rl * list_stride + g.offset(tr, tc);
+    const uint32_t first = g.offset(tr, tc);
+    const uint32_t *list = lists + (int64_t)rl * list_stride + first;
     RecT *rec_out = records + (int64_t)rl * rec_stride;
     {
         const uint4 *src = (const uint4 *)(init + (size_t)k * g.init_stride);
@@ -3000,13 +3013,32 @@ __global__ __launch_bounds__(64) void tile_sweep_kernel(
         claims[i] = 0u;
     __syncthreads();
 
-    // One batch: the bonds `cur`, with the codes of the next batch's
+    // The window of the list's entries, and the entry the next one starts at.
+    // (32-bit records: fewer steps than a window.)
+    constexpr bool WINDOWS = sizeof(RecT) == 8u;
+    const uint32_t M = 2u * g.L * (g.L - 1u);
+    uint32_t window = 0;
+    auto window_start = [&]() {
+        const uint32_t w = window / TILE_WINDOW + 1u, W = tile_windows(M);
+        return w < W ? windows[((size_t)rl * W + w) * g.K + k] - first : 0xFFFFFFFFu;
+    };
+    uint32_t next_window = WINDOWS ? window_start() : 0xFFFFFFFFu;
+
+    // One batch: the bonds `cur` (entries at `at`), with the codes of the next batch's
     // endpoints (`next`) read before its merges (a parent read early is still
     // an ancestor).
     uint32_t hint_u = TILE_OPEN, hint_v = TILE_OPEN, tag = 0, span_at = PC_NO_SPAN;
-    auto batch = [&](ENT cur, ENT next, bool active) __attribute__((always_inline)) {
+    auto batch = [&](uint32_t at, uint32_t cur, uint32_t next, bool active) __attribute__((always_inline)) {
         uint32_t t, x, y, down;
-        TileEntry<ENT>::take(cur, t, x, down);
+        TileEntry::take(cur, t, x, down);
+        if constexpr (WINDOWS) {
+            t += window;
+            while (next_window < at + 64u) {
+                t += at + lane >= next_window ? TILE_WINDOW : 0u;
+                window += TILE_WINDOW;
+                next_window = window_start();
+            }
+        }
         y = x + (down ? below : 2u);
         x = st.is_root(hint_u) ? x : hint_u;
         y = st.is_root(hint_v) ? y : hint_v;
@@ -3014,7 +3046,7 @@ __global__ __launch_bounds__(64) void tile_sweep_kernel(
         find2(st, x, cx, y, cy);
         {
             uint32_t tn, un, dn;
-            TileEntry<ENT>::take(next, tn, un, dn);
+            TileEntry::take(next, tn, un, dn);
             hint_u = st.get(un);
             hint_v = st.get(un + (dn ? below : 2u));
         }
@@ -3073,18 +3105,18 @@ __global__ __launch_bounds__(64) void tile_sweep_kernel(
     // load in a branch, or one whose register is copied at the end of the
     // loop, would be waited for at once, with the stores before it.  Lanes
     // past the end read the last entry again.
-    ENT e0 = list[min(lane, n - 1u)], e1 = list[min(64u + lane, n - 1u)];
+    uint32_t e0 = list[min(lane, n - 1u)], e1 = list[min(64u + lane, n - 1u)];
     uint32_t base = 0;
     for (; base + 128u <= n; base += 128u) {
-        const ENT a = e0;
+        const uint32_t a = e0;
         e0 = list[min(base + 128u + lane, n - 1u)];
-        batch(a, e1, true);
-        const ENT b = e1;
+        batch(base, a, e1, true);
+        const uint32_t b = e1;
         e1 = list[min(base + 192u + lane, n - 1u)];
-        batch(b, e0, true);
+        batch(base + 64u, b, e0, true);
     }
     for (; base < n; base += 64u) {
-        batch(e0, e1, base + lane < n);
+        batch(base, e0, e1, base + lane < n);
         e0 = e1;
     }
     if (lane == 0u && span_at != PC_NO_SPAN)
@@ -5652,10 +5684,9 @@ static bool tile_geo(uint32_t length, bool tiled, uint32_t num_runs, TileGeo &g)
 // The workspace of a tiled sweep of num_runs runs whose lists are held for
 // `slab` runs at a time: the offsets of its parts, and its size.
 struct TilePlan {
-    uint64_t init, open, odd, states, counts, lists, list_bytes, bytes;
+    uint64_t init, open, odd, states, counts, windows, lists, list_bytes, bytes;
     uint32_t nodes, slab;
     bool lds;       // the open nodes' codes fit LDS
-    bool short_entries;
 };
 #define TILE_OPEN_LDS_NODES 10240u  // 40 KiB of codes: two runs per CU
 #define TILE_OPEN_LDS_MOST 32768u   // 128 KiB: one run per CU
@@ -5670,14 +5701,14 @@ static TilePlan tile_plan(const TileGeo &g, uint32_t num_runs, uint32_t slab)
     // in LDS also where it holds one run per CU, if the runs are that few
     p.lds = p.nodes <= TILE_OPEN_LDS_NODES ||
             (p.nodes <= TILE_OPEN_LDS_MOST && num_runs <= 256u);
-    p.short_entries = M <= TILE_SHORT_STEPS;
     p.init = 0;
     p.open = up((uint64_t)g.K * g.init_stride * 2u);
     p.odd = p.open + up((uint64_t)p.nodes * 4u);
     p.states = p.odd + up((uint64_t)num_runs * 4u);
     p.counts = p.states + (p.lds ? 0u : up((uint64_t)num_runs * p.nodes * 4u));
-    p.lists = p.counts + up(((uint64_t)slab + TILE_SCATTER_BLOCKS) * g.K * 4u);
-    p.list_bytes = up(M * (p.short_entries ? 4u : 8u));
+    p.windows = p.counts + up(((uint64_t)slab + TILE_SCATTER_BLOCKS) * g.K * 4u);
+    p.lists = p.windows + (M > TILE_WINDOW ? up((uint64_t)slab * tile_windows((uint32_t)M) * g.K * 4u) : 0u);
+    p.list_bytes = up(M * 4u);
     p.bytes = p.lists + slab * p.list_bytes;
     return p;
 }
@@ -5709,7 +5740,7 @@ extern "C" int pc_sweep_lattice_workspace_size(uint32_t length, uint32_t num_run
     return rc;
 }
 
-template <typename ENT, typename RecT>
+template <typename RecT>
 static int tile_sweep_launch(const TileGeo &g, const TilePlan &p,
                              const uint8_t *d_node_sides, const int32_t *d_perm,
                              int64_t perm_stride, uint32_t num_runs, RecT *d_records,
@@ -5720,8 +5751,8 @@ static int tile_sweep_launch(const TileGeo &g, const TilePlan &p,
     uint16_t *init = (uint16_t *)(ws + p.init);
     uint32_t *open = (uint32_t *)(ws + p.open), *odd = (uint32_t *)(ws + p.odd);
     uint32_t *counts = (uint32_t *)(ws + p.counts);
-    ENT *lists = (ENT *)(ws + p.lists);
-    const int64_t list_stride = (int64_t)(p.list_bytes / sizeof(ENT));
+    uint32_t *windows = (uint32_t *)(ws + p.windows), *lists = (uint32_t *)(ws + p.lists);
+    const int64_t list_stride = (int64_t)(p.list_bytes / 4u);
     uint32_t bits = 0;
     while ((1u << bits) < g.K)
         ++bits;
@@ -5735,7 +5766,11 @@ static int tile_sweep_launch(const TileGeo &g, const TilePlan &p,
         // of a segment then start where a count of the earlier ones says
         uint32_t nseg = (TILE_SCATTER_BLOCKS + rn - 1u) / rn;
         nseg = std::min(nseg, (M + 16383u) / 16384u);
-        const uint32_t quant = 256u * TILE_GROUPS;
+        const bool many = g.K > TILE_MANY && M / nseg >= TILE_LONG_SEGMENT;
+        // (32-bit records come with more than TILE_MANY tiles in short
+        // segments only)
+        constexpr uint32_t MANY = sizeof(RecT) == 8u ? TILE_GROUPS_MANY : TILE_GROUPS;
+        const uint32_t quant = 256u * (many ? MANY : TILE_GROUPS);
         const uint32_t seg = ((M + nseg - 1u) / nseg + quant - 1u) / quant * quant;
         nseg = (M + seg - 1u) / seg;
         if (nseg > 1u) {
@@ -5745,13 +5780,16 @@ static int tile_sweep_launch(const TileGeo &g, const TilePlan &p,
             tile_scan_kernel<<<rn, 256, 0, s>>>(g, nseg, counts, odd + r0);
             PC_LAUNCH_CHECK("tile_scan_kernel");
         }
-        tile_scatter_kernel<ENT, RecT><<<dim3(nseg, rn), 256, 5u * g.K * 4u, s>>>(
-            g, M, bits, seg, perm, perm_stride, counts, lists, list_stride, rec, rec_stride,
-            d_span_step + r0, odd + r0);
+        auto *scatter = many ? tile_scatter_kernel<RecT, MANY>
+                             : tile_scatter_kernel<RecT, TILE_GROUPS>;
+        scatter<<<dim3(nseg, rn), 256, 5u * g.K * 4u, s>>>(
+            g, M, bits, seg, perm, perm_stride, counts, lists, list_stride, windows, rec,
+            rec_stride, d_span_step + r0, odd + r0);
         PC_LAUNCH_CHECK("tile_scatter_kernel");
         const size_t lds = TILE_CLAIM_SLOTS * 4u + g.init_stride * 2u;
-        tile_sweep_kernel<ENT, RecT><<<shuf_blocks(g.K, rn), 64, lds, s>>>(
-            g, rn, lists, list_stride, init, rec, rec_stride, d_span_step + r0, odd + r0);
+        tile_sweep_kernel<RecT><<<shuf_blocks(g.K, rn), 64, lds, s>>>(
+            g, rn, lists, list_stride, windows, init, rec, rec_stride, d_span_step + r0,
+            odd + r0);
         PC_LAUNCH_CHECK("tile_sweep_kernel");
     }
     const uint32_t threads = 64u * (1u + EVENT_FINDERS);
@@ -5797,7 +5835,7 @@ static int tile_sweep(uint32_t length, bool tiled, const uint8_t *d_node_sides,
     uint32_t slab = tile_slab(g, num_runs);
     const TilePlan one = tile_plan(g, num_runs, 1u);
     if (workspace_bytes < tile_plan(g, num_runs, slab).bytes) {
-        const uint64_t per_run = one.list_bytes + g.K * 4u;
+        const uint64_t per_run = one.list_bytes + (1u + tile_windows((uint32_t)M)) * g.K * 4u;
         const uint64_t base = one.bytes + 512u;
         slab = workspace_bytes < base ? 0u : (uint32_t)std::min<uint64_t>(
                    slab, 1u + (workspace_bytes - base) / per_run);
@@ -5817,15 +5855,11 @@ static int tile_sweep(uint32_t length, bool tiled, const uint8_t *d_node_sides,
     const bool u32rec = length * length <= kU32RecordMaxNodes;
     int rc;
     if (u32rec)
-        rc = tile_sweep_launch<uint32_t, uint32_t>(
+        rc = tile_sweep_launch<uint32_t>(
             g, p, d_node_sides, d_perm, perm_stride, num_runs, (uint32_t *)d_records,
             rec_stride, d_span_step, (char *)d_workspace, rounds, s);
-    else if (p.short_entries)
-        rc = tile_sweep_launch<uint32_t, uint64_t>(
-            g, p, d_node_sides, d_perm, perm_stride, num_runs, (uint64_t *)d_records,
-            rec_stride, d_span_step, (char *)d_workspace, rounds, s);
     else
-        rc = tile_sweep_launch<uint64_t, uint64_t>(
+        rc = tile_sweep_launch<uint64_t>(
             g, p, d_node_sides, d_perm, perm_stride, num_runs, (uint64_t *)d_records,
             rec_stride, d_span_step, (char *)d_workspace, rounds, s);
     if (rc == PC_OK && d_chunk_state)

@@ -593,3 +593,19 @@ def test_sums_at_their_bounds(gpu, N, runs):
         for k in range(7):
             assert sum(int(w) << (64 * i) for i, w in enumerate(s1[k, j])) == runs * x[k], (s, k)
             assert sum(int(w) << (64 * i) for i, w in enumerate(s2[k, j])) == runs * x[k] ** 2, (s, k)
+
+
+@pytest.mark.parametrize('length,runs,orders', [(725, 2, 'own'), (1100, 1, 'own'), (700, 80, 'random'),
+                                                (2048, 1, 'random')])
+def test_tiled_lattice_sweep_windows(gpu, length, runs, orders):
+    """More steps than a list entry tells apart (2^19): the bonds in their
+    own order and reversed, so that a tile's list lies in few windows and
+    others are empty for it, and random ones, in short segments of the steps
+    and in long ones."""
+    eng = BondEngine(_graph.square_lattice(length))
+    if orders == 'own':
+        one = np.arange(eng.M)
+        perm = eng.upload_permutations(np.stack([one, one[::-1]][:runs]))
+    else:
+        perm = eng.device_permutations(31, runs)
+    _same_sweep(*_tiled_and_untiled(eng, perm))
