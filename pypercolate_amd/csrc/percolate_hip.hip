@@ -5017,9 +5017,10 @@ __global__ __launch_bounds__(256) void fused_reduce_kernel(
 // moments[0..4] (moments as their uint64 values, like the reference's
 // structured array).
 // ---------------------------------------------------------------------------
-#ifndef WT_RUNS
-#define WT_RUNS 4
-#endif
+// 3072 runs of L = 128 over 5600 steps, 0.96 GB of columns: 0.30 ms with four
+// runs a workgroup (two 0.45, eight 0.38), 0.37 with a record at a time and one
+// row a store; a copy writes that much in 0.2.
+#define WT_RUNS 4u
 
 template <typename RecT, bool WIDE>
 __global__ __launch_bounds__(64) void window_traces_kernel(
@@ -5049,32 +5050,43 @@ __global__ __launch_bounds__(64) void window_traces_kernel(
     }
     const int64_t q = c * 64 + lane; // record index, step q + 1
     const bool valid = q < (int64_t)M;
-    for (uint32_t j = 0; j < nr; ++j) {
+    // every run's record before the first is used (past the end the last's)
+    RecT recs[WT_RUNS];
+#pragma unroll
+    for (uint32_t j = 0; j < WT_RUNS; ++j)
+        recs[j] = records[(int64_t)min(r0 + j, R - 1u) * rec_stride + min(q, (int64_t)M - 1)];
+#pragma unroll
+    for (uint32_t j = 0; j < WT_RUNS; ++j) {
+        if (j >= nr)
+            break;
         const uint32_t r = r0 + j;
         const RunState<WIDE> st0 = load_state<WIDE>(
             chunk_state + ((size_t)r * C + (size_t)c) * PC_STATE_WORDS);
-        const RecT rec = valid ? records[(int64_t)r * rec_stride + q] : (RecT)0;
+        const RecT rec = valid ? recs[j] : (RecT)0;
         const RunState<WIDE> st = advance<WIDE>(st0, Deltas<WIDE>(rec));
         MT x[7];
         observables<WIDE>(st, N, (uint64_t)(q + 1) >= span_step[r], x);
         double *row = tile[lane] + j * cols;
         int k = 0;
         if (spanning)
-            row[k++] = (double)(uint64_t)x[1];
-        row[k++] = (double)(uint64_t)x[0];
-        for (int m = 0; m < 5; ++m)
+            row[k++] = (double)(uint32_t)x[1];
+        // the largest cluster, the clusters and the sites beside it: 32 bits
+        row[k++] = (double)(uint32_t)x[0];
+        row[k++] = (double)(uint32_t)x[2];
+        row[k++] = (double)(uint32_t)x[3];
+        for (int m = 2; m < 5; ++m)
             row[k++] = (double)(uint64_t)x[2 + m];
     }
     __syncthreads();
-    const uint32_t n = nr * (uint32_t)cols;
-    for (uint32_t i = 0; i < 64u; ++i) {
-        const int64_t step = c * 64 + i + 1;
-        if (step > (int64_t)M || step < g_lo || step >= g_lo + g_len)
-            continue;
-        double *dst = out + (step - g_lo) * width + (int64_t)r0 * cols;
-        if (lane < n)
-            dst[lane] = tile[i][lane];
-    }
+    // as many rows at a time as the lanes hold
+    const uint32_t n = nr * (uint32_t)cols, rows = 64u / n;
+    const uint32_t first_row = lane / n, col = lane % n;
+    if (first_row < rows)
+        for (uint32_t i = first_row; i < 64u; i += rows) {
+            const int64_t step = c * 64 + i + 1;
+            if (step <= (int64_t)M && step >= g_lo && step < g_lo + g_len)
+                out[(step - g_lo) * width + (int64_t)r0 * cols + col] = tile[i][col];
+        }
     if (c == first_chunk && g_lo == 0 && lane < nr) {
         // step 0: max 1, no spanning, moments N - 1
         double *row = out + (int64_t)(r0 + lane) * cols;
