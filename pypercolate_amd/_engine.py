@@ -557,24 +557,42 @@ def binomial_windows(n, ps):
     return start, length
 
 
+def _p_grid(n, ps, device):
+    """Device tensors (p, window start, window length) of a float64 vector of
+    p in [0, 1], written by a kernel (pc_binomial_grid)."""
+    torch = nat.torch_cuda()
+    ps = np.ascontiguousarray(ps)
+    buf = torch.empty((3, ps.size), dtype=torch.int64, device=device)
+    d_ps = buf[2].view(torch.float64)
+    nat.check(nat.load_library().pc_binomial_grid(
+        int(n), ps.size, ctypes.c_void_p(ps.ctypes.data), nat.ptr(d_ps),
+        nat.ptr(buf[0]), nat.ptr(buf[1]), nat.stream_handle(torch)),
+        'pc_binomial_grid')
+    return d_ps, buf[0], buf[1]
+
+
 def binomial_weights(n, ps, window=True):
     """Device weights B(n, k; p), normalised, for every p: over the window
     |k - np| <= 12 sigma + 48, or over all k = 0..n with window=False."""
     torch = nat.torch_cuda()
     lib = nat.load_library()
     ps = np.atleast_1d(np.asarray(ps, dtype=np.float64))
-    if window:
-        start, length = binomial_windows(n, ps)
-    else:
-        if ps.size and not ((ps >= 0) & (ps <= 1)).all():
-            raise ValueError('p outside [0, 1]')
-        start = np.zeros(ps.size, dtype=np.int64)
-        length = np.full(ps.size, int(n) + 1, dtype=np.int64)
-    kmax = int(length.max()) if ps.size else 1
     dev = torch.device('cuda', torch.cuda.current_device())
-    d_ps = torch.from_numpy(ps.copy()).to(dev)
-    d_start = torch.from_numpy(start).to(dev)
-    d_len = torch.from_numpy(length).to(dev)
+    if window and ps.ndim == 1 and ((ps >= 0) & (ps <= 1)).all():
+        d_ps, d_start, d_len = _p_grid(n, ps, dev)
+        start, length = torch.stack((d_start, d_len)).cpu().numpy()
+    else:
+        if window:
+            start, length = binomial_windows(n, ps)
+        else:
+            if ps.size and not ((ps >= 0) & (ps <= 1)).all():
+                raise ValueError('p outside [0, 1]')
+            start = np.zeros(ps.size, dtype=np.int64)
+            length = np.full(ps.size, int(n) + 1, dtype=np.int64)
+        d_ps = torch.from_numpy(ps.copy()).to(dev)
+        d_start = torch.from_numpy(start).to(dev)
+        d_len = torch.from_numpy(length).to(dev)
+    kmax = int(length.max()) if ps.size else 1
     w = torch.empty((max(ps.size, 1), kmax), dtype=torch.float64, device=dev)
     nat.check(lib.pc_binomial_weights(int(n), ps.size, nat.ptr(d_ps),
                                       nat.ptr(d_start), nat.ptr(d_len), kmax,
@@ -695,14 +713,7 @@ class FusedPlan(object):
             order = np.argsort(ps, kind='stable')
             self.unsort = torch.from_numpy(np.argsort(order).astype(np.int64)).to(dev)
             grid = ps[order]
-        grid = np.ascontiguousarray(grid)
-        buf = torch.empty((3, self.P), dtype=torch.int64, device=dev)
-        self.d_start, self.d_len = buf[0], buf[1]
-        self.d_ps = buf[2].view(torch.float64)
-        nat.check(self.lib.pc_binomial_grid(
-            self.n, self.P, ctypes.c_void_p(grid.ctypes.data), nat.ptr(self.d_ps),
-            nat.ptr(self.d_start), nat.ptr(self.d_len), nat.stream_handle(torch)),
-            'pc_binomial_grid')
+        self.d_ps, self.d_start, self.d_len = _p_grid(self.n, grid, dev)
         if _wait:       # a plan may run on another stream than it was made on
             torch.cuda.current_stream().synchronize()
         b = ctypes.c_uint64(0)
