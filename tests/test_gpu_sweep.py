@@ -609,3 +609,17 @@ def test_tiled_lattice_sweep_windows(gpu, length, runs, orders):
     else:
         perm = eng.device_permutations(31, runs)
     _same_sweep(*_tiled_and_untiled(eng, perm))
+
+
+@pytest.mark.parametrize('runs', [300, 600])
+@pytest.mark.parametrize('M', [2, 3, 64, 65, 127, 128, 480, 1025])
+def test_randomstate_permutations_near_masks(gpu, M, runs):
+    """Many seeds at the sizes where every accepted word shifts the steps
+    that the others in its block may serve, a workgroup a run and a
+    wavefront: numpy's permutations."""
+    eng = BondEngine(_graph.GraphArrays(M + 1, np.stack(
+        [np.arange(M), np.arange(1, M + 1)], axis=1)))
+    seeds = [7 * r + M for r in range(runs)]
+    got = eng.randomstate_permutations(seeds).cpu().numpy()
+    want = np.stack([np.random.RandomState(s).permutation(M) for s in seeds])
+    np.testing.assert_array_equal(got, want)
