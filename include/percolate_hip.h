@@ -276,6 +276,19 @@ int pc_expand_traces(uint32_t num_nodes, uint32_t num_edges, uint32_t num_runs,
                      uint32_t *d_max_size, uint8_t *d_spanning,
                      uint64_t *d_moments, void *stream);
 
+/*
+ * The same as packed rows of the reference's structured array
+ * (percolate/hpc.py:34-70), little-endian, d_rows[(r * S + s) * w]: step
+ * (uint32), edge added (uint32; 0 at step 0), with `spanning` one byte 0 or
+ * 1, largest cluster (uint32), moments 0..4 (uint64); w = 53 with `spanning`,
+ * else 52.  num_edges > 0.
+ */
+int pc_expand_rows(uint32_t num_nodes, uint32_t num_edges, uint32_t num_runs,
+                   const int32_t *d_perm, int64_t perm_stride,
+                   const void *d_records, int64_t rec_stride,
+                   const uint32_t *d_span_step, const uint64_t *d_chunk_state,
+                   int32_t spanning, uint8_t *d_rows, void *stream);
+
 /* Precisions of pc_canonical_contract (element type of d_x and d_w). */
 #define PC_PREC_FP64 0        /* FP64 inputs, FP64 FMA on the vector ALUs    */
 #define PC_PREC_FP64_MFMA 1   /* FP64 inputs, v_mfma_f64_16x16x4f64          */

@@ -304,6 +304,23 @@ class BondEngine(object):
         return (mx.cpu().numpy().view(np.uint32), sp.cpu().numpy().astype(bool),
                 mom.cpu().numpy().view(np.uint64))
 
+    def host_rows(self, res, dtype):
+        """The runs as an (R, S) array of the reference's structured rows
+        (hpc.microcanonical_statistics_dtype, with or without the spanning
+        field), laid out on the device and copied once."""
+        torch = self.torch
+        R, dtype = res.num_runs, np.dtype(dtype)
+        rows = torch.empty((R * self.S * dtype.itemsize,), dtype=torch.uint8,
+                           device=self.device)
+        nat.check(self.lib.pc_expand_rows(
+            self.N, self.M, R, nat.ptr(res.perm), int(res.perm.stride(0)),
+            nat.ptr(res.records), max(self.M, 1), nat.ptr(res.span_step),
+            nat.ptr(res.chunk_state), 1 if 'has_spanning_cluster' in dtype.names else 0,
+            nat.ptr(rows), nat.stream_handle(torch)), 'pc_expand_rows')
+        out = np.empty((R * self.S,), dtype=dtype)
+        torch.from_numpy(out.view(np.uint8)).copy_(rows)
+        return out.reshape(R, self.S)
+
 
 def limbs_to_int(limbs):
     """(..., L) uint64 limb array (little-endian) -> object array of ints."""

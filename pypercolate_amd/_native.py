@@ -63,6 +63,8 @@ SIGNATURES = {
                                               _vp, _vp, _vp, _i32, _vp]),
     'pc_expand_traces': (ctypes.c_int, [_u32, _u32, _u32, _vp, _i64, _vp, _vp,
                                         _vp, _vp, _vp, _vp]),
+    'pc_expand_rows': (ctypes.c_int, [_u32, _u32, _u32, _vp, _i64, _vp, _i64,
+                                      _vp, _vp, _i32, _vp, _vp]),
     'pc_binomial_window': (ctypes.c_int, [_u32, ctypes.c_double,
                                           ctypes.POINTER(_i64),
                                           ctypes.POINTER(_i64)]),

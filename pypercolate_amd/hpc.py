@@ -88,21 +88,6 @@ def _check_sides(spanning_cluster, spanning_sides):
         )
 
 
-def _traces_to_structured(ga, perms, mx, sp, mom, spanning_cluster):
-    """(R, S) device-trace copies -> (R, S) structured arrays."""
-    R, S = mx.shape
-    out = np.empty((R, S), dtype=microcanonical_statistics_dtype(spanning_cluster))
-    out['n'] = np.arange(S, dtype=np.uint32)[np.newaxis, :]
-    out['edge'][:, 0] = 0
-    if S > 1:
-        out['edge'][:, 1:] = perms
-    if spanning_cluster:
-        out['has_spanning_cluster'] = sp
-    out['max_cluster_size'] = mx
-    out['moments'] = mom
-    return out
-
-
 def _int_seeds(seeds):
     """The seeds as uint32 values when every one is an integer in
     [0, 2**32) (RandomState's integer seeding), else None."""
@@ -131,17 +116,14 @@ def _sweep_host_perms(ga, perms, spanning_cluster):
     """Run the GPU sweep for (R, M) permutations; structured (R, S) array."""
     from ._engine import BondEngine
     R = perms.shape[0]
-    S = ga.num_edges + 1
-    if ga.num_edges == 0:
-        mx = np.ones((R, 1), dtype=np.uint32)
-        sp = np.zeros((R, 1), dtype=bool)
-        mom = np.full((R, 1, 5), ga.num_nodes - 1, dtype=np.uint64)
-        return _traces_to_structured(ga, perms, mx, sp, mom, spanning_cluster)
+    dtype = microcanonical_statistics_dtype(spanning_cluster)
+    if ga.num_edges == 0 or R == 0:
+        out = np.zeros((R, ga.num_edges + 1), dtype=dtype)
+        out['max_cluster_size'] = 1
+        out['moments'] = ga.num_nodes - 1
+        return out
     eng = BondEngine(ga)
-    res = eng.sweep(eng.upload_permutations(perms))
-    mx, sp, mom = eng.host_traces(res)
-    assert mx.shape == (R, S)
-    return _traces_to_structured(ga, perms, mx, sp, mom, spanning_cluster)
+    return eng.host_rows(eng.sweep(eng.upload_permutations(perms)), dtype)
 
 
 def bond_sample_states(
@@ -218,11 +200,8 @@ def bond_microcanonical_statistics_batch(
         return _sweep_host_perms(ga, perms, spanning_cluster)
     from ._engine import BondEngine
     eng = BondEngine(ga)
-    d_perm = _permutations(eng, seeds)
-    res = eng.sweep(d_perm)
-    mx, sp, mom = eng.host_traces(res)
-    return _traces_to_structured(ga, d_perm.cpu().numpy(), mx, sp, mom,
-                                 spanning_cluster)
+    return eng.host_rows(eng.sweep(_permutations(eng, seeds)),
+                         microcanonical_statistics_dtype(spanning_cluster))
 
 
 def _trace_columns(microcanonical_statistics):

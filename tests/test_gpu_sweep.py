@@ -623,3 +623,29 @@ def test_randomstate_permutations_near_masks(gpu, M, runs):
     got = eng.randomstate_permutations(seeds).cpu().numpy()
     want = np.stack([np.random.RandomState(s).permutation(M) for s in seeds])
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize('spanning', [True, False])
+@pytest.mark.parametrize('length', [2, 6, 9, 33, 130, 257])
+def test_structured_rows_equal_traces(gpu, length, spanning):
+    """The packed rows (53 or 52 bytes, so at every offset from a word) hold
+    the traces, the permutation and the row of step 0: narrow and wide
+    moments, 32- and 64-bit records, whole and ragged chunks, permutations
+    in a wider buffer."""
+    from pypercolate_amd import hpc
+    eng = BondEngine(_graph.square_lattice(length, spanning_cluster=spanning))
+    wide = gpu.full((5, eng.M + 3), -1, dtype=gpu.int32, device='cuda')
+    perm = eng.device_permutations(41, 5)
+    wide[:, :eng.M] = perm
+    res = eng.sweep(perm)
+    res.perm = wide[:, :eng.M]
+    rows = eng.host_rows(res, hpc.microcanonical_statistics_dtype(spanning))
+    mx, sp, mom = eng.host_traces(res)
+    assert rows.shape == mx.shape and rows.flags.writeable
+    np.testing.assert_array_equal(rows['n'], np.broadcast_to(np.arange(eng.S), mx.shape))
+    np.testing.assert_array_equal(rows['edge'][:, 1:], perm.cpu().numpy())
+    assert (rows['edge'][:, 0] == 0).all()
+    np.testing.assert_array_equal(rows['max_cluster_size'], mx)
+    np.testing.assert_array_equal(rows['moments'], mom)
+    if spanning:
+        np.testing.assert_array_equal(rows['has_spanning_cluster'], sp)
