@@ -2705,9 +2705,9 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 // more than TILE_MANY tiles, lists and lines fill in small pieces: 16 groups
 // took 1000 runs of L = 1024 (256 tiles) from 17.0 to 15.1 ms, 300 of L = 700
 // (121) 2.44 to 2.27, 1000 of L = 384 (36) 1.85 to 1.70; 600 of L = 181 (9)
-// 0.157 to 0.179, so fewer tiles keep eight, and so do segments of fewer than
-// TILE_LONG_SEGMENT steps, where a turn is a large part (200 runs of L = 256,
-// 64 tiles, segments of 22000: 0.115 to 0.138).
+// 0.157 to 0.179 and 200 of L = 256 (16) 0.115 to 0.138, so fewer tiles keep
+// eight, and so do segments of fewer than TILE_LONG_SEGMENT steps, where a
+// turn is a large part (32 runs of L = 512, the whole sweep: 2.18 to 2.15 ms).
 #define TILE_GROUPS 8u
 #define TILE_GROUPS_MANY 16u
 #define TILE_MANY 32u
@@ -5741,16 +5741,19 @@ static LatticeEdges lattice_edges(uint32_t length, bool tiled)
 //   tiled, is 0.784 and 0.842 for 4000 runs of L = 80, 0.296 and 0.252 for
 //   200; 2.68 and 2.36 for 8000 of L = 100, 7.06 and 5.05 for 10^4 of L = 128,
 //   0.66 and 0.47 for 200 of those.
-// - Tiles of at most 64 x 64 nodes, or 32 x 32 where those would leave the
-//   GPU with at most 2048 wavefronts (200 runs of L = 128: 0.52 and 0.43 ms,
-//   500 of L = 100: 0.40 and 0.38; more tiles make more events).
+// - Tiles of at most 64 x 64 nodes, or 32 x 32 up to L = 128 where those would
+//   leave the GPU with at most 2048 wavefronts: more tiles make more events.
+//   Sweep in milliseconds with 64 and 32, 200 runs of L = 128 0.479 and 0.412,
+//   600 0.547 and 0.548; 500 of L = 100 0.365 and 0.357, 1000 0.445 and 0.491;
+//   100 of L = 181 0.598 and 0.597, 200 0.629 and 0.668; 50 of L = 256 0.83 and
+//   0.89; 10 of L = 512 2.08 and 2.63.
 static bool tile_geo(uint32_t length, bool tiled, uint32_t num_runs, TileGeo &g)
 {
     if (length <= TILE_SIDE || length > TILE_MAX_LENGTH ||
         (length < TILE_LDS_LENGTH && num_runs > 1024u))
         return false;
     const uint32_t k64 = (length + TILE_SIDE - 1u) / TILE_SIDE;
-    const bool small = length <= 512u && (uint64_t)k64 * k64 * num_runs <= 2048u;
+    const bool small = length <= 128u && (uint64_t)k64 * k64 * num_runs <= 2048u;
     const uint32_t side = small ? TILE_SIDE / 2u : TILE_SIDE;
     g.lat = lattice_edges(length, tiled);
     g.L = length;
@@ -5850,8 +5853,7 @@ static int tile_sweep_launch(const TileGeo &g, const TilePlan &p,
         uint32_t nseg = (TILE_SCATTER_BLOCKS + rn - 1u) / rn;
         nseg = std::min(nseg, (M + 16383u) / 16384u);
         const bool many = g.K > TILE_MANY && M / nseg >= TILE_LONG_SEGMENT;
-        // (32-bit records come with more than TILE_MANY tiles in short
-        // segments only)
+        // (32-bit records: at most 16 tiles)
         constexpr uint32_t MANY = sizeof(RecT) == 8u ? TILE_GROUPS_MANY : TILE_GROUPS;
         const uint32_t quant = 256u * (many ? MANY : TILE_GROUPS);
         const uint32_t seg = ((M + nseg - 1u) / nseg + quant - 1u) / quant * quant;

@@ -437,9 +437,9 @@ def test_tiled_lattice_sweep_equals_untiled(gpu, length, runs):
     """The tiled sweep's records, span steps and chunk states equal those of
     the sweep with every node's code in HBM: tiles of up to 32 x 32 nodes (few
     runs) and 64 x 64, whole and ragged, state within the LDS limit, 32- and
-    64-bit records (from 257), 32- and 64-bit list entries (from 513), open
-    nodes in LDS (a run or several per CU) and in HBM (1000; 400 for more
-    than 256 runs), one workgroup per run or several."""
+    64-bit records (from 257), open nodes in LDS (a run or several per CU)
+    and in HBM (1000; 400 for more than 256 runs), one workgroup per run or
+    several."""
     eng = BondEngine(_graph.square_lattice(length))
     perm = eng.device_permutations(17, runs)
     _same_sweep(*_tiled_and_untiled(eng, perm))
