@@ -86,8 +86,8 @@ def profiled_traffic_per_add(length, runs):
 
 def large_lattice(length, runs, seed, steps=2, warmup=1):
     """The L = 1024 configuration: spanning_2d_grid(1024) (N = 1,048,576,
-    M = 2,095,104), 1000 runs from Philox seed 7, union-find state in the
-    HBM workspace (32-bit codes), 64-bit merge records, the whole per-step
+    M = 2,095,104), 1000 runs from Philox seed 7, tiled sweep (a tile's
+    state in LDS, the open nodes' in HBM), 64-bit merge records, the whole per-step
     trace reduced on the device to exact sums (moments k = 3, 4 and all
     squares in 128/192-bit).  Returns the timing and the engine and exact
     sums of the last step (the input of the canonical comparison)."""
@@ -605,6 +605,7 @@ def main(argv=None):
     adds = float(R) * M
     traffic_per_add = profiled_traffic_per_add(args.length, R)
     value = adds / (ms_per_step / 1e3)
+    tiled = 96 <= args.length <= 2048   # the tiled sweep's range
     alg_bytes = ALG_BYTES_PER_ADD_LDS if N <= 16384 else ALG_BYTES_PER_ADD_HBM
     # algorithmic bytes of the step's sweep launches over their span: the
     # launches overlap on two streams, so one launch's own duration also
@@ -630,24 +631,27 @@ def main(argv=None):
                          '-> chunk states -> exact microcanonical sums').format(
                              args.length, N, M, R),
             'length': args.length, 'runs': R, 'nodes': N, 'edges': M,
-            'parallelism': ('single GPU, one run per workgroup of {} '
-                            'wavefront(s); permutations of all runs (one '
+            'parallelism': ('single GPU, {}; permutations of all runs (one '
                             'launch; every step draws the next step\'s once '
                             'its sweeps have ended, beside its last '
                             'reductions), sub-batches of {} runs (one '
                             'residency), sweeps alternating between two '
                             'streams, reductions beside them on a third').format(
-                                2 if N >= 4096 else 1, pipe.sub),
+                                'one wavefront per run and lattice tile' if tiled
+                                else 'one run per workgroup', pipe.sub),
         },
         'roofline': {
-            'kernel': 'sweep_lds_kernel' if N <= 16384 else 'sweep_global_kernel',
+            'kernel': ('tile_scatter_kernel, tile_sweep_kernel, event_sweep_kernel'
+                       if tiled else
+                       'sweep_lds_kernel' if N <= 16384 else 'sweep_global_kernel'),
             'bound': 'hbm',
-            # what actually limits it: the union-find state is in LDS, and
-            # the resolver's dependent instruction chain (one resolver wave
-            # per SIMD at 4 runs per CU) sets the pace, not a bandwidth
-            'limiter': ('resolver dependent-instruction chain (LDS-resident '
-                        'state, issue/latency bound)' if N <= 16384 else
-                        'HBM lines of the union-find state'),
+            # what actually limits it: lists are bound by vector issue and the
+            # tiles' and events' merges by dependent LDS round trips (vector
+            # ALUs 70 % busy over the step at L = 128); at L = 1024 by records
+            # stored as parts of lines and the lines of the open nodes
+            'limiter': ('vector issue and dependent LDS round trips of the '
+                        'merges' if N <= 65536 else
+                        'part-written record lines, HBM lines of the open nodes'),
             'achieved': achieved,
             'peak': HBM_PEAK_GBS,
             'unit': 'GB/s',

@@ -192,7 +192,8 @@ class BondEngine(object):
 
     def fuse_chunk_states(self):
         """Whether the sweep should write the chunk states itself (its finder
-        wave folds the records one batch behind the resolver).  Measured on
+        wave folds the records one batch behind the resolver; a tiled sweep
+        runs the separate passes).  Measured with the untiled sweep on
         MI355X: with the union-find state in LDS the fold still lengthens the
         sweep by ~12 % (L = 128: 7.7 -> 8.7 ms for 10^4 runs), more than the
         separate pass (pc_chunk_scan) costs on another stream; with the state

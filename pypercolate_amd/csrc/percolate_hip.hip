@@ -4,8 +4,10 @@
 //
 // Pipeline for R runs on a graph with N nodes and M edges:
 //   permute (Philox-keyed bucket shuffle, or MT19937 + numpy's shuffle for
-//   bit-exact RandomState permutations) -> sweep (union-find, one run per
-//   workgroup of one or two wavefronts, merge records) -> chunk states
+//   bit-exact RandomState permutations) -> sweep (union-find: square
+//   lattices in tiles, one wavefront per run and tile, then the events
+//   between tiles; other graphs one run per workgroup of one or two
+//   wavefronts; merge records) -> chunk states
 //   (per-run state every 64
 //   steps: two passes over the records, or written by the sweep itself) ->
 //   microcanonical sums (exact Sigma x, Sigma x^2 over runs per step) or
