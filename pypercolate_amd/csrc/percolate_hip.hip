@@ -2717,11 +2717,12 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 #define TILE_WINDOW (1u << 19)  // the steps that a list entry can tell apart
 
 // Tiles of h x w nodes (the last row and column of tiles may be smaller),
-// KH x KW of them.  mh, mw divide a coordinate by h and w (high half of the
+// KH x KW of them.  mh, mw, md divide a coordinate by h and w, a bond by the
+// bonds of a row (high half of the
 // product, exact below 2^16).  Ids of a tile's border nodes: per of them.
 struct TileGeo {
     LatticeEdges lat;
-    uint32_t L, h, w, KH, KW, K, per, mh, mw, init_stride;
+    uint32_t L, h, w, KH, KW, K, per, mh, mw, md, init_stride;
     __host__ __device__ __forceinline__ uint32_t rows(uint32_t tr) const { return tr + 1u < KH ? h : L - (KH - 1u) * h; }
     __host__ __device__ __forceinline__ uint32_t cols(uint32_t tc) const { return tc + 1u < KW ? w : L - (KW - 1u) * w; }
     // internal bonds of a tile of hh x ww nodes, and the first list entry of
@@ -2790,16 +2791,22 @@ struct TileBond {
 };
 __device__ __forceinline__ TileBond tile_bond(const TileGeo &g, int32_t e)
 {
-    uint32_t r, c, down;
-    g.lat.bond((uint32_t)e, r, c, down);
+    // row and place in it, as LatticeEdges::bond: the high half of the product
+    // with ceil(2^32 / d) is the quotient or one more, below 2^32 / d bonds
+    uint32_t r = __umulhi((uint32_t)e, g.md);
+    int32_t j = e - (int32_t)(r * g.lat.d);
+    r -= j < 0 ? 1u : 0u;
+    j += j < 0 ? (int32_t)g.lat.d : 0;
+    const bool last = r + 1u == g.L;
+    const uint32_t c = last ? (uint32_t)j : (uint32_t)j >> 1;
     TileBond b;
+    b.down = last ? 0u : ~(uint32_t)j & 1u;
     b.tr = __umulhi(r, g.mh);
     const uint32_t tc = __umulhi(c, g.mw);
     b.lr = r - b.tr * g.h;
     b.lc = c - tc * g.w;
     b.k = b.tr * g.KW + tc;
-    b.down = down;
-    b.cross = down ? b.lr + 1u == g.h : b.lc + 1u == g.w;
+    b.cross = (b.down ? b.lr : b.lc) + 1u == g.h;   // h = w
     return b;
 }
 
@@ -2844,11 +2851,20 @@ __global__ __launch_bounds__(256) void tile_count_kernel(
     __syncthreads();
     const int32_t *p = perm + (int64_t)blockIdx.y * perm_stride;
     const uint32_t end = min(M, (seg + 1u) * seg_steps);
-    for (uint32_t t = seg * seg_steps + threadIdx.x; t < end; t += 256u) {
-        const uint32_t e = (uint32_t)p[t];
-        const TileBond b = tile_bond(g, (int32_t)min(e, M - 1u));
-        if (e < M && !b.cross)
-            atomicAdd(&tile_cnt[b.k], 1u);
+    // eight bonds a thread in flight (1000 runs of L = 1024: 2.0 ms, one at a
+    // time 3.8; 500 of L = 100 17 us, 35)
+    for (uint32_t t0 = seg * seg_steps + threadIdx.x; t0 < end; t0 += 8u * 256u) {
+        uint32_t e[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i)
+            e[i] = (uint32_t)p[min(t0 + i * 256u, M - 1u)];
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i) {
+            const bool ok = t0 + i * 256u < end && e[i] < M;
+            const TileBond b = tile_bond(g, (int32_t)(ok ? e[i] : 0u));
+            if (ok && !b.cross)
+                atomicAdd(&tile_cnt[b.k], 1u);
+        }
     }
     __syncthreads();
     for (uint32_t k = threadIdx.x; k < g.K; k += 256u)
@@ -2911,9 +2927,12 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(
     const uint32_t end = min(M, (seg + 1u) * seg_steps);
     int32_t e[GROUPS];
     uint32_t t0 = seg * seg_steps + wave * 64u * GROUPS + lane;
+    auto load = [&]() {
 #pragma unroll
-    for (uint32_t i = 0; i < GROUPS; ++i)
-        e[i] = t0 + i * 64u < end ? p[t0 + i * 64u] : -1;
+        for (uint32_t i = 0; i < GROUPS; ++i)
+            e[i] = p[min(t0 + i * 64u, M - 1u)];
+    };
+    load();
     for (uint32_t base = seg * seg_steps; base < end; base += 256u * GROUPS) {
         for (uint32_t k = lane; k < g.K; k += 64u)
             my[k] = 0u;
@@ -2924,37 +2943,46 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(
         }
         uint32_t ent[GROUPS];
         uint32_t at[GROUPS];   // tile | rank << 12, or all ones
+        // a turn within the segment needs no test of its steps (with that, and
+        // the row of a bond from one product and no branch, 1000 runs of L =
+        // 1024 take 14.0 ms, not 15.1; 3072 of L = 128 0.305, not 0.326)
+        auto turn = [&](auto whole) __attribute__((always_inline)) {
+            RecT *out = rec + t0;
 #pragma unroll
-        for (uint32_t i = 0; i < GROUPS; ++i) {
-            const uint32_t t = t0 + i * 64u;
-            const bool ok = (uint32_t)e[i] < M;
-            const TileBond b = tile_bond(g, ok ? e[i] : 0);
-            const bool in = ok && !b.cross;
-            const uint64_t peers = match_label(b.k, tile_bits, ballot(in));
-            at[i] = 0xFFFFFFFFu;
-            if (in) {
-                const uint32_t rank = lanes_below(peers);
-                const uint32_t before = my[b.k];
-                at[i] = b.k | ((before + rank) << 12);
-                if (rank == 0u)
-                    my[b.k] = before + (uint32_t)__popcll(peers);
+            for (uint32_t i = 0; i < GROUPS; ++i) {
+                const uint32_t t = t0 + i * 64u;
+                const bool here = decltype(whole)::value || t < end;
+                const bool ok = here && (uint32_t)e[i] < M;
+                const TileBond b = tile_bond(g, ok ? e[i] : 0);
+                const bool in = ok && !b.cross;
+                const uint64_t peers = match_label(b.k, tile_bits, ballot(in));
+                at[i] = 0xFFFFFFFFu;
+                if (in) {
+                    const uint32_t rank = lanes_below(peers);
+                    const uint32_t before = my[b.k];
+                    at[i] = b.k | ((before + rank) << 12);
+                    if (rank == 0u)
+                        my[b.k] = before + (uint32_t)__popcll(peers);
+                }
+                RecT ev = 0;
+                if (ok && b.cross) {
+                    const uint32_t hh = g.rows(b.tr);
+                    const uint32_t iu = b.k * g.per + g.border(b.lr, b.lc, hh);
+                    const uint32_t kv = b.down ? b.k + g.KW : b.k + 1u;
+                    const uint32_t iv = kv * g.per + (b.down ? b.lc : g.border(b.lr, 0u, hh));
+                    ev = EventBits<RecT>::join(iu, iv);
+                }
+                if (here)
+                    out[i * 64u] = ev;
+                ent[i] = TileEntry::make(t, b.lr * g.w + b.lc, b.down);
             }
-            RecT ev = 0;
-            if (ok && b.cross) {
-                const uint32_t hh = g.rows(b.tr);
-                const uint32_t iu = b.k * g.per + g.border(b.lr, b.lc, hh);
-                const uint32_t kv = b.down ? b.k + g.KW : b.k + 1u;
-                const uint32_t iv = kv * g.per + (b.down ? b.lc : g.border(b.lr, 0u, hh));
-                ev = EventBits<RecT>::join(iu, iv);
-            }
-            if (t < end)
-                rec[t] = ev;
-            ent[i] = TileEntry::make(t, b.lr * g.w + b.lc, b.down);
-        }
-        const uint32_t tn = t0 + 256u * GROUPS;
-#pragma unroll
-        for (uint32_t i = 0; i < GROUPS; ++i)
-            e[i] = tn + i * 64u < end ? p[tn + i * 64u] : -1;
+        };
+        if (base + 256u * GROUPS <= end)
+            turn(std::true_type());
+        else
+            turn(std::false_type());
+        t0 += 256u * GROUPS;
+        load();
         __syncthreads();
         for (uint32_t k = tid; k < g.K; k += 256u) {
             uint32_t acc = cursor[k];
@@ -2973,7 +3001,6 @@ __global__ __launch_bounds__(256) void tile_scatter_kernel(
         for (uint32_t i = 0; i < GROUPS; ++i)
             if (at[i] != 0xFFFFFFFFu)
                 list[my[at[i] & 0xFFFu] + (at[i] >> 12)] = ent[i];
-        t0 = tn;
     }
     if (nseg == 1u) {
         for (uint32_t k = tid; k < g.K; k += 256u)
@@ -5765,6 +5792,7 @@ static bool tile_geo(uint32_t length, bool tiled, uint32_t num_runs, TileGeo &g)
     g.per = 2u * g.w + 2u * (g.h - 2u);
     g.mh = (uint32_t)(((1ull << 32) + g.h - 1u) / g.h);
     g.mw = (uint32_t)(((1ull << 32) + g.w - 1u) / g.w);
+    g.md = (uint32_t)(((1ull << 32) + g.lat.d - 1u) / g.lat.d);
     g.init_stride = (g.h * g.w + 7u) & ~7u;
     return true;
 }
