@@ -122,18 +122,6 @@ __device__ __forceinline__ T wave_scan_add(T x)
     return x;
 }
 
-// Inclusive prefix maximum over the 64 lanes (unsigned, identity 0).
-__device__ __forceinline__ uint32_t wave_scan_max(uint32_t x)
-{
-    x = max(x, dpp32<DPP_ROW_SHR(1)>(x));
-    x = max(x, dpp32<DPP_ROW_SHR(2)>(x));
-    x = max(x, dpp32<DPP_ROW_SHR(4)>(x));
-    x = max(x, dpp32<DPP_ROW_SHR(8)>(x));
-    x = max(x, dpp32<DPP_ROW_BCAST15, 0xa>(x));
-    x = max(x, dpp32<DPP_ROW_BCAST31, 0xc>(x));
-    return x;
-}
-
 // Inclusive prefix scans over the 64 lanes of a chunk's state in one go: the
 // maximum mx and the sums d2, d3, d4 (32 to 128 bits), in place with DPP adds
 // and carries (one instruction per word and step; the scans' steps alternate,
@@ -2678,7 +2666,7 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 // Untiled, with every node's code in HBM, the sweep moves 342 bytes per
 // addition in random lines at L = 1024, and at L = 128 (codes in LDS) four
 // runs fill a CU.  Sweep with its chunk states, untiled and tiled: L = 1024,
-// 1000 runs 158 and 63 ms (lists 19, tiles 19, events 20, chunk states 4);
+// 1000 runs 158 and 60 ms (lists 16, tiles 19, events 20, chunk states 4);
 // L = 256, 200 runs 3.67 and 1.1; L = 181, 600 runs 2.65 and 1.1; L = 128,
 // 10^4 runs (no chunk states) 7.06 and 5.05.  The tiles are bound by vector
 // issue (60 % of a wavefront's share of its SIMD at L = 256) and dependent
@@ -2718,8 +2706,8 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 
 // Tiles of h x w nodes (the last row and column of tiles may be smaller),
 // KH x KW of them.  mh, mw, md divide a coordinate by h and w, a bond by the
-// bonds of a row (high half of the
-// product, exact below 2^16).  Ids of a tile's border nodes: per of them.
+// bonds of a row (high half of the product; exact below 2^16, tile_bond
+// corrects the bond's).  Ids of a tile's border nodes: per of them.
 struct TileGeo {
     LatticeEdges lat;
     uint32_t L, h, w, KH, KW, K, per, mh, mw, md, init_stride;
@@ -3720,7 +3708,6 @@ __global__ __launch_bounds__(64 * WAVES) void micro_sums_kernel(
     // the waves' accumulators on their way to wave 0
     constexpr uint32_t PARTS = WIDE ? 21u : 18u;
     __shared__ uint64_t part[WAVES > 1u ? PARTS : 1u][64];
-    using MT = typename Wide<WIDE>::T;
     const uint32_t c = blockIdx.x, g = blockIdx.y, lane = threadIdx.x & 63u;
     const uint32_t wave = uniform(threadIdx.x >> 6);
     const uint32_t C = (M + 63u) / 64u;
