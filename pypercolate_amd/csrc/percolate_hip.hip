@@ -4047,10 +4047,21 @@ __global__ __launch_bounds__(64) void expand_kernel(
     if (valid) {
         out_max[row] = (uint32_t)x[0];
         out_span[row] = (uint8_t)x[1];
-#pragma unroll
-        for (int k = 0; k < 5; ++k)
-            out_mom[row * 5u + k] = (uint64_t)x[2 + k];
     }
+    // the chunk's moments through LDS, so that a store takes 512 bytes in a row
+    // (500 runs of L = 100: 97 us, with 64 pieces of 8 a store 122; a copy
+    // writes their 445 MB in 91)
+    __shared__ uint64_t mom[64 * 5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+        mom[lane * 5u + k] = (uint64_t)x[2 + k];
+    __syncthreads();
+    const uint32_t n = min(64u, M - c * 64u) * 5u;
+    uint64_t *dst = out_mom + ((uint64_t)r * S + c * 64u + 1u) * 5u;
+#pragma unroll
+    for (uint32_t i = 0; i < 5u; ++i)
+        if (i * 64u + lane < n)
+            dst[i * 64u + lane] = mom[i * 64u + lane];
     if (c == 0 && lane == 0) {
         const uint64_t row0 = (uint64_t)r * S;
         out_max[row0] = 1u;
