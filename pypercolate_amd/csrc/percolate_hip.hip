@@ -3623,12 +3623,11 @@ __global__ __launch_bounds__(64) void chunk_prefix_kernel(
 // L = 128 as a pipeline: 8.3 ms, 9.5 with the form below).  Elsewhere the four
 // waves of a workgroup share 64 runs of a chunk and add up in LDS, so that a
 // fourth of the atomics remain (L = 100, 500 runs 0.121 -> 0.044 ms; L = 16,
-// 40 runs 13 -> 8 us).  Bound by vector issue: 112 to 150 instructions a
-// record.  With the squares added up limb by limb in doubles (SquareSum)
-// instead of as 128- and 192-bit integers (255 instructions), and the sums of
-// N - max left to the end, 1000 runs of L = 1024 take 7.9 ms, not 12.7 (their
-// records alone: 3.5); 600 of L = 181 0.19, not 0.26; 200 of L = 256 0.158,
-// not 0.180; a sub-batch of L = 128 beside its sweeps 0.19, not 0.21.
+// 40 runs 13 -> 8 us).  Bound by vector issue.  With the squares added up limb
+// by limb (SquareSum) instead of as 128- and 192-bit integers, and the sums of
+// N - max left to the end, 1000 runs of L = 1024 take 9.3 ms, not 12.7 (their
+// records alone: 3.5); 600 of L = 181 0.196, not 0.262; 200 of L = 256 0.147,
+// not 0.180; a sub-batch of L = 128 beside its sweeps 0.17, not 0.21.
 #define SUMS_BLOCKS 8192u
 #define SUMS_RUNS 32u
 #define SUMS_MOST 1024u   // runs a group may hold: what the bounds below allow
@@ -3653,27 +3652,23 @@ __device__ __forceinline__ u96 mul_u96(uint64_t p, uint64_t q)
     return ((u96)hi << 64) | ((u96)(uint32_t)t2 << 32) | (uint32_t)t0;
 }
 
-// Sum of the squares of numbers of K limbs of B <= 21 bits: a sum for every
+// Sum of the squares of numbers of K limbs of B <= 27 bits: a sum for every
 // product of two limbs, put together once at the end, so that a square costs
-// no carries.  The sums are doubles, whose multiply-adds run at full rate
-// (64-bit integer ones: 9.3 ms where these take 7.9), and exact: SUMS_MOST
-// products below 2^42 stay below 2^53.
+// no carries.  SUMS_MOST products below 2^54 fit 64 bits, and a product is
+// added by the instruction that forms it (in doubles, limbs of 21 bits and a
+// conversion each, 1000 runs of L = 1024 took 10.3 ms, with these 9.3).
 template <int K, int B>
 struct SquareSum {
-    static_assert(2 * B <= 42, "exact in a double");
-    double sum[K * (K + 1) / 2] = {};
+    static_assert(2 * B <= 54, "64 bits hold the sums");
+    uint64_t sum[K * (K + 1) / 2] = {};
     __device__ __forceinline__ void add(const uint32_t *limb)
     {
-        double l[K];
-#pragma unroll
-        for (int i = 0; i < K; ++i)
-            l[i] = (double)limb[i];
         int n = 0;
 #pragma unroll
         for (int i = 0; i < K; ++i)
 #pragma unroll
             for (int j = i; j < K; ++j)
-                sum[n] = __builtin_fma(l[i], l[j], sum[n]), ++n;
+                sum[n] += (uint64_t)limb[i] * limb[j], ++n;
     }
     // low 128 bits, and the word above
     __device__ __forceinline__ u128 value(uint64_t &top) const
@@ -3685,7 +3680,7 @@ struct SquareSum {
         for (int i = 0; i < K; ++i)
 #pragma unroll
             for (int j = i; j < K; ++j) {
-                const u128 v = (u128)(uint64_t)sum[n++] << (i == j ? 0 : 1);
+                const u128 v = (u128)sum[n++] << (i == j ? 0 : 1);
                 const int shift = B * (i + j);
                 const u128 part = shift < 128 ? v << (shift & 127) : (u128)0;
                 lo += part;
@@ -3773,8 +3768,7 @@ __global__ __launch_bounds__(64 * WAVES) void micro_sums_kernel(
         uint64_t n2[4] = {0, 0, 0, 0};  // sum x^2 of the same
         uint64_t m1_2 = 0, m1_3 = 0, m1_4 = 0;   // sum x: moments 2 to 4
         uint64_t sq_2 = 0;
-        SquareSum<2, 20> sq_3;
-        SquareSum<3, 18> sq_4;
+        SquareSum<2, 27> sq_3, sq_4;
         uint32_t count = 0;
         for (uint32_t r = r0 + wave; r < r1; r += WAVES) {
             const RunState<false> st0 = st_next;
@@ -3799,9 +3793,9 @@ __global__ __launch_bounds__(64 * WAVES) void micro_sums_kernel(
             m1_3 += x5;
             const uint64_t x6 = st0.s4 + d.d4 - (uint64_t)mx2 * mx2;
             m1_4 += x6;
-            const uint32_t l5[2] = {(uint32_t)x5 & 0xFFFFFu, (uint32_t)(x5 >> 20)};
-            const uint32_t l6[3] = {(uint32_t)x6 & 0x3FFFFu, (uint32_t)(x6 >> 18) & 0x3FFFFu,
-                                    (uint32_t)(x6 >> 36)};
+            constexpr uint32_t LIMB = (1u << 27) - 1u;
+            const uint32_t l5[2] = {(uint32_t)x5 & LIMB, (uint32_t)(x5 >> 27)};
+            const uint32_t l6[2] = {(uint32_t)x6 & LIMB, (uint32_t)(x6 >> 27)};
             sq_3.add(l5);
             sq_4.add(l6);
         }
@@ -3841,17 +3835,18 @@ __global__ __launch_bounds__(64 * WAVES) void micro_sums_kernel(
         // S3 is below N^3 <= 2^63 (its deltas and scan stay in 64 bits), S4
         // at most N^4 <= 2^84 (96 bits); max, #clusters - 1 and N - max are
         // at most 2^21 (group sums below 2^32, of squares below 2^53),
-        // moment 2 below 2^42, moment 3 below 2^63 and moment 4 below 2^84:
-        // two, three and four limbs of 21 bits.  The sums of N - max follow
-        // from those of max.
+        // moment 2 below 2^42, moment 3 below 2^63 and moment 4 below 2^84.
+        // The sums of N - max follow from those of max.
         uint64_t n1[5] = {0, 0, 0, 0, 0}; // sum x: max, span, #clusters - 1, N - max, moment 2
         uint64_t n2[4] = {0, 0, 0, 0};    // sum x^2 of the first four
         uint32_t s_mx = 0, s_span = 0, s_cl = 0, count = 0;
         u96 s_3 = 0, s_4 = 0;             // sum x: moments 3 and 4
-        SquareSum<2, 21> sq_2;
-        SquareSum<3, 21> sq_3;
-        SquareSum<4, 21> sq_4;
-        constexpr uint32_t LIMB = (1u << 21) - 1u;
+        // 32-bit records: N <= 2^16, moments below 2^31, 2^48 and 2^64
+        constexpr int K3 = sizeof(RecT) == 4u ? 2 : 3, K4 = sizeof(RecT) == 4u ? 3 : 4;
+        SquareSum<2, 27> sq_2;
+        SquareSum<K3, 27> sq_3;
+        SquareSum<K4, 27> sq_4;
+        constexpr uint32_t LIMB = (1u << 27) - 1u;
         for (uint32_t r = r0 + wave; r < r1; r += WAVES) {
             const uint32_t mx0 = (uint32_t)st_next.mx, merges0 = (uint32_t)st_next.merges;
             const uint64_t s2_0 = st_next.s2, s3_0 = (uint64_t)st_next.s3;
@@ -3886,11 +3881,14 @@ __global__ __launch_bounds__(64 * WAVES) void micro_sums_kernel(
             n1[4] += x4;
             s_3 += x5;
             s_4 += x6;
-            const uint32_t l4[2] = {(uint32_t)x4 & LIMB, (uint32_t)(x4 >> 21)};
-            const uint32_t l5[3] = {(uint32_t)x5 & LIMB, (uint32_t)(x5 >> 21) & LIMB,
-                                    (uint32_t)(x5 >> 42)};
-            const uint32_t l6[4] = {(uint32_t)x6 & LIMB, (uint32_t)(x6 >> 21) & LIMB,
-                                    (uint32_t)(x6 >> 42) & LIMB, (uint32_t)(x6 >> 63)};
+            const uint32_t l4[2] = {(uint32_t)x4 & LIMB, (uint32_t)(x4 >> 27)};
+            uint32_t l5[K3], l6[K4];
+#pragma unroll
+            for (int i = 0; i < K3; ++i)
+                l5[i] = (uint32_t)(x5 >> (27 * i)) & (i + 1 < K3 ? LIMB : 0xFFFFFFFFu);
+#pragma unroll
+            for (int i = 0; i < K4; ++i)
+                l6[i] = (uint32_t)(x6 >> (27 * i)) & (i + 1 < K4 ? LIMB : 0xFFFFFFFFu);
             sq_2.add(l4);
             sq_3.add(l5);
             sq_4.add(l6);

@@ -567,7 +567,8 @@ def test_device_permutation_label_bits(gpu, M):
         np.testing.assert_array_equal(got[r], want[r], err_msg='run {}'.format(r))
 
 
-@pytest.mark.parametrize('N,runs', [(16384, 2500), (16385, 1100), (1 << 21, 2)])
+@pytest.mark.parametrize('N,runs', [(16384, 2500), (16385, 1100), (65536, 1100), (65537, 3),
+                                    (1 << 21, 2)])
 def test_sums_at_their_bounds(gpu, N, runs):
     """Two clusters of half the nodes each, the largest moments there are,
     at the node counts where the sums' arithmetic changes or ends and with
