@@ -4882,6 +4882,10 @@ __global__ __launch_bounds__(64, 3) void canonical_fused_f64_kernel(
         // the row's window within the lane's range, as steps of the walk
         const int ja = (int)min(b.ka - kq0, (int64_t)1 << 30);
         const int je = (int)min(max(b.kend - kq0, (int64_t)0), (int64_t)1 << 30);
+        // A chunk before this step ends no window: the one that does, at its
+        // last step too, has to clear the weight.  (Where the lane's range
+        // ends as well, or first, the steps after it count as 0 anyway.)
+        const int jw = b.kend == kq1 ? je + 1 : je;
         double xn[FUSED_F64_UNROLL];
         // FULL: the next chunk lies in every lane's range.  (Both forms of
         // loads in one loop would be branches, whose loads are waited for
@@ -4923,7 +4927,7 @@ __global__ __launch_bounds__(64, 3) void canonical_fused_f64_kernel(
             const double w0 = b.w * ratio[0] * b.pq;
             b.w = anew ? direct : w0;
             const bool before = j + FUSED_F64_UNROLL <= ja;
-            if (ballot(before || j >= je || (j > ja && j + FUSED_F64_UNROLL <= je)) == ~0ull) {
+            if (ballot(before || j >= je || (j > ja && j + FUSED_F64_UNROLL < jw)) == ~0ull) {
                 a[0] = b.w;
 #pragma unroll
                 for (int u = 1; u < FUSED_F64_UNROLL; ++u)

@@ -185,3 +185,22 @@ def test_fused_infinite_and_nan_columns(gpu, n, ps):
     hi = np.array([(start + length)[tiles == t].max() for t in tiles])
     far = (k < lo) | (k >= hi)
     np.testing.assert_array_equal(got[far], clean[far])
+
+
+@pytest.mark.parametrize('n,at', [(40000, 19970), (40000, 20003), (200000, 100001)])
+def test_fused_short_windows(gpu, n, at):
+    """A row's sum ends with its window, wherever in the kernel's chunks that
+    is: windows of 1 to 24 steps beside a row that takes every step, so that
+    nothing else ends or starts near them."""
+    rng = np.random.RandomState(n + at)
+    x = rng.rand(n + 1, 3)
+    x[:, 0] = np.arange(n + 1)
+    ps = np.array([0.5, 0.5])
+    plan = E.FusedPlan(gpu.from_numpy(x).cuda(), ps, 'fp64_mfma')
+    for length in range(1, 25):
+        plan.d_start.copy_(gpu.tensor([0, at]))
+        plan.d_len.copy_(gpu.tensor([n + 1, length]))
+        got = plan.run().cpu().numpy()[1]
+        k = np.arange(at, at + length)
+        ref = ratio_weights(n, 0.5, k) @ x[k].astype(np.longdouble)
+        assert (np.abs(got - ref) <= TOL['fp64_mfma'] * np.abs(ref)).all(), (length, got, ref)
