@@ -100,6 +100,25 @@ class BondEngine(object):
         self.merge_rounds = 0
         self.state_mode = nat.PC_STATE_AUTO
 
+    def scratch(self, nbytes, least):
+        """A device workspace of nbytes, for calls that also do with less: at
+        most a quarter of the memory that is free, and where the GPU has no
+        room for that either, a half of it, and so on.  None if there is no
+        room for `least` bytes."""
+        torch = self.torch
+        # (asked only where it matters, and not under capture)
+        if nbytes > 1 << 28 and not torch.cuda.is_current_stream_capturing():
+            free = (torch.cuda.mem_get_info(self.device)[0] +
+                    torch.cuda.memory_reserved(self.device) -
+                    torch.cuda.memory_allocated(self.device))
+            nbytes = max(min(nbytes, free // 4), least)
+        while nbytes:
+            try:
+                return torch.empty((nbytes,), dtype=torch.uint8, device=self.device)
+            except torch.OutOfMemoryError:
+                nbytes = max(nbytes // 2, least) if nbytes > least else 0
+        return None
+
     # -- permutations -----------------------------------------------------
     def upload_permutations(self, perms):
         """(R, M) host permutations -> device int32 tensor."""
@@ -145,25 +164,34 @@ class BondEngine(object):
         return self.torch.from_numpy(seeds.astype(np.uint32).view(np.int32)).to(
             self.device)
 
-    def randomstate_permutations(self, seeds, out=None):
+    def randomstate_workspace(self, num_runs):
+        """Device workspace of randomstate_permutations for num_runs runs, or
+        for as many of them at a time as there is room for."""
+        def size(n):
+            b = ctypes.c_uint64(0)
+            nat.check(self.lib.pc_permute_randomstate_workspace_size(
+                self.M, n, ctypes.byref(b)), 'pc_permute_randomstate_workspace_size')
+            return int(b.value)
+        nbytes = size(int(num_runs))
+        return self.scratch(nbytes, size(1)) if nbytes else None
+
+    def randomstate_permutations(self, seeds, out=None, workspace=None):
         """numpy RandomState(seed).permutation(M) for every seed, drawn on
         the device (bit-identical to numpy's legacy generator).  seeds: host
-        integers, or a device vector from upload_seeds."""
+        integers, or a device vector from upload_seeds.  Any workspace will
+        do, but a smaller one than randomstate_workspace(runs) takes longer."""
         torch = self.torch
         d_seeds = seeds if torch.is_tensor(seeds) else self.upload_seeds(seeds)
         n = int(d_seeds.numel())
         if out is None:
             out = torch.empty((n, max(self.M, 1)), dtype=torch.int32,
                               device=self.device)
-        b = ctypes.c_uint64(0)
-        nat.check(self.lib.pc_permute_randomstate_workspace_size(
-            self.M, n, ctypes.byref(b)), 'pc_permute_randomstate_workspace_size')
-        wb = int(b.value)
-        workspace = (torch.empty((wb,), dtype=torch.uint8, device=self.device)
-                     if wb else None)
+        if workspace is None:
+            workspace = self.randomstate_workspace(n)
         nat.check(self.lib.pc_permute_randomstate_ws(
             nat.ptr(d_seeds), n, self.M, nat.ptr(out), max(self.M, 1),
-            nat.ptr(workspace), wb, nat.stream_handle(torch)),
+            nat.ptr(workspace), 0 if workspace is None else int(workspace.numel()),
+            nat.stream_handle(torch)),
             'pc_permute_randomstate_ws')
         return out
 
@@ -436,9 +464,10 @@ class Pipeline(object):
                            if wb else None for _ in range(min(2, nsub))]
         self.streams = _pipeline_streams(torch, dev)
         self.sweep_events = []
-        self.perm_ws = (eng.permutation_workspace(self.R if self.permute_ahead
-                                                  else self.sub)
-                        if seeds is None else None)
+        # the permutations' workspace, after the buffers that have to fit
+        self.perm_ws = (eng.permutation_workspace if seeds is None else
+                        eng.randomstate_workspace)(
+                            self.R if self.permute_ahead else self.sub)
 
     def run(self):
         """Enqueue the whole batch; the caller's stream waits for it."""
@@ -469,7 +498,8 @@ class Pipeline(object):
                     eng.device_permutations(self.seed, self.R, out=self.perm,
                                             workspace=self.perm_ws)
                 else:
-                    eng.randomstate_permutations(self.d_seeds, out=self.perm)
+                    eng.randomstate_permutations(self.d_seeds, out=self.perm,
+                                                 workspace=self.perm_ws)
                 if side:
                     have_all = torch.cuda.Event()
                     have_all.record(sp)
@@ -485,7 +515,8 @@ class Pipeline(object):
                         eng.device_permutations(self.seed, n, first_run=b0, out=perm,
                                                 workspace=self.perm_ws)
                     else:
-                        eng.randomstate_permutations(self.d_seeds[b0:b0 + n], out=perm)
+                        eng.randomstate_permutations(self.d_seeds[b0:b0 + n], out=perm,
+                                                     workspace=self.perm_ws)
                     have_perm = None
                     if side:
                         have_perm = torch.cuda.Event()
@@ -522,7 +553,8 @@ class Pipeline(object):
                                                 workspace=self.perm_ws)
                     else:
                         eng.randomstate_permutations(self.d_seeds,
-                                                     out=self.perms[1 - self.cur])
+                                                     out=self.perms[1 - self.cur],
+                                                     workspace=self.perm_ws)
         if self.prefetch:
             self.cur = 1 - self.cur
             self.prefetched = True

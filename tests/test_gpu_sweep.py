@@ -650,3 +650,43 @@ def test_structured_rows_equal_traces(gpu, length, spanning):
     np.testing.assert_array_equal(rows['moments'], mom)
     if spanning:
         np.testing.assert_array_equal(rows['has_spanning_cluster'], sp)
+
+
+@pytest.mark.parametrize('M,runs,room', [(600000, 16, 40 << 20), (40000, 300, 0)])
+def test_randomstate_permutations_without_room(gpu, M, runs, room):
+    """With room on the GPU for the workspace of some of the runs, or of
+    none, the permutations are still drawn."""
+    eng = BondEngine(_graph.GraphArrays(M + 1, np.stack(
+        [np.arange(M), np.arange(1, M + 1)], axis=1)))
+    seeds = eng.upload_seeds(range(runs))
+    out = gpu.empty((runs, M), dtype=gpu.int32, device='cuda')
+    gpu.cuda.empty_cache()
+    total = gpu.cuda.get_device_properties(0).total_memory
+    gpu.cuda.set_per_process_memory_fraction((gpu.cuda.memory_reserved() + room) / total)
+    try:
+        eng.randomstate_permutations(seeds, out=out)
+    finally:
+        gpu.cuda.set_per_process_memory_fraction(1.0)
+    for r in (0, 1, runs // 2, runs - 1):
+        np.testing.assert_array_equal(out[r].cpu().numpy(),
+                                      np.random.RandomState(r).permutation(M))
+
+
+def _allocations(gpu, call):
+    before = gpu.cuda.memory_stats()['allocation.all.allocated']
+    call()
+    gpu.cuda.synchronize()
+    return gpu.cuda.memory_stats()['allocation.all.allocated'] - before
+
+
+@pytest.mark.parametrize('ahead', [True, False])
+def test_pipeline_keeps_the_randomstate_workspace(gpu, ahead):
+    """A pipeline of numpy's permutations above 32768 edges draws them in a
+    workspace of its own: run() allocates nothing."""
+    from pypercolate_amd._engine import Pipeline
+    pipe = Pipeline(BondEngine(_graph.square_lattice(150)), 7, seeds=range(7), sub_batch=3,
+                    permute_ahead=ahead)
+    pipe.run()
+    assert _allocations(gpu, pipe.run) == 0
+    np.testing.assert_array_equal(pipe.perm[5].cpu().numpy(),
+                                  np.random.RandomState(5).permutation(pipe.engine.M))
