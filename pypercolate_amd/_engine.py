@@ -457,11 +457,14 @@ class Pipeline(object):
                                 device=dev)
         self.sum2 = torch.empty((nat.PC_COLUMNS, S, 3), dtype=torch.int64,
                                 device=dev)
-        wb = eng.workspace_bytes(self.sub)
-        # one union-find workspace (HBM state) per sweep stream in use
-        nsub = (self.R + self.sub - 1) // self.sub
+        # one workspace per sweep stream in use, for each of the sub-batches
+        # that take turns in it (the last one may be smaller than the others
+        # and need more: it can be swept in tiles where they are not)
+        sizes = [min(self.sub, self.R - b0) for b0 in range(0, self.R, self.sub)]
+        wbs = [max(eng.workspace_bytes(n) for n in set(sizes[i::2]))
+               for i in range(min(2, len(sizes)))]
         self.workspaces = [torch.empty((wb,), dtype=torch.uint8, device=dev)
-                           if wb else None for _ in range(min(2, nsub))]
+                           if wb else None for wb in wbs]
         self.streams = _pipeline_streams(torch, dev)
         self.sweep_events = []
         # the permutations' workspace, after the buffers that have to fit

@@ -690,3 +690,14 @@ def test_pipeline_keeps_the_randomstate_workspace(gpu, ahead):
     assert _allocations(gpu, pipe.run) == 0
     np.testing.assert_array_equal(pipe.perm[5].cpu().numpy(),
                                   np.random.RandomState(5).permutation(pipe.engine.M))
+
+
+@pytest.mark.parametrize('length,runs,sub', [(70, 1600, 1100), (70, 2700, 1100), (130, 7, 3)])
+def test_pipeline_allocates_nothing_in_run(gpu, length, runs, sub):
+    """run() finds a workspace for each of its sub-batches, also for a last
+    one of fewer runs that is swept in tiles where the others are not (L =
+    70, 1024 runs)."""
+    from pypercolate_amd._engine import Pipeline
+    pipe = Pipeline(BondEngine(_graph.square_lattice(length)), runs, seed=3, sub_batch=sub)
+    pipe.run()
+    assert _allocations(gpu, pipe.run) == 0
