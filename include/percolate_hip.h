@@ -110,6 +110,16 @@ int pc_sweep_lattice_workspace_size(uint32_t length, uint32_t num_runs,
                                     uint32_t state_mode, uint64_t *bytes);
 
 /*
+ * Which way pc_sweep_lattice takes with a workspace of that many bytes, 16-byte
+ * aligned: *runs is the number of runs whose bond lists its tiled sweep holds
+ * at a time, or 0 where every node's code is kept in LDS or HBM.  Host-only,
+ * no GPU work.
+ */
+int pc_sweep_lattice_tiled_runs(uint32_t length, int32_t span_on_first_merge,
+                                uint32_t num_runs, uint64_t workspace_bytes,
+                                uint32_t state_mode, uint32_t *runs);
+
+/*
  * One graph of a persistent multi-graph sweep (pc_sweep_multi): the
  * arguments pc_sweep takes for one graph, with chunk states always written.
  */

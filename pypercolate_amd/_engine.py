@@ -84,8 +84,8 @@ class BondEngine(object):
         self.lattice_sweep = bool(L) and self.N > 16384
         # lattices whose edge array is swept otherwise (state in LDS, or a
         # relabelling whose tiles are not whole): pc_sweep_lattice takes them
-        # with their sides row by row where it has a tiled sweep for them
-        # (a workspace of workspace_bytes for the number of runs)
+        # with their sides row by row where it sweeps them in tiles
+        # (tiled_runs)
         self.row_length, self.d_row_sides = 0, None
         if not self.lattice_sweep and (self.N <= 16384 or order is not None):
             self.row_length = int(getattr(graph, 'lattice_length', 0) or 0)
@@ -210,6 +210,21 @@ class BondEngine(object):
                       'pc_sweep_workspace_size')
         return int(b.value)
 
+    def tiled_runs(self, num_runs, workspace_bytes=None):
+        """How many runs sweep() takes at a time in tiles, with a workspace of
+        that many bytes (default: workspace_bytes(num_runs)); 0 where it keeps
+        every node's code in LDS or HBM."""
+        length = self.lattice_length if self.lattice_sweep else self.row_length
+        if not length:
+            return 0
+        if workspace_bytes is None:
+            workspace_bytes = self.workspace_bytes(num_runs)
+        runs = ctypes.c_uint32(0)
+        nat.check(self.lib.pc_sweep_lattice_tiled_runs(
+            length, self.span_first, num_runs, workspace_bytes, self.state_mode,
+            ctypes.byref(runs)), 'pc_sweep_lattice_tiled_runs')
+        return int(runs.value)
+
     def occupancy(self, state_mode=None):
         """Resident sweep workgroups per CU (HIP occupancy calculator)."""
         v = ctypes.c_int32(0)
@@ -256,9 +271,7 @@ class BondEngine(object):
             chunk_state = torch.empty((R, C, nat.PC_STATE_WORDS),
                                       dtype=torch.int64, device=self.device)
         st = nat.stream_handle(torch)
-        rows = (self.row_length and not self.lattice_sweep and wb and
-                self.state_mode == nat.PC_STATE_AUTO and
-                wb >= self.workspace_bytes(R) > 0)
+        rows = bool(self.row_length and wb and self.tiled_runs(R, wb))
         if self.lattice_sweep or rows:
             nat.check(self.lib.pc_sweep_lattice(
                 self.row_length if rows else self.lattice_length,

@@ -103,6 +103,8 @@ SIGNATURES = {
     'pc_sweep_multi': (ctypes.c_int, [_u32, _vp, _vp, _u64, _vp, _u64, _vp]),
     'pc_sweep_lattice_workspace_size': (ctypes.c_int, [_u32, _u32, _u32,
                                                        ctypes.POINTER(_u64)]),
+    'pc_sweep_lattice_tiled_runs': (ctypes.c_int, [_u32, _i32, _u32, _u64, _u32,
+                                                   ctypes.POINTER(_u32)]),
     'pc_sweep_lattice': (ctypes.c_int, [_u32, _i32, _vp, _i32, _vp, _i64, _u32,
                                         _vp, _i64, _vp, _vp, _u64, _u32, _u32,
                                         _vp, _vp]),

@@ -5927,10 +5927,57 @@ static int tile_sweep_launch(const TileGeo &g, const TilePlan &p,
     return PC_OK;
 }
 
-// The tiled sweep, if it takes this call: *taken tells.  Not taken: modes
-// that ask for a state or a number of wavefronts, auxiliary sides joined
-// from the first merge on, more than 2^31 grid blocks, or a workspace that
-// holds the lists of fewer than 4 runs (or of all runs).
+// Runs whose lists the tiled sweep of such a call holds at a time, 0 if it
+// does not take the call.  Not taken: modes that ask for a state or a number
+// of wavefronts, auxiliary sides joined from the first merge on, more than
+// 2^31 grid blocks, or a workspace that holds the lists of fewer than 4 runs
+// (or of all runs).
+static uint32_t tile_runs(uint32_t length, bool tiled, int32_t span_on_first_merge,
+                          uint32_t num_runs, uint64_t workspace_bytes,
+                          uint32_t state_mode, TileGeo &g)
+{
+    if (state_mode != PC_STATE_AUTO || span_on_first_merge || num_runs == 0 ||
+        !tile_geo(length, tiled, num_runs, g))
+        return 0u;
+    const uint32_t M = 2u * length * (length - 1u);
+    uint32_t slab = tile_slab(g, num_runs);
+    if (workspace_bytes < tile_plan(g, num_runs, slab).bytes) {
+        const TilePlan one = tile_plan(g, num_runs, 1u);
+        const uint64_t per_run = one.list_bytes + (1u + tile_windows(M)) * g.K * 4u;
+        const uint64_t base = one.bytes + 512u;
+        slab = workspace_bytes < base ? 0u : (uint32_t)std::min<uint64_t>(
+                   slab, 1u + (workspace_bytes - base) / per_run);
+        if (slab < std::min(num_runs, 4u))
+            return 0u;
+    }
+    // slabs of about the same size, in groups of eight runs
+    const uint32_t slabs = (num_runs + slab - 1u) / slab;
+    slab = std::min(slab, ((num_runs + slabs - 1u) / slabs + 7u) & ~7u);
+    if (slab > 65535u)
+        slab = 65528u;
+    if (tile_plan(g, num_runs, slab).bytes > workspace_bytes ||
+        (uint64_t)(slab + 7u) * g.K > 0x7FFFFFFFu)
+        return 0u;
+    return slab;
+}
+
+extern "C" int pc_sweep_lattice_tiled_runs(uint32_t length, int32_t span_on_first_merge,
+                                           uint32_t num_runs, uint64_t workspace_bytes,
+                                           uint32_t state_mode, uint32_t *runs)
+{
+    g_last_error[0] = 0;
+    if (!runs)
+        return pc_fail(PC_EINVAL, "pc_sweep_lattice_tiled_runs: runs is NULL");
+    if (length == 0 || length > 16384u)
+        return pc_fail(PC_EINVAL, "pc_sweep_lattice_tiled_runs: length must be in 1..16384");
+    TileGeo g;
+    *runs = tile_runs(length, false, span_on_first_merge, num_runs, workspace_bytes,
+                      state_mode, g);
+    return PC_OK;
+}
+
+// The tiled sweep, if it takes this call (tile_runs, and a workspace aligned
+// for it): *taken tells.
 static int tile_sweep(uint32_t length, bool tiled, const uint8_t *d_node_sides,
                       int32_t span_on_first_merge, const int32_t *d_perm,
                       int64_t perm_stride, uint32_t num_runs, void *d_records,
@@ -5943,28 +5990,14 @@ static int tile_sweep(uint32_t length, bool tiled, const uint8_t *d_node_sides,
     TileGeo g;
     const uint32_t rounds = merge_rounds ? merge_rounds : g_merge_rounds;
     const int64_t M = 2ll * length * (length - 1ll);
-    if (state_mode != PC_STATE_AUTO || span_on_first_merge || num_runs == 0 || rounds > 64 ||
-        !tile_geo(length, tiled, num_runs, g) || !d_workspace || ((uintptr_t)d_workspace & 15u) ||
-        !d_span_step || !d_perm || !d_records || perm_stride < M || rec_stride < M)
+    if (rounds > 64 || !d_workspace || ((uintptr_t)d_workspace & 15u) || !d_span_step ||
+        !d_perm || !d_records || perm_stride < M || rec_stride < M)
         return PC_OK;
-    uint32_t slab = tile_slab(g, num_runs);
-    const TilePlan one = tile_plan(g, num_runs, 1u);
-    if (workspace_bytes < tile_plan(g, num_runs, slab).bytes) {
-        const uint64_t per_run = one.list_bytes + (1u + tile_windows((uint32_t)M)) * g.K * 4u;
-        const uint64_t base = one.bytes + 512u;
-        slab = workspace_bytes < base ? 0u : (uint32_t)std::min<uint64_t>(
-                   slab, 1u + (workspace_bytes - base) / per_run);
-        if (slab < std::min(num_runs, 4u))
-            return PC_OK;
-    }
-    // slabs of about the same size, in groups of eight runs
-    const uint32_t slabs = (num_runs + slab - 1u) / slab;
-    slab = std::min(slab, ((num_runs + slabs - 1u) / slabs + 7u) & ~7u);
-    if (slab > 65535u)
-        slab = 65528u;
+    const uint32_t slab = tile_runs(length, tiled, span_on_first_merge, num_runs,
+                                    workspace_bytes, state_mode, g);
+    if (slab == 0u)
+        return PC_OK;
     const TilePlan p = tile_plan(g, num_runs, slab);
-    if (p.bytes > workspace_bytes || (uint64_t)(slab + 7u) * g.K > 0x7FFFFFFFu)
-        return PC_OK;
     *taken = true;
     hipStream_t s = as_stream(stream);
     const bool u32rec = length * length <= kU32RecordMaxNodes;

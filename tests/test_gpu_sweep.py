@@ -701,3 +701,19 @@ def test_pipeline_allocates_nothing_in_run(gpu, length, runs, sub):
     pipe = Pipeline(BondEngine(_graph.square_lattice(length)), runs, seed=3, sub_batch=sub)
     pipe.run()
     assert _allocations(gpu, pipe.run) == 0
+
+
+@pytest.mark.parametrize('length,runs,part', [(64, 9, 1), (65, 5, 1), (95, 1024, 1), (95, 1025, 1),
+                                              (128, 200, 1), (128, 200, 2), (128, 200, 400)])
+def test_lattice_sweep_way_taken(gpu, length, runs, part):
+    """A lattice whose codes fit LDS uses its workspace, or a part of it, if
+    and only if tiled_runs says that it is swept in tiles; the records are
+    the same."""
+    eng = BondEngine(_graph.square_lattice(length))
+    nbytes = (eng.workspace_bytes(runs) or 1 << 20) // part
+    ws = gpu.full((nbytes,), 0xA5, dtype=gpu.uint8, device='cuda')
+    perm = eng.device_permutations(11, runs)
+    res = eng.sweep(perm, workspace=ws, chunks=False)
+    assert bool((ws != 0xA5).any()) == (eng.tiled_runs(runs, nbytes) > 0)
+    assert (eng.tiled_runs(runs, nbytes) > 0) == (length > 64 and runs != 1025 and part < 400)
+    _same_sweep(res, eng.sweep(perm, chunks=False), chunks=False)
