@@ -210,6 +210,25 @@ class BondEngine(object):
                       'pc_sweep_workspace_size')
         return int(b.value)
 
+    def sweep_workspace(self, num_runs):
+        """Device workspace of sweep() for num_runs runs (None if it needs
+        none), or, where there is no room for the lists of all of them in
+        tiles, for fewer at a time; at the least what keeps every node's
+        code."""
+        nbytes = self.workspace_bytes(num_runs)
+        if not nbytes:
+            return None
+        b = ctypes.c_uint64(0)
+        nat.check(self.lib.pc_sweep_workspace_size(
+            self.N, num_runs, self.state_mode, ctypes.byref(b)),
+            'pc_sweep_workspace_size')
+        codes = int(b.value)
+        ws = self.scratch(nbytes, codes or self.workspace_bytes(min(num_runs, 4)))
+        if ws is None and codes:
+            raise self.torch.OutOfMemoryError(
+                'no room for the {} bytes of the nodes\' codes'.format(codes))
+        return ws
+
     def tiled_runs(self, num_runs, workspace_bytes=None):
         """How many runs sweep() takes at a time in tiles, with a workspace of
         that many bytes (default: workspace_bytes(num_runs)); 0 where it keeps
@@ -261,11 +280,9 @@ class BondEngine(object):
                                   device=self.device)
         if span_step is None:
             span_step = torch.empty((R,), dtype=torch.int32, device=self.device)
-        wb = self.workspace_bytes(R)
-        if wb and workspace is None:
-            workspace = torch.empty((wb,), dtype=torch.uint8, device=self.device)
-        elif workspace is not None:
-            wb = int(workspace.numel())
+        if workspace is None:
+            workspace = self.sweep_workspace(R)
+        wb = 0 if workspace is None else int(workspace.numel())
         if chunks and chunk_state is None:
             C = max((self.M + nat.PC_CHUNK - 1) // nat.PC_CHUNK, 1)
             chunk_state = torch.empty((R, C, nat.PC_STATE_WORDS),
@@ -474,10 +491,9 @@ class Pipeline(object):
         # that take turns in it (the last one may be smaller than the others
         # and need more: it can be swept in tiles where they are not)
         sizes = [min(self.sub, self.R - b0) for b0 in range(0, self.R, self.sub)]
-        wbs = [max(eng.workspace_bytes(n) for n in set(sizes[i::2]))
-               for i in range(min(2, len(sizes)))]
-        self.workspaces = [torch.empty((wb,), dtype=torch.uint8, device=dev)
-                           if wb else None for wb in wbs]
+        self.workspaces = [
+            eng.sweep_workspace(max(set(sizes[i::2]), key=eng.workspace_bytes))
+            for i in range(min(2, len(sizes)))]
         self.streams = _pipeline_streams(torch, dev)
         self.sweep_events = []
         # the permutations' workspace, after the buffers that have to fit

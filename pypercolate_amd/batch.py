@@ -60,9 +60,7 @@ class _LengthPlan(object):
         self.sum2 = torch.empty((nat.PC_COLUMNS, S, 3), dtype=torch.int64,
                                 device=dev)
         self.perm_ws = eng.permutation_workspace(runs)
-        wb = eng.workspace_bytes(runs)
-        self.workspace = (torch.empty((wb,), dtype=torch.uint8, device=dev)
-                          if wb else None)
+        self.workspace = eng.sweep_workspace(runs)
         self.ps = np.asarray(ps, dtype=np.float64)
         self.x = torch.empty((S, nat.PC_COLUMNS), dtype=torch.float64, device=dev)
         self.plan = (FusedPlan(self.x, self.ps, 'fp64_mfma')

@@ -717,3 +717,22 @@ def test_lattice_sweep_way_taken(gpu, length, runs, part):
     assert bool((ws != 0xA5).any()) == (eng.tiled_runs(runs, nbytes) > 0)
     assert (eng.tiled_runs(runs, nbytes) > 0) == (length > 64 and runs != 1025 and part < 400)
     _same_sweep(res, eng.sweep(perm, chunks=False), chunks=False)
+
+
+@pytest.mark.parametrize('room', [120 << 20, 0])
+def test_tiled_sweep_without_room(gpu, room):
+    """L = 128, whose codes fit LDS: with room for the lists of some of the
+    runs, or of none, the same records."""
+    eng = BondEngine(_graph.square_lattice(128))
+    perm = eng.device_permutations(13, 3000)
+    want = eng.sweep(perm, chunks=False)
+    records, span = gpu.empty_like(want.records), gpu.empty_like(want.span_step)
+    assert eng.workspace_bytes(3000) > room + (128 << 20)
+    gpu.cuda.empty_cache()
+    total = gpu.cuda.get_device_properties(0).total_memory
+    gpu.cuda.set_per_process_memory_fraction((gpu.cuda.memory_reserved() + room) / total)
+    try:
+        eng.sweep(perm, records=records, span_step=span, chunks=False)
+    finally:
+        gpu.cuda.set_per_process_memory_fraction(1.0)
+    assert gpu.equal(records, want.records) and gpu.equal(span, want.span_step)
