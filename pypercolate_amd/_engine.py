@@ -229,18 +229,19 @@ class BondEngine(object):
                 'no room for the {} bytes of the nodes\' codes'.format(codes))
         return ws
 
-    def tiled_runs(self, num_runs, workspace_bytes=None):
+    def tiled_runs(self, num_runs, workspace_bytes=None, state_mode=None):
         """How many runs sweep() takes at a time in tiles, with a workspace of
         that many bytes (default: workspace_bytes(num_runs)); 0 where it keeps
         every node's code in LDS or HBM."""
+        mode = self.state_mode if state_mode is None else state_mode
         length = self.lattice_length if self.lattice_sweep else self.row_length
         if not length:
             return 0
         if workspace_bytes is None:
-            workspace_bytes = self.workspace_bytes(num_runs)
+            workspace_bytes = self.workspace_bytes(num_runs, mode)
         runs = ctypes.c_uint32(0)
         nat.check(self.lib.pc_sweep_lattice_tiled_runs(
-            length, self.span_first, num_runs, workspace_bytes, self.state_mode,
+            length, self.span_first, num_runs, workspace_bytes, mode,
             ctypes.byref(runs)), 'pc_sweep_lattice_tiled_runs')
         return int(runs.value)
 

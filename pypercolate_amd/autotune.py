@@ -5,6 +5,8 @@ runs for every candidate
   * number of parallel conflict-free merge rounds per batch of 64 bonds,
   * union-find state placement (LDS for N <= 16384, or the HBM workspace),
   * one or two wavefronts per run (a finder beside the resolver),
+  * for square lattices that the library sweeps in tiles, its automatic mode
+    (PC_STATE_AUTO), in which it does,
 and keeps the fastest.  The sample is one residency's worth of runs (the
 HIP occupancy calculator's workgroups per CU times the number of CUs, at
 most about 2^28 bonds of buffers), so the timing sees the concurrency of a
@@ -86,13 +88,26 @@ def tune_sweep(engine, sample_runs=None, rounds=ROUND_CANDIDATES, modes=None,
     """Pick (merge_rounds, state_mode) for ``engine`` (a BondEngine), set
     them on it and return a dict with the choice and the timings.
     state_mode candidates are PC_STATE_LDS / PC_STATE_HBM, each with one
-    and with two wavefronts per run (PC_SWEEP_*).  ``max_runs``: the most
+    and with two wavefronts per run (PC_SWEEP_*), and PC_STATE_AUTO where the
+    sample is swept in tiles.  ``max_runs``: the most
     runs the caller sweeps in one launch; the sample is cut to it, and the
     cache keeps one choice per graph and cap."""
     torch = engine.torch
     device = torch.cuda.get_device_properties(engine.device)
-    key = 'tiled|{}|{}|{}'.format(device.gcnArchName, device.multi_processor_count,
-                            graph_key(engine.graph))
+    cus = device.multi_processor_count
+
+    def sample(mode):
+        # one residency of runs, capped at about 2^28 bonds of buffers
+        occ = max(engine.occupancy(mode), 1)
+        cap = max(64, (1 << 28) // max(engine.M, 1))
+        runs = sample_runs or max(1, min(occ * cus, 8192, cap))
+        return min(runs, int(max_runs)) if max_runs else runs
+
+    tiled = engine.tiled_runs(sample(nat.PC_STATE_AUTO),
+                              state_mode=nat.PC_STATE_AUTO) > 0
+    key = '{}|{}|{}'.format(device.gcnArchName, cus, graph_key(engine.graph))
+    if tiled:   # not a choice made before the tiled sweep was a candidate
+        key = 'tiled|' + key
     if max_runs:
         key += '|runs<={}'.format(int(max_runs))
     cache = _load_cache() if use_cache else {}
@@ -107,25 +122,26 @@ def tune_sweep(engine, sample_runs=None, rounds=ROUND_CANDIDATES, modes=None,
             places = [nat.PC_STATE_LDS, nat.PC_STATE_HBM]
         modes = [p | w for p in places
                  for w in (nat.PC_SWEEP_ONE_WAVE, nat.PC_SWEEP_TWO_WAVES)]
-        if engine.lattice_sweep or engine.row_length:
-            # the library's tiled sweep, with no placement asked
-            modes.insert(0, nat.PC_STATE_AUTO)
-    cus = device.multi_processor_count
+        if tiled:
+            modes.append(nat.PC_STATE_AUTO)
     timings = {}
     best = None
     for mode in modes:
-        occ = max(engine.occupancy(mode), 1)
-        # one residency of runs, capped at about 2^28 bonds of buffers
-        cap = max(64, (1 << 28) // max(engine.M, 1))
-        runs = sample_runs or max(1, min(occ * cus, 8192, cap))
-        if max_runs:
-            runs = min(runs, int(max_runs))
+        runs = sample(mode)
         perm = engine.device_permutations(seed, runs)
         records = torch.empty((runs, max(engine.M, 1)), dtype=engine.rec_torch,
                               device=engine.device)
         span = torch.empty((runs,), dtype=torch.int32, device=engine.device)
         engine.state_mode = mode
-        for r in rounds:
+        candidates = rounds
+        if mode == nat.PC_STATE_AUTO and tiled:
+            # the tiles' merges have no such rounds: timed once, with the best
+            # for the untiled sweep that the mode falls back to
+            untiled = (nat.PC_SWEEP_TWO_WAVES |
+                       (nat.PC_STATE_LDS if engine.N <= 16384 else nat.PC_STATE_HBM))
+            candidates = [max(rounds, key=lambda r: timings.get(
+                '{}/{}'.format(untiled, r), 0.0))]
+        for r in candidates:
             engine.merge_rounds = r
             ms = _time_sweep(engine, perm, records, span)
             rate = runs * engine.M / ms * 1e3

@@ -124,3 +124,34 @@ def test_tuned_knobs_do_not_change_records(gpu, tmp_path, monkeypatch, L):
                                           eng.chunk_scan(res).cpu().numpy()), (mode, r)
     # cached: a second tuning returns the stored choice
     assert tune_sweep(eng, sample_runs=64, rounds=(1, 3, 8)) == choice
+
+
+@pytest.mark.parametrize('graph,tiled', [(_graph.square_lattice(16), False),
+                                         (_graph.square_lattice(64), False),
+                                         (_graph.square_lattice(130), True),
+                                         (_graph.linear_chain(20000), False)],
+                         ids=['L16', 'L64', 'L130', 'chain'])
+def test_tuner_and_the_tiled_sweep(gpu, tmp_path, monkeypatch, graph, tiled):
+    """Choices saved before there was a tiled sweep hold for graphs that are
+    not swept in tiles, and no others; where one is, the automatic mode is
+    one candidate, timed once (its merge rounds are those of the untiled
+    sweep it falls back to), and otherwise none."""
+    import json
+    monkeypatch.setenv('PYPERCOLATE_AMD_CACHE', str(tmp_path))
+    from pypercolate_amd import autotune
+    eng = BondEngine(graph)
+    device = gpu.cuda.get_device_properties(0)
+    saved = {'merge_rounds': 6, 'state_mode': nat.PC_STATE_HBM | nat.PC_SWEEP_ONE_WAVE}
+    with open(autotune.cache_path(), 'w') as f:
+        json.dump({'{}|{}|{}'.format(device.gcnArchName, device.multi_processor_count,
+                                     autotune.graph_key(graph)): saved}, f)
+    assert (tune_sweep(eng, sample_runs=20, rounds=(1, 3)) == saved) == (not tiled)
+    eng.state_mode, eng.merge_rounds = nat.PC_STATE_AUTO, 0
+    choice = tune_sweep(eng, sample_runs=20, rounds=(1, 3), use_cache=False)
+    auto = [k for k in choice['candidates'] if k.startswith('{}/'.format(nat.PC_STATE_AUTO))]
+    assert len(auto) == (1 if tiled else 0)
+    assert choice['merge_rounds'] in (1, 3)
+    if choice['state_mode'] == nat.PC_STATE_AUTO:
+        untiled = {r: choice['candidates']['{}/{}'.format(
+            nat.PC_STATE_HBM | nat.PC_SWEEP_TWO_WAVES, r)] for r in (1, 3)}
+        assert choice['merge_rounds'] == max(untiled, key=untiled.get)
