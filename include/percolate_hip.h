@@ -172,6 +172,11 @@ int pc_sweep_multi(uint32_t num_graphs, const pc_sweep_graph *graphs,
 int pc_permute_philox_workspace_size(uint32_t num_edges, uint32_t num_runs,
                                      uint64_t *bytes);
 
+/* Resident workgroups per compute unit of pc_permute_philox's shuffles in LDS
+   (of whole runs up to 32768 edges, of a run's buckets above) when there are
+   more than the GPU holds. */
+int pc_permute_philox_occupancy(uint32_t num_edges, int32_t *blocks_per_cu);
+
 /* Where pc_sweep keeps the union-find state of a run. */
 #define PC_STATE_AUTO 0 /* LDS when num_nodes <= 16384, else HBM             */
 #define PC_STATE_LDS 1  /* 16-bit codes in LDS (num_nodes <= 16384)          */

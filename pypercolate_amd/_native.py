@@ -47,6 +47,7 @@ SIGNATURES = {
                                          _u64, _vp]),
     'pc_permute_philox_workspace_size': (ctypes.c_int, [_u32, _u32,
                                                         ctypes.POINTER(_u64)]),
+    'pc_permute_philox_occupancy': (ctypes.c_int, [_u32, ctypes.POINTER(_i32)]),
     'pc_permute_randomstate': (ctypes.c_int, [_vp, _u32, _u32, _vp, _i64, _vp]),
     'pc_permute_randomstate_ws': (ctypes.c_int, [_vp, _u32, _u32, _vp, _i64, _vp,
                                                  _u64, _vp]),

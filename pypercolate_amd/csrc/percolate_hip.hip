@@ -373,21 +373,23 @@ __device__ __forceinline__ uint64_t match_label(uint32_t label, uint32_t bits,
 }
 
 // match_label through LDS: every lane sets its bit in the mask of its label's
-// low MATCH_BITS bits, a table of the wave's own (all zero before and after),
+// low `in_lds` bits, a table of the wave's own (all zero before and after),
 // and reads the mask back; only the bits above cost a ballot, of four vector
 // instructions each.  Lanes outside `ok` get no peers.  The kernels that group
 // by label are bound by vector issue (80 to 92 % busy with a ballot for each
 // of 7 to 9 bits), so this pays: grouping by 512 labels, 2.1e9 edges, 7.1 ms
 // with ballots and labels drawn twice, 5.0; whole runs of 32512 edges (10^4)
-// 1.17 ms, 0.97 (5, 6 and 8 bits here: 1.08, 1.03 and 1.32, where the tables
-// leave room for fewer workgroups).
+// 1.17 ms, 0.97 (5, 6 and 8 bits here: 1.08, 1.03 and 1.32: a table of 8 bits
+// leaves room for fewer workgroups, one of few bits has lanes wait for each
+// other).  shuf_match_bits says where fewer bits pay.
 #define MATCH_BITS 7u
 #define MATCH_WORDS (2u << MATCH_BITS)   // 32-bit words of a wave's table
 
 __device__ __forceinline__ uint64_t match_label_lds(uint32_t label, uint32_t bits,
-                                                    bool ok, unsigned long long *table)
+                                                    bool ok, unsigned long long *table,
+                                                    uint32_t in_lds = MATCH_BITS)
 {
-    unsigned long long *slot = table + (label & ((1u << MATCH_BITS) - 1u));
+    unsigned long long *slot = table + (label & ((1u << in_lds) - 1u));
     uint64_t peers = 0;
     if (ok) {
         __hip_atomic_fetch_or(slot, 1ull << (threadIdx.x & 63u), __ATOMIC_RELAXED,
@@ -395,7 +397,7 @@ __device__ __forceinline__ uint64_t match_label_lds(uint32_t label, uint32_t bit
         peers = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    return bits > MATCH_BITS ? match_label(label >> MATCH_BITS, bits - MATCH_BITS, peers) : peers;
+    return bits > in_lds ? match_label(label >> in_lds, bits - in_lds, peers) : peers;
 }
 
 __device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
@@ -749,7 +751,8 @@ template <int W, int GPW, bool IDENT>
 __device__ void shuffle_group_lds(uint32_t n, uint32_t b, uint32_t run,
                                   uint32_t k0, uint32_t k1, int32_t *a,
                                   uint16_t *ent, uint32_t *hist, uint32_t hw,
-                                  uint32_t *wsum, unsigned long long *masks)
+                                  uint32_t *wsum, unsigned long long *masks,
+                                  uint32_t in_lds)
 {
     const uint32_t T = 64u * W, tid = threadIdx.x, wave = tid >> 6,
                    lane = tid & 63u;
@@ -763,7 +766,7 @@ __device__ void shuffle_group_lds(uint32_t n, uint32_t b, uint32_t run,
 
     for (uint32_t i = tid; i < W * hw; i += T)
         hist[i] = 0u;
-    for (uint32_t i = tid; i < W * (MATCH_WORDS / 2u); i += T)
+    for (uint32_t i = tid; i < (uint32_t)W << in_lds; i += T)
         masks[i] = 0ull;
     __syncthreads();
 
@@ -837,7 +840,7 @@ __device__ void shuffle_group_lds(uint32_t n, uint32_t b, uint32_t run,
                 const uint32_t j = g * 512u + k * 64u + lane;
                 const bool ok = j < n;
                 const uint32_t s = lb ? half16(keys[gi], k) >> (16u - lb) : 0u;
-                const uint64_t peers = match_label_lds(s, lb, ok, masks + wave * (MATCH_WORDS / 2u));
+                const uint64_t peers = match_label_lds(s, lb, ok, masks + (wave << in_lds), in_lds);
                 if (ok) {
                     const uint32_t rank = lanes_below(peers);
                     const uint32_t sh = (s & 1u) * 16u;
@@ -897,7 +900,7 @@ __device__ void shuffle_group_lds(uint32_t n, uint32_t b, uint32_t run,
 template <int W, bool IDENT>
 __global__ __launch_bounds__(64 * W) void shuffle_group_kernel(
     uint32_t k0, uint32_t k1, uint32_t first_run, uint32_t lb1, uint32_t r0,
-    uint32_t cap, const uint32_t *__restrict__ starts,
+    uint32_t cap, uint32_t in_lds, const uint32_t *__restrict__ starts,
     int32_t *__restrict__ perm, int64_t stride)
 {
     extern __shared__ uint32_t gdyn[];
@@ -906,7 +909,7 @@ __global__ __launch_bounds__(64 * W) void shuffle_group_kernel(
     constexpr int GPW = (int)(CAP / (512u * W));
     const uint32_t hw = shuf_hist_words(cap);
     unsigned long long *masks = (unsigned long long *)gdyn;
-    uint32_t *hist = gdyn + W * MATCH_WORDS, *wsum = hist + W * hw;
+    uint32_t *hist = gdyn + (2u * W << in_lds), *wsum = hist + W * hw;
     uint16_t *ent = (uint16_t *)(wsum + W);
     const uint32_t b = blockIdx.x, r = r0 + blockIdx.y;
     const uint32_t run = first_run + r;
@@ -927,12 +930,39 @@ __global__ __launch_bounds__(64 * W) void shuffle_group_kernel(
             shuffle_wide(a, n, run, b, k0, k1);
         return;
     }
-    shuffle_group_lds<W, GPW, IDENT>(n, b, run, k0, k1, a, ent, hist, hw, wsum, masks);
+    shuffle_group_lds<W, GPW, IDENT>(n, b, run, k0, k1, a, ent, hist, hw, wsum, masks,
+                                     in_lds);
 }
 
-static size_t shuf_group_lds_bytes(uint32_t W, uint32_t cap)
+// (in_lds < 0: without the tables of match_label_lds)
+static size_t shuf_group_lds_bytes(uint32_t W, uint32_t cap, int in_lds)
 {
-    return (size_t)(W * (MATCH_WORDS + shuf_hist_words(cap)) + W) * 4u + (((size_t)cap * 2u + 3u) & ~(size_t)3u);
+    const uint32_t table = in_lds < 0 ? 0u : 2u << in_lds;
+    return (size_t)(W * (table + shuf_hist_words(cap)) + W) * 4u +
+           (((size_t)cap * 2u + 3u) & ~(size_t)3u);
+}
+
+// Label bits matched through LDS in a workgroup of eight waves for a whole run
+// of `cap` edges: fewer than MATCH_BITS, but at least 5, where a CU then holds
+// as many workgroups as it would without the tables, and there are runs for
+// them (40 of 21840 edges: 26.3 us with 7, 29.2 with 5).  4000 runs, microseconds
+// with 7, 6 and 5 bits (and as the kernel was with ballots alone): 15312 edges
+// 183, 173, 172 (184); 16380 196, 194, 186 (191); 20500 252, 234, 238 (262);
+// 21424 264, 275, 247 (272); 32768 543, 403, 415 (469).  With 4 bits the lanes
+// that wait for each other cost more than the workgroup is worth: 22500 edges
+// 272 with 7, 303.
+static uint32_t shuf_match_bits(uint32_t cap, uint32_t num_runs)
+{
+    constexpr uint32_t LDS = 160u << 10, WAVES = 2048u / 512u, CUS = 256u;
+    auto resident = [&](int in_lds) {
+        return std::min<size_t>(LDS / shuf_group_lds_bytes(8, cap, in_lds), WAVES);
+    };
+    if (num_runs <= CUS * resident(MATCH_BITS))
+        return MATCH_BITS;
+    for (int bits = MATCH_BITS; bits >= 5; --bits)
+        if (resident(bits) == resident(-1))
+            return (uint32_t)bits;
+    return MATCH_BITS;
 }
 
 // ---------------------------------------------------------------------------
@@ -5556,6 +5586,30 @@ extern "C" int pc_permute_philox_workspace_size(uint32_t num_edges,
     return PC_OK;
 }
 
+extern "C" int pc_permute_philox_occupancy(uint32_t num_edges, int32_t *blocks_per_cu)
+{
+    g_last_error[0] = 0;
+    if (!blocks_per_cu)
+        return pc_fail(PC_EINVAL, "pc_permute_philox_occupancy: NULL output");
+    if (num_edges > SHUF_MAX_EDGES)
+        return pc_fail(PC_EOVERFLOW, "pc_permute_philox_occupancy: num_edges > 2^23");
+    int blocks = 0;
+    if (num_edges <= SHUF_SMALL_CAP)
+        PC_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &blocks, shuffle_group_kernel<2, true>, 128,
+            shuf_group_lds_bytes(2, num_edges, MATCH_BITS)));
+    else if (num_edges <= SHUF_WHOLE)
+        PC_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &blocks, shuffle_group_kernel<8, true>, 512,
+            shuf_group_lds_bytes(8, num_edges, shuf_match_bits(num_edges, 0xFFFFFFFFu))));
+    else
+        PC_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &blocks, shuffle_group_kernel<4, false>, 256,
+            shuf_group_lds_bytes(4, SHUF_GROUP_CAP, MATCH_BITS)));
+    *blocks_per_cu = blocks;
+    return PC_OK;
+}
+
 extern "C" int pc_permute_philox(uint64_t seed, uint64_t first_run,
                                  uint32_t num_runs, uint32_t num_edges,
                                  int32_t *d_perm, int64_t perm_stride,
@@ -5589,15 +5643,17 @@ extern "C" int pc_permute_philox(uint64_t seed, uint64_t first_run,
         const uint32_t rn = min(num_runs - r0, 65535u);
         if (lb1 == 0u && num_edges <= SHUF_SMALL_CAP) {
             shuffle_group_kernel<2, true><<<dim3(1, rn), 128,
-                                            shuf_group_lds_bytes(2, num_edges), s>>>(
-                k0, k1, fr, 0u, r0, num_edges, nullptr, d_perm, perm_stride);
+                                            shuf_group_lds_bytes(2, num_edges, MATCH_BITS),
+                                            s>>>(
+                k0, k1, fr, 0u, r0, num_edges, MATCH_BITS, nullptr, d_perm, perm_stride);
             PC_LAUNCH_CHECK("shuffle_group_kernel");
             continue;
         }
         if (lb1 == 0u) {
+            const uint32_t in_lds = shuf_match_bits(num_edges, rn);
             shuffle_group_kernel<8, true><<<dim3(1, rn), 512,
-                                            shuf_group_lds_bytes(8, num_edges), s>>>(
-                k0, k1, fr, 0u, r0, num_edges, nullptr, d_perm, perm_stride);
+                                            shuf_group_lds_bytes(8, num_edges, in_lds), s>>>(
+                k0, k1, fr, 0u, r0, num_edges, in_lds, nullptr, d_perm, perm_stride);
             PC_LAUNCH_CHECK("shuffle_group_kernel");
             continue;
         }
@@ -5612,8 +5668,9 @@ extern "C" int pc_permute_philox(uint64_t seed, uint64_t first_run,
             k0, k1, fr, num_edges, lb1, chunks, r0, rn, counts, d_perm, perm_stride);
         PC_LAUNCH_CHECK("shuffle_scatter_kernel");
         shuffle_group_kernel<4, false><<<dim3(nb1, rn), 256,
-                                         shuf_group_lds_bytes(4, SHUF_GROUP_CAP), s>>>(
-            k0, k1, fr, lb1, r0, SHUF_GROUP_CAP, starts, d_perm, perm_stride);
+                                         shuf_group_lds_bytes(4, SHUF_GROUP_CAP, MATCH_BITS),
+                                         s>>>(
+            k0, k1, fr, lb1, r0, SHUF_GROUP_CAP, MATCH_BITS, starts, d_perm, perm_stride);
         PC_LAUNCH_CHECK("shuffle_group_kernel");
     }
     return PC_OK;

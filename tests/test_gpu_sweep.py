@@ -736,3 +736,23 @@ def test_tiled_sweep_without_room(gpu, room):
     finally:
         gpu.cuda.set_per_process_memory_fraction(1.0)
     assert gpu.equal(records, want.records) and gpu.equal(span, want.span_step)
+
+
+@pytest.mark.parametrize('M,resident', [(8192, 4), (14620, 4), (16380, 4), (19404, 3), (21424, 3),
+                                        (23113, 2), (32736, 2), (32768, 2)])
+def test_shuffle_of_whole_runs_fills_the_gpu(gpu, M, resident):
+    """The masks that labels are matched in through LDS leave as many
+    workgroups on a CU as there are without them where that pays, the largest
+    runs among them, and the permutations are the oracle's with any number of
+    bits matched so (7, and in many runs of 14620 edges or more 6 or 5)."""
+    import ctypes
+    from pypercolate_amd import _native as nat
+    blocks = ctypes.c_int32(0)
+    nat.check(nat.load_library().pc_permute_philox_occupancy(M, ctypes.byref(blocks)), 'occupancy')
+    eng = BondEngine(_graph.GraphArrays(M + 1, np.stack(
+        [np.arange(M), np.arange(1, M + 1)], axis=1)))
+    want = oracle.bucket_permutations(78, 5, 3, M)
+    for runs in (3, 1100):
+        got = eng.device_permutations(seed=78, num_runs=runs, first_run=5)[:3].cpu().numpy()
+        np.testing.assert_array_equal(got, want)
+    assert blocks.value == resident
