@@ -4508,6 +4508,11 @@ __global__ __launch_bounds__(64) void contract_mfma_kernel(
 // (the X rows then came from beyond the L2, 4.7 TB/s of them) and 65 vector
 // instructions a block of 16 MFMAs instead of 12; the MFMAs alone take 1.55.
 // 128 p a tile took 1.97 ms, 128 columns 1.91, both 2.08.
+// Where the p are few and far apart, every block lies outside some row's
+// window, and the weights put in place one by one in each of them held up the
+// MFMAs: 16 p in 0.1, n = 32512, 64 columns 33.4 us, now (only in the blocks
+// where a lane's four are cut, 9 % of them, and by two rotations) 26.8; with
+// n = 130560 87 and 65.
 #define WIDE_TILE 64
 #define WIDE_KSTEP 16
 
@@ -4539,6 +4544,7 @@ __global__ __launch_bounds__(256) void contract_wide_f64_kernel(
     // four weights are read at a time, those of a shorter window apart
     const int32_t wlast = max(wlen - 4, 0);
     const double *wfour = wlen < 4 ? x : wrow;
+    const bool any_short = ballot(wlen > 0 && wlen < 4) != 0u;
     // union and intersection of the wave's windows
     int32_t any_lo = wlen > 0 ? wstart : INT32_MAX, any_hi = wlen > 0 ? wstart + wlen : 0;
     int32_t all_lo = wstart, all_hi = wstart + wlen;
@@ -4624,16 +4630,28 @@ __global__ __launch_bounds__(256) void contract_wide_f64_kernel(
             double av[4] = {a[0][0], a[0][1], a[1][0], a[1][1]};
             if (blk * KS < all_lo || blk * KS + KS > all_hi) {
                 const int32_t k = blk * KS + 4 * (int32_t)q - wstart;
-                const int32_t d = k - min(max(k, 0), wlast);
-                const double v0 = av[0], v1 = av[1], v2 = av[2], v3 = av[3];
+                const bool whole = k >= 0 && k + 4 <= wlen;
+                if (ballot(!whole && k > -4 && k < wlen)) {
+                    // some lane's four steps are partly in its window: the
+                    // weight of step e is at e + d, or (short) read by itself
+                    const int32_t d = k - min(max(k, 0), wlast);
+                    const double v[4] = {av[0], av[1], av[2], av[3]};
+                    double by1[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int32_t f = e + d;
-                    const bool in = (uint32_t)(k + e) < (uint32_t)wlen;
-                    const double v = f == 0 ? v0 : f == 1 ? v1 : f == 2 ? v2 : v3;
-                    av[e] = in ? v : 0.0;
-                    if (in && wlen < 4)
-                        av[e] = wrow[k + e];
+                    for (int e = 0; e < 4; ++e)
+                        by1[e] = d & 1 ? v[(e + 1) & 3] : v[e];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const bool in = (uint32_t)(k + e) < (uint32_t)wlen;
+                        av[e] = d & 2 ? by1[(e + 2) & 3] : by1[e];
+                        av[e] = in ? av[e] : 0.0;
+                        if (any_short && in)
+                            av[e] = wrow[k + e];
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        av[e] = whole ? av[e] : 0.0;
                 }
             }
 #pragma unroll
