@@ -3660,6 +3660,13 @@ __global__ __launch_bounds__(64) void chunk_prefix_kernel(
 // not 0.180; a sub-batch of L = 128 beside its sweeps 0.17, not 0.21.
 #define SUMS_BLOCKS 8192u
 #define SUMS_RUNS 32u
+// Few runs added to sums that are there take a wave each, as long as their
+// atomics cost less than the waves' way through LDS: up to SUMS_FEW chunks of
+// all runs, SUMS_FEW_ONE of one (16 runs of L = 16 12.6 us a call, so 11.7; 2
+// of L = 64 11.2 and 11.3, 8 of them 12.0 and 16.9; one of L = 128 12.6 and
+// 11.7, of L = 512 100 and 103).
+#define SUMS_FEW 192u
+#define SUMS_FEW_ONE 4096u
 #define SUMS_MOST 1024u   // runs a group may hold: what the bounds below allow
 
 // Product of two numbers below 2^24 (two full-rate instructions; __umul24
@@ -6189,9 +6196,10 @@ extern "C" int pc_microcanonical_sums(uint32_t num_nodes, uint32_t num_edges,
     // enough waves to fill 256 CUs several times over, and enough runs a
     // workgroup that its loop outweighs its 29 to 35 atomics a step
     const uint32_t per32 = (num_runs + SUMS_RUNS - 1u) / SUMS_RUNS;
-    const bool one_wave = (uint64_t)C * per32 >= SUMS_BLOCKS;
+    const bool few = accumulate && (uint64_t)num_runs * C <= (num_runs == 1u ? SUMS_FEW_ONE : SUMS_FEW);
+    const bool one_wave = few || (uint64_t)C * per32 >= SUMS_BLOCKS;
     uint32_t groups = C ? (SUMS_BLOCKS / (one_wave ? 1u : 4u) + C - 1u) / C : 1u;
-    groups = std::min(groups, one_wave ? per32 : (per32 + 1u) / 2u);
+    groups = std::min(groups, few ? num_runs : one_wave ? per32 : (per32 + 1u) / 2u);
     // the bounds of the sums in a group
     groups = std::max(groups, num_runs / SUMS_MOST + (num_runs % SUMS_MOST != 0u));
     const uint32_t rpg = groups ? (num_runs + groups - 1u) / groups : 0u;

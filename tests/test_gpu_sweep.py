@@ -756,3 +756,17 @@ def test_shuffle_of_whole_runs_fills_the_gpu(gpu, M, resident):
         got = eng.device_permutations(seed=78, num_runs=runs, first_run=5)[:3].cpu().numpy()
         np.testing.assert_array_equal(got, want)
     assert blocks.value == resident
+
+
+@pytest.mark.parametrize('length,sub', [(2, 1), (2, 150), (16, 24), (16, 25), (20, 1), (130, 1),
+                                        (130, 2), (300, 1), (514, 1)])
+def test_sums_of_few_runs_added(gpu, length, sub):
+    """Batches of few runs, a wavefront each, and of the next more, added one
+    after another: the sums of all runs at once."""
+    eng = BondEngine(_graph.square_lattice(length))
+    perm = eng.device_permutations(43, 3 * sub)
+    want = eng.microcanonical_sums(eng.sweep(perm))
+    sums = gpu.zeros_like(want[0]), gpu.zeros_like(want[1])
+    for r0 in range(0, 3 * sub, sub):
+        eng.microcanonical_sums(eng.sweep(perm[r0:r0 + sub]), *sums, accumulate=True)
+    assert gpu.equal(sums[0], want[0]) and gpu.equal(sums[1], want[1])
