@@ -786,9 +786,10 @@ class FusedPlan(object):
         self.P = ps.size
         self.ps = ps
         dev = self.x.device
-        if ps.ndim != 1 or not ((ps >= 0) & (ps <= 1)).all():
+        if ps.ndim != 1:
+            raise ValueError('p must be a number or a vector')
+        if not ((ps >= 0) & (ps <= 1)).all():
             binomial_windows(self.n, ps)        # raises for the first bad p
-            ps = ps.ravel()
         # a sorted grid needs no reordering of the rows
         self.unsort = None
         grid = ps

@@ -204,3 +204,13 @@ def test_fused_short_windows(gpu, n, at):
         k = np.arange(at, at + length)
         ref = ratio_weights(n, 0.5, k) @ x[k].astype(np.longdouble)
         assert (np.abs(got - ref) <= TOL['fp64_mfma'] * np.abs(ref)).all(), (length, got, ref)
+
+
+@pytest.mark.parametrize('shape', [(1, 1), (3, 1), (1, 3), (2, 2), (0, 3), (2, 1, 1)])
+def test_fused_takes_numbers_and_vectors_of_p(gpu, shape):
+    x = gpu.rand((481, 3), dtype=gpu.float64, device='cuda')
+    ps = np.full(shape, 0.5)
+    with pytest.raises(ValueError):
+        E.canonical_fused(x, ps)
+    assert E.canonical_fused(x, 0.5).shape == (1, 3)
+    assert E.canonical_fused(x, ps.ravel()).shape == (ps.size, 3)
