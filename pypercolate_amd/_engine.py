@@ -367,18 +367,26 @@ class BondEngine(object):
     def host_rows(self, res, dtype):
         """The runs as an (R, S) array of the reference's structured rows
         (hpc.microcanonical_statistics_dtype, with or without the spanning
-        field), laid out on the device and copied once."""
+        field), laid out on the device, as many runs at a time as fit 256 MB
+        or the room there is, and copied."""
         torch = self.torch
         R, dtype = res.num_runs, np.dtype(dtype)
-        rows = torch.empty((R * self.S * dtype.itemsize,), dtype=torch.uint8,
-                           device=self.device)
-        nat.check(self.lib.pc_expand_rows(
-            self.N, self.M, R, nat.ptr(res.perm), int(res.perm.stride(0)),
-            nat.ptr(res.records), max(self.M, 1), nat.ptr(res.span_step),
-            nat.ptr(res.chunk_state), 1 if 'has_spanning_cluster' in dtype.names else 0,
-            nat.ptr(rows), nat.stream_handle(torch)), 'pc_expand_rows')
+        one = self.S * dtype.itemsize
+        rows = self.scratch(min(R * one, max(1 << 28, one)), one)
+        if rows is None:
+            raise torch.OutOfMemoryError('no room for the {} bytes of a run'.format(one))
+        step = min(int(rows.numel()) // one, 65535)     # the grid's y extent
         out = np.empty((R * self.S,), dtype=dtype)
-        torch.from_numpy(out.view(np.uint8)).copy_(rows)
+        host = torch.from_numpy(out.view(np.uint8))
+        chunk_state = res.chunk_state
+        for r0 in range(0, R, step):
+            n = min(step, R - r0)
+            nat.check(self.lib.pc_expand_rows(
+                self.N, self.M, n, nat.ptr(res.perm[r0:]), int(res.perm.stride(0)),
+                nat.ptr(res.records[r0:]), max(self.M, 1), nat.ptr(res.span_step[r0:]),
+                nat.ptr(chunk_state[r0:]), 1 if 'has_spanning_cluster' in dtype.names else 0,
+                nat.ptr(rows), nat.stream_handle(torch)), 'pc_expand_rows')
+            host[r0 * one:(r0 + n) * one].copy_(rows[:n * one])
         return out.reshape(R, self.S)
 
 

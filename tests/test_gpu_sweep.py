@@ -770,3 +770,21 @@ def test_sums_of_few_runs_added(gpu, length, sub):
     for r0 in range(0, 3 * sub, sub):
         eng.microcanonical_sums(eng.sweep(perm[r0:r0 + sub]), *sums, accumulate=True)
     assert gpu.equal(sums[0], want[0]) and gpu.equal(sums[1], want[1])
+
+
+def test_structured_rows_without_room(gpu):
+    """Rows of more bytes than there is room for on the GPU, in pieces."""
+    from pypercolate_amd import hpc
+    eng = BondEngine(_graph.square_lattice(60))
+    res = eng.sweep(eng.device_permutations(47, 600))
+    dtype = hpc.microcanonical_statistics_dtype(True)
+    want = eng.host_rows(res, dtype)
+    assert want.nbytes > 200 << 20
+    gpu.cuda.empty_cache()
+    total = gpu.cuda.get_device_properties(0).total_memory
+    gpu.cuda.set_per_process_memory_fraction((gpu.cuda.memory_reserved() + (40 << 20)) / total)
+    try:
+        got = eng.host_rows(res, dtype)
+    finally:
+        gpu.cuda.set_per_process_memory_fraction(1.0)
+    assert got.tobytes() == want.tobytes()
