@@ -201,12 +201,17 @@ struct Words128 {
 SCAN_DEFINE(scan_state, SCAN_STEPS)
 SCAN_DEFINE(scan_state_rows, SCAN_ROWS)
 
+// The lanes of the mask below this one.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
 // Lanes up to and including this one with the flag set.
 __device__ __forceinline__ uint32_t scan_count(bool flag)
 {
-    const uint64_t m = __ballot(flag);
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)) + (flag ? 1u : 0u);
+    return lanes_below(__ballot(flag)) + (flag ? 1u : 0u);
 }
 
 __device__ __forceinline__ uint64_t umax64(uint64_t a, uint64_t b) { return a > b ? a : b; }
@@ -398,12 +403,6 @@ __device__ __forceinline__ uint64_t match_label_lds(uint32_t label, uint32_t bit
         __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     return bits > in_lds ? match_label(label >> in_lds, bits - in_lds, peers) : peers;
-}
-
-__device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    return (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
 }
 
 // Lemire's rejection threshold (2^w - r) mod r for w = 16 and w = 32, called
@@ -1134,13 +1133,6 @@ __device__ __forceinline__ void mt_init(uint32_t seed, uint32_t *mt)
     }
 }
 
-// The lanes of the mask below this one.
-__device__ __forceinline__ uint32_t lanes_before(uint64_t mask)
-{
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
 // Phase one.  The wave tempers 64 state words at a time (lane l holds word
 // base + l) and settles the whole block at once: for steps i, i-1, ... under
 // one mask m (the smallest all-ones mask >= i), the word of lane l serves
@@ -1169,11 +1161,11 @@ __device__ __forceinline__ uint32_t mt_settle(const uint32_t *mt, uint32_t i, in
             uint64_t acc = ballot(valid && x + 63u <= i);
             uint64_t may = ballot(valid && x <= i);
             while (acc != may) {
-                const uint32_t most = lanes_before(may), least = lanes_before(acc);
+                const uint32_t most = lanes_below(may), least = lanes_below(acc);
                 acc = ballot(valid && x + most <= i);
                 may = ballot(valid && x + least <= i);
             }
-            const uint32_t below = lanes_before(acc);
+            const uint32_t below = lanes_below(acc);
             const bool mine = (acc >> lane) & 1ull;
             const uint32_t cnt = (uint32_t)__popcll(acc);
             uint32_t used;
