@@ -635,7 +635,8 @@ def main(argv=None):
                             'launch; every step draws the next step\'s once '
                             'its sweeps have ended, beside its last '
                             'reductions), sub-batches of {} runs (one '
-                            'residency), sweeps alternating between two '
+                            'residency of the untiled sweep), sweeps '
+                            'alternating between two '
                             'streams, reductions beside them on a third').format(
                                 'one wavefront per run and lattice tile' if tiled
                                 else 'one run per workgroup', pipe.sub),

@@ -423,9 +423,11 @@ def _pipeline_streams(torch, device):
 class Pipeline(object):
     """R runs of one graph through permute -> sweep -> chunk states -> exact
     sums, in sub-batches on four streams so that the reduction of one
-    sub-batch runs beside the sweep of the next (the sweep leaves most issue
-    slots of a CU idle: its occupancy is bounded by LDS, four runs per CU at
-    N = 16384).  Stream order: permutations on the caller's stream, sweeps
+    sub-batch runs beside the sweep of the next: an untiled sweep leaves most
+    issue slots of a CU idle (its occupancy is bounded by LDS, four runs per
+    CU at N = 16384), a tiled one about half.  A sub-batch is by default what
+    the GPU holds of the untiled sweep at once; a pipeline of one sub-batch
+    runs on the caller's stream alone, unless it draws ahead.  Stream order: permutations on the caller's stream, sweeps
     alternating between two more (each waiting for its permutations; the
     next sub-batch's runs fill the CUs that the last runs of a launch leave
     idle), chunk states and sums on a fourth (each waiting for its sweep,
@@ -433,7 +435,8 @@ class Pipeline(object):
     per hardware queue of the process (HIP's default of four): streams that
     shared a queue would serialise.  HBM-state graphs get their chunk
     states from the sweep itself (BondEngine.fuse_chunk_states).  All
-    buffers are allocated up front.
+    buffers are allocated up front (without room for even one run's, the
+    RandomState workspace is asked for again in every run()).
 
     Permutations: Philox-keyed (pc_permute_philox, seed) by default, or
     with seeds= (R integers) numpy RandomState(seeds[r]).permutation(M),
@@ -466,11 +469,13 @@ class Pipeline(object):
         dev = eng.device
         M, S = eng.M, eng.S
         if sub_batch is None:
-            # one residency (runs the GPU holds at once): with the sweeps on
-            # two streams, 9.3 ms per step of 10^4 runs at L = 128 against
-            # 9.4 with 1.5 residencies, 9.5 with two and 10.6 with three
-            # (an earlier, slower sweep; smaller first or last sub-batches
-            # measured slower with the current one too)
+            # one residency of the untiled sweep (runs the GPU holds at
+            # once): with the sweeps on two streams, 9.3 ms per step of 10^4
+            # runs at L = 128 against 9.4 with 1.5 residencies, 9.5 with two
+            # and 10.6 with three (an earlier sweep, untiled; smaller first or
+            # last sub-batches measured slower too).  Tiled sweeps take the
+            # same time within 3 % with 1024 to 10^4 runs a sub-batch (L =
+            # 100, 128, 181)
             cus = torch.cuda.get_device_properties(dev).multi_processor_count
             sub_batch = max(eng.occupancy(), 1) * cus
         self.sub = max(1, min(int(sub_batch), self.R))

@@ -2691,8 +2691,8 @@ __global__ __launch_bounds__(128) void sweep_multi_kernel(
 // 1000 runs 158 and 60 ms (lists 16, tiles 19, events 20, chunk states 4);
 // L = 256, 200 runs 3.67 and 1.1; L = 181, 600 runs 2.65 and 1.1; L = 128,
 // 10^4 runs (no chunk states) 7.06 and 5.05.  The tiles are bound by vector
-// issue (60 % of a wavefront's share of its SIMD at L = 256) and dependent
-// LDS round trips, and at L = 1024 by the records, which go out in
+// issue (the vector ALUs are 48 % busy at L = 128, 43 % at L = 256) and
+// dependent LDS round trips, and at L = 1024 by the records, which go out in
 // part-written lines: rows cleared in step order by tile_scatter, so that a
 // tile writes merges only, took them from 35 to 27 ms, a claim table of 512
 // slots instead of 1024 (15 wavefronts per CU, not 13) to 23.  Codes that
@@ -4965,7 +4965,8 @@ __global__ __launch_bounds__(64, 3) void canonical_fused_f64_kernel(
             const bool fresh = j0 > 0 && j0 % FUSED_REANCHOR == 0;
             // where no row's window starts or ends in the chunk, a step is the
             // two products alone: rows before their window, past it, or past P
-            // hold weight 0
+            // hold weight 0 (past a window that their range of steps cuts
+            // short, they meet columns of 0)
             const int j = (int)j0;
             double direct = 0.0;
             const bool anew = fresh && j > ja && j < je;
@@ -5840,10 +5841,13 @@ static LatticeEdges lattice_edges(uint32_t length, bool tiled)
 // Lattices it takes, and their tiles; false otherwise.
 // - A side of at most TILE_MAX_LENGTH, and more than a tile's.
 // - Below TILE_LDS_LENGTH (a state that fits LDS several times a CU), batches
-//   of at most four runs per CU only: the sweep in milliseconds, untiled and
-//   tiled, is 0.784 and 0.842 for 4000 runs of L = 80, 0.296 and 0.252 for
-//   200; 2.68 and 2.36 for 8000 of L = 100, 7.06 and 5.05 for 10^4 of L = 128,
-//   0.66 and 0.47 for 200 of those.
+//   of at most four runs per CU only.  The sweep in microseconds, untiled and
+//   tiled: one run of L = 65 184 and 142, of L = 80 280 and 183, of L = 95 364
+//   and 219; 1024 runs 227 and 224, 318 and 292, 422 and 368; 2000 runs 252 and
+//   341, 353 and 491, 847 and 657; 8000 runs 896 and 1111, 1432 and 1580, 2426
+//   and 2148.  (From L = 88 on the tiles win at 2000 runs and more too, but not
+//   at 1500 of L = 95: 473 and 489.)  From TILE_LDS_LENGTH on 2680 and 2360 for
+//   8000 of L = 100, 7060 and 5050 for 10^4 of L = 128, 660 and 470 for 200.
 // - Tiles of at most 64 x 64 nodes, or 32 x 32 up to L = 128 where those would
 //   leave the GPU with at most 2048 wavefronts: more tiles make more events.
 //   Sweep in milliseconds with 64 and 32, 200 runs of L = 128 0.479 and 0.412,
