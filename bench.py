@@ -605,7 +605,8 @@ def main(argv=None):
     adds = float(R) * M
     traffic_per_add = profiled_traffic_per_add(args.length, R)
     value = adds / (ms_per_step / 1e3)
-    tiled = eng.tiled_runs(pipe.sub) > 0
+    tiled = eng.tiled_runs(pipe.sub, sum(int(w.numel()) for w in pipe.workspaces[:1]
+                                         if w is not None)) > 0
     alg_bytes = ALG_BYTES_PER_ADD_LDS if N <= 16384 else ALG_BYTES_PER_ADD_HBM
     # algorithmic bytes of the step's sweep launches over their span: the
     # launches overlap on two streams, so one launch's own duration also

@@ -4275,15 +4275,15 @@ __global__ __launch_bounds__(256) void binom_normalize_kernel(
 
 template <int C>
 __global__ __launch_bounds__(256) void contract_f64_kernel(
-    const double *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ start,
-    const int64_t *__restrict__ len, const double *__restrict__ w, int64_t kmax,
-    double *__restrict__ out, int32_t cols)
+    const double *__restrict__ x, int64_t S, int64_t x_stride,
+    const int64_t *__restrict__ start, const int64_t *__restrict__ len,
+    const double *__restrict__ w, int64_t kmax, double *__restrict__ out, int32_t cols)
 {
     __shared__ double part[256 / 64][C];
     const uint32_t pi = blockIdx.x;
     const double *wr = w + (int64_t)pi * kmax;
     const double *xr = x + start[pi] * x_stride;
-    const int64_t L = len[pi];
+    const int64_t L = min(len[pi], S - start[pi]);   // no rows past the last
     double acc[C];
 #pragma unroll
     for (int c = 0; c < C; ++c)
@@ -6485,13 +6485,13 @@ extern "C" int pc_canonical_contract(uint32_t num_steps, uint32_t cols,
         const double *x = (const double *)d_x, *w = (const double *)d_w;
         if (cols <= 8)
             contract_f64_kernel<8><<<num_p, 256, 0, s>>>(
-                x, x_stride, d_start, d_len, w, kmax, d_out, (int32_t)cols);
+                x, num_steps, x_stride, d_start, d_len, w, kmax, d_out, (int32_t)cols);
         else if (cols <= 16)
             contract_f64_kernel<16><<<num_p, 256, 0, s>>>(
-                x, x_stride, d_start, d_len, w, kmax, d_out, (int32_t)cols);
+                x, num_steps, x_stride, d_start, d_len, w, kmax, d_out, (int32_t)cols);
         else
             contract_f64_kernel<32><<<num_p, 256, 0, s>>>(
-                x, x_stride, d_start, d_len, w, kmax, d_out, (int32_t)cols);
+                x, num_steps, x_stride, d_start, d_len, w, kmax, d_out, (int32_t)cols);
         PC_LAUNCH_CHECK("contract_f64_kernel");
         return PC_OK;
     }

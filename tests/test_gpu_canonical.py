@@ -133,3 +133,25 @@ def test_contract_wide_windows(gpu, S, lens, C):
     y[hi + 1:] = np.nan
     z = E.contract(gpu.from_numpy(y).cuda(), wt, 'fp64_mfma').cpu().numpy()
     np.testing.assert_array_equal(z, q)
+
+
+@pytest.mark.parametrize('precision', sorted(TOL))
+@pytest.mark.parametrize('C', [7, 14, 30, 70])
+def test_contract_windows_past_the_last_step(gpu, precision, C):
+    """The C entry leaves out weights of steps past the last one, which meet no
+    row of X, in every form (the rows behind X hold NaN here)."""
+    if precision == 'fp64' and C > 32:
+        return
+    rng = np.random.RandomState(C)
+    S, lens, start = 300, np.array([40, 300, 290, 7]), np.array([270, 0, 20, 299])
+    kmax = 330
+    w = rng.rand(4, kmax)
+    buf = np.full((S + 40, C), np.nan)
+    buf[:S] = rng.rand(S, C)
+    wt = E.Weights(S - 1, np.zeros(4), gpu.from_numpy(start).cuda(),
+                   gpu.from_numpy(lens).cuda(), kmax, gpu.from_numpy(w).cuda())
+    wt.host_start, wt.host_length = start, np.minimum(lens, S - start)
+    got = E.contract(gpu.from_numpy(buf).cuda()[:S], wt, precision).cpu().numpy()
+    for i, (a, n) in enumerate(zip(start, np.minimum(lens, S - start))):
+        ref = w[i, :n] @ buf[a:a + n]
+        assert (np.abs(got[i] - ref) <= TOL[precision] * ref).all(), i
